@@ -29,11 +29,11 @@
 // partial sums are kept per tile and reduced in tile order, so a scene gives
 // bit-identical results alone and in any batch.  State and partials are
 // double-buffered by pass parity, so no decision races with its
-// publication.  Kernel boundaries are the grid-wide barriers: on MI355X a
-// kernel boundary inside a graph costs ~1.6 us, less than a grid barrier of
-// a persistent cooperative kernel (3.7 us at 128 workgroups, ~12 us at 512).
-// The host launches the graph of a chunk of passes, reads the scenes'
-// states, and repeats; scenes that have converged skip their tiles.
+// publication.  Kernel boundaries are the grid-wide barriers, in chunks of
+// passes captured as a graph: the host launches a chunk, reads the scenes'
+// states, and repeats; scenes that have converged skip their tiles.  A single
+// scene that fits the chip runs its passes resident instead, in one kernel
+// with barriers of its own (dv_apgd_resident.h).
 //
 // The same arithmetic as the reference, less traffic:
 //   * N y is not recomputed: with y_{k+1} = (1+beta) g_{k+1} - beta g_k,
@@ -160,6 +160,7 @@ struct Args {
   const int* cB;
   const int* iStart;
   const int* cStart;    // contacts of body b as body A: [cStart[b], cStart[b+1]) (rows sorted by idA)
+  const int* inc;       // resident passes: per body, its contacts << 1 | side, those as body B first
   const int* posB;      // slot of contact c in the B-side order, JB[posB[c]] = J[c]
   const int* bilIncStart;
   const int* bilInc;
@@ -179,12 +180,14 @@ struct Args {
   V4<TM>* JB;           // the same, in B-side order: body b's B incidences are
                         // [iStart[b] - cStart[b], iStart[b+1] - cStart[b+1])
   V4<TM>* tmp;
+  V4<TM>* tmpSplit;     // FP64 resident passes: tmp as they exchange it
   V4<TM>* sr;           // mixed solver: D^T of each ring slot's iterate, per body (slot k at k * nb)
   double* gHat;         // gammaHat before any iterate is accepted (ones)
   double* part1[2];     // kSlots per tile, by pass parity
   double* part3[2];     // setup and final kernels: a second kSlots per tile
   double* lq[2];        // P2's Lipschitz partials, by pass parity: one per body tile, then one
                         // per heavy body (in the heavy list's order)
+  double* lqw[2];       // resident passes: the Lipschitz sums per 64 bodies, by pass parity
   double* p1sum[2];     // single slot: P1's slots totalled by P2's last workgroup
   int nBodyTiles;       // body tiles of the scene (kTB bodies each)
 };
@@ -920,8 +923,20 @@ __global__ __launch_bounds__(kTD) void kSetupDecide(const Args<TM>* __restrict__
 // the decision of a pass: Lipschitz test, backtracking or acceptance
 // (APGD.cu:236-332), from the pass's fixed-order partial sums tot[0..15]
 
-template <bool kMixed>
-__device__ void decideStep(ApgdState& S, const double* tot, const SolveDims& D) {
+// The step sizes after either outcome, computed where they are used.
+struct LazyNext {
+  double L, theta;
+  __device__ explicit LazyNext(const ApgdState& S) : L(S.L), theta(S.theta) {}
+  __device__ double backL() const { return 2.0 * L; }
+  __device__ double backT(double Lb) const { return 1.0 / Lb; }
+  __device__ double nextL() const { return 0.9 * L; }
+  __device__ double nextT(double La) const { return 1.0 / La; }
+  __device__ double nextTheta() const { return (-(theta * theta) + theta * sqrt(theta * theta + 4.0)) / 2.0; }
+  __device__ double nextBeta(double thetaNew) const { return theta * (1.0 - theta) / (theta * theta + thetaNew); }
+};
+
+template <bool kMixed, class Next>
+__device__ void decideStep(ApgdState& S, const double* tot, const SolveDims& D, const Next& next) {
   const double* s1 = tot;           // P1 slots
   const double* s3 = tot + kSlots;  // slot 6: P2's Lipschitz term
   S.passes++;
@@ -967,22 +982,21 @@ __device__ void decideStep(ApgdState& S, const double* tot, const SolveDims& D) 
   if (backtrack && S.bt < kBacktrackCap) {
     S.bt++;
     S.backtracks++;
-    S.L = 2.0 * L;
-    S.t = 1.0 / S.L;
+    S.L = next.backL();
+    S.t = next.backT(S.L);
     S.fresh = 0;  // this pass's P1 has formed and stored N of slot cur
     return;
   }
-  const double theta = S.theta;
-  double thetaNew = (-(theta * theta) + theta * sqrt(theta * theta + 4.0)) / 2.0;
-  S.beta = theta * (1.0 - theta) / (theta * theta + thetaNew);
+  double thetaNew = next.nextTheta();
+  S.beta = next.nextBeta(thetaNew);
   if (s1[5] > 0) {
     S.restart = 1;
     thetaNew = 1.0;
   } else {
     S.restart = 0;
   }
-  S.L = 0.9 * L;
-  S.t = 1.0 / S.L;
+  S.L = next.nextL();
+  S.t = next.nextT(S.L);
   S.theta = thetaNew;
   S.prev = S.cur;
   S.cur = S.nxt;
@@ -993,6 +1007,10 @@ __device__ void decideStep(ApgdState& S, const double* tot, const SolveDims& D) 
   S.bt = 0;
   S.pendingRes = 1;
   S.fresh = 1;  // gamma_new's N is formed by the next P1, from the tmp of this pass's P2
+}
+template <bool kMixed>
+__device__ void decideStep(ApgdState& S, const double* tot, const SolveDims& D) {
+  decideStep<kMixed>(S, tot, D, LazyNext(S));
 }
 
 // ---------------------------------------------------------------------------
@@ -1453,6 +1471,8 @@ __global__ __launch_bounds__(1024) void kHeavyTable(const Args<TM>* __restrict__
   if (threadIdx.x == 0) counts[2] = base;
 }
 
+#include "dv_apgd_resident.h"
+
 // ---------------------------------------------------------------------------
 // host side
 
@@ -1572,6 +1592,7 @@ constexpr int kManySlotsN = (int)(sizeof(kManySlots) / sizeof(kManySlots[0]));
 struct TuneClass {
   std::vector<double> score;  // per candidate: us per pass per million active rows (< 0: not measured)
   int best = -1;              // the chosen candidate (-1: still measuring)
+  int solves = 0;             // finished while measuring
   Schedule sched;             // its schedule (also when read from the file)
 };
 
@@ -1657,6 +1678,7 @@ TuneClass* chooseSchedule(Engine& E, long rows, bool allowTuning) {
     return nullptr;
   }
   if (!tuningEnabled()) return nullptr;  // the first candidate, whatever the schedule file holds
+  if (single && rows <= kTC) return nullptr;  // one tile has no order to choose
   Tuner& T = tuner();
   std::lock_guard<std::mutex> lock(T.m);
   int bucket = 0;
@@ -1702,6 +1724,17 @@ bool recordCandidate(Engine& E, TuneClass& c, int i, double score) {
   E.sched = c.sched;
   persist(E.tuneKey.substr(0, E.tuneKey.find(':')), E.tuneKey, c.sched, c.score[best]);
   return true;
+}
+
+// Solves of a few passes end before a candidate's chunk counts; after
+// kMeasuredSolves of them the class takes the first candidate for this
+// process (nothing is written to the file).
+constexpr int kMeasuredSolves = 8;
+void endMeasuredSolve(Engine& E, TuneClass& c) {
+  std::lock_guard<std::mutex> lock(tuner().m);
+  if (c.best >= 0 || ++c.solves < kMeasuredSolves) return;
+  c.best = 0;
+  c.sched = (E.nSlots == 1 ? kOneSlot : kManySlots)[0];
 }
 
 const Schedule& candidate(const Engine& E, int i) { return (E.nSlots == 1 ? kOneSlot : kManySlots)[i]; }
@@ -1754,6 +1787,7 @@ void Engine::release() {
   out.release();
   states.release();
   views.release();
+  teamSync.release();
   if (outHost) (void)hipHostFree(outHost);
   outHost = nullptr;
   for (hipEvent_t& e : polled) {
@@ -1786,13 +1820,14 @@ void prepareScene(Scene& s, Args<TM>& a) {
   const long bodyTiles = std::max<long>(1, ((long)s.nb + kTB - 1) / kTB);
   // a body reduced by a workgroup has more than kHeavyDegree of the 2 nc incidences
   const long lqCap = bodyTiles + 2L * std::max(s.ncCap, 1) / kHeavyDegree + 2;
-  s.partials.reserve((size_t)4 * kSlots * tilesCap + 2 * kSlots + 2 * lqCap);
+  const long lqwCap = bodyTiles * (kTB / 64);
+  s.partials.reserve((size_t)4 * kSlots * tilesCap + 2 * kSlots + 2 * lqCap + 2 * lqwCap);
   s.work.reserve((size_t)5 * RsCap + 16);  // ring[4], gHat: FP64 in both solvers
   // TM block: rn[4], r, then J and JB (per contact), tmp and (mixed) the
   // four ring slots of D^T gamma (per body) of 4 components 32-byte aligned,
   // then (mixed) M^-1
   const size_t nbc = (size_t)std::max(s.nb, 1);
-  const size_t tmElems = (size_t)5 * RsCap + 8 + 4 * (2 * (size_t)std::max(s.ncCap, 1) + nbc + (kMixed ? 4 * nbc : 0)) +
+  const size_t tmElems = (size_t)5 * RsCap + 8 + 4 * (2 * (size_t)std::max(s.ncCap, 1) + nbc + (kMixed ? 4 : 1) * nbc) +
                          (kMixed ? nbc + 1 : 0) + 16;
   TM* WM;
   if (kMixed) {
@@ -1816,6 +1851,7 @@ void prepareScene(Scene& s, Args<TM>& a) {
   a.frame64 = s.frame.p;
   a.cap = s.ncCap;
   a.cA = s.cA.p; a.cB = s.cB.p; a.iStart = s.iStart.p; a.cStart = s.cStart.p; a.posB = s.posB.p;
+  a.inc = s.inc.p;
   a.bilIncStart = s.bilIncStart.p; a.bilInc = s.bilInc.p; a.bilA = s.bilA.p; a.bilB = s.bilB.p;
   a.heavy = s.heavy.p; a.counters = s.counters.p;
   a.minv64 = s.minv.p;
@@ -1837,6 +1873,7 @@ void prepareScene(Scene& s, Args<TM>& a) {
     a.frame = reinterpret_cast<TM*>(s.frame32.p);
     a.minv = reinterpret_cast<TM*>(a.sr + 4 * nbc);
   } else {
+    a.tmpSplit = a.tmp + nbc;
     a.frame = reinterpret_cast<TM*>(s.frame.p);
     a.minv = reinterpret_cast<TM*>(s.minv.p);
   }
@@ -1845,6 +1882,7 @@ void prepareScene(Scene& s, Args<TM>& a) {
     a.part3[k] = s.partials.p + (long)(2 * k + 1) * kSlots * tilesCap;
     a.p1sum[k] = s.partials.p + 4L * kSlots * tilesCap + k * kSlots;
     a.lq[k] = s.partials.p + 4L * kSlots * tilesCap + 2 * kSlots + k * lqCap;
+    a.lqw[k] = s.partials.p + 4L * kSlots * tilesCap + 2 * kSlots + 2 * lqCap + k * lqwCap;
   }
 }
 
@@ -2125,6 +2163,37 @@ bool engineBusy(const Engine& E) {
 
 namespace {
 
+// The resident passes of the engine's only slot (dv_apgd_resident.h), taken
+// when its team fits the chip: one workgroup to a CU, all running at once,
+// each with one row tile or, past one tile per CU, two.
+constexpr int kTeamPasses = 2048;  // of one launch
+constexpr int kTeamSkip = 16;      // solves that stay on launches after a team could not be placed
+inline int teamRows(const Engine& E, int tiles) { return tiles > std::min(kTeamMax, E.numCU) ? 2 : 1; }
+template <typename TM>
+bool teamFits(Engine& E, int slot) {
+  const Args<TM>& a = slotArgs<TM>(E, slot);
+  const int R = teamRows(E, a.nTiles), members = (a.nTiles + R - 1) / R;
+  return members <= std::min(kTeamMax, E.numCU) && a.nBodyTiles <= 64L * members;  // (32 rounds of body units)
+}
+template <typename TM>
+void launchTeam(Engine& E, hipStream_t st) {
+  const size_t need = (size_t)kTeamSync * E.nSlots;
+  if (E.teamSync.cap < need) {
+    E.teamSync.reserve(need);
+    DV_HIP(hipMemsetAsync(E.teamSync.p, 0, sizeof(u64) * E.teamSync.cap, st));
+  }
+  const Tables T = tablesOf<TM>(E, E.active);
+  const Args<TM>& a = slotArgs<TM>(E, 0);
+  const int R = teamRows(E, a.nTiles);
+  const auto kernel = a.dims.nbil ? (R == 1 ? kTeam<TM, true, 1> : kTeam<TM, true, 2>)
+                                  : (R == 1 ? kTeam<TM, false, 1> : kTeam<TM, false, 2>);
+  hipLaunchKernelGGL(kernel, dim3((a.nTiles + R - 1) / R), dim3(kTC), 0, st,
+                     reinterpret_cast<const Args<TM>*>(E.table.p), T, (const TeamItem*)nullptr, E.teamSync.p,
+                     E.teamEpoch + 1, ++E.teamLaunch, kTeamPasses);
+  DV_HIP(hipGetLastError());
+  E.teamEpoch += 2 * kTeamPasses + 2;
+}
+
 // Admit all, run chunks until every scene is done, retire all.  With
 // profiling (single scene), one chunk per solve is launched on the stream
 // with events around the chosen kernel: the first chunk after the first
@@ -2161,6 +2230,11 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
   for (Scene* s : scenes) maxIt = std::max(maxIt, s->maxIt);
   const long passCap = (long)maxIt * 64 + 4096;
   int passesBefore = 0;
+  // one slot whose schedule is decided runs resident, until a launch makes no
+  // progress (its team could not be placed)
+  const bool mayReside = n == 1 && !tc && !E.noGraph && !E.forcedRpt && teamFits<TM>(E, 0) && E.teamSkip == 0;
+  if (E.teamSkip > 0) --E.teamSkip;
+  bool resident = mayReside && !ev;  // (profiling: once the sample is taken)
   ApgdState* outH = reinterpret_cast<ApgdState*>(E.outHost);
   ApgdState* buf[2] = {outH, outH + E.nSlots};
   for (int b = 0; b < 2; ++b)
@@ -2176,7 +2250,8 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
       DV_HIP(hipEventRecord(E.tev[b][0], st));
     }
     E.chunkCand[b] = ci;
-    runChunk<TM>(E, st, timed ? ev : nullptr, prof);
+    if (resident) launchTeam<TM>(E, st);
+    else runChunk<TM>(E, st, timed ? ev : nullptr, prof);
     if (ci >= 0) DV_HIP(hipEventRecord(E.tev[b][1], st));
     DV_HIP(hipMemcpyAsync(buf[b], E.out.p, sizeof(ApgdState) * E.nSlots, hipMemcpyDeviceToHost, st));
     DV_HIP(hipEventRecord(E.polled[b], st));
@@ -2196,7 +2271,7 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
     // does not wait for the host between chunks (after the solve ends, the
     // queued chunk's passes exit at once).  While the profiling sample is
     // still to be taken, the next chunk's entry state must be known first.
-    const bool ahead = !(ev && !sampled);
+    const bool ahead = !resident && !(ev && !sampled);
     if (ahead) launch(cur ^ 1, false);
     DV_HIP(hipEventSynchronize(E.polled[cur]));
     const ApgdState* last = buf[cur];
@@ -2205,6 +2280,13 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
       DV_HIP(hipEventElapsedTime(&ms, ev[0], ev[1]));
       profStats->prof_kernel_ms += ms;
       profStats->prof_kernel_count += prof == 4 ? 1 : kProfBurst;
+    }
+    if (resident) {
+      E.launched = last[0].passes;
+      if (last[0].passes == passesBefore) {
+        resident = false;
+        E.teamSkip = kTeamSkip;
+      }
     }
     passesBefore = last[0].passes;
     int doneNow = 0;
@@ -2221,7 +2303,10 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
     }
     doneBefore = doneNow;
     activeRows = rowsLeft;
-    if (doneNow == n) break;
+    if (doneNow == n) {
+      if (tc) endMeasuredSolve(E, *tc);
+      break;
+    }
     // Once a quarter of the slots have finished since the last retirement,
     // retire them while the others iterate: the pass kernels then loop over
     // the active slots' tiles only, instead of reading the view of every
@@ -2247,6 +2332,7 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
       sampled = sampled || timed;
       launch(cur, timed);
       curTimed = timed;
+      if (timed) resident = mayReside;
     }
   }
   std::vector<int> slots;

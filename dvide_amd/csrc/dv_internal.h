@@ -149,6 +149,9 @@ struct Engine {
   DevBuf<char> out;     // ApgdState[nSlots]
   DevBuf<char> states;  // ApgdState[nSlots][2], by pass parity
   DevBuf<char> views;   // PassView[nSlots][2]: what the pass kernels read of the states
+  DevBuf<unsigned long long> teamSync;  // flags of the resident passes' teams, per slot
+  unsigned long long teamEpoch = 0, teamLaunch = 0;
+  int teamSkip = 0;     // solves to run as launches (a team could not be placed)
   void* outHost = nullptr;  // pinned copies of out: two halves, by chunk parity
   hipEvent_t polled[2] = {nullptr, nullptr};  // after each half's copy
   int outHostCap = 0;

@@ -82,8 +82,8 @@ typedef struct dv_scene dv_scene;
                                  P1: its second) that kernel runs as a captured graph of
                                  16 back-to-back launches between two events (the decide
                                  kernel once, alone, where it runs: after the chunk's
-                                 last pass for one scene); the rest run in the captured
-                                 chunk graph */
+                                 last pass for one scene); the rest run as without
+                                 profiling */
 #define DV_PARAM_ROWS_PER_THREAD 15 /* contact kernels of the graph-driven solvers: 0 the
                                        tuned choice (default), 1 or 2 contacts per thread
                                        (results agree to rounding, each choice is

@@ -1,0 +1,70 @@
+"""The resident passes against the passes as launches.
+
+A slot whose team fits the chip keeps its contacts' state in registers for
+thousands of passes; fixed rows per thread (DV_PARAM_ROWS_PER_THREAD) keep a
+scene on the launches.  Both add in the same order, so every result is equal
+bit for bit: around the edges of a row tile (512 rows), past one tile per CU
+(two rows per thread), and with the rows and bodies that take paths of their
+own (bilateral rows, a movable body with thousands of contacts, body units
+without a movable body)."""
+import copy
+
+import numpy as np
+import pytest
+
+from dvide_amd import scenes, system
+
+pytestmark = pytest.mark.gpu
+
+
+def bits_equal(x, y):
+    x = np.asarray(x, np.float64)
+    y = np.asarray(y, np.float64)
+    return x.shape == y.shape and np.array_equal(x.view(np.uint64), y.view(np.uint64))
+
+
+def layer_of(n):
+    """n spheres on a floor, one contact each."""
+    sc = scenes.layer(7, per_side=int(np.ceil(np.sqrt(n))))
+    for k in ("pos", "vel", "mass", "geom", "fixed", "family"):
+        setattr(sc, k, getattr(sc, k)[:n + 1].copy())
+    return sc
+
+
+def landed_shell():
+    sc = scenes.shell_bed(3, nx=8, ny=16, layers=1)
+    sc.pos[:, 1] -= 1e-4
+    return sc
+
+
+SCENES = {
+    "ball": scenes.ball_on_box,
+    **{f"layer_{n}": (lambda n=n: layer_of(n)) for n in (63, 511, 512, 513, 1025)},
+    "pile_6000": lambda: scenes.pile(31, 6000),
+    "free_lid": lambda: scenes.compaction(5, n=3000, width=1.5, lid=scenes.LID_FREE),
+    "bilateral_lid": lambda: scenes.compaction(5, n=1200, width=1.2, lid=scenes.LID_BILATERAL),
+    "shell": landed_shell,
+    "box_58000": lambda: scenes.compaction(2002, n=58000, width=4.0, lid=scenes.LID_NONE),
+}
+
+
+@pytest.mark.parametrize("build", [system.BUILD_FP64, system.BUILD_MIXED])
+@pytest.mark.parametrize("name", SCENES)
+def test_resident_passes_equal_the_launches(gpu, monkeypatch, name, build):
+    monkeypatch.setenv("DVIDE_TUNE", "0")  # no solve is spent on measuring schedules
+    sc = SCENES[name]()
+    out = []
+    for rows in (1, 0):
+        g = system.from_scene(copy.deepcopy(sc), build, tol=1e-7, max_iterations=150)
+        g.setRowsPerThread(rows)
+        steps = []
+        for _ in range(2):
+            g.step()
+            st = g.stats()
+            steps.append((st.num_contacts, st.iterations, st.passes, st.backtracks, st.residual, st.objective))
+        out.append((steps, g.gamma, g.v, g.p))
+        g.close()
+    assert out[0][0] == out[1][0]
+    assert out[0][0][0][0] > 0
+    for a, b in zip(out[0][1:], out[1][1:]):
+        assert bits_equal(a, b)
