@@ -301,12 +301,12 @@ int dv_scene_destroy(dv_scene* h) {
                                  &s.b, &s.gamma, &s.work, &s.partials, &s.shellNodes, &s.ptS, &s.shellF};
   for (auto* b : dbufs) b->release();
   dv::DevBuf<int>* ibufs[] = {&s.family, &s.smallIds, &s.bigIds, &s.bilA, &s.bilB, &s.bilIncStart,
-                              &s.bilInc, &s.cellItems, &s.cntUp, &s.cntDown, &s.cStart, &s.iStart,
-                              &s.scanTmp, &s.counters, &s.hostTotals, &s.cA, &s.cB, &s.inc, &s.posB,
-                              &s.heavy, &s.heavyPos, &s.bigChunks, &s.shellConn, &s.ptEl, &s.nodeIncStart,
+                              &s.bilInc, &s.cellMeta, &s.lists, &s.csr, &s.cntUp, &s.cntDown, &s.cStart, &s.iStart,
+                              &s.scanTmp, &s.counters, &s.cA, &s.cB, &s.inc, &s.posB,
+                              &s.heavy, &s.bigChunks, &s.shellConn, &s.ptEl, &s.nodeIncStart,
                               &s.nodeInc};
   for (auto* b : ibufs) b->release();
-  s.slotOf.release(); s.slotCount.release(); s.slotStart.release(); s.slotFill.release();
+  s.slotOf.release(); s.slotCount.release(); s.slotStart.release();
   s.frame32.release(); s.work32.release();
   s.engine.release();
   s.workM64.release();

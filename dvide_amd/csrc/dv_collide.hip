@@ -12,16 +12,19 @@
 // The kept set does not depend on the bins (every kept pair's AABBs overlap
 // with a margin of one envelope), so any complete broadphase yields the same
 // contacts.  Here:
-//   1. small spheres are hashed into cells of edge 2*(r_max + envelope), so a
-//      kept partner lies in one of the 27 neighbouring cells; boxes and large
-//      spheres form a short "big" list tested against every geometry;
-//   2. one pass counts, per geometry, partners with a higher index (its row
-//      of contacts) and a lower index (incidences where it is body B);
-//   3. prefix sums give each geometry's contact row offset, so the emit pass
-//      writes row i's contacts at their final canonical positions after a
-//      thread-local sort of the row (no global key sort);
-//   4. each body's incidences are listed in ascending contact order: first
-//      the contacts where it is B, then its own row.
+//   1. small spheres are sorted into the slots of a hash of cells of edge
+//      2*(r_max + envelope), so a kept partner lies in one of the 27
+//      neighbouring cells; boxes and large spheres form a short "big" list
+//      tested against every geometry;
+//   2. one walk of the neighbouring cells, sixteen lanes to a sphere, finds
+//      each sphere's partners, sorts them by id and keeps them (up to kList);
+//   3. one prefix sum over the bodies gives each geometry's contact row and
+//      incidence offsets and the list of heavy bodies;
+//   4. each sphere's row is written at its final canonical position from the
+//      kept partners (no global key sort and no second walk), with the
+//      incidences of both of its bodies: a body's incidences are listed in
+//      ascending contact order, first the contacts where it is B (its place
+//      among B's partners below is its place in B's list), then its own row.
 // The keep test and the contact record are evaluated with the shared
 // dv_geom.h code (no fused multiply-add), bit-identical to the oracle.
 #include "dv_geom.h"
@@ -35,6 +38,12 @@ namespace {
 
 constexpr int kT = 256;
 
+// What a walk reads of a small geometry, in the order of the cells: its
+// position and radius (posR), and its id, row of cells and family (meta).
+struct alignas(32) PosR {
+  double x, y, z, r;
+};
+
 struct CdArgs {
   const double* p;
   const double* geom;
@@ -42,16 +51,25 @@ struct CdArgs {
   const int* smallIds;
   const int* bigIds;
   int nb, nsmall, nbig;
-  double cs, envelope, rmaxSmall;
+  double cs, envelope;
   unsigned mask;
   int mode;
   const unsigned* slotStart;
-  const int* cellItems;
+  PosR* posR;
+  int4* meta;
 };
 
-__device__ __forceinline__ unsigned cellHash(int cx, int cy, int cz, unsigned mask) {
-  unsigned h = ((unsigned)cx * 73856093u) ^ ((unsigned)cy * 19349663u) ^ ((unsigned)cz * 83492791u);
-  return h & mask;
+// A cell's slot: a hash of its row (the cells along x) plus its place in the
+// row, so that the three cells beside each other are three slots in a row and
+// a walk takes nine ranges instead of 27.
+__device__ __forceinline__ unsigned rowHash(int cy, int cz) {
+  return ((unsigned)cy * 19349663u) ^ ((unsigned)cz * 83492791u);
+}
+// A row of cells, modulo 2^16 rows each way: among a sphere's nine rows no
+// two are equal, so a candidate belongs to one of them at most, and one
+// whose row lies 2^16 rows away is refused by the keep test.
+__device__ __forceinline__ int rowKey(int cy, int cz) {
+  return (int)(((unsigned)cy << 16) | ((unsigned)cz & 0xFFFFu));
 }
 
 __device__ __forceinline__ int cellCoord(double x, double cs) {
@@ -74,71 +92,128 @@ __device__ __forceinline__ bool keepPair(const CdArgs& a, int x, int y) {
   return narrowphase(pA, gA, pB, gB, a.envelope, a.mode, (d3*)0, (double*)0, (d3*)0) != 0;
 }
 
-// Visit every candidate partner j != g of small geometry g: the occupants of
-// the (deduplicated) hash slots of its 27 neighbour cells, then the big list.
-// Cells have edge cs = 2 (rmax + envelope) >= r_g + r_j + envelope, the
-// largest centre distance of a kept pair, so a kept partner lies in one of
-// the 27 cells around g's cell.
-template <class F>
-__device__ __forceinline__ void forEachCandidate(const CdArgs& a, int g, F&& fn) {
-  d3 pg = ldPos(a.p, g);
-  int cx = cellCoord(pg.x, a.cs), cy = cellCoord(pg.y, a.cs), cz = cellCoord(pg.z, a.cs);
-  unsigned slots[27];
-#pragma unroll
-  for (int q = 0; q < 27; ++q)
-    slots[q] = cellHash(cx + q % 3 - 1, cy + (q / 3) % 3 - 1, cz + q / 9 - 1, a.mask);
-#pragma unroll
-  for (int q = 0; q < 27; ++q) {
-    bool dup = false;
-#pragma unroll
-    for (int w = 0; w < q; ++w) dup |= (slots[w] == slots[q]);
-    if (dup) continue;
-    unsigned s0 = a.slotStart[slots[q]], s1 = a.slotStart[slots[q] + 1];
-    for (unsigned k = s0; k < s1; ++k) {
-      int j = a.cellItems[k];
-      if (j != g) fn(j);
+__device__ void insertionSort(int* x, int n) {
+  for (int i = 1; i < n; ++i) {
+    int v = x[i], j = i - 1;
+    while (j >= 0 && x[j] > v) {
+      x[j + 1] = x[j];
+      --j;
+    }
+    x[j + 1] = v;
+  }
+}
+
+__global__ __launch_bounds__(kT) void clearCells(unsigned* x, long n, int* counters) {
+  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) x[i] = 0u;
+  if (i < 8) counters[i] = 0;
+}
+
+// each small geometry's slot and its place there
+__global__ __launch_bounds__(kT) void hashSmall(CdArgs a, unsigned* slotOf, unsigned* slotCount) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= a.nsmall) return;
+  const d3 pg = ldPos(a.p, a.smallIds[t]);
+  const unsigned s =
+      (rowHash(cellCoord(pg.y, a.cs), cellCoord(pg.z, a.cs)) + (unsigned)cellCoord(pg.x, a.cs)) & a.mask;
+  slotOf[2 * (size_t)t] = s;
+  slotOf[2 * (size_t)t + 1] = atomicAdd(&slotCount[s], 1u);
+}
+
+__global__ __launch_bounds__(kT) void scatterSmall(CdArgs a, const unsigned* slotOf) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= a.nsmall) return;
+  const int g = a.smallIds[t];
+  const d3 pg = ldPos(a.p, g);
+  const unsigned pos = a.slotStart[slotOf[2 * (size_t)t]] + slotOf[2 * (size_t)t + 1];
+  a.posR[pos] = PosR{pg.x, pg.y, pg.z, a.geom[3 * (size_t)g]};
+  a.meta[pos] = make_int4(g, rowKey(cellCoord(pg.y, a.cs), cellCoord(pg.z, a.cs)), a.family[g], 0);
+}
+
+// The partners of small geometries, sixteen lanes to each: nine lanes walk a
+// row of three cells, the others test the big list.  A candidate is refused
+// by the squared distance first (with a margin far above the rounding of the
+// exact test), so that few take the exact test's square root.  The partners
+// are sorted by id and kept in lists[g * kList]; with kCsr (a sphere has more
+// than kList) every geometry's partners go to csr[iStart[g]...] instead.
+// Bound by latency at every size (dependent loads: the slots, then the
+// candidates), so by the lanes in flight; one lane to a sphere walking 27
+// cells one by one, twice, took 285 + 338 us at 112,000 spheres and 130 + 142
+// at 8,000.
+constexpr int kList = 24;
+constexpr int kLanes = 16;
+constexpr int kGroups = kT / kLanes;
+template <bool kCsr>
+__global__ __launch_bounds__(kT) void walkSmall(CdArgs a, int* cntUp, int* cntDown, int* lists, int* over,
+                                                const int* iStart, int* csr) {
+  __shared__ int found[kGroups], above[kGroups], ids[kGroups][kList];
+  const int lane = threadIdx.x % kLanes, grp = threadIdx.x / kLanes;
+  const int t = blockIdx.x * kGroups + grp;
+  const bool on = t < a.nsmall;
+  if (lane == 0) found[grp] = above[grp] = 0;
+  __syncthreads();
+  const int4 me = a.meta[on ? t : 0];
+  const PosR pr = a.posR[on ? t : 0];
+  const int g = me.x;
+  int* const out = kCsr ? csr + (on ? iStart[g] : 0) : nullptr;
+  auto keep = [&](int j) {
+    const int k = atomicAdd(&found[grp], 1);
+    if (j > g) atomicAdd(&above[grp], 1);
+    if (kCsr) out[k] = j;
+    else if (k < kList) ids[grp][k] = j;
+  };
+  if (on && lane < 9) {
+    const int cx = cellCoord(pr.x, a.cs), cy = cellCoord(pr.y, a.cs) + lane % 3 - 1;
+    const int cz = cellCoord(pr.z, a.cs) + lane / 3 - 1;
+    const int key = rowKey(cy, cz);
+    const unsigned first = (rowHash(cy, cz) + (unsigned)cx - 1u) & a.mask;
+    // slots first .. first + 2, which may wrap round the table's end
+    const unsigned T = a.mask + 1u, wrap = first + 3u > T ? first + 3u - T : 0u;
+    unsigned k = a.slotStart[first], end = a.slotStart[first + 3u - wrap];
+    for (int part = 0; part < (wrap ? 2 : 1); ++part) {
+      if (part) {
+        k = 0;
+        end = a.slotStart[wrap];
+      }
+      for (; k < end; ++k) {
+        const int4 m = a.meta[k];
+        const PosR q = a.posR[k];
+        if (m.y != key || m.x == g || (m.z == me.z && m.z != -1)) continue;
+        const d3 d = mk3(q.x - pr.x, q.y - pr.y, q.z - pr.z);
+        const double rr = pr.r + q.r, far = rr + a.envelope;
+        if (!(dot3(d, d) <= far * far * 1.00001 + 1e-30)) continue;
+        if (rr - lengthOf(d, a.mode) >= -a.envelope) keep(m.x);
+      }
+    }
+  } else if (on) {
+    for (int q = lane - 9; q < a.nbig; q += kLanes - 9) {
+      const int b = a.bigIds[q];
+      if (keepPair(a, g, b)) keep(b);
     }
   }
-  for (int q = 0; q < a.nbig; ++q) fn(a.bigIds[q]);
-}
-
-__global__ __launch_bounds__(kT) void fillU(unsigned* x, long n, unsigned v) {
-  long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] = v;
-}
-
-__global__ __launch_bounds__(kT) void hashSmall(CdArgs a, unsigned* slotOf, unsigned* slotCount) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.nsmall) return;
-  int g = a.smallIds[t];
-  d3 pg = ldPos(a.p, g);
-  unsigned s = cellHash(cellCoord(pg.x, a.cs), cellCoord(pg.y, a.cs), cellCoord(pg.z, a.cs), a.mask);
-  slotOf[t] = s;
-  atomicAdd(&slotCount[s], 1u);
-}
-
-__global__ __launch_bounds__(kT) void scatterSmall(CdArgs a, const unsigned* slotOf, unsigned* slotFill,
-                                                   int* cellItems) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.nsmall) return;
-  unsigned s = slotOf[t];
-  unsigned pos = a.slotStart[s] + atomicAdd(&slotFill[s], 1u);
-  cellItems[pos] = a.smallIds[t];
-}
-
-// per small geometry: partners above (its contact row) and below
-__global__ __launch_bounds__(kT) void countSmall(CdArgs a, int* cntUp, int* cntDown) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.nsmall) return;
-  int g = a.cellItems[t];  // spatial order: neighbouring threads share cells
-  int up = 0, down = 0;
-  forEachCandidate(a, g, [&](int j) {
-    if (keepPair(a, g, j)) {
-      if (j > g) ++up; else ++down;
+  __syncthreads();
+  const int n = found[grp];
+  if (!on) return;
+  if (kCsr) {
+    __threadfence_block();
+    if (lane == 0) insertionSort(out, n);
+    return;
+  }
+  if (lane == 0) {
+    cntUp[g] = above[grp];
+    cntDown[g] = n - above[grp];
+    if (n > kList) {
+      *over = 1;
+      lists[(size_t)g * kList] = 0;  // not a big geometry's mark
     }
-  });
-  cntUp[g] = up;
-  cntDown[g] = down;
+  }
+  if (n > kList) return;
+  for (int e = lane; e < n; e += kLanes) {
+    const int id = ids[grp][e];
+    int rank = 0;
+    for (int f = 0; f < n; ++f) rank += ids[grp][f] < id ? 1 : 0;
+    lists[(size_t)g * kList + rank] = id;
+  }
 }
 
 __device__ int blockSum(int v) {
@@ -157,8 +232,10 @@ __device__ int blockSum(int v) {
 // Big geometries (boxes, large spheres) are paired with every geometry in
 // chunks of kChunk partners: block (chunk, b) counts the kept partners of big
 // geometry b in its chunk; a per-big scan over the chunks then gives each
-// block its output offsets, so the emit pass writes the row in order.
-constexpr int kChunk = 2048;
+// block its output offsets, so the emit pass writes the row in order.  Two
+// rounds of a workgroup to a chunk: with eight, few workgroups each waited
+// for eight rounds in turn (26 + 11 us at 112,000 spheres).
+constexpr int kChunk = 512;
 
 __global__ __launch_bounds__(kT) void countBigChunks(CdArgs a, int nchunks, int* chUp, int* chDown) {
   const int b = a.bigIds[blockIdx.y];
@@ -178,25 +255,136 @@ __global__ __launch_bounds__(kT) void countBigChunks(CdArgs a, int nchunks, int*
   }
 }
 
-// per big geometry: exclusive scan of its chunk counts (in place) and totals
-__global__ void scanBigChunks(CdArgs a, int nchunks, int* chUp, int* chDown, int* cntUp, int* cntDown) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= a.nbig) return;
-  int su = 0, sd = 0;
-  for (int k = 0; k < nchunks; ++k) {
-    const int u = chUp[q * nchunks + k], d = chDown[q * nchunks + k];
-    chUp[q * nchunks + k] = su;
-    chDown[q * nchunks + k] = sd;
-    su += u;
-    sd += d;
+// per big geometry: exclusive scan of its chunk counts (in place) and totals,
+// a wavefront to each
+__global__ __launch_bounds__(64) void scanBigChunks(CdArgs a, int nchunks, int* chUp, int* chDown, int* cntUp,
+                                                    int* cntDown) {
+  const int q = blockIdx.x, lane = threadIdx.x;
+  int baseUp = 0, baseDown = 0;
+  for (int k0 = 0; k0 < nchunks; k0 += 64) {
+    const int k = k0 + lane;
+    const int u = k < nchunks ? chUp[q * nchunks + k] : 0, d = k < nchunks ? chDown[q * nchunks + k] : 0;
+    int su = u, sd = d;  // inclusive over the wavefront
+#pragma unroll
+    for (int w = 1; w < 64; w <<= 1) {
+      const int yu = __shfl_up(su, w, 64), yd = __shfl_up(sd, w, 64);
+      if (lane >= w) { su += yu; sd += yd; }
+    }
+    if (k < nchunks) {
+      chUp[q * nchunks + k] = baseUp + su - u;
+      chDown[q * nchunks + k] = baseDown + sd - d;
+    }
+    baseUp += __shfl(su, 63, 64);
+    baseDown += __shfl(sd, 63, 64);
   }
-  cntUp[a.bigIds[q]] = su;
-  cntDown[a.bigIds[q]] = sd;
+  if (lane == 0) {
+    cntUp[a.bigIds[q]] = baseUp;
+    cntDown[a.bigIds[q]] = baseDown;
+  }
 }
 
-__global__ __launch_bounds__(kT) void addCounts(const int* cntUp, const int* cntDown, int* tot, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) tot[i] = cntUp[i] + cntDown[i];
+// Offsets of every body's contact row (cStart) and incidences (iStart), and
+// the heavy bodies (more than kHeavyDegree incidences) in ascending order, so
+// that everything summed over them is summed in a fixed order: one scan of
+// three counts, tile sums and then the tiles, each workgroup of which adds up
+// the tiles before its own (past kDirectTiles, scanBodyTiles does that for
+// all).  The totals go to the host's pinned memory as well.
+constexpr int kBodyTile = 1024;
+constexpr int kDirectTiles = 1024;
+struct Counts3 {
+  int up, all, heavy;
+};
+__device__ __forceinline__ Counts3 countsOf(const int* cntUp, const int* cntDown, int g, int nb) {
+  if (g >= nb) return Counts3{0, 0, 0};
+  const int u = cntUp[g], n = u + cntDown[g];
+  return Counts3{u, n, n > kHeavyDegree ? 1 : 0};
+}
+__device__ __forceinline__ Counts3 add3c(const Counts3& a, const Counts3& b) {
+  return Counts3{a.up + b.up, a.all + b.all, a.heavy + b.heavy};
+}
+__global__ __launch_bounds__(kT) void bodyTileSums(int nb, const int* cntUp, const int* cntDown, int* sums) {
+  Counts3 s{0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < kBodyTile / kT; ++q)
+    s = add3c(s, countsOf(cntUp, cntDown, blockIdx.x * kBodyTile + q * kT + threadIdx.x, nb));
+  const int u = blockSum(s.up), n = blockSum(s.all), h = blockSum(s.heavy);
+  if (threadIdx.x == 0) {
+    sums[3 * blockIdx.x] = u;
+    sums[3 * blockIdx.x + 1] = n;
+    sums[3 * blockIdx.x + 2] = h;
+  }
+}
+// in-place exclusive scan of many tile sums by one workgroup
+__global__ __launch_bounds__(64) void scanBodyTiles(int* sums, int tiles) {
+  int base[3] = {0, 0, 0};
+  for (int k0 = 0; k0 < tiles; k0 += 64) {
+    const int k = k0 + (int)threadIdx.x;
+    for (int c = 0; c < 3; ++c) {
+      const int x = k < tiles ? sums[3 * (size_t)k + c] : 0;
+      int y = x;
+#pragma unroll
+      for (int w = 1; w < 64; w <<= 1) {
+        const int z = __shfl_up(y, w, 64);
+        if ((int)threadIdx.x >= w) y += z;
+      }
+      if (k < tiles) sums[3 * (size_t)k + c] = base[c] + y - x;
+      base[c] += __shfl(y, 63, 64);
+    }
+  }
+}
+__global__ __launch_bounds__(kT) void scanBodies(int nb, const int* cntUp, const int* cntDown, const int* sums,
+                                                 int scanned, int* cStart, int* iStart, int* heavy, int* counters,
+                                                 int* host) {
+  __shared__ int waveUp[kT / 64], waveAll[kT / 64], waveHeavy[kT / 64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tile = blockIdx.x;
+  Counts3 base{0, 0, 0};
+  if (scanned) {
+    base = Counts3{sums[3 * (size_t)tile], sums[3 * (size_t)tile + 1], sums[3 * (size_t)tile + 2]};
+  } else {
+    Counts3 s{0, 0, 0};
+    for (int k = threadIdx.x; k < tile; k += kT) s = add3c(s, Counts3{sums[3 * k], sums[3 * k + 1], sums[3 * k + 2]});
+    base = Counts3{blockSum(s.up), blockSum(s.all), blockSum(s.heavy)};
+  }
+  constexpr int kPer = kBodyTile / kT;
+  const int g0 = tile * kBodyTile + (int)threadIdx.x * kPer;
+  Counts3 v[kPer], s{0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    v[q] = countsOf(cntUp, cntDown, g0 + q, nb);
+    s = add3c(s, v[q]);
+  }
+  Counts3 x = s;  // inclusive over the wavefront
+#pragma unroll
+  for (int w = 1; w < 64; w <<= 1) {
+    const Counts3 y{__shfl_up(x.up, w, 64), __shfl_up(x.all, w, 64), __shfl_up(x.heavy, w, 64)};
+    if (lane >= w) x = add3c(x, y);
+  }
+  if (lane == 63) {
+    waveUp[wave] = x.up; waveAll[wave] = x.all; waveHeavy[wave] = x.heavy;
+  }
+  __syncthreads();
+  Counts3 e = add3c(base, Counts3{x.up - s.up, x.all - s.all, x.heavy - s.heavy});
+#pragma unroll
+  for (int w = 0; w < kT / 64; ++w)
+    if (w < wave) e = add3c(e, Counts3{waveUp[w], waveAll[w], waveHeavy[w]});
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    const int g = g0 + q;
+    if (g < nb) {
+      cStart[g] = e.up;
+      iStart[g] = e.all;
+      if (v[q].heavy) heavy[e.heavy] = g;
+    }
+    e = add3c(e, v[q]);
+    if (g == nb - 1) {
+      cStart[nb] = e.up;
+      iStart[nb] = e.all;
+      counters[2] = e.heavy;
+      host[0] = e.up;
+      host[1] = e.all;
+      host[2] = counters[3];  // a sphere's partners exceed kList
+    }
+  }
 }
 
 struct EmitOut {
@@ -206,12 +394,34 @@ struct EmitOut {
   double* gap;
   double* loc;    // 3 SoA, stride cap
   int cap;
-  int* inc;       // partner ids of lower-index contacts, converted later
+  int* inc;
+  int* posB;
+  const int* lists;  // kList sorted partners per small geometry; a big geometry's first is -1
+  const int* csr;    // or every geometry's, at iStart
   const int* cStart;
   const int* iStart;
   const int* cntUp;
   const int* cntDown;
 };
+
+__device__ __forceinline__ const int* listOf(const EmitOut& o, int g) {
+  return o.csr ? o.csr + o.iStart[g] : o.lists + (size_t)g * kList;
+}
+__device__ __forceinline__ bool isBig(const EmitOut& o, int g) { return o.lists[(size_t)g * kList] < 0; }
+
+// Contact c = (A, B) among the incidences of B, a small geometry: in the
+// order of B's partners below it.
+__device__ __forceinline__ void placeB(const EmitOut& o, int c, int A, int B) {
+  const int* L = listOf(o, B);
+  int lo = 0, hi = o.cntDown[B];
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (L[mid] < A) lo = mid + 1; else hi = mid;
+  }
+  const int i0 = o.iStart[B];
+  o.inc[i0 + lo] = (c << 1) | 1;
+  o.posB[c] = i0 - o.cStart[B] + lo;
+}
 
 __device__ __forceinline__ void writeRecord(const CdArgs& a, const EmitOut& o, int c, int A, int B) {
   d3 n, l;
@@ -230,35 +440,24 @@ __device__ __forceinline__ void writeRecord(const CdArgs& a, const EmitOut& o, i
   o.cB[c] = B;
 }
 
-__device__ void insertionSort(int* x, int n) {
-  for (int i = 1; i < n; ++i) {
-    int v = x[i], j = i - 1;
-    while (j >= 0 && x[j] > v) {
-      x[j + 1] = x[j];
-      --j;
-    }
-    x[j + 1] = v;
+// Rows of the small geometries, in id order and four lanes to each, so that a
+// wavefront writes one run of contacts.
+__global__ __launch_bounds__(kT) void emitSmall(CdArgs a, EmitOut o) {
+  const int t = (blockIdx.x * blockDim.x + threadIdx.x) >> 2, lane = threadIdx.x & 3;
+  if (t >= a.nsmall) return;
+  const int g = a.smallIds[t];
+  const int nu = o.cntUp[g], nd = o.cntDown[g], c0 = o.cStart[g], i0 = o.iStart[g];
+  const int* L = listOf(o, g);
+  for (int k = lane; k < nu; k += 4) {
+    const int j = L[nd + k], c = c0 + k;
+    writeRecord(a, o, c, g, j);
+    o.inc[i0 + nd + k] = c << 1;
+    if (!isBig(o, j)) placeB(o, c, g, j);
   }
 }
 
-__global__ __launch_bounds__(kT) void emitSmall(CdArgs a, EmitOut o) {
-  int t = blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= a.nsmall) return;
-  int g = a.cellItems[t];
-  const int c0 = o.cStart[g], i0 = o.iStart[g];
-  int up = 0, down = 0;
-  forEachCandidate(a, g, [&](int j) {
-    if (keepPair(a, g, j)) {
-      if (j > g) o.cB[c0 + up++] = j;
-      else o.inc[i0 + down++] = j;
-    }
-  });
-  insertionSort(o.cB + c0, up);
-  insertionSort(o.inc + i0, down);
-  for (int q = 0; q < up; ++q) writeRecord(a, o, c0 + q, g, o.cB[c0 + q]);
-}
-
-// big geometry rows: ordered stream compaction of each chunk's partners
+// big geometry rows: ordered stream compaction of each chunk's partners (of
+// those below it, the ids for now: placeBig)
 __global__ __launch_bounds__(kT) void emitBigChunks(CdArgs a, EmitOut o, int nchunks, const int* chUp,
                                                     const int* chDown) {
   const int b = a.bigIds[blockIdx.y];
@@ -287,7 +486,12 @@ __global__ __launch_bounds__(kT) void emitBigChunks(CdArgs a, EmitOut o, int nch
       totUp += wUp[w];
       totDown += wDown[w];
     }
-    if (isUp) writeRecord(a, o, offUp + rUp, b, j);
+    if (isUp) {
+      const int c = offUp + rUp;
+      writeRecord(a, o, c, b, j);
+      o.inc[o.iStart[b] + o.cntDown[b] + (c - o.cStart[b])] = c << 1;
+      if (!isBig(o, j)) placeB(o, c, b, j);
+    }
     if (isDown) o.inc[offDown + rDown] = j;
     __syncthreads();
     if (threadIdx.x == 0) { baseUp += totUp; baseDown += totDown; }
@@ -295,45 +499,51 @@ __global__ __launch_bounds__(kT) void emitBigChunks(CdArgs a, EmitOut o, int nch
   }
 }
 
-// incidences of body g in ascending contact order: (c << 1) | side, side 1 =
-// B (first the contacts of its lower-numbered partners' rows, then its own
-// row); and each contact's slot in the B-side order, posB[c] = (iStart[g] -
-// cStart[g]) + q for the q-th B incidence of g, so that the B incidences of
-// every body are contiguous there
-__global__ __launch_bounds__(kT) void buildIncidence(int nb, const int* cStart, const int* iStart,
-                                                     const int* cntUp, const int* cntDown,
-                                                     const int* cB, int* inc, int* posB, int* heavyFlag) {
-  int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= nb) return;
-  const int i0 = iStart[g], nd = cntDown[g], nu = cntUp[g];
-  const int b0 = i0 - cStart[g];
-  for (int q = 0; q < nd; ++q) {
-    int j = inc[i0 + q];
-    int lo = cStart[j], hi = cStart[j] + cntUp[j];
+// the incidences a big geometry has as body B, from the ids left there: the
+// contact is found in the partner's row
+__global__ __launch_bounds__(kT) void placeBig(CdArgs a, EmitOut o) {
+  const int b = a.bigIds[blockIdx.y];
+  const int i0 = o.iStart[b], nd = o.cntDown[b];
+  for (int q = blockIdx.x * kT + threadIdx.x; q < nd; q += gridDim.x * kT) {
+    const int j = o.inc[i0 + q];
+    int lo = o.cStart[j], hi = lo + o.cntUp[j];
     while (lo < hi) {
-      int mid = (lo + hi) >> 1;
-      if (cB[mid] < g) lo = mid + 1; else hi = mid;
+      const int mid = (lo + hi) >> 1;
+      if (o.cB[mid] < b) lo = mid + 1; else hi = mid;
     }
-    inc[i0 + q] = (lo << 1) | 1;
-    posB[lo] = b0 + q;
+    o.inc[i0 + q] = (lo << 1) | 1;
+    o.posB[lo] = i0 - o.cStart[b] + q;
   }
-  const int c0 = cStart[g];
-  for (int q = 0; q < nu; ++q) inc[i0 + nd + q] = (c0 + q) << 1;
-  heavyFlag[g] = nd + nu > kHeavyDegree ? 1 : 0;
 }
 
-// the bodies reduced by a whole workgroup, in ascending order (so that
-// everything summed over them is summed in a fixed order), and their count
-__global__ __launch_bounds__(kT) void compactHeavy(int nb, const int* heavyFlag, const int* pos, int* heavy,
-                                                   int* counters) {
-  int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g == 0) counters[2] = pos[nb];
-  if (g < nb && heavyFlag[g]) heavy[pos[g]] = g;
+__global__ void markBig(CdArgs a, int* lists) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < a.nbig) lists[(size_t)a.bigIds[q] * kList] = -1;
 }
 
-__global__ void zeroInt(int* x, int n) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < n) x[i] = 0;
+}  // namespace
+
+namespace {
+
+CdArgs cdArgs(Scene& s) {
+  CdArgs a;
+  a.p = s.p.p;
+  a.geom = s.geom.p;
+  a.family = s.family.p;
+  a.smallIds = s.smallIds.p;
+  a.bigIds = s.bigIds.p;
+  a.nb = s.nb;
+  a.nsmall = s.nsmall;
+  a.nbig = s.nbig;
+  a.cs = 2.0 * (s.cellSize + s.envelope);
+  if (!(a.cs > 0)) a.cs = 1.0;
+  a.envelope = s.envelope;
+  a.mask = s.hashSize - 1;
+  a.mode = s.geomMode;
+  a.slotStart = s.slotStart.p;
+  a.posR = reinterpret_cast<PosR*>(s.cellPosR.p);
+  a.meta = reinterpret_cast<int4*>(s.cellMeta.p);
+  return a;
 }
 
 }  // namespace
@@ -375,60 +585,36 @@ void collideInit(Scene& s) {
     DV_HIP(hipMemcpyAsync(s.smallIds.p, small.data(), sizeof(int) * s.nsmall, hipMemcpyHostToDevice, s.stream));
   if (s.nbig)
     DV_HIP(hipMemcpyAsync(s.bigIds.p, big.data(), sizeof(int) * s.nbig, hipMemcpyHostToDevice, s.stream));
-  s.slotOf.reserve(std::max(1, s.nsmall));
+  s.slotOf.reserve(2 * (size_t)std::max(1, s.nsmall));
   s.slotCount.reserve(T);
-  s.slotFill.reserve(T);
   s.slotStart.reserve(T + 1);
-  s.cellItems.reserve(std::max(1, s.nsmall));
+  s.cellPosR.reserve(4 * (size_t)std::max(1, s.nsmall));
+  s.cellMeta.reserve(4 * (size_t)std::max(1, s.nsmall));
+  s.lists.reserve((size_t)kList * std::max(1, s.nb));
   s.cntUp.reserve(s.nb + 1);
   s.cntDown.reserve(s.nb + 1);
   s.cStart.reserve(s.nb + 1);
   s.iStart.reserve(s.nb + 1);
   s.counters.reserve(8);
   s.heavy.reserve(s.nb + 1);
-  s.heavyPos.reserve(s.nb + 1);
+  const CdArgs a = cdArgs(s);
+  hipLaunchKernelGGL(markBig, dim3(blocksFor(s.nbig, 64)), dim3(64), 0, s.stream, a, s.lists.p);
   DV_HIP(hipStreamSynchronize(s.stream));
 }
-
-namespace {
-
-CdArgs cdArgs(Scene& s) {
-  CdArgs a;
-  a.p = s.p.p;
-  a.geom = s.geom.p;
-  a.family = s.family.p;
-  a.smallIds = s.smallIds.p;
-  a.bigIds = s.bigIds.p;
-  a.nb = s.nb;
-  a.nsmall = s.nsmall;
-  a.nbig = s.nbig;
-  a.cs = 2.0 * (s.cellSize + s.envelope);
-  a.rmaxSmall = s.cellSize;
-  if (!(a.cs > 0)) a.cs = 1.0;
-  a.envelope = s.envelope;
-  a.mask = s.hashSize - 1;
-  a.mode = s.geomMode;
-  a.slotStart = s.slotStart.p;
-  a.cellItems = s.cellItems.p;
-  return a;
-}
-
-}  // namespace
 
 void collideCount(Scene& s) {
   const hipStream_t st = s.stream;
   const CdArgs a = cdArgs(s);
   const unsigned T = s.hashSize;
 
-  hipLaunchKernelGGL(zeroInt, dim3(1), dim3(64), 0, st, s.counters.p, 8);
+  hipLaunchKernelGGL(clearCells, dim3(blocksFor(T, kT)), dim3(kT), 0, st, s.slotCount.p, s.nsmall ? (long)T : 0L,
+                     s.counters.p);
   if (s.nsmall) {
-    hipLaunchKernelGGL(fillU, dim3(blocksFor(T, kT)), dim3(kT), 0, st, s.slotCount.p, (long)T, 0u);
-    hipLaunchKernelGGL(fillU, dim3(blocksFor(T, kT)), dim3(kT), 0, st, s.slotFill.p, (long)T, 0u);
     hipLaunchKernelGGL(hashSmall, dim3(blocksFor(s.nsmall, kT)), dim3(kT), 0, st, a, s.slotOf.p, s.slotCount.p);
     exclusiveScanU(s, s.slotCount.p, s.slotStart.p, (int)T);
-    hipLaunchKernelGGL(scatterSmall, dim3(blocksFor(s.nsmall, kT)), dim3(kT), 0, st, a, s.slotOf.p,
-                       s.slotFill.p, s.cellItems.p);
-    hipLaunchKernelGGL(countSmall, dim3(blocksFor(s.nsmall, kT)), dim3(kT), 0, st, a, s.cntUp.p, s.cntDown.p);
+    hipLaunchKernelGGL(scatterSmall, dim3(blocksFor(s.nsmall, kT)), dim3(kT), 0, st, a, (const unsigned*)s.slotOf.p);
+    hipLaunchKernelGGL(walkSmall<false>, dim3(blocksFor(s.nsmall, kGroups)), dim3(kT), 0, st, a, s.cntUp.p, s.cntDown.p,
+                       s.lists.p, s.counters.p + 3, (const int*)nullptr, (int*)nullptr);
   }
   const int nchunks = blocksFor(s.nb, kChunk);
   s.bigChunks.reserve((size_t)2 * std::max(1, s.nbig * nchunks));
@@ -436,18 +622,18 @@ void collideCount(Scene& s) {
   int* chDown = s.bigChunks.p + (size_t)std::max(1, s.nbig * nchunks);
   if (s.nbig) {
     hipLaunchKernelGGL(countBigChunks, dim3(nchunks, s.nbig), dim3(kT), 0, st, a, nchunks, chUp, chDown);
-    hipLaunchKernelGGL(scanBigChunks, dim3(blocksFor(s.nbig, 64)), dim3(64), 0, st, a, nchunks, chUp, chDown,
-                       s.cntUp.p, s.cntDown.p);
+    hipLaunchKernelGGL(scanBigChunks, dim3(s.nbig), dim3(64), 0, st, a, nchunks, chUp, chDown, s.cntUp.p, s.cntDown.p);
   }
-  // contact rows and incidence offsets
-  s.scanTmp.reserve(16);
-  exclusiveScan(s, s.cntUp.p, s.cStart.p, s.nb);
-  DevBuf<int>& tot = s.hostTotals;  // reuse as n-sized temp of up+down
-  tot.reserve(s.nb + 1);
-  hipLaunchKernelGGL(addCounts, dim3(blocksFor(s.nb, kT)), dim3(kT), 0, st, s.cntUp.p, s.cntDown.p, tot.p, s.nb);
-  exclusiveScan(s, tot.p, s.iStart.p, s.nb);
-  DV_HIP(hipMemcpyAsync(s.pinned, s.cStart.p + s.nb, sizeof(int), hipMemcpyDeviceToHost, st));
-  DV_HIP(hipMemcpyAsync(s.pinned + 1, s.iStart.p + s.nb, sizeof(int), hipMemcpyDeviceToHost, st));
+  // contact rows and incidence offsets, heavy bodies, and the totals for the host
+  const int tiles = blocksFor(s.nb, kBodyTile);
+  s.scanTmp.reserve(3 * (size_t)tiles);
+  s.pinned[0] = s.pinned[1] = s.pinned[2] = 0;  // (a scene without bodies)
+  hipLaunchKernelGGL(bodyTileSums, dim3(tiles), dim3(kT), 0, st, s.nb, (const int*)s.cntUp.p, (const int*)s.cntDown.p,
+                     s.scanTmp.p);
+  if (tiles > kDirectTiles) hipLaunchKernelGGL(scanBodyTiles, dim3(1), dim3(64), 0, st, s.scanTmp.p, tiles);
+  hipLaunchKernelGGL(scanBodies, dim3(tiles), dim3(kT), 0, st, s.nb, (const int*)s.cntUp.p, (const int*)s.cntDown.p,
+                     (const int*)s.scanTmp.p, tiles > kDirectTiles ? 1 : 0, s.cStart.p, s.iStart.p, s.heavy.p,
+                     s.counters.p, s.pinned);
 }
 
 void collideEmit(Scene& s) {
@@ -475,20 +661,23 @@ void collideEmit(Scene& s) {
     s.posB.reserve(cap);
     s.ncCap = cap;
   }
+  const bool csr = s.pinned[2] != 0;
+  if (csr) {
+    s.csr.reserve(std::max(1, ninc));
+    hipLaunchKernelGGL(walkSmall<true>, dim3(blocksFor(s.nsmall, kGroups)), dim3(kT), 0, st, a, s.cntUp.p, s.cntDown.p,
+                       s.lists.p, s.counters.p + 3, (const int*)s.iStart.p, s.csr.p);
+  }
   EmitOut o;
   o.cA = s.cA.p; o.cB = s.cB.p; o.frame = s.frame.p; o.gap = s.gap.p; o.loc = s.loc.p;
   o.cap = s.ncCap;
-  o.inc = s.inc.p;
+  o.inc = s.inc.p; o.posB = s.posB.p;
+  o.lists = s.lists.p; o.csr = csr ? s.csr.p : nullptr;
   o.cStart = s.cStart.p; o.iStart = s.iStart.p; o.cntUp = s.cntUp.p; o.cntDown = s.cntDown.p;
-  if (s.nsmall) hipLaunchKernelGGL(emitSmall, dim3(blocksFor(s.nsmall, kT)), dim3(kT), 0, st, a, o);
-  if (s.nbig)
+  if (s.nsmall) hipLaunchKernelGGL(emitSmall, dim3(blocksFor(4L * s.nsmall, kT)), dim3(kT), 0, st, a, o);
+  if (s.nbig) {
     hipLaunchKernelGGL(emitBigChunks, dim3(nchunks, s.nbig), dim3(kT), 0, st, a, o, nchunks, chUp, chDown);
-  int* heavyFlag = s.hostTotals.p;  // free again after the offsets' scans
-  hipLaunchKernelGGL(buildIncidence, dim3(blocksFor(s.nb, kT)), dim3(kT), 0, st, s.nb, s.cStart.p,
-                     s.iStart.p, s.cntUp.p, s.cntDown.p, s.cB.p, s.inc.p, s.posB.p, heavyFlag);
-  exclusiveScan(s, heavyFlag, s.heavyPos.p, s.nb);
-  hipLaunchKernelGGL(compactHeavy, dim3(blocksFor(s.nb, kT)), dim3(kT), 0, st, s.nb, (const int*)heavyFlag,
-                     (const int*)s.heavyPos.p, s.heavy.p, s.counters.p);
+    hipLaunchKernelGGL(placeBig, dim3(16, s.nbig), dim3(kT), 0, st, a, o);
+  }
   DV_HIP(hipGetLastError());
 }
 

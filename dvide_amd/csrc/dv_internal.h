@@ -224,13 +224,13 @@ struct Scene {
   DevBuf<int> bilIncStart, bilInc;  // per body: (row<<3)|(comp<<1)|sign
 
   // --- collision detection work
-  DevBuf<unsigned> slotOf, slotCount, slotStart, slotFill;
-  DevBuf<int> cellItems;
-  DevBuf<double> cellPosR;  // 4 per sorted small geometry
+  DevBuf<unsigned> slotOf, slotCount, slotStart;
+  DevBuf<double> cellPosR;  // 4 per sorted small geometry: position, radius
+  DevBuf<int> cellMeta;     // 4 per sorted small geometry: id, row of cells, family, -
+  DevBuf<int> lists, csr;   // each geometry's sorted partners (dv_collide.hip)
   DevBuf<int> cntUp, cntDown, cStart, iStart, scanTmp;
-  DevBuf<int> counters;     // [0] nc, [1] ninc, [2] nHeavy
-  DevBuf<int> hostTotals;
-  int* pinned = nullptr;    // pinned host copy of counters
+  DevBuf<int> counters;     // [2] nHeavy, [3] a partner list overflowed
+  int* pinned = nullptr;    // pinned: contacts, incidences, overflow of the last count
 
   // --- contacts (canonical (idA, idB) order)
   int nc = 0, ncCap = 0;
@@ -242,7 +242,6 @@ struct Scene {
   DevBuf<int> inc;       // per-body incidences (contact << 1 | side)
   DevBuf<int> posB;      // per contact: its slot in the B-side order (see buildIncidence)
   DevBuf<int> heavy;     // bodies processed by a whole workgroup, ascending
-  DevBuf<int> heavyPos;  // their positions in `heavy` (exclusive scan of the flags)
   DevBuf<int> bigChunks; // per (big geometry, chunk) partner counts
 
   // --- system of the step (flat rows: nbil bilateral, then 3 per contact)
@@ -311,8 +310,7 @@ std::vector<int> enginePoll(Engine& E, hipStream_t st);
 void engineRetire(Engine& E, const std::vector<int>& slots, hipStream_t st);
 bool engineBusy(const Engine& E);
 
-// scans (dv_scan.hip): exclusive scan of n ints, out has n+1 entries
-void exclusiveScan(Scene& s, const int* in, int* out, int n);
+// scan (dv_scan.hip): exclusive scan of n numbers, out has n+1 entries
 void exclusiveScanU(Scene& s, const unsigned* in, unsigned* out, int n);
 
 inline int blocksFor(long n, int t) { return (int)((n + t - 1) / t) > 0 ? (int)((n + t - 1) / t) : 1; }

@@ -1,10 +1,10 @@
 // Device-wide exclusive prefix sums (out[i] = sum in[0..i), out[n] = total),
-// used for the cell-slot offsets and the contact/incidence offsets of the
-// collision pipeline (the reference's thrust::inclusive_scan calls,
-// CollisionDetector.cu:586,605,614,650 and System.cu:1357).
+// used for the cell-slot offsets of the collision pipeline (the reference's
+// thrust::inclusive_scan calls, CollisionDetector.cu:586,605,614,650).
 //
-// Three passes over 1024-element tiles: tile sums, a scan of the tile sums
-// (recursively), and the tile-local scans with their offsets added.  Each
+// Passes over 1024-element tiles: tile sums, then the tile-local scans, each
+// block first adding up the tile sums before its own.  Past kDirect tiles
+// (a million elements) the tile sums are scanned first, recursively.  Each
 // 256-thread block scans its tile with 64-wide wavefront shuffles.
 #include "dv_internal.h"
 
@@ -14,6 +14,7 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kPer = 4;
 constexpr int kTile = kThreads * kPer;
+constexpr int kDirect = 1024;
 
 template <typename T>
 __device__ T blockExclusiveScan(T v, T* total) {
@@ -52,7 +53,7 @@ __global__ __launch_bounds__(kThreads) void tileSums(const T* __restrict__ in, T
 
 template <typename T>
 __global__ __launch_bounds__(kThreads) void tileScan(const T* __restrict__ in, T* __restrict__ out,
-                                                     const T* __restrict__ offs, int n) {
+                                                     const T* __restrict__ offs, int direct, int n) {
   const long base = (long)blockIdx.x * kTile + threadIdx.x * kPer;
   T vals[kPer];
   T s = 0;
@@ -61,8 +62,15 @@ __global__ __launch_bounds__(kThreads) void tileScan(const T* __restrict__ in, T
     vals[q] = (base + q < n) ? in[base + q] : 0;
     s += vals[q];
   }
-  T tot;
-  T ex = blockExclusiveScan<T>(s, &tot) + (offs ? offs[blockIdx.x] : 0);
+  T tot, before = 0;
+  if (direct) {  // offs holds the tile sums themselves
+    T part = 0;
+    for (int k = threadIdx.x; k < (int)blockIdx.x; k += kThreads) part += offs[k];
+    blockExclusiveScan<T>(part, &before);
+  } else if (offs) {
+    before = offs[blockIdx.x];
+  }
+  T ex = blockExclusiveScan<T>(s, &tot) + before;
 #pragma unroll
   for (int q = 0; q < kPer; ++q) {
     if (base + q < n) out[base + q] = ex;
@@ -75,14 +83,18 @@ template <typename T>
 void scanImpl(hipStream_t st, const T* in, T* out, int n, std::vector<T*>& scratch, int depth) {
   const int tiles = blocksFor(n, kTile);
   if (tiles == 1) {
-    hipLaunchKernelGGL(tileScan<T>, dim3(1), dim3(kThreads), 0, st, in, out, (const T*)nullptr, n);
+    hipLaunchKernelGGL(tileScan<T>, dim3(1), dim3(kThreads), 0, st, in, out, (const T*)nullptr, 0, n);
     return;
   }
   T* sums = scratch[2 * depth];
   T* sumsScan = scratch[2 * depth + 1];
   hipLaunchKernelGGL(tileSums<T>, dim3(tiles), dim3(kThreads), 0, st, in, sums, n);
+  if (tiles <= kDirect) {
+    hipLaunchKernelGGL(tileScan<T>, dim3(tiles), dim3(kThreads), 0, st, in, out, (const T*)sums, 1, n);
+    return;
+  }
   scanImpl<T>(st, sums, sumsScan, tiles, scratch, depth + 1);
-  hipLaunchKernelGGL(tileScan<T>, dim3(tiles), dim3(kThreads), 0, st, in, out, (const T*)sumsScan, n);
+  hipLaunchKernelGGL(tileScan<T>, dim3(tiles), dim3(kThreads), 0, st, in, out, (const T*)sumsScan, 0, n);
 }
 
 template <typename T>
@@ -113,7 +125,6 @@ void scanTop(Scene& s, const T* in, T* out, int n) {
 
 }  // namespace
 
-void exclusiveScan(Scene& s, const int* in, int* out, int n) { scanTop<int>(s, in, out, n); }
 void exclusiveScanU(Scene& s, const unsigned* in, unsigned* out, int n) {
   scanTop<unsigned>(s, in, out, n);
 }

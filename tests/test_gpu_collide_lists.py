@@ -1,0 +1,104 @@
+"""Collision detection where its paths part: partner lists that hold a
+sphere's partners and that do not (24 fit), big geometries before, among and
+after the small ones, and cells on both sides of the origin.  The contact set
+is the oracle's bit for bit, and so is the Schur product, which reads every
+body's incidence list; the pass kernels' product reads the B-side order."""
+import numpy as np
+import pytest
+
+import oracle
+from dvide_amd import scenes, system
+from tests.helpers import both, pair_keys, rel
+
+pytestmark = pytest.mark.gpu
+
+
+def _scene(geoms, pos, seed, family=None):
+    rng = np.random.default_rng(seed)
+    n = len(geoms)
+    geom = np.zeros((n, 3))
+    for i, g in enumerate(geoms):
+        geom[i, :len(np.atleast_1d(g))] = g
+    sc = scenes.cloud(1, n=8)
+    sc.pos, sc.vel = np.array(pos, float), rng.normal(0.0, 0.1, (n, 3))
+    sc.mass, sc.geom = rng.uniform(0.5, 2.0, n), geom
+    sc.fixed = np.zeros(n, np.int32)
+    sc.family = np.full(n, -1, np.int32) if family is None else np.asarray(family, np.int32)
+    sc.bil_dofs, sc.bil_info = np.zeros((0, 2), np.int32), np.zeros((0, 2))
+    return sc
+
+
+def swarm(hubs, around, hub_radius):
+    """Spheres of `hub_radius` with `around` spheres of radius 0.05 each
+    touching them from all sides, hubs and others in shuffled order, beside a
+    line of single spheres (which keep the median radius small)."""
+    rng = np.random.default_rng(17 + around)
+    pos, rad = [], []
+    for k in range(hubs):
+        c = np.array([3.0 * (k - hubs / 2), -1.0, 0.5])
+        pos.append(c)
+        rad.append(hub_radius)
+        u = rng.normal(size=(around, 3))
+        u /= np.linalg.norm(u, axis=1)[:, None]
+        pos += list(c + u * (hub_radius + 0.05) * rng.uniform(0.97, 1.0, (around, 1)))
+        rad += [0.05] * around
+    line = np.arange(1500)
+    pos += list(np.stack([0.0995 * (line - 700), np.full(line.size, 4.0), 0.001 * np.sin(line)], 1))
+    rad += [0.05] * line.size
+    order = rng.permutation(len(rad))
+    return _scene([rad[i] for i in order], [pos[i] for i in order], 3)
+
+
+def mixed_order(seed):
+    """A cloud with large spheres and boxes first, in the middle and last,
+    some geometries in collision families."""
+    rng = np.random.default_rng(seed)
+    n = 1200
+    pos = rng.uniform(-0.9, 0.9, (n, 3))
+    geoms = [rng.uniform(0.03, 0.05) for _ in range(n)]
+    for i, g in ((0, (1.2, 0.05, 1.2)), (1, 0.3), (n // 2, 0.35), (n // 2 + 1, (0.2, 0.3, 0.1)), (n - 2, 0.4),
+                 (n - 1, (1.2, 0.05, 1.2))):
+        geoms[i] = g
+    pos[0], pos[n - 1] = (0, -0.95, 0), (0, 0.95, 0)
+    return _scene(geoms, pos, seed, rng.choice([-1, -1, -1, 1, 2], n))
+
+
+SCENES = {
+    "lists_24": lambda: swarm(5, 23, 0.19),
+    "lists_25": lambda: swarm(5, 26, 0.19),
+    "lists_90": lambda: swarm(3, 90, 0.2),
+    "big_order": lambda: mixed_order(5),
+    "one_sphere": lambda: _scene([0.05, (1, 0.1, 1)], [(0, 0.15, 0), (0, 0, 0)], 1),
+    "boxes_only": lambda: _scene([(1, 0.1, 1), (1, 0.1, 1)], [(0, 0.15, 0), (0, 0, 0)], 1),
+}
+
+
+@pytest.mark.parametrize("name", SCENES)
+def test_contacts_and_incidences_match_the_oracle(gpu, name):
+    o, g = both(SCENES[name]())
+    for _ in range(2):  # the second time with the first's lists in place
+        nc = o.assemble()
+        assert g.assemble() == nc
+        if name == "boxes_only":
+            assert nc == 0
+            return
+        a0, b0, n0, l0 = o.contacts()
+        a1, b1, n1, l1 = g.contacts()
+        assert np.array_equal(pair_keys(a0, b0), pair_keys(a1, b1))
+        # (a sphere whose centre lies inside a box has no normal: NaN on both sides)
+        assert np.array_equal(n0, n1, equal_nan=True) and np.array_equal(l0, l1, equal_nan=True)
+        most = np.bincount(np.concatenate([a0, b0]).astype(int)).max()
+        assert (most > 24) == (name not in ("lists_24", "one_sphere")), most
+        x = np.random.default_rng(11).normal(size=3 * nc)
+        ref = o.schur(x)
+        assert np.array_equal(g.schur_product(x), ref, equal_nan=True)
+        # the same products in FP64, in another order: sums of at most a few
+        # hundred terms, so rounding of a few hundred ulps
+        y = g.pass_product(x, system.BUILD_FP64)
+        fine = np.isfinite(ref)
+        assert np.array_equal(fine, np.isfinite(y)) and rel(y[fine], ref[fine]) < 1e-13
+        if name != "one_sphere":
+            p = o.vec(oracle.P)
+            p[0::3] += 0.01
+            o.set_vec(oracle.P, p)
+            g.set_vector(system.VEC_P, p)
