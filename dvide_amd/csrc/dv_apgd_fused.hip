@@ -1788,6 +1788,7 @@ void Engine::release() {
   states.release();
   views.release();
   teamSync.release();
+  teamItems.release();
   if (outHost) (void)hipHostFree(outHost);
   outHost = nullptr;
   for (hipEvent_t& e : polled) {
@@ -1988,12 +1989,66 @@ Plan<TM> activePlan(Engine& E) {
   return P;
 }
 
+// The resident passes (dv_apgd_resident.h).  A slot's team is one workgroup
+// per row tile, or per two: one workgroup fills a CU, so once the tiles
+// outnumber the CUs two rows per thread do more work per exchange (48 scenes
+// of 1,000 to 20,000 contacts, 545 tiles, 233 passes: 6.0 ms as launches, 2.7
+// so; 512 scenes, 8.1 million contacts: 372 ms and 322).  The members of a team must all be
+// running, so a team may be no larger than the chip; the teams of a launch
+// may be, since they are placed in order and the first to end make room.
+constexpr int kTeamPasses = 2048;     // of one launch of a single scene
+constexpr int kTeamPassesMany = 512;  // of several scenes: a team waits for the room of those before it
+constexpr int kTeamPassesServed = 64; // of a server, which admits and completes between launches
+constexpr int kTeamSkip = 16;         // solves that stay on launches after a team could not be placed
+
+// Every active slot's team, uploaded for the launches to come; teamRows 0
+// where a slot has none (its passes, and the others', then run as launches).
+template <typename TM>
+void buildTeams(Engine& E, hipStream_t st) {
+  const int most = std::min(kTeamMax, E.numCU);
+  long tiles = 0;
+  for (int slot : E.active.hSlots) tiles += slotArgs<TM>(E, slot).nTiles;
+  const int R = tiles > E.numCU ? 2 : 1;
+  std::vector<TeamItem> items;
+  E.teamRows = E.active.hSlots.empty() ? 0 : R;
+  E.teamBil = false;
+  for (int slot : E.active.hSlots) {
+    const Args<TM>& a = slotArgs<TM>(E, slot);
+    const int members = (a.nTiles + R - 1) / R;
+    if (members > most || a.nBodyTiles > 64L * members) E.teamRows = 0;  // (32 rounds of body units)
+    for (int k = 0; k < members; ++k) items.push_back(TeamItem{slot, k, members, 0});
+    E.teamBil = E.teamBil || a.dims.nbil > 0;
+  }
+  E.hTeams.assign(reinterpret_cast<const char*>(items.data()), reinterpret_cast<const char*>(items.data() + items.size()));
+  if (!E.teamRows) return;
+  E.teamItems.reserve(E.hTeams.size());
+  DV_HIP(hipMemcpyAsync(E.teamItems.p, E.hTeams.data(), E.hTeams.size(), hipMemcpyHostToDevice, st));
+}
+template <typename TM>
+void launchTeams(Engine& E, hipStream_t st, int passes) {
+  const size_t need = (size_t)kTeamSync * E.nSlots;
+  if (E.teamSync.cap < need) {
+    E.teamSync.reserve(need);
+    DV_HIP(hipMemsetAsync(E.teamSync.p, 0, sizeof(u64) * E.teamSync.cap, st));
+  }
+  const Tables T = tablesOf<TM>(E, E.active);
+  const auto kernel = E.teamBil ? (E.teamRows == 1 ? kTeam<TM, true, 1> : kTeam<TM, true, 2>)
+                                : (E.teamRows == 1 ? kTeam<TM, false, 1> : kTeam<TM, false, 2>);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(E.hTeams.size() / sizeof(TeamItem))), dim3(kTC), 0, st,
+                     reinterpret_cast<const Args<TM>*>(E.table.p), T,
+                     reinterpret_cast<const TeamItem*>(E.teamItems.p), E.teamSync.p, E.teamEpoch + 1, ++E.teamLaunch,
+                     passes, E.nSlots == 1 ? kFormTicks : kFormTicksMany);
+  DV_HIP(hipGetLastError());
+  E.teamEpoch += 2 * (unsigned long long)passes + 2;
+}
+
 template <typename TM>
 void rebuildActive(Engine& E, hipStream_t st) {
   E.active.hSlots.clear();
   for (int i = 0; i < E.nSlots; ++i)
     if (slotArgs<TM>(E, i).active) E.active.hSlots.push_back(i);
   buildSet<TM>(E, E.active, st);
+  buildTeams<TM>(E, st);
 }
 
 template <typename TM>
@@ -2136,8 +2191,17 @@ void engineStartAdmitted(Engine& E, hipStream_t st) {
 }
 
 void engineRunChunk(Engine& E, hipStream_t st) {
-  if (E.mixed) runChunk<float>(E, st, nullptr, 0);
-  else runChunk<double>(E, st, nullptr, 0);
+  // resident, unless the last such launch made no progress (enginePoll)
+  const bool resident = E.teamRows && !E.noGraph && E.teamSkip == 0;
+  E.ranResident = resident;
+  if (E.teamSkip > 0) --E.teamSkip;
+  if (resident) {
+    if (E.mixed) launchTeams<float>(E, st, kTeamPassesServed);
+    else launchTeams<double>(E, st, kTeamPassesServed);
+  } else {
+    if (E.mixed) runChunk<float>(E, st, nullptr, 0);
+    else runChunk<double>(E, st, nullptr, 0);
+  }
 }
 
 std::vector<int> enginePoll(Engine& E, hipStream_t st) {
@@ -2145,8 +2209,17 @@ std::vector<int> enginePoll(Engine& E, hipStream_t st) {
   DV_HIP(hipMemcpyAsync(outH, E.out.p, sizeof(ApgdState) * E.nSlots, hipMemcpyDeviceToHost, st));
   DV_HIP(hipStreamSynchronize(st));
   std::vector<int> done;
+  long passes = 0;
+  bool some = false;
   for (int i = 0; i < E.nSlots; ++i)
-    if (E.slotScene[i] && outH[i].done) done.push_back(i);
+    if (E.slotScene[i]) {
+      if (outH[i].done) done.push_back(i);
+      passes += outH[i].passes;
+      some = some || outH[i].passes > 0;
+    }
+  if (E.ranResident && some && done.empty() && passes == E.polledPasses) E.teamSkip = kTeamSkip;
+  E.polledPasses = passes;
+  E.ranResident = false;
   return done;
 }
 
@@ -2162,37 +2235,6 @@ bool engineBusy(const Engine& E) {
 }
 
 namespace {
-
-// The resident passes of the engine's only slot (dv_apgd_resident.h), taken
-// when its team fits the chip: one workgroup to a CU, all running at once,
-// each with one row tile or, past one tile per CU, two.
-constexpr int kTeamPasses = 2048;  // of one launch
-constexpr int kTeamSkip = 16;      // solves that stay on launches after a team could not be placed
-inline int teamRows(const Engine& E, int tiles) { return tiles > std::min(kTeamMax, E.numCU) ? 2 : 1; }
-template <typename TM>
-bool teamFits(Engine& E, int slot) {
-  const Args<TM>& a = slotArgs<TM>(E, slot);
-  const int R = teamRows(E, a.nTiles), members = (a.nTiles + R - 1) / R;
-  return members <= std::min(kTeamMax, E.numCU) && a.nBodyTiles <= 64L * members;  // (32 rounds of body units)
-}
-template <typename TM>
-void launchTeam(Engine& E, hipStream_t st) {
-  const size_t need = (size_t)kTeamSync * E.nSlots;
-  if (E.teamSync.cap < need) {
-    E.teamSync.reserve(need);
-    DV_HIP(hipMemsetAsync(E.teamSync.p, 0, sizeof(u64) * E.teamSync.cap, st));
-  }
-  const Tables T = tablesOf<TM>(E, E.active);
-  const Args<TM>& a = slotArgs<TM>(E, 0);
-  const int R = teamRows(E, a.nTiles);
-  const auto kernel = a.dims.nbil ? (R == 1 ? kTeam<TM, true, 1> : kTeam<TM, true, 2>)
-                                  : (R == 1 ? kTeam<TM, false, 1> : kTeam<TM, false, 2>);
-  hipLaunchKernelGGL(kernel, dim3((a.nTiles + R - 1) / R), dim3(kTC), 0, st,
-                     reinterpret_cast<const Args<TM>*>(E.table.p), T, (const TeamItem*)nullptr, E.teamSync.p,
-                     E.teamEpoch + 1, ++E.teamLaunch, kTeamPasses);
-  DV_HIP(hipGetLastError());
-  E.teamEpoch += 2 * kTeamPasses + 2;
-}
 
 // Admit all, run chunks until every scene is done, retire all.  With
 // profiling (single scene), one chunk per solve is launched on the stream
@@ -2229,10 +2271,10 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
   int maxIt = 1;
   for (Scene* s : scenes) maxIt = std::max(maxIt, s->maxIt);
   const long passCap = (long)maxIt * 64 + 4096;
-  int passesBefore = 0;
-  // one slot whose schedule is decided runs resident, until a launch makes no
-  // progress (its team could not be placed)
-  const bool mayReside = n == 1 && !tc && !E.noGraph && !E.forcedRpt && teamFits<TM>(E, 0) && E.teamSkip == 0;
+  long passesBefore = 0;
+  // a class whose schedule is decided runs resident, until a launch makes no
+  // progress (no team could be placed)
+  const bool mayReside = !tc && !E.noGraph && !E.forcedRpt && E.teamRows && E.teamSkip == 0;
   if (E.teamSkip > 0) --E.teamSkip;
   bool resident = mayReside && !ev;  // (profiling: once the sample is taken)
   ApgdState* outH = reinterpret_cast<ApgdState*>(E.outHost);
@@ -2250,7 +2292,7 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
       DV_HIP(hipEventRecord(E.tev[b][0], st));
     }
     E.chunkCand[b] = ci;
-    if (resident) launchTeam<TM>(E, st);
+    if (resident) launchTeams<TM>(E, st, n == 1 ? kTeamPasses : kTeamPassesMany);
     else runChunk<TM>(E, st, timed ? ev : nullptr, prof);
     if (ci >= 0) DV_HIP(hipEventRecord(E.tev[b][1], st));
     DV_HIP(hipMemcpyAsync(buf[b], E.out.p, sizeof(ApgdState) * E.nSlots, hipMemcpyDeviceToHost, st));
@@ -2281,14 +2323,20 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
       profStats->prof_kernel_ms += ms;
       profStats->prof_kernel_count += prof == 4 ? 1 : kProfBurst;
     }
+    long passesNow = 0;
+    int passesMost = 0;
+    for (int i = 0; i < n; ++i) {
+      passesNow += last[i].passes;
+      passesMost = std::max(passesMost, last[i].passes);
+    }
     if (resident) {
-      E.launched = last[0].passes;
-      if (last[0].passes == passesBefore) {
+      E.launched = passesMost;
+      if (passesNow == passesBefore) {
         resident = false;
         E.teamSkip = kTeamSkip;
       }
     }
-    passesBefore = last[0].passes;
+    passesBefore = passesNow;
     int doneNow = 0;
     double rowsLeft = 0;
     for (int i = 0; i < n; ++i) {

@@ -36,6 +36,7 @@ constexpr int kTeamSync = 16 + kTeamMax;
 // A team whose members are not all running after this long gives up (the
 // 100 MHz wall clock): the slot's passes then run as launches.
 constexpr unsigned long long kFormTicks = 200000ull;         // 2 ms
+constexpr unsigned long long kFormTicksMany = 10000000ull;   // 100 ms: several scenes' teams wait for room
 // No wait of a formed team lasts this long; a member that sees it ends.
 constexpr unsigned long long kBarrierTicks = 1000000000ull;  // 10 s
 
@@ -145,12 +146,12 @@ __device__ __forceinline__ bool teamWait(const u64* flags, int W, u64 epoch, int
 // the first proposal of the launch holds for all.  Members wait for nothing
 // else before this, so a team that cannot be placed whole (other work holds
 // part of the chip) ends instead of waiting for ever.
-__device__ __forceinline__ bool teamForm(u64* sync, int rank, int W, u64 epoch, u64 launch, int* bad) {
+__device__ __forceinline__ bool teamForm(u64* sync, int rank, int W, u64 epoch, u64 launch, u64 ticks, int* bad) {
   __shared__ u64 outcome;
   if (W == 1) return true;
   u64* flags = sync + 16;
   if (threadIdx.x == 0) coStore(flags + rank, epoch);
-  const bool all = teamWait(flags, W, epoch, kFormTicks, bad);
+  const bool all = teamWait(flags, W, epoch, ticks, bad);
   if (threadIdx.x == 0) {
     u64 cur = coLoad(sync);
     while ((cur >> 1) != launch) {
@@ -278,7 +279,7 @@ __device__ __forceinline__ PassView uniformView(const PassView& s) {
 // per pass on 256,000 contacts, where two rows per thread take 17.8.
 template <typename TM, bool kBil, int R>
 __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, Tables T, const TeamItem* items,
-                                                u64* sync, u64 epoch, u64 launch, int passes) {
+                                                u64* sync, u64 epoch, u64 launch, int passes, u64 formTicks) {
   constexpr bool kMixed = sizeof(TM) < sizeof(double);
   constexpr int NF = kMixed ? 6 : 3;
   constexpr unsigned kUsed = kP1Slots<TM>;
@@ -286,7 +287,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
   constexpr int kWT = kTP / 64;      // of a heavy body's sum
   constexpr int kUnits = kTB / 64;   // body units of a body tile
   static_assert(kW == kSlots && kSlots == 8 && kUnits == 4, "a wavefront for each total; two loads to a body tile");
-  const TeamItem me = items ? items[blockIdx.x] : TeamItem{0, (int)blockIdx.x, (int)gridDim.x, 0};
+  const TeamItem me = items[blockIdx.x];
   const Args<TM>& a = A[me.slot];
   const SolveDims& D = a.dims;
   const int W = me.members, rank = me.rank, nTiles = a.nTiles;
@@ -323,7 +324,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
     drainStores();
     __syncthreads();
   }
-  if (!teamForm(sy, rank, W, epoch, launch, &bad)) return;
+  if (!teamForm(sy, rank, W, epoch, launch, formTicks, &bad)) return;
 
   // this thread's rows: row u of tile R rank + u
   struct Row {

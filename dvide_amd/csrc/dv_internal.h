@@ -151,7 +151,13 @@ struct Engine {
   DevBuf<char> views;   // PassView[nSlots][2]: what the pass kernels read of the states
   DevBuf<unsigned long long> teamSync;  // flags of the resident passes' teams, per slot
   unsigned long long teamEpoch = 0, teamLaunch = 0;
-  int teamSkip = 0;     // solves to run as launches (a team could not be placed)
+  DevBuf<char> teamItems;  // the active slots' teams, and their host copy
+  std::vector<char> hTeams;
+  int teamRows = 0;     // their row tiles per workgroup (0: some slot has no team)
+  bool teamBil = false; // some have bilateral rows
+  int teamSkip = 0;     // solves (or chunks) to run as launches: no team could be placed
+  bool ranResident = false;  // a server's last chunk
+  long polledPasses = 0;     // of its slots, when last polled
   void* outHost = nullptr;  // pinned copies of out: two halves, by chunk parity
   hipEvent_t polled[2] = {nullptr, nullptr};  // after each half's copy
   int outHostCap = 0;

@@ -68,3 +68,46 @@ def test_resident_passes_equal_the_launches(gpu, monkeypatch, name, build):
     assert out[0][0][0][0] > 0
     for a, b in zip(out[0][1:], out[1][1:]):
         assert bits_equal(a, b)
+
+
+def _launched(sc, build, steps):
+    g = system.from_scene(copy.deepcopy(sc), build, tol=1e-7, max_iterations=150)
+    g.setRowsPerThread(1)
+    for _ in range(steps):
+        g.step()
+    out = (g.stats().iterations, g.gamma, g.v, g.p)
+    g.close()
+    return out
+
+
+@pytest.mark.parametrize("how", ["batch", "server"])
+@pytest.mark.parametrize("names", [("ball", "layer_513", "pile_6000", "bilateral_lid", "free_lid"),
+                                   ("layer_63", "pile_6000", "box_58000", "shell", "box_58000", "layer_1025")])
+def test_teams_side_by_side_equal_the_launches(gpu, monkeypatch, names, how):
+    """Several scenes' teams in one launch (one row per thread, and with the
+    large scenes, which outnumber the chip's CUs, two): every member as its
+    launches alone leave it, whichever rows and neighbours it has."""
+    monkeypatch.setenv("DVIDE_TUNE", "0")
+    build, steps = system.BUILD_MIXED, 2
+    scs = [SCENES[n]() for n in names]
+    members = [system.from_scene(copy.deepcopy(sc), build, tol=1e-7, max_iterations=150) for sc in scs]
+    if how == "batch":
+        b = system.Batch(build)
+        for g in members:
+            b.add(g)
+        for _ in range(steps):
+            b.step()
+        b.close()
+    else:
+        srv = system.Server(build, max_slots=4)
+        for _ in range(steps):
+            for g in members:
+                srv.submit(g)
+            assert len(srv.drain()) == len(members)
+        srv.close()
+    for sc, g in zip(scs, members):
+        ref = _launched(sc, build, steps)
+        assert g.stats().iterations == ref[0]
+        for a, b in zip((g.gamma, g.v, g.p), ref[1:]):
+            assert bits_equal(a, b)
+        g.close()
