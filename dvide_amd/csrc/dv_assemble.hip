@@ -9,7 +9,7 @@
 // B's; D^T's rows: bilateral rows ascending, then contacts ascending with the
 // n, u, v rows in turn), and add them one by one from 0.0 without fused
 // multiply-adds, so they round exactly like the oracle's COO SpMV.
-#include "dv_internal.h"
+#include "dv_exact.h"
 
 namespace dv {
 namespace {
@@ -82,57 +82,39 @@ __global__ __launch_bounds__(kT) void kRowsD(RowArgs a, const double* __restrict
   }
 }
 
-struct GatherArgs {
-  int nb, nbil, cap;
-  const double* frame;
-  const int* iStart;
-  const int* inc;
-  const int* bilIncStart;
-  const int* bilInc;
-  const double* minv;
-};
-
 // f = D^T x and tmp = M^-1 f per body, terms in D^T row order.  With
-// skipFixed, bodies with M^-1 = 0 get tmp = +0 without the sum (0.0 + 0*f).
-__global__ __launch_bounds__(kT) void kGatherDT(GatherArgs a, const double* __restrict__ x,
-                                                double* __restrict__ fOut, double* __restrict__ tmpOut,
-                                                int skipFixed, int skipHeavy) {
-  int g = blockIdx.x * blockDim.x + threadIdx.x;
-  if (g >= a.nb) return;
-  if (skipHeavy && a.iStart[g + 1] - a.iStart[g] > kHeavyDegree) return;
+// skipFixed, bodies with M^-1 = 0 get tmp = +0 without the sum (0.0 + 0*f);
+// with skipHeavy, the heavy bodies are left to kGatherHeavy.
+__global__ __launch_bounds__(kGatherT) void kGatherDT(GatherArgs a, const double* __restrict__ x,
+                                                      double* __restrict__ fOut, double* __restrict__ tmpOut,
+                                                      int skipFixed, int skipHeavy, int lightBlocks) {
+  __shared__ double sh[64][9];
+  auto row = [&](long r) { return x[r]; };
+  if ((int)blockIdx.x >= lightBlocks) {
+    for (int h = blockIdx.x - lightBlocks; !skipHeavy && h < a.counters[2]; h += kHeavyBlocks) {
+      const int g = a.heavy[h], q = threadIdx.x;
+      const double mi = a.minv[g];
+      const bool fixed = skipFixed && mi == 0;
+      const double s = fixed ? 0.0 : gatherHeavy(a, g, row, sh);
+      if (q >= 3) continue;
+      if (fOut && !fixed) fOut[3 * g + q] = s;
+      if (tmpOut) {
+        double t = 0.0;
+        if (!fixed) t = t + mi * s;
+        tmpOut[3 * g + q] = t;
+      }
+    }
+    return;
+  }
+  const int g = blockIdx.x * kGatherT + threadIdx.x;
+  if (g >= a.nb || a.iStart[g + 1] - a.iStart[g] > kHeavyDegree) return;
   const double mi = a.minv[g];
   if (skipFixed && mi == 0) {
     tmpOut[3 * g] = 0.0; tmpOut[3 * g + 1] = 0.0; tmpOut[3 * g + 2] = 0.0;
     return;
   }
-  double s0 = 0.0, s1 = 0.0, s2 = 0.0;
-  for (int k = a.bilIncStart[g]; k < a.bilIncStart[g + 1]; ++k) {
-    const int e = a.bilInc[k];
-    const int row = e >> 3, comp = (e >> 1) & 3;
-    const double val = (e & 1) ? -1.0 : 1.0;
-    const double t = val * x[row];
-    if (comp == 0) s0 = s0 + t;
-    else if (comp == 1) s1 = s1 + t;
-    else s2 = s2 + t;
-  }
-  const long S = a.cap;
-  for (int k = a.iStart[g]; k < a.iStart[g + 1]; ++k) {
-    const int e = a.inc[k];
-    const int c = e >> 1;
-    const bool sideB = e & 1;
-    const long base = a.nbil + 3L * c;
-#pragma unroll
-    for (int rr = 0; rr < 3; ++rr) {
-      const double xr = x[base + rr];
-      double v0 = a.frame[(3 * rr + 0) * S + c];
-      double v1 = a.frame[(3 * rr + 1) * S + c];
-      double v2 = a.frame[(3 * rr + 2) * S + c];
-      if (sideB) { v0 = -v0; v1 = -v1; v2 = -v2; }
-      s0 = s0 + v0 * xr;
-      s1 = s1 + v1 * xr;
-      s2 = s2 + v2 * xr;
-    }
-  }
+  double s0, s1, s2;
+  gatherSums(a, g, row, s0, s1, s2);
   if (fOut) { fOut[3 * g] = s0; fOut[3 * g + 1] = s1; fOut[3 * g + 2] = s2; }
   if (tmpOut) {
     double t0 = 0.0, t1 = 0.0, t2 = 0.0;
@@ -251,14 +233,6 @@ RowArgs rowArgs(Scene& s) {
   return a;
 }
 
-GatherArgs gatherArgs(Scene& s) {
-  GatherArgs a;
-  a.nb = s.nb; a.nbil = s.nbil; a.cap = s.ncCap;
-  a.frame = s.frame.p; a.iStart = s.iStart.p; a.inc = s.inc.p;
-  a.bilIncStart = s.bilIncStart.p; a.bilInc = s.bilInc.p; a.minv = s.minv.p;
-  return a;
-}
-
 }  // namespace
 
 void fillDevice(Scene& s, double* x, long n, double v) {
@@ -295,9 +269,10 @@ void buildR(Scene& s) {
                      (const double*)s.b.p, s.r.p);
 }
 
-void gatherExact(Scene& s, const double* x, double* fOut, double* tmpOut, bool skipFixed) {
-  hipLaunchKernelGGL(kGatherDT, dim3(blocksFor(s.nb, kT)), dim3(kT), 0, s.stream, gatherArgs(s), x, fOut, tmpOut,
-                     skipFixed ? 1 : 0, 0);
+static void gatherExact(Scene& s, const double* x, double* fOut, double* tmpOut, bool skipFixed) {
+  const GatherArgs a = gatherArgs(s);
+  hipLaunchKernelGGL(kGatherDT, dim3(gatherBlocks(a) + kHeavyBlocks), dim3(kGatherT), 0, s.stream, a, x, fOut, tmpOut,
+                     skipFixed ? 1 : 0, 0, gatherBlocks(a));
 }
 
 // y = D (M^-1 (D^T x))  (APGD.cu:81-87)
@@ -307,10 +282,6 @@ void schurExact(Scene& s, const double* x, double* y) {
   if (items)
     hipLaunchKernelGGL(kRowsD, dim3(blocksFor(items, kT)), dim3(kT), 0, s.stream, rowArgs(s), (const double*)s.tmp.p,
                        (const double*)nullptr, y);
-}
-
-void minvTimes(Scene& s, const double* x, double* y) {
-  if (s.nb) hipLaunchKernelGGL(kMinv, dim3(blocksFor(3L * s.nb, kT)), dim3(kT), 0, s.stream, s.nb, s.minv.p, x, y);
 }
 
 void rowsD(Scene& s, const double* x, const double* badd, double* y) {
@@ -324,9 +295,10 @@ void updateState(Scene& s, bool haveRows, bool exactOrder) {
     if (exactOrder) {
       gatherExact(s, s.gamma.p, s.fContact.p, nullptr, false);
     } else {
-      hipLaunchKernelGGL(kGatherDT, dim3(blocksFor(s.nb, kT)), dim3(kT), 0, s.stream, gatherArgs(s),
-                         (const double*)s.gamma.p, s.fContact.p, (double*)nullptr, 0, 1);
-      hipLaunchKernelGGL(kGatherHeavy, dim3(64), dim3(kT), 0, s.stream, gatherArgs(s), (const int*)s.heavy.p,
+      const GatherArgs a = gatherArgs(s);
+      hipLaunchKernelGGL(kGatherDT, dim3(gatherBlocks(a)), dim3(kGatherT), 0, s.stream, a,
+                         (const double*)s.gamma.p, s.fContact.p, (double*)nullptr, 0, 1, gatherBlocks(a));
+      hipLaunchKernelGGL(kGatherHeavy, dim3(64), dim3(kT), 0, s.stream, a, (const int*)s.heavy.p,
                          (const int*)s.counters.p, (const double*)s.gamma.p, s.fContact.p);
     }
   }

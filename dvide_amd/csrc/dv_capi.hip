@@ -309,6 +309,9 @@ int dv_scene_destroy(dv_scene* h) {
   s.slotOf.release(); s.slotCount.release(); s.slotStart.release();
   s.frame32.release(); s.work32.release();
   s.engine.release();
+  s.plainGraph.reset();
+  s.plainState.release();
+  if (s.plainHost) (void)hipHostFree(s.plainHost);
   s.workM64.release();
   if (s.pinned) (void)hipHostFree(s.pinned);
   for (auto& e : s.ev)

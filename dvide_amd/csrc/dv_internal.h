@@ -259,10 +259,13 @@ struct Scene {
   DevBuf<float> work32;  // products and matrix data of the mixed solver
   DevBuf<double> partials;
   Engine engine;               // the graph-driven solver of this scene alone
+  DevBuf<char> plainState;     // the plain solver's arguments and state
+  void* plainHost = nullptr;   // pinned: two copies of the state, the arguments
+  GraphCache plainGraph;       // its captured chunk of passes
 
   // --- statistics of the last step
   dv_stats stats{};
-  hipEvent_t ev[6] = {};
+  hipEvent_t ev[7] = {};  // [0..4] phases of a step, [5], [6] the plain solver's chunks
 };
 
 // collision detection + incidence lists (dv_collide.hip)
@@ -286,11 +289,9 @@ void buildK(Scene& s);
 void buildR(Scene& s);
 void updateState(Scene& s, bool haveRows, bool exactOrder);
 void schurExact(Scene& s, const double* x, double* y);  // device pointers, flat R
-void gatherExact(Scene& s, const double* x, double* fOut, double* tmpOut, bool skipFixed);
 void ensureRowBuffers(Scene& s);
 void fillDevice(Scene& s, double* x, long n, double v);
 void rowsD(Scene& s, const double* x, const double* badd, double* y);
-void minvTimes(Scene& s, const double* x, double* y);  // y = M^-1 x per DOF
 
 // solvers (dv_apgd_plain.hip, dv_apgd_fused.hip)
 void solvePlain(Scene& s);

@@ -50,8 +50,8 @@ typedef struct dv_scene dv_scene;
 /* APGD builds (DV_PARAM_APGD_BUILD); each runs APGD::solve (APGD.cu:164-361) */
 #define DV_APGD_FP64 0  /* device-resident state machine in hipGraph chunks, FP64 (default) */
 #define DV_APGD_MIXED 1 /* same, FP32 D/M^-1/products, FP64 iterates, tests and update */
-#define DV_APGD_PLAIN 2 /* host-driven FP64, one kernel per CUSP operation; the build
-                           that runs anti-relaxation */
+#define DV_APGD_PLAIN 2 /* FP64, every operation rounded as the reference's CUSP calls
+                           round it; the build that runs anti-relaxation */
 
 /* double parameters (dv_set_param / dv_get_param) */
 #define DV_PARAM_H 0          /* time step              System::setTimeStep, System.cu:135 */
