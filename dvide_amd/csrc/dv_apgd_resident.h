@@ -379,6 +379,14 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
   const BodyRuns<TM> first = bodyRuns(a, u0 < nU ? (long)u0 * 64 + lane : (long)D.nb);
 #pragma unroll
   for (int k = 0; k < kRun; ++k) shIds[k][tid] = contactOf(a, first, k);
+  // (the launches read the D^T gamma ring of fixed bodies too, times zero)
+  if (kMixed)
+    for (int u = u0; u < nU; u += W * kW) {
+      const int g = u * 64 + lane;
+      if (g < D.nb && gl(a.minv)[g] == (TM)0)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) st4(a.sr, (long)k * D.nb + g, V4<TM>{0, 0, 0, 0});
+    }
   unsigned live = 0;
   for (int j = 0, u = u0; u < nU; ++j, u += W * kW) {
     if (__any(bodyRuns(a, (long)u * 64 + lane).sums)) live |= 1u << j;
