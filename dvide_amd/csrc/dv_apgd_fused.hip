@@ -539,10 +539,29 @@ __device__ __forceinline__ void zero(double (&acc)[kSlots]) {
 }
 
 // loop of a workgroup over the row tiles (uniform across the workgroup)
-#define TILE_LOOP(T) \
-  for (int ti_ = tilesOf(T, (T).counts[0], gridDim.x).first, te_ = tilesOf(T, (T).counts[0], gridDim.x).end, \
-           ts_ = tilesOf(T, (T).counts[0], gridDim.x).step;                                                 \
+#define TILE_LOOP(T, n) \
+  for (int ti_ = tilesOf(T, n, gridDim.x).first, te_ = tilesOf(T, n, gridDim.x).end, \
+           ts_ = tilesOf(T, n, gridDim.x).step;                                      \
        ti_ < te_; ti_ += ts_)
+
+// What the launch tables hold for several slots, a single slot's table entry
+// says as well: its solves build and upload none.  That took about twenty
+// small copies and three kernels out of a solve, and with the finalisation
+// queued behind the passes one of its waits: a solve of 2 passes went from
+// 158 us to 71 us, of 6 passes on 1000 spheres from 188 us to 106 us.
+template <typename TM>
+__device__ __forceinline__ int rowTiles(const Args<TM>* A, const Tables& T) {
+  return T.single ? A[0].nTiles : T.counts[0];
+}
+template <typename TM>
+__device__ __forceinline__ int heavyCount(const Args<TM>* A, const Tables& T) {
+  return T.single ? gl(A[0].counters)[2] : T.counts[2];
+}
+template <typename TM>
+__device__ __forceinline__ int2 heavyRef(const Args<TM>* A, const Tables& T, int k) {
+  return T.single ? make_int2(0, gl(A[0].heavy)[k]) : T.heavy[k];
+}
+__device__ __forceinline__ int slotOf(const Tables& T) { return T.single ? 0 : T.slots[blockIdx.x]; }
 
 __device__ __forceinline__ Tile rowTile(const Tables& T, int k) {
   return T.single ? Tile{0, k * kTC} : T.items[k];
@@ -589,7 +608,7 @@ __device__ __forceinline__ TileRange tilesOf(const Tables& T, int nt, int nw) {
 template <typename TM>
 __global__ __launch_bounds__(kTC) void kSetup1(const Args<TM>* __restrict__ A, Tables T) {
   constexpr bool kMixed = sizeof(TM) < sizeof(double);
-  TILE_LOOP(T) {
+  TILE_LOOP(T, rowTiles(A, T)) {
     const Tile tile = rowTile(T, ti_);
     const Args<TM>& a = A[tile.scene];
     const SolveDims& D = a.dims;
@@ -762,8 +781,8 @@ __global__ __launch_bounds__(kTB) void kBody(const Args<TM>* __restrict__ A, Tab
   if (T.single) {  // as in kP1
     const PassView S = loadView(T, 0, sIdx);
     const Args<TM>& a = A[0];
-    const int nt = T.counts[1];
-    if (!(which == 2 && viewDone(S))) {
+    const int nt = a.nBodyTiles;
+    if (!(which == 2 ? viewDone(S) : which == 3 && !viewDone(S))) {
       const TileRange tr = tilesOf(T, nt, nw);
       for (int ti = tr.first; ti < tr.end; ti += tr.step) tileBody(Tile{0, ti * kTB}, S, a);
     }
@@ -772,19 +791,19 @@ __global__ __launch_bounds__(kTB) void kBody(const Args<TM>* __restrict__ A, Tab
     for (int ti = tr.first; ti < tr.end; ti += tr.step) {
       const Tile tile = bodyTile(T, ti);
       const PassView S = loadView(T, tile.scene, sIdx);
-      if (which == 2 && viewDone(S)) continue;
+      if (which == 2 ? viewDone(S) : which == 3 && !viewDone(S)) continue;
       tileBody(tile, S, A[tile.scene]);
     }
   }
-  for (int hq = blockIdx.x, nh = T.counts[2]; hq < nh; hq += nw) {
-    const int2 ref = T.heavy[hq];
+  for (int hq = blockIdx.x, nh = heavyCount(A, T); hq < nh; hq += nw) {
+    const int2 ref = heavyRef(A, T, hq);
     const PassView S = loadView(T, ref.x, sIdx);
-    if (which == 2 && viewDone(S)) continue;
+    if (which == 2 ? viewDone(S) : which == 3 && !viewDone(S)) continue;
     const Args<TM>& a = A[ref.x];
     const int g = ref.y;
     const TM mi = bodyMinv(a, g, which);
     // this body's slot among the Lipschitz partials, after the body tiles'
-    double* lqSlot = which == 2 ? a.lq[sIdx ^ 1] + a.nBodyTiles + T.heavyIdx[hq] : nullptr;
+    double* lqSlot = which == 2 ? a.lq[sIdx ^ 1] + a.nBodyTiles + (T.single ? hq : T.heavyIdx[hq]) : nullptr;
     if (mi == (TM)0) {
       if (threadIdx.x == 0) {
         V4<TM> out;
@@ -837,7 +856,7 @@ __global__ __launch_bounds__(kTB) void kBody(const Args<TM>* __restrict__ A, Tab
 // |N d|^2 into part3[1]; J = F^T gamma_0
 template <typename TM>
 __global__ __launch_bounds__(kTC) void kSetup3(const Args<TM>* __restrict__ A, Tables T) {
-  TILE_LOOP(T) {
+  TILE_LOOP(T, rowTiles(A, T)) {
     const Tile tile = rowTile(T, ti_);
     const Args<TM>& a = A[tile.scene];
     const SolveDims& D = a.dims;
@@ -866,7 +885,7 @@ __global__ __launch_bounds__(kTC) void kSetup3(const Args<TM>* __restrict__ A, T
 // N gamma_0 into rn[0]
 template <typename TM>
 __global__ __launch_bounds__(kTC) void kSetup5(const Args<TM>* __restrict__ A, Tables T) {
-  TILE_LOOP(T) {
+  TILE_LOOP(T, rowTiles(A, T)) {
     const Tile tile = rowTile(T, ti_);
     const Args<TM>& a = A[tile.scene];
     const SolveDims& D = a.dims;
@@ -890,7 +909,7 @@ __global__ __launch_bounds__(kTC) void kSetup5(const Args<TM>* __restrict__ A, T
 // written to both parity slots; one wavefront per scene
 template <typename TM>
 __global__ __launch_bounds__(kTD) void kSetupDecide(const Args<TM>* __restrict__ A, Tables T) {
-  const int slot = T.slots[blockIdx.x];
+  const int slot = slotOf(T);
   const Args<TM>& a = A[slot];
   double tot[2 * kSlots];
   reduceAll(a.part1[0], a.part3[0], a.nTiles, tot);
@@ -1287,7 +1306,7 @@ __global__ __launch_bounds__(kTC / R, (kP1MinWaves<TM, R>)) void kP1(const Args<
     tileBody(tile, S, a, ia, ib, tA, tB, pr);
     return;
   }
-  TILE_LOOP(T) {
+  TILE_LOOP(T, rowTiles(A, T)) {
     const Tile tile = rowTile(T, ti_);
     const PassView S = loadView(T, tile.scene, par ^ 1);
     if (viewDone(S)) continue;
@@ -1363,16 +1382,18 @@ __global__ __launch_bounds__(kTP) void kDecide(const Args<TM>* __restrict__ A, T
 
 // ---------------------------------------------------------------------------
 // gamma := gammaHat (APGD.cu:358) and objectiveCCP (APGD.cu:353-354); the
-// final state is st[fin]
+// final state is st[fin].  A slot whose solve has not ended is left alone: a
+// resident solve queues these behind its passes, before it knows.
 
 template <typename TM>
 __global__ __launch_bounds__(kTC) void kFin1(const Args<TM>* __restrict__ A, Tables T, int fin) {
-  TILE_LOOP(T) {
+  TILE_LOOP(T, rowTiles(A, T)) {
     const Tile tile = rowTile(T, ti_);
     const Args<TM>& a = A[tile.scene];
     const SolveDims& D = a.dims;
     const long items = (long)D.nc + D.nbil;
     const long q = (long)tile.start + threadIdx.x;
+    if (!STATE(T, tile.scene, fin).done) continue;
     const int hatSrc = STATE(T, tile.scene, fin).hatSrc;
     const DV_GLOBAL double* hatV = gl(hatSrc >= 0 ? a.ring[hatSrc] : a.gHat);
     double acc[kSlots];
@@ -1400,9 +1421,10 @@ __global__ __launch_bounds__(kTC) void kFin1(const Args<TM>* __restrict__ A, Tab
 }
 
 template <typename TM>
-__global__ __launch_bounds__(kTC) void kFin3(const Args<TM>* __restrict__ A, Tables T) {
-  TILE_LOOP(T) {
+__global__ __launch_bounds__(kTC) void kFin3(const Args<TM>* __restrict__ A, Tables T, int fin) {
+  TILE_LOOP(T, rowTiles(A, T)) {
     const Tile tile = rowTile(T, ti_);
+    if (!STATE(T, tile.scene, fin).done) continue;
     const Args<TM>& a = A[tile.scene];
     const SolveDims& D = a.dims;
     const long items = (long)D.nc + D.nbil;
@@ -1428,7 +1450,8 @@ __global__ __launch_bounds__(kTC) void kFin3(const Args<TM>* __restrict__ A, Tab
 
 template <typename TM>
 __global__ __launch_bounds__(kTD) void kFinDecide(const Args<TM>* __restrict__ A, Tables T, int fin) {
-  const int slot = T.slots[blockIdx.x];
+  const int slot = slotOf(T);
+  if (!STATE(T, slot, fin).done) return;
   const Args<TM>& a = A[slot];
   double tot[2 * kSlots];
   reduceAll(a.part1[0], a.part3[0], a.nTiles, tot);
@@ -1893,9 +1916,11 @@ Args<TM>& slotArgs(Engine& E, int slot) {
 }
 
 // Tiles of the slots in set.hSlots, uploaded with the device slot list and
-// the heavy-body table (built on the device from the slots' counters).
+// the heavy-body table (built on the device from the slots' counters); a
+// single slot needs none of it.
 template <typename TM>
 void buildSet(Engine& E, TileSet& set, hipStream_t st) {
+  if (E.nSlots == 1) return;
   set.hItems.clear();
   set.hBodies.clear();
   long heavyCap = 1;
@@ -2020,7 +2045,7 @@ void buildTeams(Engine& E, hipStream_t st) {
     E.teamBil = E.teamBil || a.dims.nbil > 0;
   }
   E.hTeams.assign(reinterpret_cast<const char*>(items.data()), reinterpret_cast<const char*>(items.data() + items.size()));
-  if (!E.teamRows) return;
+  if (!E.teamRows || E.nSlots == 1) return;  // (a single slot's workgroups know their places)
   E.teamItems.reserve(E.hTeams.size());
   DV_HIP(hipMemcpyAsync(E.teamItems.p, E.hTeams.data(), E.hTeams.size(), hipMemcpyHostToDevice, st));
 }
@@ -2036,7 +2061,7 @@ void launchTeams(Engine& E, hipStream_t st, int passes) {
                                 : (E.teamRows == 1 ? kTeam<TM, false, 1> : kTeam<TM, false, 2>);
   hipLaunchKernelGGL(kernel, dim3((unsigned)(E.hTeams.size() / sizeof(TeamItem))), dim3(kTC), 0, st,
                      reinterpret_cast<const Args<TM>*>(E.table.p), T,
-                     reinterpret_cast<const TeamItem*>(E.teamItems.p), E.teamSync.p, E.teamEpoch + 1, ++E.teamLaunch,
+                     E.nSlots == 1 ? nullptr : reinterpret_cast<const TeamItem*>(E.teamItems.p), E.teamSync.p, E.teamEpoch + 1, ++E.teamLaunch,
                      passes, E.nSlots == 1 ? kFormTicks : kFormTicksMany);
   DV_HIP(hipGetLastError());
   E.teamEpoch += 2 * (unsigned long long)passes + 2;
@@ -2102,10 +2127,9 @@ void runChunk(Engine& E, hipStream_t st, hipEvent_t* ev, int prof) {
   E.launched += kPassesPerChunk;
 }
 
-// gamma := gammaHat and the objective for the slots, then their statistics
+// gamma := gammaHat and the objective of the slots whose solves have ended
 template <typename TM>
-void retireSlots(Engine& E, const std::vector<int>& slots, hipStream_t st) {
-  if (slots.empty()) return;
+void finishSlots(Engine& E, const std::vector<int>& slots, hipStream_t st) {
   E.retire.hSlots = slots;
   buildSet<TM>(E, E.retire, st);
   const Args<TM>* A = reinterpret_cast<const Args<TM>*>(E.table.p);
@@ -2114,12 +2138,14 @@ void retireSlots(Engine& E, const std::vector<int>& slots, hipStream_t st) {
   grids<TM>(E, E.retire, gc, gb);
   const int fin = 1;  // a chunk's last pass (parity 1) decides into st[1]
   hipLaunchKernelGGL(kFin1<TM>, dim3(gc), dim3(kTC), 0, st, A, T, fin);
-  hipLaunchKernelGGL((kBody<TM, 3>), dim3(gb), dim3(kTB), 0, st, A, T, 0);
-  hipLaunchKernelGGL(kFin3<TM>, dim3(gc), dim3(kTC), 0, st, A, T);
+  hipLaunchKernelGGL((kBody<TM, 3>), dim3(gb), dim3(kTB), 0, st, A, T, fin);
+  hipLaunchKernelGGL(kFin3<TM>, dim3(gc), dim3(kTC), 0, st, A, T, fin);
   hipLaunchKernelGGL(kFinDecide<TM>, dim3((int)slots.size()), dim3(kTD), 0, st, A, T, fin);
-  ApgdState* outH = reinterpret_cast<ApgdState*>(E.outHost);
-  DV_HIP(hipMemcpyAsync(outH, E.out.p, sizeof(ApgdState) * E.nSlots, hipMemcpyDeviceToHost, st));
-  DV_HIP(hipStreamSynchronize(st));
+}
+
+// the statistics of finished slots, from their states read back
+template <typename TM>
+void recordSlots(Engine& E, const std::vector<int>& slots, const ApgdState* outH) {
   for (int slot : slots) {
     Scene& s = *E.slotScene[slot];
     const ApgdState& S = outH[slot];
@@ -2137,6 +2163,17 @@ void retireSlots(Engine& E, const std::vector<int>& slots, hipStream_t st) {
     slotArgs<TM>(E, slot).active = 0;
     E.slotScene[slot] = nullptr;
   }
+}
+
+template <typename TM>
+void retireSlots(Engine& E, const std::vector<int>& slots, hipStream_t st) {
+  if (slots.empty()) return;
+  finishSlots<TM>(E, slots, st);
+  ApgdState* outH = reinterpret_cast<ApgdState*>(E.outHost);
+  DV_HIP(hipMemcpyAsync(outH, E.out.p, sizeof(ApgdState) * E.nSlots, hipMemcpyDeviceToHost, st));
+  DV_HIP(hipStreamSynchronize(st));
+  recordSlots<TM>(E, slots, outH);
+  if (E.nSlots == 1) return;  // (the next solve opens the engine anew)
   uploadTable<TM>(E, st);
   rebuildActive<TM>(E, st);
 }
@@ -2284,6 +2321,7 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
   // a chunk, then the copy of the states after it into buf[b]; while the
   // class is being measured, the chunk runs the next unmeasured candidate
   // schedule between two timing events
+  bool ranResident[2] = {false, false};
   auto launch = [&](int b, bool timed) {
     const int ci = tc ? nextCandidate(*tc, E.chunkCand[b ^ 1]) : -1;
     if (ci >= 0) {
@@ -2292,8 +2330,13 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
       DV_HIP(hipEventRecord(E.tev[b][0], st));
     }
     E.chunkCand[b] = ci;
-    if (resident) launchTeams<TM>(E, st, n == 1 ? kTeamPasses : kTeamPassesMany);
-    else runChunk<TM>(E, st, timed ? ev : nullptr, prof);
+    if (resident) {
+      launchTeams<TM>(E, st, n == 1 ? kTeamPasses : kTeamPassesMany);
+      if (n == 1) finishSlots<TM>(E, {0}, st);  // (nothing is done unless the solve has ended)
+    } else {
+      runChunk<TM>(E, st, timed ? ev : nullptr, prof);
+    }
+    ranResident[b] = resident;
     if (ci >= 0) DV_HIP(hipEventRecord(E.tev[b][1], st));
     DV_HIP(hipMemcpyAsync(buf[b], E.out.p, sizeof(ApgdState) * E.nSlots, hipMemcpyDeviceToHost, st));
     DV_HIP(hipEventRecord(E.polled[b], st));
@@ -2329,20 +2372,20 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
       passesNow += last[i].passes;
       passesMost = std::max(passesMost, last[i].passes);
     }
-    if (resident) {
-      E.launched = passesMost;
-      if (passesNow == passesBefore) {
-        resident = false;
-        E.teamSkip = kTeamSkip;
-      }
-    }
-    passesBefore = passesNow;
     int doneNow = 0;
     double rowsLeft = 0;
     for (int i = 0; i < n; ++i) {
       if (last[i].done) ++doneNow;
       else rowsLeft += (double)slotRows[i];
     }
+    if (ranResident[cur]) {
+      E.launched = passesMost;
+      if (passesNow == passesBefore && doneNow < n) {
+        resident = false;
+        E.teamSkip = kTeamSkip;
+      }
+    }
+    passesBefore = passesNow;
     if (tc && E.chunkCand[cur] >= 0 && doneNow == doneBefore && doneNow < n) {
       float ms = 0;
       DV_HIP(hipEventElapsedTime(&ms, E.tev[cur][0], E.tev[cur][1]));
@@ -2353,6 +2396,10 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
     activeRows = rowsLeft;
     if (doneNow == n) {
       if (tc) endMeasuredSolve(E, *tc);
+      if (n == 1 && ranResident[cur]) {
+        recordSlots<TM>(E, {0}, last);
+        return;
+      }
       break;
     }
     // Once a quarter of the slots have finished since the last retirement,

@@ -287,7 +287,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
   constexpr int kWT = kTP / 64;      // of a heavy body's sum
   constexpr int kUnits = kTB / 64;   // body units of a body tile
   static_assert(kW == kSlots && kSlots == 8 && kUnits == 4, "a wavefront for each total; two loads to a body tile");
-  const TeamItem me = items[blockIdx.x];
+  const TeamItem me = items ? items[blockIdx.x] : TeamItem{0, (int)blockIdx.x, (int)gridDim.x, 0};
   const Args<TM>& a = A[me.slot];
   const SolveDims& D = a.dims;
   const int W = me.members, rank = me.rank, nTiles = a.nTiles;
