@@ -180,14 +180,15 @@ struct Args {
   V4<TM>* JB;           // the same, in B-side order: body b's B incidences are
                         // [iStart[b] - cStart[b], iStart[b+1] - cStart[b+1])
   V4<TM>* tmp;
-  V4<TM>* tmpSplit;     // FP64 resident passes: tmp as they exchange it
+  V4<TM>* tmpX;         // resident passes: tmp as they exchange it (J in its own memory, and JB's)
   V4<TM>* sr;           // mixed solver: D^T of each ring slot's iterate, per body (slot k at k * nb)
   double* gHat;         // gammaHat before any iterate is accepted (ones)
   double* part1[2];     // kSlots per tile, by pass parity
   double* part3[2];     // setup and final kernels: a second kSlots per tile
   double* lq[2];        // P2's Lipschitz partials, by pass parity: one per body tile, then one
                         // per heavy body (in the heavy list's order)
-  double* lqw[2];       // resident passes: the Lipschitz sums per 64 bodies, by pass parity
+  double* partX;        // resident passes, for either pass parity: P1's partial sums as exchanged,
+  double* lqX;          // and the Lipschitz sums per body tile, then per heavy body
   double* p1sum[2];     // single slot: P1's slots totalled by P2's last workgroup
   int nBodyTiles;       // body tiles of the scene (kTB bodies each)
 };
@@ -242,8 +243,8 @@ __device__ __forceinline__ bool viewDone(const PassView& S) {
 template <int kCtrl>
 __device__ __forceinline__ double dppMove(double v) {
   const long long b = __builtin_bit_cast(long long, v);
-  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, kCtrl, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), kCtrl, 0xF, 0xF, true);
+  const int lo = __builtin_amdgcn_mov_dpp((int)b, kCtrl, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp((int)(b >> 32), kCtrl, 0xF, 0xF, true);
   return __builtin_bit_cast(double, ((long long)hi << 32) | (unsigned)lo);
 }
 __device__ __forceinline__ double laneValue(double v, int lane) {
@@ -675,20 +676,29 @@ __device__ __forceinline__ TM bodyMinv(const Args<TM>& a, int g, int which, bool
 // Delta = gamma_new - y.  The mixed solver keeps s in ring slot nxt.
 template <typename TM>
 __device__ __forceinline__ double lipschitzTerm(const Args<TM>& a, int g, const PassView& S, TM mi, TM s0, TM s1,
-                                                TM s2) {
+                                                TM s2, const V4<TM>& c, const V4<TM>& p) {
   constexpr bool kMixed = sizeof(TM) < sizeof(double);
   if (!kMixed) return (double)s0 * (double)(mi * s0) + (double)s1 * (double)(mi * s1) + (double)s2 * (double)(mi * s2);
-  const long nb = a.dims.nb;
-  const V4<TM> c = ld4(a.sr, S.cur * nb + g), p = ld4(a.sr, S.prev * nb + g);
   V4<TM> sn;
   sn.x = s0; sn.y = s1; sn.z = s2; sn.w = 0;
-  st4(a.sr, S.nxt * nb + g, sn);
+  st4(a.sr, S.nxt * (long)a.dims.nb + g, sn);
   const bool mom = !(S.flags & kViewRestart);
   const double bp = 1.0 + S.beta, bm = -S.beta;
   const double d0 = (double)s0 - (mom ? bp * (double)c.x + bm * (double)p.x : (double)c.x);
   const double d1 = (double)s1 - (mom ? bp * (double)c.y + bm * (double)p.y : (double)c.y);
   const double d2 = (double)s2 - (mom ? bp * (double)c.z + bm * (double)p.z : (double)c.z);
   return (double)mi * (d0 * d0 + d1 * d1 + d2 * d2);
+}
+template <typename TM>
+__device__ __forceinline__ double lipschitzTerm(const Args<TM>& a, int g, const PassView& S, TM mi, TM s0, TM s1,
+                                                TM s2) {
+  constexpr bool kMixed = sizeof(TM) < sizeof(double);
+  V4<TM> c, p;
+  if (kMixed) {  // D^T gamma_k and D^T gamma_{k-1}
+    c = ld4(a.sr, S.cur * (long)a.dims.nb + g);
+    p = ld4(a.sr, S.prev * (long)a.dims.nb + g);
+  }
+  return lipschitzTerm(a, g, S, mi, s0, s1, s2, c, p);
 }
 
 template <typename TM, int which>
@@ -946,6 +956,7 @@ __global__ __launch_bounds__(kTD) void kSetupDecide(const Args<TM>* __restrict__
 struct LazyNext {
   double L, theta;
   __device__ explicit LazyNext(const ApgdState& S) : L(S.L), theta(S.theta) {}
+  __device__ LazyNext(double L, double theta) : L(L), theta(theta) {}
   __device__ double backL() const { return 2.0 * L; }
   __device__ double backT(double Lb) const { return 1.0 / Lb; }
   __device__ double nextL() const { return 0.9 * L; }
@@ -1843,15 +1854,15 @@ void prepareScene(Scene& s, Args<TM>& a) {
   const long tilesCap = std::max<long>(1, (itemsCap + kTC - 1) / kTC);
   const long bodyTiles = std::max<long>(1, ((long)s.nb + kTB - 1) / kTB);
   // a body reduced by a workgroup has more than kHeavyDegree of the 2 nc incidences
-  const long lqCap = bodyTiles + 2L * std::max(s.ncCap, 1) / kHeavyDegree + 2;
-  const long lqwCap = bodyTiles * (kTB / 64);
-  s.partials.reserve((size_t)4 * kSlots * tilesCap + 2 * kSlots + 2 * lqCap + 2 * lqwCap);
+  const long lqCap = (bodyTiles + 2L * std::max(s.ncCap, 1) / kHeavyDegree + 2) / 2 * 2;
+  s.partials.reserve((size_t)(4 + 4) * kSlots * tilesCap + 2 * kSlots + (2 + 4) * lqCap);  // (exchanged: 16 bytes)
   s.work.reserve((size_t)5 * RsCap + 16);  // ring[4], gHat: FP64 in both solvers
-  // TM block: rn[4], r, then J and JB (per contact), tmp and (mixed) the
-  // four ring slots of D^T gamma (per body) of 4 components 32-byte aligned,
-  // then (mixed) M^-1
+  // TM block: rn[4], r, then J and JB (per contact; J as the resident passes
+  // exchange it takes the bilateral rows too), tmp, tmp exchanged and (mixed)
+  // the four ring slots of D^T gamma (per body) of 4 components 32-byte
+  // aligned, then (mixed) M^-1
   const size_t nbc = (size_t)std::max(s.nb, 1);
-  const size_t tmElems = (size_t)5 * RsCap + 8 + 4 * (2 * (size_t)std::max(s.ncCap, 1) + nbc + (kMixed ? 4 : 1) * nbc) +
+  const size_t tmElems = (size_t)5 * RsCap + 8 + 4 * (2 * (size_t)std::max(s.ncCap, 1) + s.nbil + 2 * nbc + (kMixed ? 4 : 0) * nbc) +
                          (kMixed ? nbc + 1 : 0) + 16;
   TM* WM;
   if (kMixed) {
@@ -1891,13 +1902,13 @@ void prepareScene(Scene& s, Args<TM>& a) {
   uintptr_t p = (reinterpret_cast<uintptr_t>(after) + 31) & ~uintptr_t(31);
   a.J = reinterpret_cast<V4<TM>*>(p);
   a.JB = a.J + std::max<long>(s.ncCap, 1);
-  a.tmp = a.JB + std::max<long>(s.ncCap, 1);
+  a.tmp = a.JB + std::max<long>(s.ncCap, 1) + s.nbil;
+  a.tmpX = a.tmp + nbc;
   if (kMixed) {
-    a.sr = a.tmp + nbc;
+    a.sr = a.tmpX + nbc;
     a.frame = reinterpret_cast<TM*>(s.frame32.p);
     a.minv = reinterpret_cast<TM*>(a.sr + 4 * nbc);
   } else {
-    a.tmpSplit = a.tmp + nbc;
     a.frame = reinterpret_cast<TM*>(s.frame.p);
     a.minv = reinterpret_cast<TM*>(s.minv.p);
   }
@@ -1906,8 +1917,9 @@ void prepareScene(Scene& s, Args<TM>& a) {
     a.part3[k] = s.partials.p + (long)(2 * k + 1) * kSlots * tilesCap;
     a.p1sum[k] = s.partials.p + 4L * kSlots * tilesCap + k * kSlots;
     a.lq[k] = s.partials.p + 4L * kSlots * tilesCap + 2 * kSlots + k * lqCap;
-    a.lqw[k] = s.partials.p + 4L * kSlots * tilesCap + 2 * kSlots + 2 * lqCap + k * lqwCap;
   }
+  a.partX = s.partials.p + 4L * kSlots * tilesCap + 2 * kSlots + 2 * lqCap;
+  a.lqX = a.partX + 4L * kSlots * tilesCap;
 }
 
 template <typename TM>
@@ -2021,7 +2033,7 @@ Plan<TM> activePlan(Engine& E) {
 // so; 512 scenes, 8.1 million contacts: 372 ms and 322).  The members of a team must all be
 // running, so a team may be no larger than the chip; the teams of a launch
 // may be, since they are placed in order and the first to end make room.
-constexpr int kTeamPasses = 2048;     // of one launch of a single scene
+constexpr int kTeamPasses = 2048;     // of one launch of a single scene (tags: 2 p + 3 < 65,536)
 constexpr int kTeamPassesMany = 512;  // of several scenes: a team waits for the room of those before it
 constexpr int kTeamPassesServed = 64; // of a server, which admits and completes between launches
 constexpr int kTeamSkip = 16;         // solves that stay on launches after a team could not be placed
@@ -2041,6 +2053,7 @@ void buildTeams(Engine& E, hipStream_t st) {
     const Args<TM>& a = slotArgs<TM>(E, slot);
     const int members = (a.nTiles + R - 1) / R;
     if (members > most || a.nBodyTiles > 64L * members) E.teamRows = 0;  // (32 rounds of body units)
+    if (a.cap + a.dims.nbil > 1L << 26) E.teamRows = 0;  // (32-bit offsets into the exchanged J)
     for (int k = 0; k < members; ++k) items.push_back(TeamItem{slot, k, members, 0});
     E.teamBil = E.teamBil || a.dims.nbil > 0;
   }
@@ -2061,10 +2074,9 @@ void launchTeams(Engine& E, hipStream_t st, int passes) {
                                 : (E.teamRows == 1 ? kTeam<TM, false, 1> : kTeam<TM, false, 2>);
   hipLaunchKernelGGL(kernel, dim3((unsigned)(E.hTeams.size() / sizeof(TeamItem))), dim3(kTC), 0, st,
                      reinterpret_cast<const Args<TM>*>(E.table.p), T,
-                     E.nSlots == 1 ? nullptr : reinterpret_cast<const TeamItem*>(E.teamItems.p), E.teamSync.p, E.teamEpoch + 1, ++E.teamLaunch,
-                     passes, E.nSlots == 1 ? kFormTicks : kFormTicksMany);
+                     E.nSlots == 1 ? nullptr : reinterpret_cast<const TeamItem*>(E.teamItems.p), E.teamSync.p,
+                     ++E.teamLaunch, passes, E.nSlots == 1 ? kFormTicks : kFormTicksMany);
   DV_HIP(hipGetLastError());
-  E.teamEpoch += 2 * (unsigned long long)passes + 2;
 }
 
 template <typename TM>

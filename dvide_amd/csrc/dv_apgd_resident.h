@@ -1,26 +1,30 @@
 // The resident passes: thousands of passes of a slot in one launch, its
 // contacts' state in registers and its workgroups exchanging what the other
-// half of a pass needs through device-scope stores and flags.
+// half of a pass needs through device-scope stores.
 //
 // Included by dv_apgd_fused.hip after the pass kernels, whose arithmetic and
 // summation orders it repeats bit for bit (a slot may run some chunks here
 // and others as P1/P2 launches, and ends in the same state).
 //
 // Why: a pass as two launches costs two kernel boundaries and a reload of the
-// whole state.  A grid barrier used to cost more, because an agent-scope
-// release writes back the L2; but the data that crosses workgroups is small
-// (J and tmp), and stored at device scope it needs no write-back.  Such a
-// barrier takes 1.1 us among 8 workgroups, 1.3 among 32, 2.0 among 64 and 3.0
-// among 256, and an exchange of 16 bytes per thread another 0.9 to 2.7.
-// us per pass, launches -> resident (piles of the given contacts):
-//   contacts    200   2,400   18,000  64,000  126,000  160,000  256,000
-//   FP64       10.7    13.9     15.5    17.1     21.0     26.0     27.2
-//          ->   5.4     9.2     10.2    11.8     14.2     18.3     23.3
-//   mixed       8.8    11.7     12.9    13.6     16.1     18.9     20.7
-//          ->   4.5     7.9      8.4    10.0     11.9     14.6     17.8
-// What a pass waits for (18,000 contacts, mixed): P1 0.8 us, draining J 0.8,
-// the partial sums under the flags' flight 1.1, P2 1.5, draining tmp and the
-// flags 1.6, the totals and the decision 1.1.
+// whole state.  What crosses workgroups is small (J, tmp and the sums), and
+// stored at device scope it needs no write-back of the L2.  Exchanged under a
+// grid barrier it still cost a chain of store, drain, flag, poll and load,
+// 2.5 to 3 us twice a pass; so the entries carry the pass's tag themselves, a
+// reader waits for just those that it needs, and the step of the next pass is
+// taken before this one is decided.
+// us per pass as launches, resident with two barriers a pass, and so (piles
+// of the given contacts):
+//   contacts    200   2,400   18,000  64,000  126,000  256,000
+//   FP64       10.7    13.9     15.5    17.1     21.0     27.2
+//               5.4     9.2     10.2    11.8     14.2     23.3
+//               4.7     7.7      7.4     9.0     12.1     19.4
+//   mixed       8.8    11.7     12.9    13.6     16.1     20.7
+//               4.5     7.9      8.4    10.0     11.9     17.8
+//               3.7     5.6      5.7     6.6      8.2     12.6
+// Where a pass of 18,000 contacts spends them (mixed, one wavefront's clock):
+// J's loads 1.1 us, the bodies' sums 0.5, waiting for tmp 0.7, the next step
+// 0.4, its sums 1.0, waiting for the totals 0.7, the decision 1.0.
 #pragma once
 
 // A workgroup's place: member `rank` of the `members` of slot `slot`'s team.
@@ -29,16 +33,14 @@ struct TeamItem {
 };
 
 // Per slot, in 64-bit words: the formation's outcome, then one flag per
-// member.  Flags hold epochs that only grow, so nothing is cleared between
-// launches.
+// member.  Flags hold the launch's number, which only grows, so nothing is
+// cleared between launches.
 constexpr int kTeamMax = 256;
 constexpr int kTeamSync = 16 + kTeamMax;
 // A team whose members are not all running after this long gives up (the
 // 100 MHz wall clock): the slot's passes then run as launches.
 constexpr unsigned long long kFormTicks = 200000ull;         // 2 ms
 constexpr unsigned long long kFormTicksMany = 10000000ull;   // 100 ms: several scenes' teams wait for room
-// No wait of a formed team lasts this long; a member that sees it ends.
-constexpr unsigned long long kBarrierTicks = 1000000000ull;  // 10 s
 
 using u64 = unsigned long long;
 
@@ -65,41 +67,185 @@ template <typename TM>
 struct V3 {
   TM x, y, z;
 };
-// An exchanged array of n 3-vectors.  FP32: padded to 16 bytes.  FP64: the x
-// and y of all entries, then the z, so that a wavefront's stores are two
-// contiguous runs (padded to 32 bytes they were two half-filled ones, and took
-// twice as long to drain).  Entry kNone reads as zero without touching
-// memory: its offset lies past the bound that the hardware checks.
-constexpr int kNone = -1;
+// What crosses workgroups carries its own arrival: every aligned 8-byte word
+// of an exchanged entry holds 48 bits of it and a 16-bit tag that names the
+// pass, and a reader loads until all words carry the tag it waits for.  A word
+// of 8 bytes arrives whole, and no order between words or stores is needed,
+// so nothing is drained and no flag follows the data.  A launch clears the
+// tags before its members meet, so tags need not differ between launches.
+__device__ __forceinline__ int lowTagged(int hi, unsigned tag) { return (hi & 0xFFFF) | (int)tag; }
+__device__ __forceinline__ int highTagged(int hi, unsigned tag) { return (int)((unsigned)hi >> 16 | tag); }
+// (a's low half above b's, and a's high half above b's low half)
+__device__ __forceinline__ int lowLow(int a, int b) { return (int)__builtin_amdgcn_perm((unsigned)a, (unsigned)b, 0x05040100u); }
+__device__ __forceinline__ int highLow(int a, int b) { return (int)__builtin_amdgcn_perm((unsigned)a, (unsigned)b, 0x07060100u); }
+__device__ __forceinline__ i32x2 wordsOf(double v) { return __builtin_bit_cast(i32x2, v); }
+__device__ __forceinline__ double doubleOf(int lo, int hi) { return __builtin_bit_cast(double, i32x2{lo, hi}); }
+constexpr int kNone = -1;  // no entry: reads as zero and stores nothing, without touching memory
+constexpr int kPastEnd = 0x7FFFFF00;  // an offset past every bound, which the hardware checks
+
+// n 3-vectors.  FP32: 16 bytes, (x, y's high half) and (z, y's low half).
+// FP64: 32 bytes, the low 48 bits of x, y and z, then the high 16 of the
+// three, as two arrays of 16-byte halves, so that a wavefront's stores are
+// contiguous runs.
 template <typename TM>
 struct CoArray {
   static constexpr int kSplit = sizeof(TM) == 8;
-  __amdgpu_buffer_rsrc_t r, rz;
+  static constexpr int kHalves = kSplit ? 2 : 1;
+  struct Raw {
+    i32x4 h[kHalves];
+  };
+  __amdgpu_buffer_rsrc_t r, r1;
   __device__ CoArray(void* p, long n)
       : r(__builtin_amdgcn_make_buffer_rsrc(p, 0, (int)(16 * n), 0x00027000)),
-        rz(__builtin_amdgcn_make_buffer_rsrc((char*)p + 16 * n, 0, kSplit ? (int)(8 * n) : 0, 0x00027000)) {}
-  __device__ __forceinline__ V3<TM> ld(int i) const {
-    const i32x4 a = __builtin_amdgcn_raw_buffer_load_b128(r, i == kNone ? 0x7FFFFF00 : 16 * i, 0, kDeviceScope);
+        r1(__builtin_amdgcn_make_buffer_rsrc((char*)p + (kSplit ? 16 * n : 0), 0, (int)(16 * n), 0x00027000)) {}
+  __device__ __forceinline__ Raw ld(int i) const {
+    const int o = i == kNone ? kPastEnd : 16 * i;
+    Raw w;
+    w.h[0] = __builtin_amdgcn_raw_buffer_load_b128(r, o, 0, kDeviceScope);
+    if constexpr (kSplit) w.h[1] = __builtin_amdgcn_raw_buffer_load_b128(r1, o, 0, kDeviceScope);
+    return w;
+  }
+  __device__ __forceinline__ void st(int i, TM x, TM y, TM z, unsigned tag) const {
+    const int o = i == kNone ? kPastEnd : 16 * i;
     if constexpr (kSplit) {
-      const i32x2 b = __builtin_amdgcn_raw_buffer_load_b64(rz, i == kNone ? 0x7FFFFF00 : 8 * i, 0, kDeviceScope);
-      return V3<TM>{__builtin_bit_cast(double, i32x2{a.x, a.y}), __builtin_bit_cast(double, i32x2{a.z, a.w}),
-                    __builtin_bit_cast(double, b)};
+      const i32x2 a = wordsOf(x), b = wordsOf(y), c = wordsOf(z);
+      const i32x4 h0{a.x, lowTagged(a.y, tag), b.x, lowTagged(b.y, tag)};
+      const i32x4 h1{c.x, lowTagged(c.y, tag), (int)((unsigned)a.y >> 16 | ((unsigned)b.y & 0xFFFF0000u)), highTagged(c.y, tag)};
+      __builtin_amdgcn_raw_buffer_store_b128(h0, r, o, 0, kDeviceScope);
+      __builtin_amdgcn_raw_buffer_store_b128(h1, r1, o, 0, kDeviceScope);
     } else {
-      const int x = a.x, y = a.y, z = a.z;
+      const int b = __builtin_bit_cast(int, y);
+      const i32x4 h{__builtin_bit_cast(int, x), highTagged(b, tag), __builtin_bit_cast(int, z), lowTagged(b, tag)};
+      __builtin_amdgcn_raw_buffer_store_b128(h, r, o, 0, kDeviceScope);
+    }
+  }
+  static __device__ __forceinline__ V3<TM> value(const Raw& w) {
+    const i32x4 a = w.h[0];
+    if constexpr (kSplit) {
+      const i32x4 b = w.h[1];
+      return V3<TM>{doubleOf(a.x, lowLow(b.z, a.y)), doubleOf(a.z, highLow(b.z, a.w)), doubleOf(b.x, lowLow(b.w, b.y))};
+    } else {
+      const int x = a.x, y = lowLow(a.y, a.w), z = a.z;
       return V3<TM>{__builtin_bit_cast(float, x), __builtin_bit_cast(float, y), __builtin_bit_cast(float, z)};
     }
   }
-  __device__ __forceinline__ void st(int i, TM x, TM y, TM z) const {
-    if constexpr (kSplit) {
-      const i32x2 a = __builtin_bit_cast(i32x2, x), b = __builtin_bit_cast(i32x2, y);
-      __builtin_amdgcn_raw_buffer_store_b128(i32x4{a.x, a.y, b.x, b.y}, r, 16 * i, 0, kDeviceScope);
-      __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(i32x2, z), rz, 8 * i, 0, kDeviceScope);
-    } else {
-      const V4<TM> v{x, y, z, (TM)0};
-      __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(i32x4, v), r, 16 * i, 0, kDeviceScope);
-    }
+  // 0 in the upper half where the entry carries the tag
+  static __device__ __forceinline__ unsigned missing(int i, const Raw& w, unsigned tag) {
+    unsigned m = 0;
+#pragma unroll
+    for (int h = 0; h < kHalves; ++h) m |= ((unsigned)w.h[h].y ^ tag) | ((unsigned)w.h[h].w ^ tag);
+    return i == kNone ? 0u : m;
+  }
+  // a bilateral row's gamma in the same form
+  __device__ __forceinline__ void stDouble(int i, double v, unsigned tag) const {
+    const i32x2 a = wordsOf(v);
+    const int lo = a.x, hi = a.y;  // (a vector's element, bit-cast in place, reads element 0)
+    if constexpr (kSplit) st(i, v, 0.0, 0.0, tag);
+    else st(i, __builtin_bit_cast(float, lo), __builtin_bit_cast(float, hi), 0.0f, tag);
+  }
+  static __device__ __forceinline__ double asDouble(const Raw& w) {
+    const V3<TM> v = value(w);
+    if constexpr (kSplit) return v.x;
+    else return doubleOf(__builtin_bit_cast(int, v.x), __builtin_bit_cast(int, v.y));
   }
 };
+// One double as an exchanged entry of 16 bytes.
+__device__ __forceinline__ i32x4 taggedDouble(double v, unsigned tag) {
+  const i32x2 a = wordsOf(v);
+  return i32x4{a.x, lowTagged(a.y, tag), (int)((unsigned)a.y >> 16), (int)tag};
+}
+__device__ __forceinline__ double valueOf(const i32x4& w) { return doubleOf(w.x, lowLow(w.z, w.y)); }
+__device__ __forceinline__ unsigned missing(const i32x4& w, unsigned tag) {
+  return ((unsigned)w.y ^ tag) | ((unsigned)w.w ^ tag);
+}
+
+__device__ __forceinline__ float exactFma(float x, float y, float z) { return __builtin_fmaf(x, y, z); }
+__device__ __forceinline__ double exactFma(double x, double y, double z) { return __builtin_fma(x, y, z); }
+
+// projectCone<double> without its branches, which every wavefront takes all
+// of, and with 1 / mu and mu^2 + 1 formed once: the same results.
+struct Cone {
+  double mu, inverse, den;
+  __device__ explicit Cone(double m) : mu(m), inverse(1.0 / m), den(m * m + 1.0) {}
+  __device__ __forceinline__ void project(double& g0, double& g1, double& g2) const {
+    const double gn = g0;
+    if (mu == 0) {
+      g1 = 0; g2 = 0;
+      if (gn < 0) g0 = 0;
+      return;
+    }
+    const double gt = __builtin_sqrt(g1 * g1 + g2 * g2);
+    const bool inside = gt < mu * gn;
+    const bool polar = (gt < -inverse * gn) | (fabs(gn) < 10e-15);
+    const double gnp = (gt * mu + gn) / den;
+    const double q = gnp * mu / gt;
+    g0 = inside ? g0 : polar ? 0.0 : gnp;
+    g1 = inside ? g1 : polar ? 0.0 : q * g1;
+    g2 = inside ? g2 : polar ? 0.0 : q * g2;
+  }
+  __device__ __forceinline__ double residual(double g0, double g1, double g2, double w0, double w1, double w2,
+                                             double gdiff, double ig) const {
+    double z0 = 1.0 * g0 + (-gdiff) * w0, z1 = 1.0 * g1 + (-gdiff) * w1, z2 = 1.0 * g2 + (-gdiff) * w2;
+    project(z0, z1, z2);
+    const double e0 = ig * g0 + (-ig) * z0, e1 = ig * g1 + (-ig) * z1, e2 = ig * g2 + (-ig) * z2;
+    const double sum = e0 + e1 + e2;
+    return sum == sum ? fmax(fabs(e0), fmax(fabs(e1), fabs(e2))) : INFINITY;
+  }
+};
+
+// A wait of the whole wavefront: load() until nothing is missing(), which
+// loads of what has been asked for already may show at once.  It ends after
+// kMostLoads loads (at 0.2 us or more each, some seconds) and then marks the
+// member lost, whose other waits end after one.  (One way out, for all lanes
+// together: loops with more kept what they load in three copies of its
+// registers.)
+constexpr int kMostLoads = 1 << 25;
+__device__ __forceinline__ bool someMissing(unsigned m) { return __any(m >= 0x10000u); }
+// (Otherwise the compiler carries the parts of what was loaded out of the wait
+// in further registers.)
+__device__ __forceinline__ void pinned(i32x4& w) { asm volatile("" : "+v"(w)); }
+template <class Missing, class Load>
+__device__ __forceinline__ void waitFor(int* bad, const Missing& missing, const Load& load) {
+  if (!missing()) return;
+  int left = __builtin_amdgcn_readfirstlane(__hip_atomic_load(bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) ? 1 : kMostLoads;
+  do {
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);  // (the loads stay in the loop)
+    __builtin_amdgcn_s_sleep(10);  // (others' loads first: 0.1 to 0.6 us a pass)
+    load();
+    --left;
+  } while ((int)missing() & (int)(left > 0));
+  if (left <= 0) __hip_atomic_store(bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+// N entries of an array, once each carries the tag (kNone: nothing to wait
+// for); awaitRest where they have been loaded once already.
+template <typename TM, int N>
+__device__ __forceinline__ void loadEntries(const CoArray<TM>& A, const int (&id)[N], typename CoArray<TM>::Raw (&w)[N]) {
+#pragma unroll
+  for (int k = 0; k < N; ++k) w[k] = A.ld(id[k]);
+}
+template <typename TM, int N>
+__device__ __forceinline__ void awaitRest(const CoArray<TM>& A, const int (&id)[N], unsigned tag, int* bad,
+                                          typename CoArray<TM>::Raw (&w)[N]) {
+  waitFor(
+      bad,
+      [&] {
+        unsigned m = 0;
+#pragma unroll
+        for (int k = 0; k < N; ++k) m |= A.missing(id[k], w[k], tag);
+        return someMissing(m);
+      },
+      [&] { loadEntries(A, id, w); });
+#pragma unroll
+  for (int k = 0; k < N; ++k)
+#pragma unroll
+    for (int h = 0; h < CoArray<TM>::kHalves; ++h) pinned(w[k].h[h]);
+}
+template <typename TM, int N>
+__device__ __forceinline__ void await(const CoArray<TM>& A, const int (&id)[N], unsigned tag, int* bad,
+                                      typename CoArray<TM>::Raw (&w)[N]) {
+  loadEntries(A, id, w);
+  awaitRest(A, id, tag, bad, w);
+}
 
 // Waits until this wavefront's stores have reached device scope (vmcnt 0;
 // not as inline asm, beside which the compiler keeps half of the registers
@@ -110,58 +256,39 @@ __device__ __forceinline__ void drainStores() {
   __atomic_signal_fence(__ATOMIC_SEQ_CST);
 }
 
-// Every member's flag at `epoch`, or false after `ticks`.
-__device__ __forceinline__ bool teamWait(const u64* flags, int W, u64 epoch, u64 ticks, int* bad) {
+// All members are running and have cleared their entries, or none goes on: a
+// member that has seen every flag proposes to go, one that has waited too
+// long proposes to give up, and the first proposal of the launch holds for
+// all.  Members wait for nothing else before this, so a team that cannot be
+// placed whole (other work holds part of the chip) ends instead of waiting
+// for ever.
+__device__ __forceinline__ bool teamForm(u64* sync, int rank, int W, u64 launch, u64 ticks) {
+  __shared__ u64 outcome;
+  __shared__ int late;
+  if (threadIdx.x == 0) late = 0;
+  drainStores();
+  __syncthreads();
+  if (W == 1) return true;
+  u64* flags = sync + 16;
+  if (threadIdx.x == 0) coStore(flags + rank, launch);
   for (int i = threadIdx.x; i < W; i += kTC) {
-    if (coLoad(flags + i) >= epoch) continue;
     const u64 t0 = wall_clock64();
-    for (int k = 1; coLoad(flags + i) < epoch; ++k)
+    for (int k = 1; coLoad(flags + i) < launch; ++k)
       if ((k & 63) == 0 && wall_clock64() - t0 > ticks) {
-        *bad = 1;
+        late = 1;
         break;
       }
   }
   __syncthreads();
-  return *bad == 0;
-}
-
-// Barrier of a formed team, in two halves: what a member stored before it
-// arrives, every member loads after the wait; work that the others do not
-// need yet goes between the two.
-__device__ __forceinline__ void teamArrive(u64* flags, int rank, int W, u64 epoch) {
-  drainStores();
-  __syncthreads();
-  if (W > 1 && threadIdx.x == 0) coStore(flags + rank, epoch);
-}
-__device__ __forceinline__ bool teamWait(const u64* flags, int W, u64 epoch, int* bad) {
-  if (W == 1) {
-    __syncthreads();
-    return true;
-  }
-  return teamWait(flags, W, epoch, kBarrierTicks, bad);
-}
-
-// All members are running, or none goes on: a member that has seen every
-// flag proposes to go, one that has waited too long proposes to give up, and
-// the first proposal of the launch holds for all.  Members wait for nothing
-// else before this, so a team that cannot be placed whole (other work holds
-// part of the chip) ends instead of waiting for ever.
-__device__ __forceinline__ bool teamForm(u64* sync, int rank, int W, u64 epoch, u64 launch, u64 ticks, int* bad) {
-  __shared__ u64 outcome;
-  if (W == 1) return true;
-  u64* flags = sync + 16;
-  if (threadIdx.x == 0) coStore(flags + rank, epoch);
-  const bool all = teamWait(flags, W, epoch, ticks, bad);
   if (threadIdx.x == 0) {
     u64 cur = coLoad(sync);
     while ((cur >> 1) != launch) {
-      const u64 want = 2 * launch + (all ? 1 : 0);
+      const u64 want = 2 * launch + (late ? 0 : 1);
       if (__hip_atomic_compare_exchange_strong(gl(sync), &cur, want, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT))
         cur = want;
     }
     outcome = cur;
-    *bad = 0;
   }
   __syncthreads();
   return (outcome & 1) != 0;
@@ -199,10 +326,11 @@ template <typename TM>
 __device__ __forceinline__ int contactOf(const Args<TM>& a, const BodyRuns<TM>& b, int k) {
   return k >= b.n ? kNone : k < b.nd ? gl(a.inc)[b.k0 + k] >> 1 : b.c0 + k - b.nd;
 }
-// A body's contacts in flight together.  A settled pile has 4.7 to a body and
-// seldom more than 8, and each load more costs every body of the wavefront
-// its issue (two runs of 8 loaded side by side took P2 0.5 us longer).
-constexpr int kRun = 8;
+// A body's contacts in flight together.  A settled pile has 4.7 to a body, but
+// of 64 bodies some have more than 8, and a second round of loads costs them
+// all another flight: us per pass with 6, 8, 10 and 12 at 18,000 contacts 6.6,
+// 6.3, 6.1 and 6.1 (mixed), 8.9, 8.5, 8.1 and 8.8 (FP64).
+constexpr int kRun = 10;
 
 // Wavefront totals in waveSum's and waveMax's order, valid in lane 63 only:
 // past the rows of 16 lanes the partners come by row broadcasts instead of
@@ -232,8 +360,8 @@ constexpr int kLast = 63;
 // the decision.
 struct StepNext {
   double Lb, tb, La, ta, thetaNew, beta;
-  __device__ explicit StepNext(const ApgdState& S) {
-    const LazyNext n(S);
+  __device__ StepNext(double L, double theta) {
+    const LazyNext n(L, theta);
     Lb = n.backL(); tb = n.backT(Lb);
     La = n.nextL(); ta = n.nextT(La);
     thetaNew = n.nextTheta();
@@ -266,314 +394,429 @@ __device__ __forceinline__ PassView uniformView(const PassView& s) {
 
 // `passes` passes (fewer once the solve has ended) of every slot in items, R
 // row tiles per workgroup (R rows per thread).  Per pass a member
-//   takes P1's step on its tiles, from registers (the iterates, N gamma and r
-//     stay there, the frame in LDS), stores J and arrives; then, while the others
-//     arrive, writes the iterate and N gamma back (memory is complete at
-//     every pass end) and forms its partial sums;
+//   has P1's step on its tiles, from registers (the iterates, N gamma and r
+//     stay there, the frame in LDS), and J stored; forms its partial sums;
 //   takes P2 on its body units (64 bodies to a wavefront, the team's units
-//     dealt out evenly), stores tmp and the units' Lipschitz sums, arrives,
-//     and computes the next step sizes of either outcome while it waits;
-//   decides the pass from the team's partial sums, as kDecide does.
+//     dealt out evenly) as their contacts' J arrive; stores tmp and the units'
+//     Lipschitz sums;
+//   takes the next pass's step as its bodies' tmp arrive, on the guess that
+//     this pass is accepted without a restart (then the next step size and
+//     momentum do not depend on the pass's sums), and stores its J;
+//   decides the pass from the team's partial sums, as kDecide does, and takes
+//     the step again where the guess was wrong, under a second tag.
+// The decision takes every member's sums, so it is also what keeps a member
+// from storing over what another still reads: J of a contact is stored again
+// only after tmp of its bodies, which is formed from it, has arrived, and tmp
+// only after J of the body's contacts, formed from it; the partial sums
+// alternate between two places.
+// The iterates go back to memory when the launch ends, and gammaHat's when it
+// leaves the registers.
 // Two wavefronts per SIMD (up to 256 VGPRs, one workgroup to a CU): held to
 // 128, so that a CU takes two, the mixed kernel spilled 20 and took 26.3 us
-// per pass on 256,000 contacts, where two rows per thread take 17.8.
+// per pass on 256,000 contacts, where two rows per thread take 12.6.  (Two
+// rows in FP64 have no registers for a second step: without the guess.)
 template <typename TM, bool kBil, int R>
 __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, Tables T, const TeamItem* items,
-                                                u64* sync, u64 epoch, u64 launch, int passes, u64 formTicks) {
+                                                u64* sync, u64 launch, int passes, u64 formTicks) {
   constexpr bool kMixed = sizeof(TM) < sizeof(double);
+  constexpr bool kGuess = kMixed || R == 1;
   constexpr int NF = kMixed ? 6 : 3;
   constexpr unsigned kUsed = kP1Slots<TM>;
   constexpr int kW = kTC / 64;       // wavefronts
   constexpr int kWT = kTP / 64;      // of a heavy body's sum
   constexpr int kUnits = kTB / 64;   // body units of a body tile
-  static_assert(kW == kSlots && kSlots == 8 && kUnits == 4, "a wavefront for each total; two loads to a body tile");
+  using Raw = typename CoArray<TM>::Raw;
+  static_assert(kW == 2 * kUnits && kW == kSlots && kSlots == 8 && kUnits == 4, "a wavefront for each total; a body tile's units to a lane");
   const TeamItem me = items ? items[blockIdx.x] : TeamItem{0, (int)blockIdx.x, (int)gridDim.x, 0};
   const Args<TM>& a = A[me.slot];
   const SolveDims& D = a.dims;
   const int W = me.members, rank = me.rank, nTiles = a.nTiles;
   u64* sy = sync + (long)me.slot * kTeamSync;
-  u64* flags = sy + 16;
   __shared__ int bad;
-  __shared__ double shP[R][kW][kSlots], shTot[kW], shH[kWT][3];
-  __shared__ ApgdState shS;  // the state and its view: registers are for the rows and bodies
-  __shared__ PassView shV;
-  __shared__ double shNext[6];
+  __shared__ double shP[2][R][kW][kSlots], shTot[2][kW], shLq[2][kWT], shH[kWT][3];
+  // the state before and after a pass; and, like the sums, for either parity:
+  // a pass has one barrier, before its decision, which every wavefront takes
+  __shared__ ApgdState shS[2];
+  __shared__ double shNext[2][6];
+  __shared__ double shUnit[32][kW];  // the units' Lipschitz sums, and how many of a tile's are there
+  __shared__ int unitCount[32][2];
+  __shared__ int nextFor;  // the pass that they belong to
   // per thread, kept here instead of in registers: the rows' frames and the
   // first body's contacts
   __shared__ TM shF[R][9][kTC];
   __shared__ int shIds[kRun][kTC];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (tid < 64) unitCount[tid / 2][tid % 2] = 0;
   if (tid == 0) {
     bad = 0;
-    shS = STATE(T, me.slot, 1);
-    shV = viewOf(shS);
+    nextFor = -1;
+    shS[0] = STATE(T, me.slot, 1);
   }
   __syncthreads();
-  if (shS.done) return;  // the same for every member
-  PassView V = uniformView(shV);
-  const CoArray<TM> J(a.J, a.cap), tmp(kMixed ? (void*)a.tmp : (void*)a.tmpSplit, D.nb);
+  if (shS[0].done) return;  // the same for every member
+  PassView V = uniformView(viewOf(shS[0]));
+  double L = shS[0].L, theta = shS[0].theta;
+  const long cap = a.cap;
+  const CoArray<TM> J(a.J, cap + D.nbil), tmp(a.tmpX, D.nb);
   const int nBT = a.nBodyTiles, nHeavy = gl(a.counters)[2], nl = nBT + nHeavy;
-  const int nU = kUnits * nBT, u0 = rank + W * wave;  // body units (below)
-  if (!kMixed) {  // M^-1 D^T gamma as the launches left it, into the exchanged form
-    for (int u = u0; u < nU; u += W * kW) {
-      const int g = u * 64 + lane;
-      if (g >= D.nb) continue;
-      const V4<TM> t = ld4(a.tmp, g);
-      tmp.st(g, t.x, t.y, t.z);
-    }
-    drainStores();
-    __syncthreads();
-  }
-  if (!teamForm(sy, rank, W, epoch, launch, formTicks, &bad)) return;
+  // body units of 64 bodies: a wavefront's in iteration j is of tile
+  // rank + W (2 j + half)
+  const int half = wave / kUnits, nU = kUnits * nBT;
+  const int u0 = kUnits * (rank + W * half) + wave % kUnits, uStep = 2 * kUnits * W;
+  // P1's partial sums (slot s of tile k at s nTiles + k) and the body tiles'
+  // and the heavy bodies' Lipschitz sums, by pass parity
+  const __amdgpu_buffer_rsrc_t rPart = __builtin_amdgcn_make_buffer_rsrc(a.partX, 0, 2 * 16 * kSlots * nTiles, 0x00027000);
+  const __amdgpu_buffer_rsrc_t rLq = __builtin_amdgcn_make_buffer_rsrc(a.lqX, 0, 2 * 16 * nl, 0x00027000);
+  auto postPart = [&](int par, int i, double v, unsigned tag) {
+    __builtin_amdgcn_raw_buffer_store_b128(taggedDouble(v, tag), rPart, 16 * i, par * 16 * kSlots * nTiles, kDeviceScope);
+  };
+  auto postLq = [&](int par, int i, double v, unsigned tag) {
+    __builtin_amdgcn_raw_buffer_store_b128(taggedDouble(v, tag), rLq, 16 * i, par * 16 * nl, kDeviceScope);
+  };
 
   // this thread's rows: row u of tile R rank + u
   struct Row {
-    int c, ia, ib, f0, fs;  // the contact and its bodies; row 0, and the step to rows 1 and 2
+    int e, ia, ib;  // its entry of J, and the tmp of its bodies (kNone: fixed)
+    int ca, cb;     // bilateral: the components
     bool valid, bil;
-    TM rv[3], nk[3], nm[3];
-    double gk[3], gm[3], gn[3];
+    TM rv[3], nk[3], nm[3], nn[3];
+    double gk[3], gm[3], gn[3], gs[3];
   };
   Row row[R];
-  const long cap = a.cap;
+  auto flatOf = [&](int u, int rr) {  // row rr's place in a row vector
+    const long q = ((long)rank * R + u) * kTC + tid;
+    return kBil && q >= D.nc ? (long)BROW(a, q - D.nc) : ROW(a, rr, q);
+  };
 #pragma unroll
   for (int u = 0; u < R; ++u) {
     Row& w = row[u];
     const long q = ((long)rank * R + u) * kTC + tid;
     w.valid = q < (long)D.nc + D.nbil;
-    w.bil = kBil && q >= D.nc;
-    w.c = w.valid && !w.bil ? (int)q : 0;
-    w.f0 = w.valid ? (int)(w.bil ? BROW(a, q - D.nc) : q) : 0;
-    w.fs = w.valid && !w.bil ? (int)cap : 0;
-    w.ia = gl(a.cA)[w.c];
-    w.ib = gl(a.cB)[w.c];
-    if (kBil && w.valid && w.bil) {  // the two DOFs
-      w.ia = gl(a.bilA)[q - D.nc];
-      w.ib = gl(a.bilB)[q - D.nc];
+    w.bil = kBil && w.valid && q >= D.nc;
+    const int c = w.valid && !w.bil ? (int)q : 0;
+    w.e = w.bil ? (int)(cap + (q - D.nc)) : w.valid ? c : kNone;
+    w.ia = gl(a.cA)[c];
+    w.ib = gl(a.cB)[c];
+    w.ca = w.cb = 0;
+    if (kBil && w.bil) {  // the two DOFs
+      const int da = gl(a.bilA)[q - D.nc], db = gl(a.bilB)[q - D.nc];
+      w.ia = da / 3;
+      w.ca = da % 3;
+      w.ib = db < 0 ? w.ia : db / 3;
+      w.cb = db < 0 ? -1 : db % 3;
     }
+    if (!w.valid || gl(a.minv)[w.ia] == (TM)0) w.ia = kNone;
+    if (!w.valid || w.cb < 0 || gl(a.minv)[w.ib] == (TM)0) w.ib = kNone;
     TM fc[6], F[9];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) fc[k] = k < NF ? gl(a.frame)[k * cap + w.c] : (TM)0;
+    for (int k = 0; k < 6; ++k) fc[k] = k < NF ? gl(a.frame)[k * cap + c] : (TM)0;
     frameFrom(fc, D.geomMode, F);
 #pragma unroll
     for (int k = 0; k < 9; ++k) shF[u][k][tid] = F[k];
 #pragma unroll
     for (int rr = 0; rr < 3; ++rr) {
-      const long f = w.f0 + (long)rr * w.fs;
-      w.rv[rr] = gl(a.r)[f];
-      w.gk[rr] = gl(a.ring[0] + V.cur * a.ringStride)[f];
-      w.gm[rr] = gl(a.ring[0] + V.prev * a.ringStride)[f];
-      w.nk[rr] = gl(a.rn[0] + V.cur * a.ringStride)[f];  // (not formed yet if fresh: replaced below)
-      w.nm[rr] = gl(a.rn[0] + V.prev * a.ringStride)[f];
-      w.gn[rr] = 0;
+      // (a thread without a row has one of zeros, which adds zero to every sum)
+      const bool on = w.valid && !(w.bil && rr);
+      const long f = on ? flatOf(u, rr) : 0;
+      w.rv[rr] = on ? gl(a.r)[f] : (TM)0;
+      w.gk[rr] = on ? gl(a.ring[0] + V.cur * a.ringStride)[f] : 0.0;
+      w.gm[rr] = on ? gl(a.ring[0] + V.prev * a.ringStride)[f] : 0.0;
+      w.nk[rr] = on ? gl(a.rn[0] + V.cur * a.ringStride)[f] : (TM)0;  // (not formed yet if fresh: replaced below)
+      w.nm[rr] = on ? gl(a.rn[0] + V.prev * a.ringStride)[f] : (TM)0;
+      w.gn[rr] = w.gs[rr] = 0;
+      w.nn[rr] = 0;
     }
+    J.st(w.e, 0, 0, 0, 0);
   }
-  auto tmpOf = [&](int dof) {
-    const V3<TM> t = tmp.ld(dof / 3);
-    const int k = dof % 3;
-    return k == 0 ? t.x : (k == 1 ? t.y : t.z);
+  // the iterate in registers back to its ring slot
+  auto storeIterate = [&](int slot, int u, const double (&g)[3]) {
+    const Row& w = row[u];
+    if (!w.valid) return;
+#pragma unroll
+    for (int rr = 0; rr < 3; ++rr)
+      if (!(w.bil && rr)) gl(a.ring[0] + slot * a.ringStride)[flatOf(u, rr)] = g[rr];
   };
 
-  // body units: unit rank + W (wave + kW j) in iteration j.  A unit without a
-  // movable light body is left out: its tmp is zero from the setup on, and so
-  // are its sums.
+  // (a unit without a movable light body only has a zero sum)
   const BodyRuns<TM> first = bodyRuns(a, u0 < nU ? (long)u0 * 64 + lane : (long)D.nb);
 #pragma unroll
   for (int k = 0; k < kRun; ++k) shIds[k][tid] = contactOf(a, first, k);
-  // (the launches read the D^T gamma ring of fixed bodies too, times zero)
-  if (kMixed)
-    for (int u = u0; u < nU; u += W * kW) {
-      const int g = u * 64 + lane;
-      if (g < D.nb && gl(a.minv)[g] == (TM)0)
-#pragma unroll
-        for (int k = 0; k < 4; ++k) st4(a.sr, (long)k * D.nb + g, V4<TM>{0, 0, 0, 0});
-    }
   unsigned live = 0;
-  for (int j = 0, u = u0; u < nU; ++j, u += W * kW) {
-    if (__any(bodyRuns(a, (long)u * 64 + lane).sums)) live |= 1u << j;
-    else if (lane == 0) {
-      coStore(a.lqw[0] + u, 0.0);
-      coStore(a.lqw[1] + u, 0.0);
-    }
+  for (int j = 0, u = u0; u < nU; ++j, u += uStep) {
+    const int g = u * 64 + lane;
+    if (__any(bodyRuns(a, (long)g).sums)) live |= 1u << j;
+    if (g < D.nb) tmp.st(g, 0, 0, 0, 0);
+    if (wave % kUnits == 0 && lane == kLast)
+      for (int k = 0; k < 2; ++k) postLq(k, u / kUnits, 0.0, 0);
+    // (the launches read the D^T gamma ring of fixed bodies too, times zero)
+    if (kMixed && g < D.nb && gl(a.minv)[g] == (TM)0)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) st4(a.sr, (long)k * D.nb + g, V4<TM>{0, 0, 0, 0});
   }
+  for (int h = rank + W * tid; h < nHeavy; h += W * kTC)
+    for (int k = 0; k < 2; ++k) postLq(k, nBT + h, 0.0, 0);
   bool liveHeavy = false;
-  for (int h = rank; h < nHeavy; h += W) {
-    if (gl(a.minv)[gl(a.heavy)[h]] != (TM)0) liveHeavy = true;
-    else if (tid == 0) {
-      coStore(a.lq[0] + nBT + h, 0.0);
-      coStore(a.lq[1] + nBT + h, 0.0);
-    }
+  for (int h = rank; h < nHeavy; h += W) liveHeavy = liveHeavy || gl(a.minv)[gl(a.heavy)[h]] != (TM)0;
+  // lane l of the last wavefront posts the zero sum of fixed body rank + W l
+  auto isFixed = [&](int h) { return h < nHeavy && gl(a.minv)[gl(a.heavy)[h]] == (TM)0; };
+  const bool fixedHeavy = wave == kW - 1 && isFixed(rank + W * lane);
+  if (tid < R * kSlots) {
+    const int u = tid / kSlots, s = tid % kSlots;
+    if (R * rank + u < nTiles)
+      for (int k = 0; k < 2; ++k) postPart(k, s * nTiles + R * rank + u, 0.0, 0);
   }
+  if (!teamForm(sy, rank, W, launch, formTicks)) return;
 
-  u64 ep = epoch;
+  // y, N y and g of a row (formed once for the step and again for the sums,
+  // rather than kept)
+  auto momentum = [&](bool mom, double beta, double gk, double gm, TM nk, TM nm, TM rv, double& y, double& ny,
+                      double& gg) {
+    if (mom) {
+      const double bp = 1.0 + beta, bm = -beta;
+      y = bp * gk + bm * gm;
+      ny = bp * (double)nk + bm * (double)nm;
+    } else {
+      y = gk;
+      ny = (double)nk;
+    }
+    gg = 1.0 * ny + 1.0 * (double)rv;
+  };
+  const Cone cone(D.mu);
+  // P1's step of row u from (gk, gm, nk, nm) into out, and its J
+  auto step = [&](int u, const double (&gk)[3], const double (&gm)[3], const TM (&nk)[3], const TM (&nm)[3], bool mom,
+                  double beta, double t, double (&out)[3], unsigned tag) {
+    const Row& w = row[u];
+#pragma unroll
+    for (int rr = 0; rr < 3; ++rr) {
+      double y, ny, gg;
+      momentum(mom, beta, gk[rr], gm[rr], nk[rr], nm[rr], w.rv[rr], y, ny, gg);
+      out[rr] = 1.0 * y + (-t) * gg;
+    }
+    if (w.bil) {
+      J.stDouble(w.e, out[0], tag);
+    } else {
+      cone.project(out[0], out[1], out[2]);
+      const TM x0 = (TM)out[0], x1 = (TM)out[1], x2 = (TM)out[2];
+      TM F[9];
+#pragma unroll
+      for (int k = 0; k < 9; ++k) F[k] = shF[u][k][tid];
+      J.st(w.e, F[0] * x0 + F[3] * x1 + F[6] * x2, F[1] * x0 + F[4] * x1 + F[7] * x2,
+           F[2] * x0 + F[5] * x1 + F[8] * x2, tag);
+    }
+  };
+  // N gamma of row u from its bodies' M^-1 D^T gamma
+  auto rowsN = [&](int u, const V3<TM>& tA, const V3<TM>& tB, TM (&out)[3]) {
+    const Row& w = row[u];
+    if (w.bil) {
+      auto comp = [](const V3<TM>& t, int k) { return k == 0 ? t.x : (k == 1 ? t.y : t.z); };
+      out[0] = comp(tA, w.ca) - (w.cb < 0 ? (TM)0 : comp(tB, w.cb));
+    } else {
+      TM F[9];
+#pragma unroll
+      for (int k = 0; k < 9; ++k) F[k] = shF[u][k][tid];
+      rowsOfTmp(F, V4<TM>{tA.x, tA.y, tA.z, (TM)0}, V4<TM>{tB.x, tB.y, tB.z, (TM)0}, out[0], out[1], out[2]);
+    }
+  };
+  auto rowsOfArrived = [&](unsigned tag, bool next) {
+    int id[2 * R];
+    Raw t[2 * R];
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      id[2 * u] = row[u].ia;
+      id[2 * u + 1] = row[u].ib;
+    }
+    await(tmp, id, tag, &bad, t);
+#pragma unroll
+    for (int u = 0; u < R; ++u) rowsN(u, tmp.value(t[2 * u]), tmp.value(t[2 * u + 1]), next ? row[u].nn : row[u].nk);
+  };
+
+  // the partial sums of the step from (gk, gm, nk, nm) to gn, in P1's order
+  auto sumsOf = [&](int to, int u, const double (&gk)[3], const double (&gm)[3], const double (&gn)[3],
+                    const TM (&nk)[3], const TM (&nm)[3], bool mom, double beta) {
+    const Row& w = row[u];
+    double acc[kSlots];
+    zero(acc);
+    const double w0 = (double)nk[0] + (double)w.rv[0];
+    if (w.bil) {
+      double e;
+      if (D.nc) {
+        const double z = 1.0 * gk[0] + (-D.gdiff) * w0;
+        const double ig = D.igdiff;
+        e = fabs(ig * gk[0] + (-ig) * z);
+      } else {
+        e = fabs(w0);
+      }
+      acc[7] = fmax(acc[7], e == e ? e : INFINITY);
+    } else {
+      const double w1 = (double)nk[1] + (double)w.rv[1];
+      const double w2 = (double)nk[2] + (double)w.rv[2];
+      acc[7] = fmax(acc[7], cone.residual(gk[0], gk[1], gk[2], w0, w1, w2, D.gdiff, D.igdiff));
+    }
+#pragma unroll
+    for (int rr = 0; rr < 3; ++rr) {
+      double y, ny, gg;
+      momentum(mom, beta, gk[rr], gm[rr], nk[rr], nm[rr], w.rv[rr], y, ny, gg);
+      const double dy = gn[rr] - y;
+      if (!kMixed) {
+        acc[0] += gn[rr] * (double)w.rv[rr];
+        acc[1] += y * ny;
+        acc[2] += y * (double)w.rv[rr];
+        acc[3] += gg * dy;
+      }
+      acc[4] += dy * dy;
+      acc[5] += gg * (gn[rr] - gk[rr]);
+    }
+#pragma unroll
+    for (int s = 0; s < kSlots; ++s) {
+      if (!((kUsed >> s) & 1u)) continue;
+      const double v = s == kSlots - 1 ? lastMax(acc[s]) : lastSum(acc[s]);
+      if (lane == kLast) shP[to][u][wave][s] = v;
+    }
+  };
+
+  int ends = 0;        // which state is the last
+  bool taken = false;  // this pass's step was taken on the last one's guess
   for (int p = 0; p < passes; ++p) {
     const int par = p & 1;
-    const bool mom = !(V.flags & kViewRestart), fresh = (V.flags & kViewFresh) != 0;
-    const double bp = 1.0 + V.beta, bm = -V.beta;
-    double* const Gn = a.ring[0] + V.nxt * a.ringStride;
-    // y, N y and g of a row (formed once for the step and again for the sums,
-    // rather than kept across the arrival)
-    auto momentum = [&](const Row& w, int rr, double& y, double& ny, double& gg) {
-      if (mom) {
-        y = bp * w.gk[rr] + bm * w.gm[rr];
-        ny = bp * (double)w.nk[rr] + bm * (double)w.nm[rr];
-      } else {
-        y = w.gk[rr];
-        ny = (double)w.nk[rr];
-      }
-      gg = 1.0 * ny + 1.0 * (double)w.rv[rr];
-    };
+    const unsigned tag = (unsigned)(2 * p + 2) << 16;
+    unsigned tagJ = tag;
+    const bool mom = !(V.flags & kViewRestart);
     // ---- P1
-    if (fresh) {
-      V3<TM> tA[R], tB[R];
+    if (!taken) {
+      if (p == 0) {
+        if (V.flags & kViewFresh) {  // tmp as the launches or the last resident passes left it
 #pragma unroll
-      for (int u = 0; u < R; ++u)
-        if (!row[u].bil) {
-          tA[u] = tmp.ld(row[u].valid ? row[u].ia : kNone);
-          tB[u] = tmp.ld(row[u].valid ? row[u].ib : kNone);
+          for (int u = 0; u < R; ++u) {
+            const V4<TM> z{0, 0, 0, 0};
+            const V4<TM> tA = row[u].ia == kNone ? z : ld4(a.tmp, row[u].ia);
+            const V4<TM> tB = row[u].ib == kNone ? z : ld4(a.tmp, row[u].ib);
+            rowsN(u, V3<TM>{tA.x, tA.y, tA.z}, V3<TM>{tB.x, tB.y, tB.z}, row[u].nk);
+          }
         }
+      } else if (kGuess) {
+        tagJ |= 1u << 16;
+      } else if (V.flags & kViewFresh) {
+        rowsOfArrived(tag - (2u << 16), false);
+      }
 #pragma unroll
       for (int u = 0; u < R; ++u) {
         Row& w = row[u];
-        if (!w.valid) continue;
-        if (w.bil) {
-          w.nk[0] = tmpOf(w.ia);
-          if (w.ib >= 0) w.nk[0] -= tmpOf(w.ib);
-        } else {
-          TM F[9];
-#pragma unroll
-          for (int k = 0; k < 9; ++k) F[k] = shF[u][k][tid];
-          rowsOfTmp(F, V4<TM>{tA[u].x, tA[u].y, tA[u].z, (TM)0}, V4<TM>{tB[u].x, tB[u].y, tB[u].z, (TM)0}, w.nk[0],
-                    w.nk[1], w.nk[2]);
-        }
+        step(u, w.gk, w.gm, w.nk, w.nm, mom, V.beta, V.t, w.gn, tagJ);
+        sumsOf(par, u, w.gk, w.gm, w.gn, w.nk, w.nm, mom, V.beta);
       }
+      __syncthreads();
     }
+    // the tiles' partial sums, by the last wavefront (which has the fewest
+    // body units)
+    if (wave == kW - 1 && lane < R * kSlots && ((kUsed >> (lane % kSlots)) & 1u)) {
+      const int u = lane / kSlots, s = lane % kSlots;
+      double t[kW];
 #pragma unroll
-    for (int u = 0; u < R; ++u) {
-      Row& w = row[u];
-      if (!w.valid) continue;
+      for (int w = 0; w < kW; ++w) t[w] = shP[par][u][w][s];
+      double v = t[0];
 #pragma unroll
-      for (int rr = 0; rr < 3; ++rr) {
-        if (w.bil && rr) continue;
-        double y, ny, gg;
-        momentum(w, rr, y, ny, gg);
-        w.gn[rr] = 1.0 * y + (-V.t) * gg;
-      }
-      if (w.bil) {
-        coStore(Gn + w.f0, w.gn[0]);  // P2 reads it
-      } else {
-        projectCone<double>(w.gn[0], w.gn[1], w.gn[2], D.mu);
-        const TM x0 = (TM)w.gn[0], x1 = (TM)w.gn[1], x2 = (TM)w.gn[2];
-        TM F[9];
-#pragma unroll
-        for (int k = 0; k < 9; ++k) F[k] = shF[u][k][tid];
-        J.st(w.c, F[0] * x0 + F[3] * x1 + F[6] * x2, F[1] * x0 + F[4] * x1 + F[7] * x2,
-             F[2] * x0 + F[5] * x1 + F[8] * x2);
-      }
+      for (int w = 1; w < kW; ++w) v = s == kSlots - 1 ? fmax(v, t[w]) : v + t[w];
+      if (R * rank + u < nTiles) postPart(par, s * nTiles + R * rank + u, v, tag);
     }
-    teamArrive(flags, rank, W, ++ep);
-    // what the others need only after P2: N gamma_k, gamma_new and the
-    // partial sums, in P1's order
-#pragma unroll
-    for (int u = 0; u < R; ++u) {
-      const Row& w = row[u];
-      double acc[kSlots];
-      zero(acc);
-      if (w.valid) {
-        const int nr = w.bil ? 1 : 3;
-        DV_GLOBAL TM* Nw = gl(a.rn[0] + V.cur * a.ringStride);
-#pragma unroll
-        for (int rr = 0; rr < 3; ++rr) {
-          if (rr >= nr) continue;
-          const long f = w.f0 + (long)rr * w.fs;
-          if (fresh) Nw[f] = w.nk[rr];
-          if (!w.bil) gl(Gn)[f] = w.gn[rr];
-        }
-        const double w0 = (double)w.nk[0] + (double)w.rv[0];
-        if (w.bil) {
-          double e;
-          if (D.nc) {
-            const double z = 1.0 * w.gk[0] + (-D.gdiff) * w0;
-            const double ig = D.igdiff;
-            e = fabs(ig * w.gk[0] + (-ig) * z);
-          } else {
-            e = fabs(w0);
-          }
-          acc[7] = fmax(acc[7], e == e ? e : INFINITY);
-        } else {
-          const double w1 = (double)w.nk[1] + (double)w.rv[1];
-          const double w2 = (double)w.nk[2] + (double)w.rv[2];
-          acc[7] = fmax(acc[7], residualContact(w.gk[0], w.gk[1], w.gk[2], w0, w1, w2, D.mu, D.gdiff, D.igdiff));
-        }
-#pragma unroll
-        for (int rr = 0; rr < 3; ++rr) {
-          if (rr >= nr) continue;
-          double y, ny, gg;
-          momentum(w, rr, y, ny, gg);
-          const double dy = w.gn[rr] - y;
-          if (!kMixed) {
-            acc[0] += w.gn[rr] * (double)w.rv[rr];
-            acc[1] += y * ny;
-            acc[2] += y * (double)w.rv[rr];
-            acc[3] += gg * dy;
-          }
-          acc[4] += dy * dy;
-          acc[5] += gg * (w.gn[rr] - w.gk[rr]);
-        }
-      }
-#pragma unroll
-      for (int s = 0; s < kSlots; ++s) {
-        if (!((kUsed >> s) & 1u)) continue;
-        const double v = s == kSlots - 1 ? lastMax(acc[s]) : lastSum(acc[s]);
-        if (lane == kLast) shP[u][wave][s] = v;
-      }
-    }
-    if (!teamWait(flags, W, ep, &bad)) break;
+    if (fixedHeavy) postLq(par, nBT + rank + W * lane, 0.0, tag);
+    for (int h = rank + W * (64 + lane); wave == kW - 1 && h < nHeavy; h += W * 64)
+      if (isFixed(h)) postLq(par, nBT + h, 0.0, tag);
 
-    // ---- P2 (every load before a store: a wait for a load also waits for
-    // the stores before it)
-    const double* X = Gn + 3 * cap;  // bilateral rows of gamma_new
-    for (int j = 0, u = u0; u < nU; ++j, u += W * kW) {
-      if (!((live >> j) & 1u)) continue;
-      const BodyRuns<TM> b = j == 0 ? first : bodyRuns(a, (long)u * 64 + lane);
-      int id[kRun];
-      if (j == 0) {
-#pragma unroll
-        for (int k = 0; k < kRun; ++k) id[k] = shIds[k][tid];
-      } else {
-#pragma unroll
-        for (int k = 0; k < kRun; ++k) id[k] = contactOf(a, b, k);
+    // the step sizes of either outcome, by a wavefront that has time
+    if (wave == kW - 2) {
+      const StepNext n(L, theta);
+      if (lane == 0) {
+        n.store(shNext[par]);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        __hip_atomic_store(&nextFor, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
       }
-      V3<TM> v[kRun];
-#pragma unroll
-      for (int k = 0; k < kRun; ++k) v[k] = J.ld(id[k]);
-      TM s0 = 0, s1 = 0, s2 = 0;
+    }
+
+    // ---- P2
+    auto bilateral = [&](const BodyRuns<TM>& b, TM (&s)[3]) {
       for (int k = b.b0; kBil && k < b.b1; ++k) {
         const int e = gl(a.bilInc)[k];
-        const double x = coLoad(X + (e >> 3));
-        const TM t = (TM)((e & 1) ? -x : x);
+        const int i[1] = {(int)cap + (e >> 3)};
+        Raw x[1];
+        await(J, i, tagJ, &bad, x);
+        const double g = J.asDouble(x[0]);
+        const TM t = (TM)((e & 1) ? -g : g);
         const int comp = (e >> 1) & 3;
-        if (comp == 0) s0 += t; else if (comp == 1) s1 += t; else s2 += t;
+        if (comp == 0) s[0] += t; else if (comp == 1) s[1] += t; else s[2] += t;
       }
-      for (int kb = 0;;) {
+    };
+    auto contacts = [&](const BodyRuns<TM>& b, int kb, const Raw (&v)[kRun], TM (&s)[3]) {
 #pragma unroll
-        for (int k = 0; k < kRun; ++k) {
-          if (kb + k >= b.n) continue;
-          if (kb + k < b.nd) {
-            s0 -= v[k].x; s1 -= v[k].y; s2 -= v[k].z;
-          } else {
-            s0 += v[k].x; s1 += v[k].y; s2 += v[k].z;
-          }
-        }
-        kb += kRun;
-        if (kb >= b.n) break;
-#pragma unroll
-        for (int k = 0; k < kRun; ++k) v[k] = J.ld(contactOf(a, b, kb + k));
+      for (int k = 0; k < kRun; ++k) {
+        // (past the body's contacts zero, which changes no sum that began with zero)
+        const V3<TM> t = J.value(v[k]);
+        const TM sign = kb + k < b.nd ? -1 : 1;  // (times it is exact)
+        s[0] = exactFma(t.x, sign, s[0]); s[1] = exactFma(t.y, sign, s[1]); s[2] = exactFma(t.z, sign, s[2]);
       }
-      const double term = lastSum(b.sums ? lipschitzTerm(a, b.g, V, b.mi, s0, s1, s2) : 0.0);
-      if (b.sums) tmp.st(b.g, b.mi * s0, b.mi * s1, b.mi * s2);
-      if (lane == kLast) coStore(a.lqw[par] + u, term);
+    };
+    auto moreContacts = [&](const BodyRuns<TM>& b, int kb, TM (&s)[3]) {  // from its kb-th on
+      for (; __any(kb < b.n); kb += kRun) {
+        int id[kRun];
+        Raw v[kRun];
+#pragma unroll
+        for (int k = 0; k < kRun; ++k) id[k] = contactOf(a, b, kb + k);
+        await(J, id, tagJ, &bad, v);
+        contacts(b, kb, v, s);
+      }
+    };
+    // a unit's Lipschitz sum; the last of a tile's four posts the tile's
+    auto postUnit = [&](int j, int u, double term) {
+      if (lane != kLast) return;
+      shUnit[j][wave] = term;
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      const int before = __hip_atomic_fetch_add(&unitCount[j][half], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      __atomic_signal_fence(__ATOMIC_SEQ_CST);
+      if (before != kUnits - 1) return;
+      __hip_atomic_store(&unitCount[j][half], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+      const double* t = &shUnit[j][kUnits * half];
+      postLq(par, u / kUnits, ((t[0] + t[1]) + t[2]) + t[3], tag);
+    };
+    auto finish = [&](const BodyRuns<TM>& b, int j, int u, const TM (&s)[3], const V4<TM>& c, const V4<TM>& p) {
+      if (b.sums) tmp.st(b.g, b.mi * s[0], b.mi * s[1], b.mi * s[2], tag);
+      const double term = lastSum(b.sums ? lipschitzTerm(a, b.g, V, b.mi, s[0], s[1], s[2], c, p) : 0.0);
+      postUnit(j, u, term);
+    };
+    auto loadRing = [&](int g, V4<TM>& c, V4<TM>& p) {  // D^T gamma_k and D^T gamma_{k-1}
+      if (!kMixed) return;
+      c = ld4(a.sr, V.cur * (long)D.nb + g);
+      p = ld4(a.sr, V.prev * (long)D.nb + g);
+    };
+    if (live & 1u) {
+      int id[kRun];
+      Raw v[kRun];
+      V4<TM> c, p;
+#pragma unroll
+      for (int k = 0; k < kRun; ++k) id[k] = shIds[k][tid];
+      loadRing(first.g, c, p);
+      loadEntries(J, id, v);
+      awaitRest(J, id, tagJ, &bad, v);
+      TM s[3] = {0, 0, 0};
+      bilateral(first, s);
+      contacts(first, 0, v, s);
+      moreContacts(first, kRun, s);
+      finish(first, 0, u0, s, c, p);
+    } else if (u0 < nU) {
+      postUnit(0, u0, 0.0);
     }
-    // movable bodies with many contacts, by the first kTP threads
+    for (int j = 1, u = u0 + uStep; u < nU; ++j, u += uStep) {
+      if (!((live >> j) & 1u)) {
+        postUnit(j, u, 0.0);
+        continue;
+      }
+      const BodyRuns<TM> b = bodyRuns(a, (long)u * 64 + lane);
+      V4<TM> c, p;
+      loadRing(b.g, c, p);
+      TM s[3] = {0, 0, 0};
+      bilateral(b, s);
+      moreContacts(b, 0, s);
+      finish(b, j, u, s, c, p);
+    }
+    // bodies with many contacts, by the first kTP threads
     for (int h = rank; liveHeavy && h < nHeavy; h += W) {
       const int g = gl(a.heavy)[h];
       const TM mi = gl(a.minv)[g];
@@ -581,29 +824,37 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       const int k0 = gl(a.iStart)[g], n = gl(a.iStart)[g + 1] - k0;
       const int c0 = gl(a.cStart)[g], c1 = gl(a.cStart)[g + 1];
       const int nd = n - (c1 - c0);
+      V4<TM> c, p;
+      loadRing(g, c, p);
       if (tid < kTP) {
         double hx = 0, hy = 0, hz = 0;
         for (int kb = tid; kb < n; kb += 4 * kTP) {
-          V3<TM> v[4];
+          int id[4];
+          Raw v[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int k = kb + i * kTP;
-            v[i] = J.ld(k < nd ? gl(a.inc)[k0 + k] >> 1 : k < n ? c0 + k - nd : kNone);
+            id[i] = k < nd ? gl(a.inc)[k0 + k] >> 1 : k < n ? c0 + k - nd : kNone;
           }
+          await(J, id, tagJ, &bad, v);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int k = kb + i * kTP;
             if (k >= n) continue;
             const double sg = k < nd ? -1.0 : 1.0;
-            hx += sg * (double)v[i].x;
-            hy += sg * (double)v[i].y;
-            hz += sg * (double)v[i].z;
+            const V3<TM> t = J.value(v[i]);
+            hx += sg * (double)t.x;
+            hy += sg * (double)t.y;
+            hz += sg * (double)t.z;
           }
         }
         if (kBil && tid == 0) {
           for (int k = gl(a.bilIncStart)[g]; k < gl(a.bilIncStart)[g + 1]; ++k) {
             const int e = gl(a.bilInc)[k];
-            const double x = coLoad(X + (e >> 3)), t = (e & 1) ? -x : x;
+            const int i[1] = {(int)cap + (e >> 3)};
+            Raw x[1];
+            await(J, i, tagJ, &bad, x);
+            const double v = J.asDouble(x[0]), t = (e & 1) ? -v : v;
             const int comp = (e >> 1) & 3;
             if (comp == 0) hx += t; else if (comp == 1) hy += t; else hz += t;
           }
@@ -621,121 +872,164 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
           for (int w = 1; w < kWT; ++w) v += shH[w][s];
           t[s] = (TM)v;
         }
-        tmp.st(g, mi * t[0], mi * t[1], mi * t[2]);
-        coStore(a.lq[par] + nBT + h, lipschitzTerm(a, g, V, mi, t[0], t[1], t[2]));
+        tmp.st(g, mi * t[0], mi * t[1], mi * t[2], tag);
+        postLq(par, nBT + h, lipschitzTerm(a, g, V, mi, t[0], t[1], t[2], c, p), tag);
       }
       __syncthreads();
     }
-    // the tiles' partial sums, by the last wavefront (which has the fewest
-    // body units)
-    if (wave == kW - 1 && lane < R * kSlots && ((kUsed >> (lane % kSlots)) & 1u)) {
-      const int u = lane / kSlots, s = lane % kSlots;
-      double v = shP[u][0][s];
-      for (int w = 1; w < kW; ++w) v = s == kSlots - 1 ? fmax(v, shP[u][w][s]) : v + shP[u][w][s];
-      if (R * rank + u < nTiles) coStore(a.part1[par] + ((long)R * rank + u) * kSlots + s, v);
-    }
-    teamArrive(flags, rank, W, ++ep);
-    if (tid == 0) StepNext(shS).store(shNext);
-    if (!teamWait(flags, W, ep, &bad)) break;
 
-    // ---- the decision, by every member.  Wavefront s totals slot s of P1's
-    // partials, and wavefront 6 (whose slot is not used) the Lipschitz terms,
-    // in reduceSlots' order: lane l of its wavefront w adds entries 64 w + l,
-    // 64 w + l + kTP, ..., and the wavefronts' sums are added in order (past
-    // the entries they are zero, and left out).
-    if (wave == 6) {
-      const auto rq = __builtin_amdgcn_make_buffer_rsrc(a.lqw[par], 0, 8 * nU, 0x00027000);
-      const auto rh = __builtin_amdgcn_make_buffer_rsrc(a.lq[par], 0, 8 * nl, 0x00027000);
-      double v[kWT] = {0, 0, 0, 0};
-      for (int b0 = 0; b0 < nl; b0 += kTP) {
-        i32x4 x[kWT][2];  // a body tile's units, or a heavy body's term and zeros; all loads first
+    // ---- the next pass's step, should this one be accepted without a restart
+    const bool guess = kGuess && p + 1 < passes;
+    if (guess) rowsOfArrived(tag, true);
+    while (__any(__hip_atomic_load(&nextFor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != p)) {
+    }  // (its wavefront waits for nothing before that)
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    const double tNext = uniformDouble(shNext[par][3]), betaNext = uniformDouble(shNext[par][5]);
+    // The team's sums, in reduceSlots' order: lane l of its wavefront i adds
+    // entries 64 i + l, 64 i + l + kTP, ..., and the wavefronts' sums are added
+    // in order (past the entries they are zero, and left out).  Here wavefront
+    // s totals slot s of P1's partials, and wavefront 6 - i is wavefront i for
+    // the Lipschitz terms.
+    const int il = 6 - wave;
+    const bool sumsPart = (kUsed >> wave) & 1u, sumsLq = il >= 0 && il < kWT && 64 * il < nl;
+    i32x4 xp[kWT], xl;  // a slot of four tiles; a body tile's or a heavy body's sum
+    auto loadPart = [&](int b0) {
 #pragma unroll
-        for (int i = 0; i < kWT; ++i) {
-          if (b0 + 64 * i >= nl) break;
-          const int w = b0 + 64 * i + lane;
-          if (w < nBT) {
-            x[i][0] = __builtin_amdgcn_raw_buffer_load_b128(rq, 8 * kUnits * w, 0, kDeviceScope);
-            x[i][1] = __builtin_amdgcn_raw_buffer_load_b128(rq, 8 * kUnits * w, 16, kDeviceScope);
-          } else {  // (past nl: zero, by the bound)
-            const i32x2 t = __builtin_amdgcn_raw_buffer_load_b64(rh, 8 * w, 0, kDeviceScope);
-            x[i][0] = i32x4{t.x, t.y, 0, 0};
-            x[i][1] = i32x4{0, 0, 0, 0};
-          }
-        }
-#pragma unroll
-        for (int i = 0; i < kWT; ++i) {
-          if (b0 + 64 * i >= nl) break;
-          double t = __builtin_bit_cast(double, i32x2{x[i][0].x, x[i][0].y});
-          t += __builtin_bit_cast(double, i32x2{x[i][0].z, x[i][0].w});
-          t += __builtin_bit_cast(double, i32x2{x[i][1].x, x[i][1].y});
-          t += __builtin_bit_cast(double, i32x2{x[i][1].z, x[i][1].w});
-          v[i] += t;
-        }
+      for (int i = 0; i < kWT; ++i) {
+        const int w = b0 + 64 * i + lane;
+        xp[i] = __builtin_amdgcn_raw_buffer_load_b128(rPart, w >= nTiles ? kPastEnd : 16 * (wave * nTiles + w),
+                                                      par * 16 * kSlots * nTiles, kDeviceScope);
       }
-      double total = lastSum(v[0]);
-      for (int i = 1; i < kWT && 64 * i < nl; ++i) total += lastSum(v[i]);
-      if (lane == kLast) shTot[wave] = total;
-    } else if ((kUsed >> wave) & 1u) {
-      const auto rp = __builtin_amdgcn_make_buffer_rsrc(a.part1[par], 0, 8 * kSlots * nTiles, 0x00027000);
+    };
+    auto loadLq = [&](int b0) {
+      const int w = b0 + 64 * il + lane;
+      xl = __builtin_amdgcn_raw_buffer_load_b128(rLq, w >= nl ? kPastEnd : 16 * w, par * 16 * nl, kDeviceScope);
+    };
+    if (guess) {
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        Row& w = row[u];
+        step(u, w.gn, w.gk, w.nn, w.nk, true, betaNext, tNext, w.gs, tag + (2u << 16));
+      }
+    }
+    if (guess)
+#pragma unroll
+      for (int u = 0; u < R; ++u) {
+        const Row& w = row[u];
+        sumsOf(par ^ 1, u, w.gn, w.gk, w.gs, w.nn, w.nk, true, betaNext);
+      }
+    if (sumsPart) loadPart(0);
+    if (sumsLq) loadLq(0);
+    if (sumsPart) {
       double v[kWT] = {0, 0, 0, 0};
       for (int b0 = 0; b0 < nTiles; b0 += kTP) {
-        double x[kWT];
+        if (b0) loadPart(b0);
+        waitFor(
+            &bad,
+            [&] {
+              unsigned m = 0;
 #pragma unroll
-        for (int i = 0; i < kWT; ++i) {
-          if (b0 + 64 * i >= nTiles) break;
-          const int w = b0 + 64 * i + lane;  // (past nTiles: zero, by the bound)
-          x[i] = __builtin_bit_cast(double, (i32x2)__builtin_amdgcn_raw_buffer_load_b64(rp, 8 * kSlots * w + 8 * wave, 0,
-                                                                                        kDeviceScope));
-        }
+              for (int i = 0; i < kWT; ++i) m |= b0 + 64 * i + lane < nTiles ? missing(xp[i], tag) : 0u;
+              return someMissing(m);
+            },
+            [&] { loadPart(b0); });
 #pragma unroll
-        for (int i = 0; i < kWT; ++i) {
-          if (b0 + 64 * i >= nTiles) break;
-          v[i] = wave == kSlots - 1 ? fmax(v[i], x[i]) : v[i] + x[i];
-        }
+        for (int i = 0; i < kWT; ++i) pinned(xp[i]);
+#pragma unroll
+        for (int i = 0; i < kWT; ++i) v[i] = wave == kSlots - 1 ? fmax(v[i], valueOf(xp[i])) : v[i] + valueOf(xp[i]);
       }
       double total = wave == kSlots - 1 ? lastMax(v[0]) : lastSum(v[0]);
       for (int i = 1; i < kWT && 64 * i < nTiles; ++i)
         total = wave == kSlots - 1 ? fmax(total, lastMax(v[i])) : total + lastSum(v[i]);
-      if (lane == kLast) shTot[wave] = total;
+      if (lane == kLast) shTot[par][wave] = total;
     }
-    __syncthreads();
-    if (tid == 0) {
-      double tot[2 * kSlots];
-#pragma unroll
-      for (int s = 0; s < 2 * kSlots; ++s) tot[s] = 0.0;
-#pragma unroll
-      for (int s = 0; s < kSlots; ++s)
-        if ((kUsed >> s) & 1u) tot[s] = shTot[s];
-      tot[kSlots + 6] = shTot[6];
-      ApgdState S = shS;
-      decideStep<kMixed>(S, tot, D, StepNext(shNext));
-      shS = S;
-      shV = viewOf(S);
+    if (sumsLq) {
+      double v = 0;
+      for (int b0 = 0; b0 + 64 * il < nl; b0 += kTP) {
+        if (b0) loadLq(b0);
+        const int w = b0 + 64 * il + lane;
+        waitFor(
+            &bad, [&] { return someMissing(w < nl ? missing(xl, tag) : 0u); }, [&] { loadLq(b0); });
+        pinned(xl);
+        v += valueOf(xl);
+      }
+      const double total = lastSum(v);
+      if (lane == kLast) shLq[par][il] = total;
     }
+
+
+    // ---- the decision, by every member's every wavefront
     __syncthreads();
-    V = uniformView(shV);
-    if (V.flags & kViewDone) break;
+    const bool lost = bad != 0;  // (set by waits only, which all lie before this point)
+    double tot[2 * kSlots];
+#pragma unroll
+    for (int k = 0; k < 2 * kSlots; ++k) tot[k] = 0.0;
+#pragma unroll
+    for (int k = 0; k < kSlots; ++k)
+      if ((kUsed >> k) & 1u) tot[k] = shTot[par][k];
+    tot[kSlots + 6] = shLq[par][0];
+    for (int i = 1; i < kWT && 64 * i < nl; ++i) tot[kSlots + 6] += shLq[par][i];
+    ApgdState S = shS[par];
+    decideStep<kMixed>(S, tot, D, StepNext(shNext[par]));
+    if (tid == 0) shS[par ^ 1] = S;
+    const int dropped = V.prev;
+    V = uniformView(viewOf(S));
+    L = S.L;
+    theta = S.theta;
+    ends = par ^ 1;
+    if (lost || (V.flags & kViewDone)) break;
+    taken = false;
     if (V.flags & kViewFresh) {  // accepted: gamma_new becomes gamma_k (a backtrack keeps both)
+      const bool keep = __builtin_amdgcn_readfirstlane(S.hatSrc) == dropped;  // gammaHat leaves the registers
+      taken = kGuess && !(V.flags & kViewRestart) && V.t == tNext && V.beta == betaNext;
 #pragma unroll
-      for (int u = 0; u < R; ++u)
+      for (int u = 0; u < R; ++u) {
+        Row& w = row[u];
+        if (keep) storeIterate(dropped, u, w.gm);
 #pragma unroll
         for (int rr = 0; rr < 3; ++rr) {
-          row[u].gm[rr] = row[u].gk[rr];
-          row[u].nm[rr] = row[u].nk[rr];
-          row[u].gk[rr] = row[u].gn[rr];
+          w.gm[rr] = w.gk[rr];
+          w.nm[rr] = w.nk[rr];
+          w.gk[rr] = w.gn[rr];
+          if (kGuess) {
+            w.nk[rr] = w.nn[rr];
+            w.gn[rr] = w.gs[rr];
+          }
         }
+      }
     }
   }
-  if (!kMixed) {  // M^-1 D^T gamma back for the launches
-    for (int u = u0; u < nU; u += W * kW) {
-      const int g = u * 64 + lane;
-      if (g >= D.nb) continue;
-      const V3<TM> t = tmp.ld(g);
+  // what the launches, or the next resident passes, read
+#pragma unroll
+  for (int u = 0; u < R; ++u) {
+    const Row& w = row[u];
+    if (V.prev != V.cur) storeIterate(V.prev, u, w.gm);
+    storeIterate(V.cur, u, w.gk);
+    if (!w.valid) continue;
+#pragma unroll
+    for (int rr = 0; rr < 3; ++rr) {
+      if (w.bil && rr) continue;
+      const long f = flatOf(u, rr);
+      if (V.prev != V.cur) gl(a.rn[0] + V.prev * a.ringStride)[f] = w.nm[rr];
+      if (!(V.flags & kViewFresh)) gl(a.rn[0] + V.cur * a.ringStride)[f] = w.nk[rr];
+    }
+  }
+  if (V.flags & kViewFresh) {  // (from the thread's own stores)
+    for (int u = u0; u < nU; u += uStep) {
+      const BodyRuns<TM> b = bodyRuns(a, (long)u * 64 + lane);
+      if (!b.sums) continue;
+      const V3<TM> t = tmp.value(tmp.ld(b.g));
+      st4(a.tmp, b.g, V4<TM>{t.x, t.y, t.z, (TM)0});
+    }
+    for (int h = rank; tid == 0 && h < nHeavy; h += W) {
+      const int g = gl(a.heavy)[h];
+      if (gl(a.minv)[g] == (TM)0) continue;
+      const V3<TM> t = tmp.value(tmp.ld(g));
       st4(a.tmp, g, V4<TM>{t.x, t.y, t.z, (TM)0});
     }
   }
   if (rank == 0 && tid == 0) {
-    ApgdState S = shS;
+    ApgdState S = shS[ends];
     if (bad) {  // a member was lost (never seen): the solve ends as diverged
       S.done = 1;
       S.best = INFINITY;

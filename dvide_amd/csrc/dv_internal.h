@@ -150,7 +150,7 @@ struct Engine {
   DevBuf<char> states;  // ApgdState[nSlots][2], by pass parity
   DevBuf<char> views;   // PassView[nSlots][2]: what the pass kernels read of the states
   DevBuf<unsigned long long> teamSync;  // flags of the resident passes' teams, per slot
-  unsigned long long teamEpoch = 0, teamLaunch = 0;
+  unsigned long long teamLaunch = 0;
   DevBuf<char> teamItems;  // the active slots' teams, and their host copy
   std::vector<char> hTeams;
   int teamRows = 0;     // their row tiles per workgroup (0: some slot has no team)

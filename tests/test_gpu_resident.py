@@ -37,6 +37,15 @@ def landed_shell():
     return sc
 
 
+def ball_on_a_layer():
+    """A large sphere on some thirty small ones: more contacts than a round of
+    a body's loads, fewer than make a body's sum a workgroup's."""
+    sc = layer_of(256)
+    sc.geom[-1, 0] = 2.0
+    sc.pos[-1] = (0.0, 2.02, 0.0)
+    return sc
+
+
 SCENES = {
     "ball": scenes.ball_on_box,
     **{f"layer_{n}": (lambda n=n: layer_of(n)) for n in (63, 511, 512, 513, 1025)},
@@ -44,6 +53,7 @@ SCENES = {
     "free_lid": lambda: scenes.compaction(5, n=3000, width=1.5, lid=scenes.LID_FREE),
     "bilateral_lid": lambda: scenes.compaction(5, n=1200, width=1.2, lid=scenes.LID_BILATERAL),
     "shell": landed_shell,
+    "ball_on_a_layer": ball_on_a_layer,
     "box_58000": lambda: scenes.compaction(2002, n=58000, width=4.0, lid=scenes.LID_NONE),
 }
 
@@ -111,3 +121,23 @@ def test_teams_side_by_side_equal_the_launches(gpu, monkeypatch, names, how):
         for a, b in zip((g.gamma, g.v, g.p), ref[1:]):
             assert bits_equal(a, b)
         g.close()
+
+
+@pytest.mark.parametrize("build", [system.BUILD_FP64, system.BUILD_MIXED])
+@pytest.mark.parametrize("name", ["pile_6000", "bilateral_lid"])
+def test_passes_past_one_launch_equal_the_launches(gpu, monkeypatch, name, build):
+    """A launch runs 2048 passes; the next takes up the iterates, N gamma and
+    M^-1 D^T gamma that it left in memory (also after a backtrack)."""
+    monkeypatch.setenv("DVIDE_TUNE", "0")
+    out = []
+    for rows in (1, 0):
+        g = system.from_scene(SCENES[name](), build, tol=1e-300, max_iterations=2500)
+        g.setRowsPerThread(rows)
+        g.step()
+        st = g.stats()
+        out.append(((st.iterations, st.passes, st.backtracks), g.gamma, g.v, g.p))
+        g.close()
+    assert out[0][0] == out[1][0]
+    assert out[0][0][1] > 2048
+    for a, b in zip(out[0][1:], out[1][1:]):
+        assert bits_equal(a, b)
