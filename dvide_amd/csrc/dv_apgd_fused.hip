@@ -2033,6 +2033,12 @@ Plan<TM> activePlan(Engine& E) {
 // so; 512 scenes, 8.1 million contacts: 372 ms and 322).  The members of a team must all be
 // running, so a team may be no larger than the chip; the teams of a launch
 // may be, since they are placed in order and the first to end make room.
+// Workgroups go to the chip's eight L2s in turn, so the places of a scene's
+// small team are chosen eight apart (several scenes' teams, which fill the chip
+// between them, gained nothing so): us per pass of one scene spread over all and on one, FP64
+// and mixed, 3 tiles 7.4 and 7.0, 5.5 and 5.2; 5 tiles 7.5 and 7.0, 5.8 and
+// 5.3; 10 tiles 7.5 and 7.3, 5.8 and 5.5; 19 tiles 7.7 and 8.7, 5.8 and 6.0.
+constexpr int kXcdMost = 10;
 constexpr int kTeamPasses = 2048;     // of one launch of a single scene (tags: 2 p + 3 < 65,536)
 constexpr int kTeamPassesMany = 512;  // of several scenes: a team waits for the room of those before it
 constexpr int kTeamPassesServed = 64; // of a server, which admits and completes between launches
@@ -2072,9 +2078,11 @@ void launchTeams(Engine& E, hipStream_t st, int passes) {
   const Tables T = tablesOf<TM>(E, E.active);
   const auto kernel = E.teamBil ? (E.teamRows == 1 ? kTeam<TM, true, 1> : kTeam<TM, true, 2>)
                                 : (E.teamRows == 1 ? kTeam<TM, false, 1> : kTeam<TM, false, 2>);
-  hipLaunchKernelGGL(kernel, dim3((unsigned)(E.hTeams.size() / sizeof(TeamItem))), dim3(kTC), 0, st,
+  const int places = (int)(E.hTeams.size() / sizeof(TeamItem));
+  const int stride = E.nSlots == 1 && places <= kXcdMost ? kXcds : 1;
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(places * stride)), dim3(kTC), 0, st,
                      reinterpret_cast<const Args<TM>*>(E.table.p), T,
-                     E.nSlots == 1 ? nullptr : reinterpret_cast<const TeamItem*>(E.teamItems.p), E.teamSync.p,
+                     E.nSlots == 1 ? nullptr : reinterpret_cast<const TeamItem*>(E.teamItems.p), stride, E.teamSync.p,
                      ++E.teamLaunch, passes, E.nSlots == 1 ? kFormTicks : kFormTicksMany);
   DV_HIP(hipGetLastError());
 }

@@ -416,7 +416,7 @@ __device__ __forceinline__ PassView uniformView(const PassView& s) {
 // per pass on 256,000 contacts, where two rows per thread take 12.6.  (Two
 // rows in FP64 have no registers for a second step: without the guess.)
 template <typename TM, bool kBil, int R>
-__global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, Tables T, const TeamItem* items,
+__global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, Tables T, const TeamItem* items, int stride,
                                                 u64* sync, u64 launch, int passes, u64 formTicks) {
   constexpr bool kMixed = sizeof(TM) < sizeof(double);
   constexpr bool kGuess = kMixed || R == 1;
@@ -427,7 +427,9 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
   constexpr int kUnits = kTB / 64;   // body units of a body tile
   using Raw = typename CoArray<TM>::Raw;
   static_assert(kW == 2 * kUnits && kW == kSlots && kSlots == 8 && kUnits == 4, "a wavefront for each total; a body tile's units to a lane");
-  const TeamItem me = items ? items[blockIdx.x] : TeamItem{0, (int)blockIdx.x, (int)gridDim.x, 0};
+  // (a single team needs no list: every stride-th workgroup is a member)
+  if (!items && (int)blockIdx.x % stride) return;
+  const TeamItem me = items ? items[blockIdx.x] : TeamItem{0, (int)blockIdx.x / stride, (int)gridDim.x / stride, 0};
   const Args<TM>& a = A[me.slot];
   const SolveDims& D = a.dims;
   const int W = me.members, rank = me.rank, nTiles = a.nTiles;
