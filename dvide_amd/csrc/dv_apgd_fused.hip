@@ -675,19 +675,25 @@ __device__ __forceinline__ TM bodyMinv(const Args<TM>& a, int g, int which, bool
 // per-body D^T gamma (gamma_k on a restart), whose sum is Delta' N Delta for
 // Delta = gamma_new - y.  The mixed solver keeps s in ring slot nxt.
 template <typename TM>
-__device__ __forceinline__ double lipschitzTerm(const Args<TM>& a, int g, const PassView& S, TM mi, TM s0, TM s1,
-                                                TM s2, const V4<TM>& c, const V4<TM>& p) {
+__device__ __forceinline__ double lipschitzOf(TM mi, TM s0, TM s1, TM s2, const V4<TM>& c, const V4<TM>& p, bool mom,
+                                              double beta) {
   constexpr bool kMixed = sizeof(TM) < sizeof(double);
   if (!kMixed) return (double)s0 * (double)(mi * s0) + (double)s1 * (double)(mi * s1) + (double)s2 * (double)(mi * s2);
-  V4<TM> sn;
-  sn.x = s0; sn.y = s1; sn.z = s2; sn.w = 0;
-  st4(a.sr, S.nxt * (long)a.dims.nb + g, sn);
-  const bool mom = !(S.flags & kViewRestart);
-  const double bp = 1.0 + S.beta, bm = -S.beta;
+  const double bp = 1.0 + beta, bm = -beta;
   const double d0 = (double)s0 - (mom ? bp * (double)c.x + bm * (double)p.x : (double)c.x);
   const double d1 = (double)s1 - (mom ? bp * (double)c.y + bm * (double)p.y : (double)c.y);
   const double d2 = (double)s2 - (mom ? bp * (double)c.z + bm * (double)p.z : (double)c.z);
   return (double)mi * (d0 * d0 + d1 * d1 + d2 * d2);
+}
+template <typename TM>
+__device__ __forceinline__ double lipschitzTerm(const Args<TM>& a, int g, const PassView& S, TM mi, TM s0, TM s1,
+                                                TM s2, const V4<TM>& c, const V4<TM>& p) {
+  if (sizeof(TM) < sizeof(double)) {
+    V4<TM> sn;
+    sn.x = s0; sn.y = s1; sn.z = s2; sn.w = 0;
+    st4(a.sr, S.nxt * (long)a.dims.nb + g, sn);
+  }
+  return lipschitzOf(mi, s0, s1, s2, c, p, !(S.flags & kViewRestart), S.beta);
 }
 template <typename TM>
 __device__ __forceinline__ double lipschitzTerm(const Args<TM>& a, int g, const PassView& S, TM mi, TM s0, TM s1,

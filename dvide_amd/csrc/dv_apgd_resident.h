@@ -11,20 +11,24 @@
 // stored at device scope it needs no write-back of the L2.  Exchanged under a
 // grid barrier it still cost a chain of store, drain, flag, poll and load,
 // 2.5 to 3 us twice a pass; so the entries carry the pass's tag themselves, a
-// reader waits for just those that it needs, and the step of the next pass is
-// taken before this one is decided.
-// us per pass as launches, resident with two barriers a pass, and so (piles
-// of the given contacts):
-//   contacts    200   2,400   18,000  64,000  126,000  256,000
-//   FP64       10.7    13.9     15.5    17.1     21.0     27.2
-//               5.4     9.2     10.2    11.8     14.2     23.3
-//               4.7     7.7      7.4     9.0     12.1     19.4
-//   mixed       8.8    11.7     12.9    13.6     16.1     20.7
-//               4.5     7.9      8.4    10.0     11.9     17.8
-//               3.7     5.6      5.7     6.6      8.2     12.6
-// Where a pass of 18,000 contacts spends them (mixed, one wavefront's clock):
-// J's loads 1.1 us, the bodies' sums 0.5, waiting for tmp 0.7, the next step
-// 0.4, its sums 1.0, waiting for the totals 0.7, the decision 1.0.
+// reader waits for just those that it needs, and the step of the next pass and
+// its bodies' sums are taken before this one is decided.
+// us per pass as launches, resident with two barriers a pass, with the step
+// alone taken ahead, and so (piles of the given contacts):
+//   contacts    134     440   1,630  11,900  41,800  82,400  168,000
+//   FP64       10.7            13.9    15.5    17.1    21.0    27.2
+//               5.4             9.2    10.2    11.8    14.2    23.3
+//               4.6     5.7     6.6     7.2     8.1     9.8    17.5
+//               4.6     5.2     5.7     6.8     7.8     9.4    17.5
+//   mixed       8.8            11.7    12.9    13.6    16.1    20.7
+//               4.5             7.9     8.4    10.0    11.9    17.8
+//               3.7     4.1     5.1     5.4     6.0     6.8    10.8
+//               3.8     3.8     4.3     4.9     5.4     5.8     9.6
+// Where a pass of 11,900 contacts spends its 11,700 cycles (mixed, a wavefront
+// with bodies): tmp's arrival 1,300, the next step 1,000, its sums 1,900, the
+// contacts' J and the bodies' sums 2,500, the totals and the barrier 800, the
+// decision and the change of registers 2,000, steps taken again (13% of the
+// passes) 700.
 #pragma once
 
 // A workgroup's place: member `rank` of the `members` of slot `slot`'s team.
@@ -193,27 +197,40 @@ struct Cone {
   }
 };
 
-// A wait of the whole wavefront: load() until nothing is missing(), which
-// loads of what has been asked for already may show at once.  It ends after
+// A wait of the whole wavefront: load() until nothing is missing() in any lane,
+// which loads of what has been asked for already may show at once; with kLanes
+// only lanes with something missing load again (us per pass of 82,400 contacts
+// in FP64 without and with: 11.1 and 10.5; with two rows a thread it costs
+// registers, and 17.4 became 18.0).  It ends after
 // kMostLoads loads (at 0.2 us or more each, some seconds) and then marks the
 // member lost, whose other waits end after one.  (One way out, for all lanes
 // together: loops with more kept what they load in three copies of its
 // registers.)
 constexpr int kMostLoads = 1 << 25;
-__device__ __forceinline__ bool someMissing(unsigned m) { return __any(m >= 0x10000u); }
+__device__ __forceinline__ bool someMissing(unsigned m, unsigned least = 0x10000u) { return __any(m >= least); }
+// An entry of a step taken on a guess is also there once the right step has
+// replaced it (its tag is the guess's, plus one): what it holds is not used.
+constexpr unsigned kOrReplaced = 0x20000u;
 // (Otherwise the compiler carries the parts of what was loaded out of the wait
 // in further registers.)
 __device__ __forceinline__ void pinned(i32x4& w) { asm volatile("" : "+v"(w)); }
-template <class Missing, class Load>
-__device__ __forceinline__ void waitFor(int* bad, const Missing& missing, const Load& load) {
-  if (!missing()) return;
+// Ends the wait for loads here.  Loads and stores complete in their order, so
+// one that is left unused on some path is waited for, with every store since,
+// wherever the compiler uses its registers next.
+template <typename TM>
+__device__ __forceinline__ void settled(const V4<TM>& v) { asm volatile("" : : "v"(v.x), "v"(v.y), "v"(v.z)); }
+template <bool kLanes, class Missing, class Load>
+__device__ __forceinline__ void waitFor(int* bad, unsigned least, const Missing& missing, const Load& load) {
+  unsigned m = missing();
+  if (!someMissing(m, least)) return;
   int left = __builtin_amdgcn_readfirstlane(__hip_atomic_load(bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)) ? 1 : kMostLoads;
   do {
     __atomic_signal_fence(__ATOMIC_SEQ_CST);  // (the loads stay in the loop)
     __builtin_amdgcn_s_sleep(10);  // (others' loads first: 0.1 to 0.6 us a pass)
-    load();
+    if (!kLanes || m >= least) load();
+    m = missing();
     --left;
-  } while ((int)missing() & (int)(left > 0));
+  } while ((int)someMissing(m, least) & (int)(left > 0));
   if (left <= 0) __hip_atomic_store(bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 // N entries of an array, once each carries the tag (kNone: nothing to wait
@@ -223,16 +240,16 @@ __device__ __forceinline__ void loadEntries(const CoArray<TM>& A, const int (&id
 #pragma unroll
   for (int k = 0; k < N; ++k) w[k] = A.ld(id[k]);
 }
-template <typename TM, int N>
+template <bool kLanes, typename TM, int N>
 __device__ __forceinline__ void awaitRest(const CoArray<TM>& A, const int (&id)[N], unsigned tag, int* bad,
-                                          typename CoArray<TM>::Raw (&w)[N]) {
-  waitFor(
-      bad,
+                                          typename CoArray<TM>::Raw (&w)[N], unsigned least = 0x10000u) {
+  waitFor<kLanes>(
+      bad, least,
       [&] {
         unsigned m = 0;
 #pragma unroll
         for (int k = 0; k < N; ++k) m |= A.missing(id[k], w[k], tag);
-        return someMissing(m);
+        return m;
       },
       [&] { loadEntries(A, id, w); });
 #pragma unroll
@@ -240,11 +257,11 @@ __device__ __forceinline__ void awaitRest(const CoArray<TM>& A, const int (&id)[
 #pragma unroll
     for (int h = 0; h < CoArray<TM>::kHalves; ++h) pinned(w[k].h[h]);
 }
-template <typename TM, int N>
+template <bool kLanes, typename TM, int N>
 __device__ __forceinline__ void await(const CoArray<TM>& A, const int (&id)[N], unsigned tag, int* bad,
-                                      typename CoArray<TM>::Raw (&w)[N]) {
+                                      typename CoArray<TM>::Raw (&w)[N], unsigned least = 0x10000u) {
   loadEntries(A, id, w);
-  awaitRest(A, id, tag, bad, w);
+  awaitRest<kLanes>(A, id, tag, bad, w, least);
 }
 
 // Waits until this wavefront's stores have reached device scope (vmcnt 0;
@@ -401,28 +418,40 @@ __device__ __forceinline__ PassView uniformView(const PassView& s) {
 //     Lipschitz sums;
 //   takes the next pass's step as its bodies' tmp arrive, on the guess that
 //     this pass is accepted without a restart (then the next step size and
-//     momentum do not depend on the pass's sums), and stores its J;
+//     momentum do not depend on the pass's sums), and stores its J; and, on
+//     the same guess, P2 on the wavefront's first unit, whose tmp is then on
+//     its way while the pass is decided;
 //   decides the pass from the team's partial sums, as kDecide does, and takes
-//     the step again where the guess was wrong, under a second tag.
-// The decision takes every member's sums, so it is also what keeps a member
-// from storing over what another still reads: J of a contact is stored again
-// only after tmp of its bodies, which is formed from it, has arrived, and tmp
-// only after J of the body's contacts, formed from it; the partial sums
-// alternate between two places.
+//     the step and the unit again where the guess was wrong, under a second
+//     tag.
+// What keeps a member from storing over what another still reads: J of a
+// contact is stored again only after tmp of its bodies, which is formed from
+// it, has arrived, and tmp only after J of the body's contacts, formed from
+// it; a step taken again stores over one that a slower member may still wait
+// for, which takes either for its guess and drops what it made of it.  The
+// partial sums alternate between two places, and are stored after a decision,
+// which takes every member's.
 // The iterates go back to memory when the launch ends, and gammaHat's when it
 // leaves the registers.
 // Two wavefronts per SIMD (up to 256 VGPRs, one workgroup to a CU): held to
 // 128, so that a CU takes two, the mixed kernel spilled 20 and took 26.3 us
 // per pass on 256,000 contacts, where two rows per thread take 12.6.  (Two
 // rows in FP64 have no registers for a second step: without the guess.)
+// In FP64 a large team's members wait for J, twice as long, with loads that
+// take the others' room: us per pass with the unit taken ahead and not, 82
+// members (41,800 contacts) 8.2 and 7.8, 162 (82,400) 10.5 and 9.4, but 24
+// (11,900) 6.8 and 7.2; mixed 5.4 and 6.0, 5.8 and 6.8, 4.9 and 5.4.
+constexpr int kAheadMost = 64;
 template <typename TM, bool kBil, int R>
 __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, Tables T, const TeamItem* items, int stride,
                                                 u64* sync, u64 launch, int passes, u64 formTicks) {
   constexpr bool kMixed = sizeof(TM) < sizeof(double);
   constexpr bool kGuess = kMixed || R == 1;
+  constexpr bool kLanes = R == 1;
   constexpr int NF = kMixed ? 6 : 3;
   constexpr unsigned kUsed = kP1Slots<TM>;
   constexpr int kW = kTC / 64;       // wavefronts
+  constexpr int kStateWave = kW - 2;
   constexpr int kWT = kTP / 64;      // of a heavy body's sum
   constexpr int kUnits = kTB / 64;   // body units of a body tile
   using Raw = typename CoArray<TM>::Raw;
@@ -439,10 +468,11 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
   // the state before and after a pass; and, like the sums, for either parity:
   // a pass has one barrier, before its decision, which every wavefront takes
   __shared__ ApgdState shS[2];
-  __shared__ double shNext[2][6];
+  __shared__ double shTol;
+  __shared__ int shMaxIt;
+  __shared__ double shNext[3][6];  // (a pass's, the next one's, and the last one's, still read)
   __shared__ double shUnit[32][kW];  // the units' Lipschitz sums, and how many of a tile's are there
   __shared__ int unitCount[32][2];
-  __shared__ int nextFor;  // the pass that they belong to
   // per thread, kept here instead of in registers: the rows' frames and the
   // first body's contacts
   __shared__ TM shF[R][9][kTC];
@@ -451,13 +481,13 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
   if (tid < 64) unitCount[tid / 2][tid % 2] = 0;
   if (tid == 0) {
     bad = 0;
-    nextFor = -1;
+    shTol = a.dims.tol;
+    shMaxIt = a.dims.maxIt;
     shS[0] = STATE(T, me.slot, 1);
   }
   __syncthreads();
   if (shS[0].done) return;  // the same for every member
   PassView V = uniformView(viewOf(shS[0]));
-  double L = shS[0].L, theta = shS[0].theta;
   const long cap = a.cap;
   const CoArray<TM> J(a.J, cap + D.nbil), tmp(a.tmpX, D.nb);
   const int nBT = a.nBodyTiles, nHeavy = gl(a.counters)[2], nl = nBT + nHeavy;
@@ -627,7 +657,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       id[2 * u] = row[u].ia;
       id[2 * u + 1] = row[u].ib;
     }
-    await(tmp, id, tag, &bad, t);
+    await<kLanes>(tmp, id, tag, &bad, t);
 #pragma unroll
     for (int u = 0; u < R; ++u) rowsN(u, tmp.value(t[2 * u]), tmp.value(t[2 * u + 1]), next ? row[u].nn : row[u].nk);
   };
@@ -676,9 +706,73 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
     }
   };
 
+  auto bilateral = [&](const BodyRuns<TM>& b, unsigned tagJ, unsigned least, TM (&s)[3]) {
+    for (int k = b.b0; kBil && k < b.b1; ++k) {
+      const int e = gl(a.bilInc)[k];
+      const int i[1] = {(int)cap + (e >> 3)};
+      Raw x[1];
+      await<kLanes>(J, i, tagJ, &bad, x, least);
+      const double g = J.asDouble(x[0]);
+      const TM t = (TM)((e & 1) ? -g : g);
+      const int comp = (e >> 1) & 3;
+      if (comp == 0) s[0] += t; else if (comp == 1) s[1] += t; else s[2] += t;
+    }
+  };
+  auto contacts = [&](const BodyRuns<TM>& b, int kb, const Raw (&v)[kRun], TM (&s)[3]) {
+#pragma unroll
+    for (int k = 0; k < kRun; ++k) {
+      // (past the body's contacts zero, which changes no sum that began with zero)
+      const V3<TM> t = J.value(v[k]);
+      const TM sign = kb + k < b.nd ? -1 : 1;  // (times it is exact)
+      s[0] = exactFma(t.x, sign, s[0]); s[1] = exactFma(t.y, sign, s[1]); s[2] = exactFma(t.z, sign, s[2]);
+    }
+  };
+  auto moreContacts = [&](const BodyRuns<TM>& b, int kb, unsigned tagJ, unsigned least, TM (&s)[3]) {  // from its kb-th on
+    for (; __any(kb < b.n); kb += kRun) {
+      int id[kRun];
+      Raw v[kRun];
+#pragma unroll
+      for (int k = 0; k < kRun; ++k) id[k] = contactOf(a, b, kb + k);
+      await<kLanes>(J, id, tagJ, &bad, v, least);
+      contacts(b, kb, v, s);
+    }
+  };
+  // P2 on this wavefront's first unit, whose D^T gamma_k and D^T gamma_{k-1}
+  // stay in registers (mixed; dn the pass's, dg the guessed pass's)
+  V4<TM> dc{0, 0, 0, 0}, dp{0, 0, 0, 0}, dn{0, 0, 0, 0}, dg{0, 0, 0, 0};
+  double firstTerm = 0;
+  if (kMixed && first.sums) {
+    dc = ld4(a.sr, V.cur * (long)D.nb + first.g);
+    dp = ld4(a.sr, V.prev * (long)D.nb + first.g);
+  }
+  const bool ahead = kGuess && (kMixed || W <= kAheadMost);
+  auto firstUnit = [&](unsigned tagJ, unsigned least, const V4<TM>& c, const V4<TM>& p, bool mom, double beta, V4<TM>& out) {
+    if (!(live & 1u)) return;
+    int id[kRun];
+    Raw v[kRun];
+#pragma unroll
+    for (int k = 0; k < kRun; ++k) id[k] = shIds[k][tid];
+    await<kLanes>(J, id, tagJ, &bad, v, least);
+    TM s[3] = {0, 0, 0};
+    bilateral(first, tagJ, least, s);
+    contacts(first, 0, v, s);
+    moreContacts(first, kRun, tagJ, least, s);
+    if (first.sums) tmp.st(first.g, first.mi * s[0], first.mi * s[1], first.mi * s[2], tagJ);
+    firstTerm = lastSum(first.sums ? lipschitzOf(first.mi, s[0], s[1], s[2], c, p, mom, beta) : 0.0);
+    if (kMixed) out = V4<TM>{s[0], s[1], s[2], 0};
+  };
+
+  // the step sizes of a pass's either outcome, by a wavefront that has time
+  // (as for the state)
+  auto stepSizes = [&](int to, double fromL, double fromTheta) {
+    if (wave != kStateWave) return;
+    const StepNext n(fromL, fromTheta);
+    if (lane == 0) n.store(shNext[to]);
+  };
+
   int ends = 0;        // which state is the last
   bool taken = false;  // this pass's step was taken on the last one's guess
-  for (int p = 0; p < passes; ++p) {
+  for (int p = 0, sizes = 0; p < passes; ++p, sizes = sizes == 2 ? 0 : sizes + 1) {
     const int par = p & 1;
     const unsigned tag = (unsigned)(2 * p + 2) << 16;
     unsigned tagJ = tag;
@@ -706,6 +800,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
         step(u, w.gk, w.gm, w.nk, w.nm, mom, V.beta, V.t, w.gn, tagJ);
         sumsOf(par, u, w.gk, w.gm, w.gn, w.nk, w.nm, mom, V.beta);
       }
+      stepSizes(sizes, shS[par].L, shS[par].theta);  // (which its wavefront has stored)
       __syncthreads();
     }
     // the tiles' partial sums, by the last wavefront (which has the fewest
@@ -724,48 +819,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
     for (int h = rank + W * (64 + lane); wave == kW - 1 && h < nHeavy; h += W * 64)
       if (isFixed(h)) postLq(par, nBT + h, 0.0, tag);
 
-    // the step sizes of either outcome, by a wavefront that has time
-    if (wave == kW - 2) {
-      const StepNext n(L, theta);
-      if (lane == 0) {
-        n.store(shNext[par]);
-        __atomic_signal_fence(__ATOMIC_SEQ_CST);
-        __hip_atomic_store(&nextFor, p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-      }
-    }
-
     // ---- P2
-    auto bilateral = [&](const BodyRuns<TM>& b, TM (&s)[3]) {
-      for (int k = b.b0; kBil && k < b.b1; ++k) {
-        const int e = gl(a.bilInc)[k];
-        const int i[1] = {(int)cap + (e >> 3)};
-        Raw x[1];
-        await(J, i, tagJ, &bad, x);
-        const double g = J.asDouble(x[0]);
-        const TM t = (TM)((e & 1) ? -g : g);
-        const int comp = (e >> 1) & 3;
-        if (comp == 0) s[0] += t; else if (comp == 1) s[1] += t; else s[2] += t;
-      }
-    };
-    auto contacts = [&](const BodyRuns<TM>& b, int kb, const Raw (&v)[kRun], TM (&s)[3]) {
-#pragma unroll
-      for (int k = 0; k < kRun; ++k) {
-        // (past the body's contacts zero, which changes no sum that began with zero)
-        const V3<TM> t = J.value(v[k]);
-        const TM sign = kb + k < b.nd ? -1 : 1;  // (times it is exact)
-        s[0] = exactFma(t.x, sign, s[0]); s[1] = exactFma(t.y, sign, s[1]); s[2] = exactFma(t.z, sign, s[2]);
-      }
-    };
-    auto moreContacts = [&](const BodyRuns<TM>& b, int kb, TM (&s)[3]) {  // from its kb-th on
-      for (; __any(kb < b.n); kb += kRun) {
-        int id[kRun];
-        Raw v[kRun];
-#pragma unroll
-        for (int k = 0; k < kRun; ++k) id[k] = contactOf(a, b, kb + k);
-        await(J, id, tagJ, &bad, v);
-        contacts(b, kb, v, s);
-      }
-    };
     // a unit's Lipschitz sum; the last of a tile's four posts the tile's
     auto postUnit = [&](int j, int u, double term) {
       if (lane != kLast) return;
@@ -779,7 +833,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       postLq(par, u / kUnits, ((t[0] + t[1]) + t[2]) + t[3], tag);
     };
     auto finish = [&](const BodyRuns<TM>& b, int j, int u, const TM (&s)[3], const V4<TM>& c, const V4<TM>& p) {
-      if (b.sums) tmp.st(b.g, b.mi * s[0], b.mi * s[1], b.mi * s[2], tag);
+      if (b.sums) tmp.st(b.g, b.mi * s[0], b.mi * s[1], b.mi * s[2], tagJ);
       const double term = lastSum(b.sums ? lipschitzTerm(a, b.g, V, b.mi, s[0], s[1], s[2], c, p) : 0.0);
       postUnit(j, u, term);
     };
@@ -788,23 +842,8 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       c = ld4(a.sr, V.cur * (long)D.nb + g);
       p = ld4(a.sr, V.prev * (long)D.nb + g);
     };
-    if (live & 1u) {
-      int id[kRun];
-      Raw v[kRun];
-      V4<TM> c, p;
-#pragma unroll
-      for (int k = 0; k < kRun; ++k) id[k] = shIds[k][tid];
-      loadRing(first.g, c, p);
-      loadEntries(J, id, v);
-      awaitRest(J, id, tagJ, &bad, v);
-      TM s[3] = {0, 0, 0};
-      bilateral(first, s);
-      contacts(first, 0, v, s);
-      moreContacts(first, kRun, s);
-      finish(first, 0, u0, s, c, p);
-    } else if (u0 < nU) {
-      postUnit(0, u0, 0.0);
-    }
+    if (!(taken && ahead)) firstUnit(tagJ, 0x10000u, dc, dp, mom, V.beta, dn);
+    if (u0 < nU) postUnit(0, u0, firstTerm);  // (zero where nothing is live)
     for (int j = 1, u = u0 + uStep; u < nU; ++j, u += uStep) {
       if (!((live >> j) & 1u)) {
         postUnit(j, u, 0.0);
@@ -814,8 +853,12 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       V4<TM> c, p;
       loadRing(b.g, c, p);
       TM s[3] = {0, 0, 0};
-      bilateral(b, s);
-      moreContacts(b, 0, s);
+      bilateral(b, tagJ, 0x10000u, s);
+      moreContacts(b, 0, tagJ, 0x10000u, s);
+      if (kMixed) {
+        settled(c);
+        settled(p);
+      }
       finish(b, j, u, s, c, p);
     }
     // bodies with many contacts, by the first kTP threads
@@ -838,7 +881,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
             const int k = kb + i * kTP;
             id[i] = k < nd ? gl(a.inc)[k0 + k] >> 1 : k < n ? c0 + k - nd : kNone;
           }
-          await(J, id, tagJ, &bad, v);
+          await<kLanes>(J, id, tagJ, &bad, v);
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
             const int k = kb + i * kTP;
@@ -855,7 +898,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
             const int e = gl(a.bilInc)[k];
             const int i[1] = {(int)cap + (e >> 3)};
             Raw x[1];
-            await(J, i, tagJ, &bad, x);
+            await<kLanes>(J, i, tagJ, &bad, x);
             const double v = J.asDouble(x[0]), t = (e & 1) ? -v : v;
             const int comp = (e >> 1) & 3;
             if (comp == 0) hx += t; else if (comp == 1) hy += t; else hz += t;
@@ -866,6 +909,10 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
           shH[wave][0] = hx; shH[wave][1] = hy; shH[wave][2] = hz;
         }
       }
+      if (kMixed) {
+        settled(c);
+        settled(p);
+      }
       __syncthreads();
       if (tid == 0) {
         TM t[3];
@@ -874,7 +921,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
           for (int w = 1; w < kWT; ++w) v += shH[w][s];
           t[s] = (TM)v;
         }
-        tmp.st(g, mi * t[0], mi * t[1], mi * t[2], tag);
+        tmp.st(g, mi * t[0], mi * t[1], mi * t[2], tagJ);
         postLq(par, nBT + h, lipschitzTerm(a, g, V, mi, t[0], t[1], t[2], c, p), tag);
       }
       __syncthreads();
@@ -882,11 +929,8 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
 
     // ---- the next pass's step, should this one be accepted without a restart
     const bool guess = kGuess && p + 1 < passes;
-    if (guess) rowsOfArrived(tag, true);
-    while (__any(__hip_atomic_load(&nextFor, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) != p)) {
-    }  // (its wavefront waits for nothing before that)
-    __atomic_signal_fence(__ATOMIC_SEQ_CST);
-    const double tNext = uniformDouble(shNext[par][3]), betaNext = uniformDouble(shNext[par][5]);
+    if (guess) rowsOfArrived(tagJ, true);
+    const double tNext = uniformDouble(shNext[sizes][3]), betaNext = uniformDouble(shNext[sizes][5]);
     // The team's sums, in reduceSlots' order: lane l of its wavefront i adds
     // entries 64 i + l, 64 i + l + kTP, ..., and the wavefronts' sums are added
     // in order (past the entries they are zero, and left out).  Here wavefront
@@ -920,19 +964,21 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
         const Row& w = row[u];
         sumsOf(par ^ 1, u, w.gn, w.gk, w.gs, w.nn, w.nk, true, betaNext);
       }
+    if (guess) stepSizes(sizes == 2 ? 0 : sizes + 1, shNext[sizes][2], shNext[sizes][4]);  // (those of the guessed outcome)
     if (sumsPart) loadPart(0);
     if (sumsLq) loadLq(0);
+    if (guess && ahead) firstUnit(tag + (2u << 16), kOrReplaced, dn, dc, true, betaNext, dg);
     if (sumsPart) {
       double v[kWT] = {0, 0, 0, 0};
       for (int b0 = 0; b0 < nTiles; b0 += kTP) {
         if (b0) loadPart(b0);
-        waitFor(
-            &bad,
+        waitFor<false>(
+            &bad, 0x10000u,
             [&] {
               unsigned m = 0;
 #pragma unroll
               for (int i = 0; i < kWT; ++i) m |= b0 + 64 * i + lane < nTiles ? missing(xp[i], tag) : 0u;
-              return someMissing(m);
+              return m;
             },
             [&] { loadPart(b0); });
 #pragma unroll
@@ -950,8 +996,8 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       for (int b0 = 0; b0 + 64 * il < nl; b0 += kTP) {
         if (b0) loadLq(b0);
         const int w = b0 + 64 * il + lane;
-        waitFor(
-            &bad, [&] { return someMissing(w < nl ? missing(xl, tag) : 0u); }, [&] { loadLq(b0); });
+        waitFor<false>(
+            &bad, 0x10000u, [&] { return w < nl ? missing(xl, tag) : 0u; }, [&] { loadLq(b0); });
         pinned(xl);
         v += valueOf(xl);
       }
@@ -962,28 +1008,89 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
 
     // ---- the decision, by every member's every wavefront
     __syncthreads();
-    const bool lost = bad != 0;  // (set by waits only, which all lie before this point)
-    double tot[2 * kSlots];
+    const bool lost = __builtin_amdgcn_readfirstlane(bad) != 0;  // (set by waits only, which all lie before this point)
+    const ApgdState& before = shS[par];
+    double lq = shLq[par][0];
 #pragma unroll
-    for (int k = 0; k < 2 * kSlots; ++k) tot[k] = 0.0;
-#pragma unroll
-    for (int k = 0; k < kSlots; ++k)
-      if ((kUsed >> k) & 1u) tot[k] = shTot[par][k];
-    tot[kSlots + 6] = shLq[par][0];
-    for (int i = 1; i < kWT && 64 * i < nl; ++i) tot[kSlots + 6] += shLq[par][i];
-    ApgdState S = shS[par];
-    decideStep<kMixed>(S, tot, D, StepNext(shNext[par]));
-    if (tid == 0) shS[par ^ 1] = S;
+    for (int i = 1; i < kWT; ++i) {
+      const double more = lq + shLq[par][i];
+      lq = 64 * i < nl ? more : lq;
+    }
     const int dropped = V.prev;
-    V = uniformView(viewOf(S));
-    L = S.L;
-    theta = S.theta;
+    bool keep = false;  // gammaHat leaves the registers
+    // most passes are accepted without a restart, as decideStep has it
+    // (all loads at once, and no branch between them)
+    const double res = shTot[par][kSlots - 1], best = before.best, tol = shTol, stepL = before.L;
+    const int pending = before.pendingRes, it = before.it, maxIt = shMaxIt, hatBefore = before.hatSrc;
+    double t[6];
+#pragma unroll
+    for (int k = 0; k < 6; ++k) t[k] = (kUsed >> k) & 1u ? shTot[par][k] : 0.0;
+    const bool better = res < best;
+    bool goesOn = (pending != 0) & (res < INFINITY) & !((better ? res : best) < tol) & (it < maxIt) & !(t[5] > 0);
+    if (kMixed) {
+      goesOn = goesOn & !(lq >= stepL * t[4]);
+    } else {
+      const double obj1 = 0.5 * lq + t[0], nrm = sqrt(t[4]);
+      double obj2 = 0.5 * t[1] + t[2];
+      obj2 += t[3] + 0.5 * stepL * (nrm * nrm);
+      goesOn = goesOn & !(obj1 >= obj2);
+    }
+    if (__any(goesOn)) {  // (alike in all lanes)
+      const int hat = __any(better) ? V.cur : __builtin_amdgcn_readfirstlane(hatBefore);
+      V.prev = V.cur;
+      V.cur = V.nxt;
+      V.nxt = __builtin_ctz(~(1u << V.cur | 1u << V.prev | 1u << hat));
+      V.flags = kViewFresh;
+      V.t = tNext;
+      V.beta = betaNext;
+      keep = hat == dropped;
+      if (wave == kStateWave) {
+        ApgdState S = before;
+        const StepNext n(shNext[sizes]);
+        S.passes++;
+        S.best = better ? res : best;
+        S.hatSrc = hat;
+        S.beta = n.beta;
+        S.restart = 0;
+        S.L = n.La;
+        S.t = n.ta;
+        S.theta = n.thetaNew;
+        S.prev = V.prev;
+        S.cur = V.cur;
+        S.nxt = V.nxt;
+        S.it++;
+        S.bt = 0;
+        S.pendingRes = 1;
+        S.fresh = 1;
+        if (lane == 0) shS[par ^ 1] = S;
+      }
+    } else {
+      double tot[2 * kSlots];
+#pragma unroll
+      for (int k = 0; k < 2 * kSlots; ++k) tot[k] = 0.0;
+#pragma unroll
+      for (int k = 0; k < kSlots; ++k)
+        if ((kUsed >> k) & 1u) tot[k] = shTot[par][k];
+      tot[kSlots + 6] = lq;
+      ApgdState S = before;
+      SolveDims limits = D;  // (of these two only, and not from memory)
+      limits.tol = shTol;
+      limits.maxIt = shMaxIt;
+      decideStep<kMixed>(S, tot, limits, StepNext(shNext[sizes]));
+      if (wave == kStateWave && lane == 0) shS[par ^ 1] = S;
+      V = uniformView(viewOf(S));
+      keep = __builtin_amdgcn_readfirstlane(S.hatSrc) == dropped;
+    }
     ends = par ^ 1;
     if (lost || (V.flags & kViewDone)) break;
     taken = false;
     if (V.flags & kViewFresh) {  // accepted: gamma_new becomes gamma_k (a backtrack keeps both)
-      const bool keep = __builtin_amdgcn_readfirstlane(S.hatSrc) == dropped;  // gammaHat leaves the registers
       taken = kGuess && !(V.flags & kViewRestart) && V.t == tNext && V.beta == betaNext;
+      if (kMixed) {
+        dp = dc;
+        dc = dn;
+        dn = dg;
+      }
 #pragma unroll
       for (int u = 0; u < R; ++u) {
         Row& w = row[u];
@@ -1016,7 +1123,13 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       if (!(V.flags & kViewFresh)) gl(a.rn[0] + V.cur * a.ringStride)[f] = w.nk[rr];
     }
   }
-  if (V.flags & kViewFresh) {  // (from the thread's own stores)
+  if (kMixed && first.sums) {
+    if (V.prev != V.cur) st4(a.sr, V.prev * (long)D.nb + first.g, dp);
+    st4(a.sr, V.cur * (long)D.nb + first.g, dc);
+  }
+  // (from the thread's own stores; after the last decision of a solve nothing
+  // reads tmp, and it may hold a guess)
+  if ((V.flags & (kViewFresh | kViewDone)) == kViewFresh) {
     for (int u = u0; u < nU; u += uStep) {
       const BodyRuns<TM> b = bodyRuns(a, (long)u * 64 + lane);
       if (!b.sums) continue;
@@ -1030,7 +1143,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       st4(a.tmp, g, V4<TM>{t.x, t.y, t.z, (TM)0});
     }
   }
-  if (rank == 0 && tid == 0) {
+  if (rank == 0 && tid == 64 * kStateWave) {
     ApgdState S = shS[ends];
     if (bad) {  // a member was lost (never seen): the solve ends as diverged
       S.done = 1;
