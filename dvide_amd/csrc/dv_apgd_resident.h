@@ -441,6 +441,10 @@ __device__ __forceinline__ PassView uniformView(const PassView& s) {
 // take the others' room: us per pass with the unit taken ahead and not, 82
 // members (41,800 contacts) 8.2 and 7.8, 162 (82,400) 10.5 and 9.4, but 24
 // (11,900) 6.8 and 7.2; mixed 5.4 and 6.0, 5.8 and 6.8, 4.9 and 5.4.
+// Where bodies outnumber contacts so far that both wavefronts of a SIMD have a
+// unit, their waits cannot hide behind each other's steps: a shell's 19,200
+// spheres with 20,100 contacts 6.4 ahead and 6.1 not; but with two rows a thread
+// (112,000 spheres, 256,000 contacts) 10.7 ahead and 12.0 not.
 constexpr int kAheadMost = 64;
 template <typename TM, bool kBil, int R>
 __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, Tables T, const TeamItem* items, int stride,
@@ -473,6 +477,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
   __shared__ double shNext[3][6];  // (a pass's, the next one's, and the last one's, still read)
   __shared__ double shUnit[32][kW];  // the units' Lipschitz sums, and how many of a tile's are there
   __shared__ int unitCount[32][2];
+  __shared__ u64 liveTiles;  // bit t: tile rank + W t has a unit with a movable light body
   // per thread, kept here instead of in registers: the rows' frames and the
   // first body's contacts
   __shared__ TM shF[R][9][kTC];
@@ -481,6 +486,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
   if (tid < 64) unitCount[tid / 2][tid % 2] = 0;
   if (tid == 0) {
     bad = 0;
+    liveTiles = 0;
     shTol = a.dims.tol;
     shMaxIt = a.dims.maxIt;
     shS[0] = STATE(T, me.slot, 1);
@@ -569,14 +575,16 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       if (!(w.bil && rr)) gl(a.ring[0] + slot * a.ringStride)[flatOf(u, rr)] = g[rr];
   };
 
-  // (a unit without a movable light body only has a zero sum)
   const BodyRuns<TM> first = bodyRuns(a, u0 < nU ? (long)u0 * 64 + lane : (long)D.nb);
 #pragma unroll
   for (int k = 0; k < kRun; ++k) shIds[k][tid] = contactOf(a, first, k);
   unsigned live = 0;
   for (int j = 0, u = u0; u < nU; ++j, u += uStep) {
     const int g = u * 64 + lane;
-    if (__any(bodyRuns(a, (long)g).sums)) live |= 1u << j;
+    if (__any(bodyRuns(a, (long)g).sums)) {
+      live |= 1u << j;
+      if (lane == 0) __hip_atomic_fetch_or(&liveTiles, 1ull << (2 * j + half), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
     if (g < D.nb) tmp.st(g, 0, 0, 0, 0);
     if (wave % kUnits == 0 && lane == kLast)
       for (int k = 0; k < 2; ++k) postLq(k, u / kUnits, 0.0, 0);
@@ -598,6 +606,15 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       for (int k = 0; k < 2; ++k) postPart(k, s * nTiles + R * rank + u, 0.0, 0);
   }
   if (!teamForm(sy, rank, W, launch, formTicks)) return;
+  // The zero sums of tiles of fixed bodies only are posted by lane t of the
+  // last wavefront; of the others, a unit without a movable light body has a
+  // zero sum.
+  const u64 tiles = liveTiles;
+  unsigned units = 0;  // this wavefront's units of live tiles
+  for (int j = 0, u = u0; u < nU; ++j, u += uStep)
+    if ((tiles >> (2 * j + half)) & 1u) units |= 1u << j;
+  units = __builtin_amdgcn_readfirstlane(units);
+  const bool fixedTile = wave == kW - 1 && rank + W * lane < nBT && !((tiles >> lane) & 1u);
 
   // y, N y and g of a row (formed once for the step and again for the sums,
   // rather than kept)
@@ -745,7 +762,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
     dc = ld4(a.sr, V.cur * (long)D.nb + first.g);
     dp = ld4(a.sr, V.prev * (long)D.nb + first.g);
   }
-  const bool ahead = kGuess && (kMixed || W <= kAheadMost);
+  const bool ahead = kGuess && (R == 2 || __popcll(tiles) <= 1) && (kMixed || W <= kAheadMost);
   auto firstUnit = [&](unsigned tagJ, unsigned least, const V4<TM>& c, const V4<TM>& p, bool mom, double beta, V4<TM>& out) {
     if (!(live & 1u)) return;
     int id[kRun];
@@ -815,6 +832,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       for (int w = 1; w < kW; ++w) v = s == kSlots - 1 ? fmax(v, t[w]) : v + t[w];
       if (R * rank + u < nTiles) postPart(par, s * nTiles + R * rank + u, v, tag);
     }
+    if (fixedTile) postLq(par, rank + W * lane, 0.0, tag);
     if (fixedHeavy) postLq(par, nBT + rank + W * lane, 0.0, tag);
     for (int h = rank + W * (64 + lane); wave == kW - 1 && h < nHeavy; h += W * 64)
       if (isFixed(h)) postLq(par, nBT + h, 0.0, tag);
@@ -843,8 +861,9 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       p = ld4(a.sr, V.prev * (long)D.nb + g);
     };
     if (!(taken && ahead)) firstUnit(tagJ, 0x10000u, dc, dp, mom, V.beta, dn);
-    if (u0 < nU) postUnit(0, u0, firstTerm);  // (zero where nothing is live)
-    for (int j = 1, u = u0 + uStep; u < nU; ++j, u += uStep) {
+    if (units & 1u) postUnit(0, u0, firstTerm);  // (zero where nothing is live)
+    for (unsigned left = units & ~1u; left; left &= left - 1) {
+      const int j = __builtin_ctz(left), u = u0 + j * uStep;
       if (!((live >> j) & 1u)) {
         postUnit(j, u, 0.0);
         continue;
