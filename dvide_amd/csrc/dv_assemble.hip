@@ -17,25 +17,20 @@ namespace {
 constexpr int kT = 256;
 
 // k = M v + h f - h f_elastic  (System.cu:1411-1417, 1502-1514; f_elastic = 0 for bodies)
+// and y = M^-1 k (diagonal COO: 0.0 + minv * k)
 __global__ __launch_bounds__(kT) void kBuildK(int nb, const double* __restrict__ minv,
                                               const double* __restrict__ v, const double* __restrict__ f,
-                                              double* __restrict__ k, double h) {
+                                              double* __restrict__ k, double* __restrict__ y, double h) {
   int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i >= 3 * nb) return;
-  double m = minv[i / 3];
-  if (m != 0) m = 1.0 / m;
+  const double mi = minv[i / 3];
+  const double m = mi != 0 ? 1.0 / mi : mi;
   double kk = m * v[i];
   const double fEl = 0.0;
-  k[i] = (h * f[i] + (-h) * fEl) + 1.0 * kk;
-}
-
-// y = M^-1 x per DOF (diagonal COO: 0.0 + minv * x)
-__global__ __launch_bounds__(kT) void kMinv(int nb, const double* __restrict__ minv,
-                                            const double* __restrict__ x, double* __restrict__ y) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= 3 * nb) return;
+  kk = (h * f[i] + (-h) * fEl) + 1.0 * kk;
+  k[i] = kk;
   double s = 0.0;
-  s = s + minv[i / 3] * x[i];
+  s = s + mi * kk;
   y[i] = s;
 }
 
@@ -48,16 +43,15 @@ struct RowArgs {
   const int* bilB;
 };
 
-// y = D x  (+ optional b: y = 1.0*b + D x), one thread per contact / bilateral row
-__global__ __launch_bounds__(kT) void kRowsD(RowArgs a, const double* __restrict__ x,
-                                             const double* __restrict__ badd, double* __restrict__ y) {
-  int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= a.nc + a.nbil) return;
+// row q of D x, one thread per contact / bilateral row; put(row, value) takes
+// its values
+template <class Put>
+__device__ __forceinline__ void rowOfD(const RowArgs& a, int q, const double* __restrict__ x, const Put& put) {
   if (q < a.nbil) {
     double s = 0.0;
     s = s + 1.0 * x[a.bilA[q]];
     if (a.bilB[q] >= 0) s = s + (-1.0) * x[a.bilB[q]];
-    y[q] = badd ? 1.0 * badd[q] + s : s;
+    put(q, 0, s);
     return;
   }
   const int c = q - a.nbil;
@@ -77,9 +71,16 @@ __global__ __launch_bounds__(kT) void kRowsD(RowArgs a, const double* __restrict
     s = s + (-f0) * xb0;
     s = s + (-f1) * xb1;
     s = s + (-f2) * xb2;
-    const int row = a.nbil + 3 * c + rr;
-    y[row] = badd ? 1.0 * badd[row] + s : s;
+    put(a.nbil + 3 * c + rr, rr, s);
   }
+}
+
+// y = D x  (+ optional b: y = 1.0*b + D x)
+__global__ __launch_bounds__(kT) void kRowsD(RowArgs a, const double* __restrict__ x,
+                                             const double* __restrict__ badd, double* __restrict__ y) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= a.nc + a.nbil) return;
+  rowOfD(a, q, x, [&](int row, int, double s) { y[row] = badd ? 1.0 * badd[row] + s : s; });
 }
 
 // f = D^T x and tmp = M^-1 f per body, terms in D^T row order.  With
@@ -175,26 +176,30 @@ __global__ __launch_bounds__(kT) void kGatherHeavy(GatherArgs a, const int* heav
 }
 
 // b: bilateral rows violation / h (System.cu:1526-1544), contact rows
-// (gap/h, 0, 0) (System.cu:1516-1524)
-__global__ __launch_bounds__(kT) void kStab(int nc, int nbil, const double* __restrict__ gap,
-                                            const int* bilA, const int* bilB, const double* bilVel,
-                                            const double* bilT0, const double* bilP0,
-                                            const double* __restrict__ p, double h, double time,
-                                            double* __restrict__ b) {
-  int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nc + nbil) return;
-  if (q < nbil) {
+// (gap/h, 0, 0) (System.cu:1516-1524); and r = D M^-1 k + b.  Launches bound
+// the assembly of small scenes: k, M^-1 k, b and r in four took 25 us of one
+// sphere's step, in two 12.
+__global__ __launch_bounds__(kT) void kBuildR(RowArgs a, const double* __restrict__ gap, const double* bilVel,
+                                              const double* bilT0, const double* bilP0,
+                                              const double* __restrict__ p, const double* __restrict__ x, double h,
+                                              double time, double* __restrict__ b, double* __restrict__ r) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= a.nc + a.nbil) return;
+  double first;
+  if (q < a.nbil) {
     double vel = bilVel[q], t0 = bilT0[q];
     if (time < t0) vel = 0;
-    double viol = bilB[q] < 0 ? p[bilA[q]] - bilP0[q] - vel * (time - t0)
-                              : p[bilA[q]] - p[bilB[q]] - vel * (time - t0);
-    b[q] = viol / h;
-    return;
+    double viol = a.bilB[q] < 0 ? p[a.bilA[q]] - bilP0[q] - vel * (time - t0)
+                                : p[a.bilA[q]] - p[a.bilB[q]] - vel * (time - t0);
+    first = viol / h;
+  } else {
+    first = gap[q - a.nbil] / h;
   }
-  const int c = q - nbil;
-  b[nbil + 3 * c] = gap[c] / h;
-  b[nbil + 3 * c + 1] = 0;
-  b[nbil + 3 * c + 2] = 0;
+  rowOfD(a, q, x, [&](int row, int rr, double s) {
+    const double bb = rr ? 0.0 : first;
+    b[row] = bb;
+    r[row] = 1.0 * bb + s;
+  });
 }
 
 // v = M^-1 (k + f_c), f_c /= h, p += h v  (System.cu:570-581)
@@ -241,7 +246,7 @@ void fillDevice(Scene& s, double* x, long n, double v) {
 
 void buildK(Scene& s) {
   hipLaunchKernelGGL(kBuildK, dim3(blocksFor(3L * s.nb, kT)), dim3(kT), 0, s.stream, s.nb, s.minv.p, s.v.p,
-                     s.f.p, s.k.p, s.h);
+                     s.f.p, s.k.p, s.tmp.p, s.h);
 }
 
 void ensureRowBuffers(Scene& s) {
@@ -256,17 +261,14 @@ void ensureRowBuffers(Scene& s) {
   s.gammaLen = R;
 }
 
-// r = D M^-1 k + b  (System.cu:1561-1580)
+// r = D M^-1 k + b  (System.cu:1561-1580), from the M^-1 k that buildK left in
+// tmp
 void buildR(Scene& s) {
   ensureRowBuffers(s);
-  const hipStream_t st = s.stream;
-  hipLaunchKernelGGL(kMinv, dim3(blocksFor(3L * s.nb, kT)), dim3(kT), 0, st, s.nb, s.minv.p, s.k.p, s.tmp.p);
   const int items = s.nc + s.nbil;
   if (items == 0) return;
-  hipLaunchKernelGGL(kStab, dim3(blocksFor(items, kT)), dim3(kT), 0, st, s.nc, s.nbil, s.gap.p, s.bilA.p,
-                     s.bilB.p, s.bilVel.p, s.bilT0.p, s.bilP0.p, s.p.p, s.h, s.time, s.b.p);
-  hipLaunchKernelGGL(kRowsD, dim3(blocksFor(items, kT)), dim3(kT), 0, st, rowArgs(s), (const double*)s.tmp.p,
-                     (const double*)s.b.p, s.r.p);
+  hipLaunchKernelGGL(kBuildR, dim3(blocksFor(items, kT)), dim3(kT), 0, s.stream, rowArgs(s), s.gap.p, s.bilVel.p,
+                     s.bilT0.p, s.bilP0.p, s.p.p, (const double*)s.tmp.p, s.h, s.time, s.b.p, s.r.p);
 }
 
 static void gatherExact(Scene& s, const double* x, double* fOut, double* tmpOut, bool skipFixed) {

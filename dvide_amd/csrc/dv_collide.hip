@@ -130,6 +130,76 @@ __global__ __launch_bounds__(kT) void scatterSmall(CdArgs a, const unsigned* slo
   a.meta[pos] = make_int4(g, rowKey(cellCoord(pg.y, a.cs), cellCoord(pg.z, a.cs)), a.family[g], 0);
 }
 
+// The same in one workgroup, the counts in LDS, for a table of up to kSortMost
+// slots: clearing, hashing, two scan kernels and scattering are five launches
+// of 3 to 5 us each, whatever the scene's size.  Collision detection of a step
+// with the launches and so (and with the merged ones below): one sphere 66 and
+// 40 us, 1,000 spheres 85 and 52, 4,000 78 and 67; with a larger table one
+// workgroup takes longer than the launches: 8,001 spheres 96, against 77.
+constexpr int kSortT = 1024;
+constexpr int kSortMost = 8192;  // slots: 4,096 small geometries at most
+__global__ __launch_bounds__(kSortT) void sortSmall(CdArgs a, unsigned* slotStart, int* counters) {
+  constexpr int kPer = kSortMost / kSortT;       // slots of a thread
+  constexpr int kOwn = kSortMost / 2 / kSortT;   // its geometries
+  __shared__ unsigned count[kSortMost];
+  __shared__ unsigned waveSums[kSortT / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int T = (int)a.mask + 1;
+  for (int k = tid; k < T; k += kSortT) count[k] = 0;
+  if (tid < 8) counters[tid] = 0;
+  __syncthreads();
+  int id[kOwn], key[kOwn];
+  unsigned slot[kOwn], place[kOwn];
+  d3 pos[kOwn];
+#pragma unroll
+  for (int q = 0; q < kOwn; ++q) {
+    const int t = q * kSortT + tid;
+    id[q] = t < a.nsmall ? a.smallIds[t] : -1;
+    if (id[q] < 0) continue;
+    pos[q] = ldPos(a.p, id[q]);
+    const int cy = cellCoord(pos[q].y, a.cs), cz = cellCoord(pos[q].z, a.cs);
+    slot[q] = (rowHash(cy, cz) + (unsigned)cellCoord(pos[q].x, a.cs)) & a.mask;
+    key[q] = rowKey(cy, cz);
+    place[q] = atomicAdd(&count[slot[q]], 1u);
+  }
+  __syncthreads();
+  // exclusive scan: T / kSortT slots to a thread
+  const int per = T / kSortT;
+  unsigned sum = 0, v[kPer];
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    v[q] = q < per ? count[tid * per + q] : 0u;
+    sum += v[q];
+  }
+  unsigned x = sum;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const unsigned y = __shfl_up(x, d, 64);
+    if (lane >= d) x += y;
+  }
+  if (lane == 63) waveSums[wave] = x;
+  __syncthreads();
+  unsigned at = x - sum;
+#pragma unroll
+  for (int w = 0; w < kSortT / 64; ++w) at += w < wave ? waveSums[w] : 0u;
+#pragma unroll
+  for (int q = 0; q < kPer; ++q) {
+    if (q >= per) continue;
+    count[tid * per + q] = at;
+    slotStart[tid * per + q] = at;
+    at += v[q];
+  }
+  if (tid == kSortT - 1) slotStart[T] = at;
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kOwn; ++q) {
+    if (id[q] < 0) continue;
+    const unsigned k = count[slot[q]] + place[q];
+    a.posR[k] = PosR{pos[q].x, pos[q].y, pos[q].z, a.geom[3 * (size_t)id[q]]};
+    a.meta[k] = make_int4(id[q], key[q], a.family[id[q]], 0);
+  }
+}
+
 // The partners of small geometries, sixteen lanes to each: nine lanes walk a
 // row of three cells, the others test the big list.  A candidate is refused
 // by the squared distance first (with a margin far above the rounding of the
@@ -144,8 +214,8 @@ constexpr int kList = 24;
 constexpr int kLanes = 16;
 constexpr int kGroups = kT / kLanes;
 template <bool kCsr>
-__global__ __launch_bounds__(kT) void walkSmall(CdArgs a, int* cntUp, int* cntDown, int* lists, int* over,
-                                                const int* iStart, int* csr) {
+__device__ void walkSmall(const CdArgs& a, int* cntUp, int* cntDown, int* lists, int* over, const int* iStart,
+                          int* csr) {
   __shared__ int found[kGroups], above[kGroups], ids[kGroups][kList];
   const int lane = threadIdx.x % kLanes, grp = threadIdx.x / kLanes;
   const int t = blockIdx.x * kGroups + grp;
@@ -237,9 +307,10 @@ __device__ int blockSum(int v) {
 // for eight rounds in turn (26 + 11 us at 112,000 spheres).
 constexpr int kChunk = 512;
 
-__global__ __launch_bounds__(kT) void countBigChunks(CdArgs a, int nchunks, int* chUp, int* chDown) {
-  const int b = a.bigIds[blockIdx.y];
-  const int j0 = blockIdx.x * kChunk, j1 = min(a.nb, j0 + kChunk);
+__device__ void countBigChunk(const CdArgs& a, int q, int chunk, int nchunks, int* chUp, int* chDown, int* cntUp,
+                              int* cntDown) {
+  const int b = a.bigIds[q];
+  const int j0 = chunk * kChunk, j1 = min(a.nb, j0 + kChunk);
   int up = 0, down = 0;
   for (int j = j0 + threadIdx.x; j < j1; j += kT) {
     if (j == b) continue;
@@ -250,9 +321,29 @@ __global__ __launch_bounds__(kT) void countBigChunks(CdArgs a, int nchunks, int*
   up = blockSum(up);
   down = blockSum(down);
   if (threadIdx.x == 0) {
-    chUp[blockIdx.y * nchunks + blockIdx.x] = up;
-    chDown[blockIdx.y * nchunks + blockIdx.x] = down;
+    const bool only = nchunks == 1;  // then there is nothing to scan
+    chUp[q * nchunks + chunk] = only ? 0 : up;
+    chDown[q * nchunks + chunk] = only ? 0 : down;
+    if (only) {
+      cntUp[b] = up;
+      cntDown[b] = down;
+    }
   }
+}
+
+// The walk of the small geometries in the first walkBlocks workgroups and the
+// big ones' chunks in the others, which need nothing of each other.
+__global__ __launch_bounds__(kT) void countPartners(CdArgs a, int walkBlocks, int nchunks, int* cntUp, int* cntDown,
+                                                    int* lists, int* over, int* chUp, int* chDown) {
+  if ((int)blockIdx.x < walkBlocks) {
+    walkSmall<false>(a, cntUp, cntDown, lists, over, nullptr, nullptr);
+  } else {
+    const int k = (int)blockIdx.x - walkBlocks;
+    countBigChunk(a, k / nchunks, k % nchunks, nchunks, chUp, chDown, cntUp, cntDown);
+  }
+}
+__global__ __launch_bounds__(kT) void listPartners(CdArgs a, int* over, const int* iStart, int* csr) {
+  walkSmall<true>(a, nullptr, nullptr, nullptr, over, iStart, csr);
 }
 
 // per big geometry: exclusive scan of its chunk counts (in place) and totals,
@@ -288,9 +379,10 @@ __global__ __launch_bounds__(64) void scanBigChunks(CdArgs a, int nchunks, int* 
 // that everything summed over them is summed in a fixed order: one scan of
 // three counts, tile sums and then the tiles, each workgroup of which adds up
 // the tiles before its own (past kDirectTiles, scanBodyTiles does that for
-// all).  The totals go to the host's pinned memory as well.
+// all; up to kCountTiles, the counts before it themselves, a launch less).  The totals go to the host's pinned memory as well.
 constexpr int kBodyTile = 1024;
 constexpr int kDirectTiles = 1024;
+constexpr int kCountTiles = 8;
 struct Counts3 {
   int up, all, heavy;
 };
@@ -333,12 +425,16 @@ __global__ __launch_bounds__(64) void scanBodyTiles(int* sums, int tiles) {
   }
 }
 __global__ __launch_bounds__(kT) void scanBodies(int nb, const int* cntUp, const int* cntDown, const int* sums,
-                                                 int scanned, int* cStart, int* iStart, int* heavy, int* counters,
+                                                 int tiles, int* cStart, int* iStart, int* heavy, int* counters,
                                                  int* host) {
   __shared__ int waveUp[kT / 64], waveAll[kT / 64], waveHeavy[kT / 64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tile = blockIdx.x;
   Counts3 base{0, 0, 0};
-  if (scanned) {
+  if (tiles <= kCountTiles) {
+    Counts3 s{0, 0, 0};
+    for (int g = threadIdx.x; g < tile * kBodyTile; g += kT) s = add3c(s, countsOf(cntUp, cntDown, g, nb));
+    base = Counts3{blockSum(s.up), blockSum(s.all), blockSum(s.heavy)};
+  } else if (tiles > kDirectTiles) {
     base = Counts3{sums[3 * (size_t)tile], sums[3 * (size_t)tile + 1], sums[3 * (size_t)tile + 2]};
   } else {
     Counts3 s{0, 0, 0};
@@ -442,7 +538,7 @@ __device__ __forceinline__ void writeRecord(const CdArgs& a, const EmitOut& o, i
 
 // Rows of the small geometries, in id order and four lanes to each, so that a
 // wavefront writes one run of contacts.
-__global__ __launch_bounds__(kT) void emitSmall(CdArgs a, EmitOut o) {
+__device__ void emitSmall(const CdArgs& a, const EmitOut& o) {
   const int t = (blockIdx.x * blockDim.x + threadIdx.x) >> 2, lane = threadIdx.x & 3;
   if (t >= a.nsmall) return;
   const int g = a.smallIds[t];
@@ -456,16 +552,29 @@ __global__ __launch_bounds__(kT) void emitSmall(CdArgs a, EmitOut o) {
   }
 }
 
-// big geometry rows: ordered stream compaction of each chunk's partners (of
-// those below it, the ids for now: placeBig)
-__global__ __launch_bounds__(kT) void emitBigChunks(CdArgs a, EmitOut o, int nchunks, const int* chUp,
-                                                    const int* chDown) {
-  const int b = a.bigIds[blockIdx.y];
-  const int j0 = blockIdx.x * kChunk, j1 = min(a.nb, j0 + kChunk);
+// Contact c = (A, B) of a small geometry A with a big one B above it: A's
+// contacts are its partners above it, in order.
+__device__ __forceinline__ int contactWith(const EmitOut& o, int A, int B) {
+  const int* L = listOf(o, A);
+  const int nd = o.cntDown[A];
+  int lo = nd, hi = nd + o.cntUp[A];
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (L[mid] < B) lo = mid + 1; else hi = mid;
+  }
+  return o.cStart[A] + lo - nd;
+}
+
+// big geometry rows: ordered stream compaction of each chunk's partners, and
+// its incidences as body B (of big partners below it, ~id for now: placeBig)
+__device__ void emitBigChunk(const CdArgs& a, const EmitOut& o, int q, int chunk, int nchunks, const int* chUp,
+                             const int* chDown) {
+  const int b = a.bigIds[q];
+  const int j0 = chunk * kChunk, j1 = min(a.nb, j0 + kChunk);
   __shared__ int baseUp, baseDown;
   if (threadIdx.x == 0) {
-    baseUp = o.cStart[b] + chUp[blockIdx.y * nchunks + blockIdx.x];
-    baseDown = o.iStart[b] + chDown[blockIdx.y * nchunks + blockIdx.x];
+    baseUp = o.cStart[b] + chUp[q * nchunks + chunk];
+    baseDown = o.iStart[b] + chDown[q * nchunks + chunk];
   }
   __syncthreads();
   __shared__ int wUp[kT / 64], wDown[kT / 64];
@@ -492,20 +601,42 @@ __global__ __launch_bounds__(kT) void emitBigChunks(CdArgs a, EmitOut o, int nch
       o.inc[o.iStart[b] + o.cntDown[b] + (c - o.cStart[b])] = c << 1;
       if (!isBig(o, j)) placeB(o, c, b, j);
     }
-    if (isDown) o.inc[offDown + rDown] = j;
+    if (isDown) {
+      const int i = offDown + rDown;
+      if (isBig(o, j)) {
+        o.inc[i] = ~j;
+      } else {
+        const int c = contactWith(o, j, b);
+        o.inc[i] = (c << 1) | 1;
+        o.posB[c] = i - o.cStart[b];
+      }
+    }
     __syncthreads();
     if (threadIdx.x == 0) { baseUp += totUp; baseDown += totDown; }
     __syncthreads();
   }
 }
 
-// the incidences a big geometry has as body B, from the ids left there: the
-// contact is found in the partner's row
+// All rows: the small geometries' in the first smallBlocks workgroups.
+__global__ __launch_bounds__(kT) void emitContacts(CdArgs a, EmitOut o, int smallBlocks, int nchunks, const int* chUp,
+                                                   const int* chDown) {
+  if ((int)blockIdx.x < smallBlocks) {
+    emitSmall(a, o);
+  } else {
+    const int k = (int)blockIdx.x - smallBlocks;
+    emitBigChunk(a, o, k / nchunks, k % nchunks, nchunks, chUp, chDown);
+  }
+}
+
+// The incidences a big geometry has as body B with other big ones, from the
+// ids left there, once the rows are written: the contact is found in the
+// partner's row.  (Boxes never collide with each other.)
 __global__ __launch_bounds__(kT) void placeBig(CdArgs a, EmitOut o) {
   const int b = a.bigIds[blockIdx.y];
   const int i0 = o.iStart[b], nd = o.cntDown[b];
   for (int q = blockIdx.x * kT + threadIdx.x; q < nd; q += gridDim.x * kT) {
-    const int j = o.inc[i0 + q];
+    if (o.inc[i0 + q] >= 0) continue;
+    const int j = ~o.inc[i0 + q];
     int lo = o.cStart[j], hi = lo + o.cntUp[j];
     while (lo < hi) {
       const int mid = (lo + hi) >> 1;
@@ -575,6 +706,8 @@ void collideInit(Scene& s) {
   }
   s.nsmall = (int)small.size();
   s.nbig = (int)big.size();
+  s.bigPairs = false;
+  for (int i : big) s.bigPairs = s.bigPairs || (s.nbig > 1 && s.hGeom[3 * i + 1] == 0);
   s.cellSize = rmax;  // scaled with the envelope at each step
   unsigned T = 1024;
   while (T < 2u * (unsigned)std::max(1, s.nsmall)) T <<= 1;
@@ -607,32 +740,34 @@ void collideCount(Scene& s) {
   const CdArgs a = cdArgs(s);
   const unsigned T = s.hashSize;
 
-  hipLaunchKernelGGL(clearCells, dim3(blocksFor(T, kT)), dim3(kT), 0, st, s.slotCount.p, s.nsmall ? (long)T : 0L,
-                     s.counters.p);
-  if (s.nsmall) {
+  if (T <= (unsigned)kSortMost) {
+    hipLaunchKernelGGL(sortSmall, dim3(1), dim3(kSortT), 0, st, a, s.slotStart.p, s.counters.p);
+  } else {
+    hipLaunchKernelGGL(clearCells, dim3(blocksFor(T, kT)), dim3(kT), 0, st, s.slotCount.p, (long)T, s.counters.p);
     hipLaunchKernelGGL(hashSmall, dim3(blocksFor(s.nsmall, kT)), dim3(kT), 0, st, a, s.slotOf.p, s.slotCount.p);
     exclusiveScanU(s, s.slotCount.p, s.slotStart.p, (int)T);
     hipLaunchKernelGGL(scatterSmall, dim3(blocksFor(s.nsmall, kT)), dim3(kT), 0, st, a, (const unsigned*)s.slotOf.p);
-    hipLaunchKernelGGL(walkSmall<false>, dim3(blocksFor(s.nsmall, kGroups)), dim3(kT), 0, st, a, s.cntUp.p, s.cntDown.p,
-                       s.lists.p, s.counters.p + 3, (const int*)nullptr, (int*)nullptr);
   }
   const int nchunks = blocksFor(s.nb, kChunk);
   s.bigChunks.reserve((size_t)2 * std::max(1, s.nbig * nchunks));
   int* chUp = s.bigChunks.p;
   int* chDown = s.bigChunks.p + (size_t)std::max(1, s.nbig * nchunks);
-  if (s.nbig) {
-    hipLaunchKernelGGL(countBigChunks, dim3(nchunks, s.nbig), dim3(kT), 0, st, a, nchunks, chUp, chDown);
+  const int walkBlocks = s.nsmall ? blocksFor(s.nsmall, kGroups) : 0;
+  if (walkBlocks + s.nbig)
+    hipLaunchKernelGGL(countPartners, dim3(walkBlocks + s.nbig * nchunks), dim3(kT), 0, st, a, walkBlocks, nchunks,
+                       s.cntUp.p, s.cntDown.p, s.lists.p, s.counters.p + 3, chUp, chDown);
+  if (s.nbig && nchunks > 1)
     hipLaunchKernelGGL(scanBigChunks, dim3(s.nbig), dim3(64), 0, st, a, nchunks, chUp, chDown, s.cntUp.p, s.cntDown.p);
-  }
   // contact rows and incidence offsets, heavy bodies, and the totals for the host
   const int tiles = blocksFor(s.nb, kBodyTile);
   s.scanTmp.reserve(3 * (size_t)tiles);
   s.pinned[0] = s.pinned[1] = s.pinned[2] = 0;  // (a scene without bodies)
-  hipLaunchKernelGGL(bodyTileSums, dim3(tiles), dim3(kT), 0, st, s.nb, (const int*)s.cntUp.p, (const int*)s.cntDown.p,
-                     s.scanTmp.p);
+  if (tiles > kCountTiles)
+    hipLaunchKernelGGL(bodyTileSums, dim3(tiles), dim3(kT), 0, st, s.nb, (const int*)s.cntUp.p, (const int*)s.cntDown.p,
+                       s.scanTmp.p);
   if (tiles > kDirectTiles) hipLaunchKernelGGL(scanBodyTiles, dim3(1), dim3(64), 0, st, s.scanTmp.p, tiles);
   hipLaunchKernelGGL(scanBodies, dim3(tiles), dim3(kT), 0, st, s.nb, (const int*)s.cntUp.p, (const int*)s.cntDown.p,
-                     (const int*)s.scanTmp.p, tiles > kDirectTiles ? 1 : 0, s.cStart.p, s.iStart.p, s.heavy.p,
+                     (const int*)s.scanTmp.p, tiles, s.cStart.p, s.iStart.p, s.heavy.p,
                      s.counters.p, s.pinned);
 }
 
@@ -664,8 +799,8 @@ void collideEmit(Scene& s) {
   const bool csr = s.pinned[2] != 0;
   if (csr) {
     s.csr.reserve(std::max(1, ninc));
-    hipLaunchKernelGGL(walkSmall<true>, dim3(blocksFor(s.nsmall, kGroups)), dim3(kT), 0, st, a, s.cntUp.p, s.cntDown.p,
-                       s.lists.p, s.counters.p + 3, (const int*)s.iStart.p, s.csr.p);
+    hipLaunchKernelGGL(listPartners, dim3(blocksFor(s.nsmall, kGroups)), dim3(kT), 0, st, a, s.counters.p + 3,
+                       (const int*)s.iStart.p, s.csr.p);
   }
   EmitOut o;
   o.cA = s.cA.p; o.cB = s.cB.p; o.frame = s.frame.p; o.gap = s.gap.p; o.loc = s.loc.p;
@@ -673,11 +808,11 @@ void collideEmit(Scene& s) {
   o.inc = s.inc.p; o.posB = s.posB.p;
   o.lists = s.lists.p; o.csr = csr ? s.csr.p : nullptr;
   o.cStart = s.cStart.p; o.iStart = s.iStart.p; o.cntUp = s.cntUp.p; o.cntDown = s.cntDown.p;
-  if (s.nsmall) hipLaunchKernelGGL(emitSmall, dim3(blocksFor(4L * s.nsmall, kT)), dim3(kT), 0, st, a, o);
-  if (s.nbig) {
-    hipLaunchKernelGGL(emitBigChunks, dim3(nchunks, s.nbig), dim3(kT), 0, st, a, o, nchunks, chUp, chDown);
-    hipLaunchKernelGGL(placeBig, dim3(16, s.nbig), dim3(kT), 0, st, a, o);
-  }
+  const int smallBlocks = s.nsmall ? blocksFor(4L * s.nsmall, kT) : 0;
+  if (smallBlocks + s.nbig)
+    hipLaunchKernelGGL(emitContacts, dim3(smallBlocks + s.nbig * nchunks), dim3(kT), 0, st, a, o, smallBlocks, nchunks,
+                       (const int*)chUp, (const int*)chDown);
+  if (s.bigPairs) hipLaunchKernelGGL(placeBig, dim3(16, s.nbig), dim3(kT), 0, st, a, o);
   DV_HIP(hipGetLastError());
 }
 

@@ -251,6 +251,7 @@ struct Scene {
   DevBuf<int> inc;       // per-body incidences (contact << 1 | side)
   DevBuf<int> posB;      // per contact: its slot in the B-side order (see buildIncidence)
   DevBuf<int> heavy;     // bodies processed by a whole workgroup, ascending
+  bool bigPairs = false; // two big geometries may collide (not both are boxes)
   DevBuf<int> bigChunks; // per (big geometry, chunk) partner counts
 
   // --- system of the step (flat rows: nbil bilateral, then 3 per contact)

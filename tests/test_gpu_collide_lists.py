@@ -63,6 +63,15 @@ def mixed_order(seed):
     return _scene(geoms, pos, seed, rng.choice([-1, -1, -1, 1, 2], n))
 
 
+def row_on_a_floor(n):
+    """n touching spheres in a row on a fixed box."""
+    k = np.arange(n)
+    pos = np.stack([0.0995 * (k - n // 3), np.full(n, 0.149), 0.001 * np.sin(k)], 1)
+    sc = _scene([(0.1 * n, 0.1, 1.0)] + [0.05] * n, [(0.0, 0.0, 0.0)] + list(pos), 7)
+    sc.fixed[0] = 1
+    return sc
+
+
 SCENES = {
     "lists_24": lambda: swarm(5, 23, 0.19),
     "lists_25": lambda: swarm(5, 26, 0.19),
@@ -70,6 +79,9 @@ SCENES = {
     "big_order": lambda: mixed_order(5),
     "one_sphere": lambda: _scene([0.05, (1, 0.1, 1)], [(0, 0.15, 0), (0, 0, 0)], 1),
     "boxes_only": lambda: _scene([(1, 0.1, 1), (1, 0.1, 1)], [(0, 0.15, 0), (0, 0, 0)], 1),
+    # one and two chunks of a big geometry's partners; cells sorted by one
+    # workgroup or not; body tiles added up from counts or from tile sums
+    **{f"row_{n}": (lambda n=n: row_on_a_floor(n)) for n in (511, 512, 4096, 4097, 8191, 8192)},
 }
 
 
