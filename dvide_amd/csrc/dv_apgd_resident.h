@@ -19,7 +19,7 @@
 //   FP64       10.7            13.9    15.5    17.1    21.0    27.2
 //               5.4             9.2    10.2    11.8    14.2    23.3
 //               4.6     5.7     6.6     7.2     8.1     9.8    17.5
-//               4.6     5.2     5.7     6.8     7.8     9.4    17.5
+//               4.6     5.2     5.7     6.8     7.8     9.4    14.6
 //   mixed       8.8            11.7    12.9    13.6    16.1    20.7
 //               4.5             7.9     8.4    10.0    11.9    17.8
 //               3.7     4.1     5.1     5.4     6.0     6.8    10.8
@@ -347,7 +347,12 @@ __device__ __forceinline__ int contactOf(const Args<TM>& a, const BodyRuns<TM>& 
 // of 64 bodies some have more than 8, and a second round of loads costs them
 // all another flight: us per pass with 6, 8, 10 and 12 at 18,000 contacts 6.6,
 // 6.3, 6.1 and 6.1 (mixed), 8.9, 8.5, 8.1 and 8.8 (FP64).
-constexpr int kRun = 10;
+constexpr int kRunMost = 10;
+// Two rows a thread in FP64 have no registers for ten: with 10, 8, 6, 5 and 4 at
+// 168,000 contacts 16.6, 15.7, 14.9, 14.6 and 14.8 us, at 216,000 17.7, 17.7,
+// 16.8, 16.2 and 16.3 (one row a thread, 11,900: 6.9 with 10, 7.0 with 9, 7.3
+// with 8; mixed with two rows, 9.6 with 10, 10.0 with 8, 9.8 with 6).
+constexpr int kRunTwo = 5;
 
 // Wavefront totals in waveSum's and waveMax's order, valid in lane 63 only:
 // past the rows of 16 lanes the partners come by row broadcasts instead of
@@ -435,22 +440,26 @@ __device__ __forceinline__ PassView uniformView(const PassView& s) {
 // leaves the registers.
 // Two wavefronts per SIMD (up to 256 VGPRs, one workgroup to a CU): held to
 // 128, so that a CU takes two, the mixed kernel spilled 20 and took 26.3 us
-// per pass on 256,000 contacts, where two rows per thread take 12.6.  (Two
-// rows in FP64 have no registers for a second step: without the guess.)
+// per pass on 256,000 contacts, where two rows per thread take 10.7.
+// Two rows in FP64 have room for the second step with gamma_{k-1} and its
+// N gamma in LDS and five contacts of a body in flight: 17.4 us without the
+// step, 14.6 with it.  (Mixed they stay in registers: 9.4 us, in LDS 9.6.)
 // In FP64 a large team's members wait for J, twice as long, with loads that
 // take the others' room: us per pass with the unit taken ahead and not, 82
 // members (41,800 contacts) 8.2 and 7.8, 162 (82,400) 10.5 and 9.4, but 24
 // (11,900) 6.8 and 7.2; mixed 5.4 and 6.0, 5.8 and 6.8, 4.9 and 5.4.
 // Where bodies outnumber contacts so far that both wavefronts of a SIMD have a
 // unit, their waits cannot hide behind each other's steps: a shell's 19,200
-// spheres with 20,100 contacts 6.4 ahead and 6.1 not; but with two rows a thread
-// (112,000 spheres, 256,000 contacts) 10.7 ahead and 12.0 not.
+// spheres with 20,100 contacts 6.4 ahead and 6.1 not.  With two rows a thread
+// all units go ahead: 112,000 spheres, 256,000 contacts 10.7 ahead and 12.0
+// not (mixed); 168,000 contacts 16.7 and 17.7 (FP64).
 constexpr int kAheadMost = 64;
 template <typename TM, bool kBil, int R>
 __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, Tables T, const TeamItem* items, int stride,
                                                 u64* sync, u64 launch, int passes, u64 formTicks) {
   constexpr bool kMixed = sizeof(TM) < sizeof(double);
-  constexpr bool kGuess = kMixed || R == 1;
+  constexpr int kRun = !kMixed && R == 2 ? kRunTwo : kRunMost;
+  constexpr bool kOldInLds = !kMixed && R == 2;
   constexpr bool kLanes = R == 1;
   constexpr int NF = kMixed ? 6 : 3;
   constexpr unsigned kUsed = kP1Slots<TM>;
@@ -482,6 +491,9 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
   // first body's contacts
   __shared__ TM shF[R][9][kTC];
   __shared__ int shIds[kRun][kTC];
+  // and gamma_{k-1} and its N gamma, which only a step taken again reads
+  __shared__ double shGm[kOldInLds ? R : 1][3][kOldInLds ? kTC : 1];
+  __shared__ TM shNm[kOldInLds ? R : 1][3][kOldInLds ? kTC : 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   if (tid < 64) unitCount[tid / 2][tid % 2] = 0;
   if (tid == 0) {
@@ -521,6 +533,30 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
     double gk[3], gm[3], gn[3], gs[3];
   };
   Row row[R];
+  auto keepOld = [&](int u, const double (&g)[3], const TM (&n)[3]) {
+#pragma unroll
+    for (int rr = 0; rr < 3; ++rr) {
+      if constexpr (kOldInLds) {
+        shGm[u][rr][tid] = g[rr];
+        shNm[u][rr][tid] = n[rr];
+      } else {
+        row[u].gm[rr] = g[rr];
+        row[u].nm[rr] = n[rr];
+      }
+    }
+  };
+  auto loadOld = [&](int u, double (&g)[3], TM (&n)[3]) {
+#pragma unroll
+    for (int rr = 0; rr < 3; ++rr) {
+      if constexpr (kOldInLds) {
+        g[rr] = shGm[u][rr][tid];
+        n[rr] = shNm[u][rr][tid];
+      } else {
+        g[rr] = row[u].gm[rr];
+        n[rr] = row[u].nm[rr];
+      }
+    }
+  };
   auto flatOf = [&](int u, int rr) {  // row rr's place in a row vector
     const long q = ((long)rank * R + u) * kTC + tid;
     return kBil && q >= D.nc ? (long)BROW(a, q - D.nc) : ROW(a, rr, q);
@@ -551,6 +587,8 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
     frameFrom(fc, D.geomMode, F);
 #pragma unroll
     for (int k = 0; k < 9; ++k) shF[u][k][tid] = F[k];
+    double gm[3];
+    TM nm[3];
 #pragma unroll
     for (int rr = 0; rr < 3; ++rr) {
       // (a thread without a row has one of zeros, which adds zero to every sum)
@@ -558,12 +596,13 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       const long f = on ? flatOf(u, rr) : 0;
       w.rv[rr] = on ? gl(a.r)[f] : (TM)0;
       w.gk[rr] = on ? gl(a.ring[0] + V.cur * a.ringStride)[f] : 0.0;
-      w.gm[rr] = on ? gl(a.ring[0] + V.prev * a.ringStride)[f] : 0.0;
+      gm[rr] = on ? gl(a.ring[0] + V.prev * a.ringStride)[f] : 0.0;
       w.nk[rr] = on ? gl(a.rn[0] + V.cur * a.ringStride)[f] : (TM)0;  // (not formed yet if fresh: replaced below)
-      w.nm[rr] = on ? gl(a.rn[0] + V.prev * a.ringStride)[f] : (TM)0;
+      nm[rr] = on ? gl(a.rn[0] + V.prev * a.ringStride)[f] : (TM)0;
       w.gn[rr] = w.gs[rr] = 0;
       w.nn[rr] = 0;
     }
+    keepOld(u, gm, nm);
     J.st(w.e, 0, 0, 0, 0);
   }
   // the iterate in registers back to its ring slot
@@ -666,7 +705,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
       rowsOfTmp(F, V4<TM>{tA.x, tA.y, tA.z, (TM)0}, V4<TM>{tB.x, tB.y, tB.z, (TM)0}, out[0], out[1], out[2]);
     }
   };
-  auto rowsOfArrived = [&](unsigned tag, bool next) {
+  auto rowsOfArrived = [&](unsigned tag) {
     int id[2 * R];
     Raw t[2 * R];
 #pragma unroll
@@ -676,7 +715,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
     }
     await<kLanes>(tmp, id, tag, &bad, t);
 #pragma unroll
-    for (int u = 0; u < R; ++u) rowsN(u, tmp.value(t[2 * u]), tmp.value(t[2 * u + 1]), next ? row[u].nn : row[u].nk);
+    for (int u = 0; u < R; ++u) rowsN(u, tmp.value(t[2 * u]), tmp.value(t[2 * u + 1]), row[u].nn);
   };
 
   // the partial sums of the step from (gk, gm, nk, nm) to gn, in P1's order
@@ -762,7 +801,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
     dc = ld4(a.sr, V.cur * (long)D.nb + first.g);
     dp = ld4(a.sr, V.prev * (long)D.nb + first.g);
   }
-  const bool ahead = kGuess && (R == 2 || __popcll(tiles) <= 1) && (kMixed || W <= kAheadMost);
+  const bool ahead = (R == 2 || __popcll(tiles) <= 1) && (kMixed || R == 2 || W <= kAheadMost);
   auto firstUnit = [&](unsigned tagJ, unsigned least, const V4<TM>& c, const V4<TM>& p, bool mom, double beta, V4<TM>& out) {
     if (!(live & 1u)) return;
     int id[kRun];
@@ -806,16 +845,17 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
             rowsN(u, V3<TM>{tA.x, tA.y, tA.z}, V3<TM>{tB.x, tB.y, tB.z}, row[u].nk);
           }
         }
-      } else if (kGuess) {
+      } else {
         tagJ |= 1u << 16;
-      } else if (V.flags & kViewFresh) {
-        rowsOfArrived(tag - (2u << 16), false);
       }
 #pragma unroll
       for (int u = 0; u < R; ++u) {
         Row& w = row[u];
-        step(u, w.gk, w.gm, w.nk, w.nm, mom, V.beta, V.t, w.gn, tagJ);
-        sumsOf(par, u, w.gk, w.gm, w.gn, w.nk, w.nm, mom, V.beta);
+        double gm[3];
+        TM nm[3];
+        loadOld(u, gm, nm);
+        step(u, w.gk, gm, w.nk, nm, mom, V.beta, V.t, w.gn, tagJ);
+        sumsOf(par, u, w.gk, gm, w.gn, w.nk, nm, mom, V.beta);
       }
       stepSizes(sizes, shS[par].L, shS[par].theta);  // (which its wavefront has stored)
       __syncthreads();
@@ -947,8 +987,8 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
     }
 
     // ---- the next pass's step, should this one be accepted without a restart
-    const bool guess = kGuess && p + 1 < passes;
-    if (guess) rowsOfArrived(tagJ, true);
+    const bool guess = p + 1 < passes;
+    if (guess) rowsOfArrived(tagJ);
     const double tNext = uniformDouble(shNext[sizes][3]), betaNext = uniformDouble(shNext[sizes][5]);
     // The team's sums, in reduceSlots' order: lane l of its wavefront i adds
     // entries 64 i + l, 64 i + l + kTP, ..., and the wavefronts' sums are added
@@ -1104,7 +1144,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
     if (lost || (V.flags & kViewDone)) break;
     taken = false;
     if (V.flags & kViewFresh) {  // accepted: gamma_new becomes gamma_k (a backtrack keeps both)
-      taken = kGuess && !(V.flags & kViewRestart) && V.t == tNext && V.beta == betaNext;
+      taken = !(V.flags & kViewRestart) && V.t == tNext && V.beta == betaNext;
       if (kMixed) {
         dp = dc;
         dc = dn;
@@ -1113,16 +1153,18 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
 #pragma unroll
       for (int u = 0; u < R; ++u) {
         Row& w = row[u];
-        if (keep) storeIterate(dropped, u, w.gm);
+        if (keep) {
+          double gm[3];
+          TM nm[3];
+          loadOld(u, gm, nm);
+          storeIterate(dropped, u, gm);
+        }
+        keepOld(u, w.gk, w.nk);
 #pragma unroll
         for (int rr = 0; rr < 3; ++rr) {
-          w.gm[rr] = w.gk[rr];
-          w.nm[rr] = w.nk[rr];
           w.gk[rr] = w.gn[rr];
-          if (kGuess) {
-            w.nk[rr] = w.nn[rr];
-            w.gn[rr] = w.gs[rr];
-          }
+          w.nk[rr] = w.nn[rr];
+          w.gn[rr] = w.gs[rr];
         }
       }
     }
@@ -1131,14 +1173,17 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
 #pragma unroll
   for (int u = 0; u < R; ++u) {
     const Row& w = row[u];
-    if (V.prev != V.cur) storeIterate(V.prev, u, w.gm);
+    double gm[3];
+    TM nm[3];
+    loadOld(u, gm, nm);
+    if (V.prev != V.cur) storeIterate(V.prev, u, gm);
     storeIterate(V.cur, u, w.gk);
     if (!w.valid) continue;
 #pragma unroll
     for (int rr = 0; rr < 3; ++rr) {
       if (w.bil && rr) continue;
       const long f = flatOf(u, rr);
-      if (V.prev != V.cur) gl(a.rn[0] + V.prev * a.ringStride)[f] = w.nm[rr];
+      if (V.prev != V.cur) gl(a.rn[0] + V.prev * a.ringStride)[f] = nm[rr];
       if (!(V.flags & kViewFresh)) gl(a.rn[0] + V.cur * a.ringStride)[f] = w.nk[rr];
     }
   }
