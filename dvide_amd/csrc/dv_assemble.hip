@@ -84,15 +84,14 @@ __global__ __launch_bounds__(kT) void kRowsD(RowArgs a, const double* __restrict
 }
 
 // f = D^T x and tmp = M^-1 f per body, terms in D^T row order.  With
-// skipFixed, bodies with M^-1 = 0 get tmp = +0 without the sum (0.0 + 0*f);
-// with skipHeavy, the heavy bodies are left to kGatherHeavy.
+// skipFixed, bodies with M^-1 = 0 get tmp = +0 without the sum (0.0 + 0*f).
 __global__ __launch_bounds__(kGatherT) void kGatherDT(GatherArgs a, const double* __restrict__ x,
                                                       double* __restrict__ fOut, double* __restrict__ tmpOut,
-                                                      int skipFixed, int skipHeavy, int lightBlocks) {
+                                                      int skipFixed, int lightBlocks) {
   __shared__ double sh[64][9];
   auto row = [&](long r) { return x[r]; };
   if ((int)blockIdx.x >= lightBlocks) {
-    for (int h = blockIdx.x - lightBlocks; !skipHeavy && h < a.counters[2]; h += kHeavyBlocks) {
+    for (int h = blockIdx.x - lightBlocks; h < a.counters[2]; h += kHeavyBlocks) {
       const int g = a.heavy[h], q = threadIdx.x;
       const double mi = a.minv[g];
       const bool fixed = skipFixed && mi == 0;
@@ -124,16 +123,90 @@ __global__ __launch_bounds__(kGatherT) void kGatherDT(GatherArgs a, const double
   }
 }
 
-// f = D^T x for the bodies of the heavy list (more than kHeavyDegree
-// incidences), one workgroup each, FP64 sums in a fixed tree order; used by
-// the update of the persistent solvers in place of the sequential sums.
-__global__ __launch_bounds__(kT) void kGatherHeavy(GatherArgs a, const int* heavy, const int* counters,
-                                                   const double* __restrict__ x, double* __restrict__ fOut) {
-  const int nHeavy = counters[2];
+// b: bilateral rows violation / h (System.cu:1526-1544), contact rows
+// (gap/h, 0, 0) (System.cu:1516-1524); and r = D M^-1 k + b.  Launches bound
+// the assembly of small scenes: k, M^-1 k, b and r in four took 25 us of one
+// sphere's step, in two 12.
+__global__ __launch_bounds__(kT) void kBuildR(RowArgs a, const double* __restrict__ gap, const double* bilVel,
+                                              const double* bilT0, const double* bilP0,
+                                              const double* __restrict__ p, const double* __restrict__ x, double h,
+                                              double time, double* __restrict__ b, double* __restrict__ r) {
+  const int q = blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= a.nc + a.nbil) return;
+  double first;
+  if (q < a.nbil) {
+    double vel = bilVel[q], t0 = bilT0[q];
+    if (time < t0) vel = 0;
+    double viol = a.bilB[q] < 0 ? p[a.bilA[q]] - bilP0[q] - vel * (time - t0)
+                                : p[a.bilA[q]] - p[a.bilB[q]] - vel * (time - t0);
+    first = viol / h;
+  } else {
+    first = gap[q - a.nbil] / h;
+  }
+  rowOfD(a, q, x, [&](int row, int rr, double s) {
+    const double bb = rr ? 0.0 : first;
+    b[row] = bb;
+    r[row] = 1.0 * bb + s;
+  });
+}
+
+// v = M^-1 (k + f_c), f_c /= h, p += h v  (System.cu:570-581)
+struct UpdateArgs {
+  int nb;
+  const double* minv;
+  const double* k;
+  double* fc;
+  double* v;
+  double* p;
+  double h;
+};
+// DOF i, whose contact impulse is f
+__device__ __forceinline__ void updateDof(const UpdateArgs& u, int i, double mi, double f) {
+  const double t = 1.0 * u.k[i] + 1.0 * f;
+  double vv = 0.0;
+  vv = vv + mi * t;
+  u.fc[i] = (1.0 / u.h) * f;
+  u.v[i] = vv;
+  u.p[i] = u.h * vv + u.p[i];
+}
+__global__ __launch_bounds__(kT) void kUpdate(UpdateArgs u, int haveRows) {
+  int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= 3 * u.nb) return;
+  const double mi = u.minv[i / 3];
+  if (haveRows) {
+    updateDof(u, i, mi, u.fc[i]);
+    return;
+  }
+  double vv = 0.0;
+  vv = vv + mi * u.k[i];
+  u.fc[i] = 0.0;
+  u.v[i] = vv;
+  u.p[i] = u.h * vv + u.p[i];
+}
+
+// The update with f_c = D^T gamma formed as it is used: the bodies' sums in
+// D^T row order (by one wavefront of a workgroup: 64 bodies each spread a small
+// scene over more CUs), and in the first kHeavyBlocks workgroups those of the heavy
+// list (more than kHeavyDegree incidences), one workgroup each, FP64 sums in
+// a fixed tree order.  In one launch: gather, heavy bodies and update in three
+// took 10 us of one sphere's step and 30 of 1,000 spheres'.
+__global__ __launch_bounds__(kT) void kGatherUpdate(GatherArgs a, const double* __restrict__ x, UpdateArgs u) {
+  if (blockIdx.x >= kHeavyBlocks) {
+    const int g = ((int)blockIdx.x - kHeavyBlocks) * kGatherT + threadIdx.x;
+    if (threadIdx.x >= kGatherT || g >= a.nb || a.iStart[g + 1] - a.iStart[g] > kHeavyDegree) return;
+    const double mi = u.minv[g];
+    double s0, s1, s2;
+    gatherSums(a, g, [&](long r) { return x[r]; }, s0, s1, s2);
+    updateDof(u, 3 * g, mi, s0);
+    updateDof(u, 3 * g + 1, mi, s1);
+    updateDof(u, 3 * g + 2, mi, s2);
+    return;
+  }
+  const int nHeavy = a.counters[2];
   __shared__ double red[kT / 64][3];
   const long S = a.cap;
-  for (int hq = blockIdx.x; hq < nHeavy; hq += gridDim.x) {
-    const int g = heavy[hq];
+  for (int hq = blockIdx.x; hq < nHeavy; hq += kHeavyBlocks) {
+    const int g = a.heavy[hq];
     double s0 = 0, s1 = 0, s2 = 0;
     for (int k = a.iStart[g] + threadIdx.x; k < a.iStart[g + 1]; k += kT) {
       const int e = a.inc[k];
@@ -169,60 +242,10 @@ __global__ __launch_bounds__(kT) void kGatherHeavy(GatherArgs a, const int* heav
     if (threadIdx.x < 3) {
       double v = 0;
       for (int w = 0; w < kT / 64; ++w) v += red[w][threadIdx.x];
-      fOut[3 * g + threadIdx.x] = v;
+      updateDof(u, 3 * g + threadIdx.x, u.minv[g], v);
     }
     __syncthreads();
   }
-}
-
-// b: bilateral rows violation / h (System.cu:1526-1544), contact rows
-// (gap/h, 0, 0) (System.cu:1516-1524); and r = D M^-1 k + b.  Launches bound
-// the assembly of small scenes: k, M^-1 k, b and r in four took 25 us of one
-// sphere's step, in two 12.
-__global__ __launch_bounds__(kT) void kBuildR(RowArgs a, const double* __restrict__ gap, const double* bilVel,
-                                              const double* bilT0, const double* bilP0,
-                                              const double* __restrict__ p, const double* __restrict__ x, double h,
-                                              double time, double* __restrict__ b, double* __restrict__ r) {
-  const int q = blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= a.nc + a.nbil) return;
-  double first;
-  if (q < a.nbil) {
-    double vel = bilVel[q], t0 = bilT0[q];
-    if (time < t0) vel = 0;
-    double viol = a.bilB[q] < 0 ? p[a.bilA[q]] - bilP0[q] - vel * (time - t0)
-                                : p[a.bilA[q]] - p[a.bilB[q]] - vel * (time - t0);
-    first = viol / h;
-  } else {
-    first = gap[q - a.nbil] / h;
-  }
-  rowOfD(a, q, x, [&](int row, int rr, double s) {
-    const double bb = rr ? 0.0 : first;
-    b[row] = bb;
-    r[row] = 1.0 * bb + s;
-  });
-}
-
-// v = M^-1 (k + f_c), f_c /= h, p += h v  (System.cu:570-581)
-__global__ __launch_bounds__(kT) void kUpdate(int nb, const double* __restrict__ minv,
-                                              const double* __restrict__ k, double* __restrict__ fc,
-                                              double* __restrict__ v, double* __restrict__ p, double h,
-                                              int haveRows) {
-  int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= 3 * nb) return;
-  const double mi = minv[i / 3];
-  double vv;
-  if (haveRows) {
-    double t = 1.0 * k[i] + 1.0 * fc[i];
-    vv = 0.0;
-    vv = vv + mi * t;
-    fc[i] = (1.0 / h) * fc[i];
-  } else {
-    vv = 0.0;
-    vv = vv + mi * k[i];
-    fc[i] = 0.0;
-  }
-  v[i] = vv;
-  p[i] = h * vv + p[i];
 }
 
 __global__ __launch_bounds__(kT) void kFillD(double* x, long n, double val) {
@@ -274,7 +297,7 @@ void buildR(Scene& s) {
 static void gatherExact(Scene& s, const double* x, double* fOut, double* tmpOut, bool skipFixed) {
   const GatherArgs a = gatherArgs(s);
   hipLaunchKernelGGL(kGatherDT, dim3(gatherBlocks(a) + kHeavyBlocks), dim3(kGatherT), 0, s.stream, a, x, fOut, tmpOut,
-                     skipFixed ? 1 : 0, 0, gatherBlocks(a));
+                     skipFixed ? 1 : 0, gatherBlocks(a));
 }
 
 // y = D (M^-1 (D^T x))  (APGD.cu:81-87)
@@ -293,19 +316,15 @@ void rowsD(Scene& s, const double* x, const double* badd, double* y) {
 }
 
 void updateState(Scene& s, bool haveRows, bool exactOrder) {
-  if (haveRows) {
-    if (exactOrder) {
-      gatherExact(s, s.gamma.p, s.fContact.p, nullptr, false);
-    } else {
-      const GatherArgs a = gatherArgs(s);
-      hipLaunchKernelGGL(kGatherDT, dim3(gatherBlocks(a)), dim3(kGatherT), 0, s.stream, a,
-                         (const double*)s.gamma.p, s.fContact.p, (double*)nullptr, 0, 1, gatherBlocks(a));
-      hipLaunchKernelGGL(kGatherHeavy, dim3(64), dim3(kT), 0, s.stream, a, (const int*)s.heavy.p,
-                         (const int*)s.counters.p, (const double*)s.gamma.p, s.fContact.p);
-    }
+  const UpdateArgs u{s.nb, s.minv.p, s.k.p, s.fContact.p, s.v.p, s.p.p, s.h};
+  if (haveRows && !exactOrder) {
+    const GatherArgs a = gatherArgs(s);
+    hipLaunchKernelGGL(kGatherUpdate, dim3(kHeavyBlocks + gatherBlocks(a)), dim3(kT), 0, s.stream, a,
+                       (const double*)s.gamma.p, u);
+    return;
   }
-  hipLaunchKernelGGL(kUpdate, dim3(blocksFor(3L * s.nb, kT)), dim3(kT), 0, s.stream, s.nb, s.minv.p, s.k.p,
-                     s.fContact.p, s.v.p, s.p.p, s.h, haveRows ? 1 : 0);
+  if (haveRows) gatherExact(s, s.gamma.p, s.fContact.p, nullptr, false);
+  hipLaunchKernelGGL(kUpdate, dim3(blocksFor(3L * s.nb, kT)), dim3(kT), 0, s.stream, u, haveRows ? 1 : 0);
 }
 
 }  // namespace dv
