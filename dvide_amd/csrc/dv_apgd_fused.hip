@@ -31,9 +31,9 @@
 // double-buffered by pass parity, so no decision races with its
 // publication.  Kernel boundaries are the grid-wide barriers, in chunks of
 // passes captured as a graph: the host launches a chunk, reads the scenes'
-// states, and repeats; scenes that have converged skip their tiles.  A single
-// scene that fits the chip runs its passes resident instead, in one kernel
-// with barriers of its own (dv_apgd_resident.h).
+// states, and repeats; scenes that have converged skip their tiles.  Scenes
+// that fit the chip run their passes resident instead, each with a team of
+// workgroups in one kernel (dv_apgd_resident.h).
 //
 // The same arithmetic as the reference, less traffic:
 //   * N y is not recomputed: with y_{k+1} = (1+beta) g_{k+1} - beta g_k,
@@ -2033,7 +2033,8 @@ Plan<TM> activePlan(Engine& E) {
 }
 
 // The resident passes (dv_apgd_resident.h).  A slot's team is one workgroup
-// per row tile, or per two: one workgroup fills a CU, so once the tiles
+// per row tile, or per two, or, mixed and past two a CU (262,144 rows on 256
+// CUs), per three: one workgroup fills a CU, so once the tiles
 // outnumber the CUs two rows per thread do more work per exchange (48 scenes
 // of 1,000 to 20,000 contacts, 545 tiles, 233 passes: 6.0 ms as launches, 2.7
 // so; 512 scenes, 8.1 million contacts: 372 ms and 322).  The members of a team must all be
@@ -2057,7 +2058,10 @@ void buildTeams(Engine& E, hipStream_t st) {
   const int most = std::min(kTeamMax, E.numCU);
   long tiles = 0;
   for (int slot : E.active.hSlots) tiles += slotArgs<TM>(E, slot).nTiles;
-  const int R = tiles > E.numCU ? 2 : 1;
+  int R = tiles > E.numCU ? 2 : 1;
+  if (E.mixed)  // (three rows in FP64 have no room in LDS)
+    for (int slot : E.active.hSlots)
+      if (slotArgs<TM>(E, slot).nTiles > 2L * most) R = 3;
   std::vector<TeamItem> items;
   E.teamRows = E.active.hSlots.empty() ? 0 : R;
   E.teamBil = false;
@@ -2082,8 +2086,10 @@ void launchTeams(Engine& E, hipStream_t st, int passes) {
     DV_HIP(hipMemsetAsync(E.teamSync.p, 0, sizeof(u64) * E.teamSync.cap, st));
   }
   const Tables T = tablesOf<TM>(E, E.active);
-  const auto kernel = E.teamBil ? (E.teamRows == 1 ? kTeam<TM, true, 1> : kTeam<TM, true, 2>)
-                                : (E.teamRows == 1 ? kTeam<TM, false, 1> : kTeam<TM, false, 2>);
+  auto kernel = E.teamBil ? (E.teamRows == 1 ? kTeam<TM, true, 1> : kTeam<TM, true, 2>)
+                          : (E.teamRows == 1 ? kTeam<TM, false, 1> : kTeam<TM, false, 2>);
+  if constexpr (sizeof(TM) < sizeof(double))
+    if (E.teamRows == 3) kernel = E.teamBil ? kTeam<TM, true, 3> : kTeam<TM, false, 3>;
   const int places = (int)(E.hTeams.size() / sizeof(TeamItem));
   const int stride = E.nSlots == 1 && places <= kXcdMost ? kXcds : 1;
   hipLaunchKernelGGL(kernel, dim3((unsigned)(places * stride)), dim3(kTC), 0, st,

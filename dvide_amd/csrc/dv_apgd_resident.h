@@ -348,7 +348,7 @@ __device__ __forceinline__ int contactOf(const Args<TM>& a, const BodyRuns<TM>& 
 // all another flight: us per pass with 6, 8, 10 and 12 at 18,000 contacts 6.6,
 // 6.3, 6.1 and 6.1 (mixed), 8.9, 8.5, 8.1 and 8.8 (FP64).
 constexpr int kRunMost = 10;
-// Two rows a thread in FP64 have no registers for ten: with 10, 8, 6, 5 and 4 at
+// Two rows a thread in FP64 (and three, mixed) have no registers for ten: with 10, 8, 6, 5 and 4 at
 // 168,000 contacts 16.6, 15.7, 14.9, 14.6 and 14.8 us, at 216,000 17.7, 17.7,
 // 16.8, 16.2 and 16.3 (one row a thread, 11,900: 6.9 with 10, 7.0 with 9, 7.3
 // with 8; mixed with two rows, 9.6 with 10, 10.0 with 8, 9.8 with 6).
@@ -444,6 +444,9 @@ __device__ __forceinline__ PassView uniformView(const PassView& s) {
 // Two rows in FP64 have room for the second step with gamma_{k-1} and its
 // N gamma in LDS and five contacts of a body in flight: 17.4 us without the
 // step, 14.6 with it.  (Mixed they stay in registers: 9.4 us, in LDS 9.6.)
+// Three rows, mixed: 268,000 contacts 22.4 us as launches and 16.8 so, 327,000
+// 24.0 and 18.0, 383,000 25.4 and 19.6.  (In FP64 the frames and the old
+// iterates of three rows do not fit LDS.)
 // In FP64 a large team's members wait for J, twice as long, with loads that
 // take the others' room: us per pass with the unit taken ahead and not, 82
 // members (41,800 contacts) 8.2 and 7.8, 162 (82,400) 10.5 and 9.4, but 24
@@ -458,8 +461,8 @@ template <typename TM, bool kBil, int R>
 __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, Tables T, const TeamItem* items, int stride,
                                                 u64* sync, u64 launch, int passes, u64 formTicks) {
   constexpr bool kMixed = sizeof(TM) < sizeof(double);
-  constexpr int kRun = !kMixed && R == 2 ? kRunTwo : kRunMost;
-  constexpr bool kOldInLds = !kMixed && R == 2;
+  constexpr int kRun = R == 1 || (kMixed && R == 2) ? kRunMost : kRunTwo;
+  constexpr bool kOldInLds = R > (kMixed ? 2 : 1);
   constexpr bool kLanes = R == 1;
   constexpr int NF = kMixed ? 6 : 3;
   constexpr unsigned kUsed = kP1Slots<TM>;
@@ -801,7 +804,7 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
     dc = ld4(a.sr, V.cur * (long)D.nb + first.g);
     dp = ld4(a.sr, V.prev * (long)D.nb + first.g);
   }
-  const bool ahead = (R == 2 || __popcll(tiles) <= 1) && (kMixed || R == 2 || W <= kAheadMost);
+  const bool ahead = (R > 1 || __popcll(tiles) <= 1) && (kMixed || R > 1 || W <= kAheadMost);
   auto firstUnit = [&](unsigned tagJ, unsigned least, const V4<TM>& c, const V4<TM>& p, bool mom, double beta, V4<TM>& out) {
     if (!(live & 1u)) return;
     int id[kRun];

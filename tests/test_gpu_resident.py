@@ -3,8 +3,8 @@
 A slot whose team fits the chip keeps its contacts' state in registers for
 thousands of passes; fixed rows per thread (DV_PARAM_ROWS_PER_THREAD) keep a
 scene on the launches.  Both add in the same order, so every result is equal
-bit for bit: around the edges of a row tile (512 rows), past one tile per CU
-(two rows per thread), and with the rows and bodies that take paths of their
+bit for bit: around the edges of a row tile (512 rows), past one and two tiles
+per CU (two rows per thread, and three), and with the rows and bodies that take paths of their
 own (bilateral rows, a movable body with thousands of contacts, body units
 without a movable body)."""
 import copy
@@ -55,6 +55,9 @@ SCENES = {
     "shell": landed_shell,
     "ball_on_a_layer": ball_on_a_layer,
     "box_58000": lambda: scenes.compaction(2002, n=58000, width=4.0, lid=scenes.LID_NONE),
+    # past two rows per thread on 256 CUs
+    "box_118000": lambda: scenes.compaction(2002, n=118000, width=5.1, lid=scenes.LID_NONE),
+    "bilateral_118000": lambda: scenes.compaction(2002, n=118000, width=5.1, lid=scenes.LID_BILATERAL),
 }
 
 
