@@ -13,8 +13,8 @@ pressed pile costs.
 
 The headline `value` is time-steps/s of the mixed-precision solver (FP32
 D, M^-1 and products, FP64 iterates, tests and update).  The same run times
-the FP64 graph-driven solver and the plain FP64 solver (one kernel per
-vector operation, host-driven like the reference's CUSP calls) from the same
+the FP64 graph-driven solver and the plain FP64 solver (the reference's
+operations in the oracle's order) from the same
 initial state, and the CPU oracle on the host cores.
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--cpu-steps S] [--no-cpu]
