@@ -588,8 +588,10 @@ __global__ __launch_bounds__(kTC, 2) void kTeam(const Args<TM>* __restrict__ A, 
 #pragma unroll
     for (int k = 0; k < 6; ++k) fc[k] = k < NF ? gl(a.frame)[k * cap + c] : (TM)0;
     frameFrom(fc, D.geomMode, F);
+    // (no contact, no frame: without contacts in the scene the memory of
+    // contact 0 may hold anything, and NaN times the row's zeros is NaN)
 #pragma unroll
-    for (int k = 0; k < 9; ++k) shF[u][k][tid] = F[k];
+    for (int k = 0; k < 9; ++k) shF[u][k][tid] = w.valid && !w.bil ? F[k] : (TM)0;
     double gm[3];
     TM nm[3];
 #pragma unroll
