@@ -2099,6 +2099,17 @@ void launchTeams(Engine& E, hipStream_t st, int passes) {
   DV_HIP(hipGetLastError());
 }
 
+// A slot's passes as read after a chunk that ran with ranRows row tiles per
+// workgroup (0: as launches).
+void notePasses(Engine& E, int slot, int passes, int ranRows) {
+  Engine::SlotRun& r = E.slotRun[slot];
+  if (ranRows && passes > r.passes) {
+    r.resident += passes - r.passes;
+    r.teamRows = ranRows;
+  }
+  r.passes = passes;
+}
+
 template <typename TM>
 void rebuildActive(Engine& E, hipStream_t st) {
   E.active.hSlots.clear();
@@ -2186,6 +2197,8 @@ void recordSlots(Engine& E, const std::vector<int>& slots, const ApgdState* outH
     s.stats.residual = S.best;
     s.stats.objective = S.objective;
     s.stats.passes = S.passes;
+    s.residentPasses = E.slotRun[slot].resident;
+    s.teamRows = E.slotRun[slot].teamRows;
     s.stats.rows_per_thread = E.sched.rpt;
     s.stats.xcd_order = E.sched.xcd;
     s.stats.wg_per_cu_contacts = E.nSlots > 1 ? E.sched.wgc : 0;
@@ -2214,6 +2227,7 @@ template <typename TM>
 void openT(Engine& E, int nSlots) {
   E.hostTable.assign(sizeof(Args<TM>) * nSlots, 0);  // every slot inactive
   E.slotScene.assign(nSlots, nullptr);
+  E.slotRun.assign(nSlots, Engine::SlotRun{});
   E.table.reserve(sizeof(Args<TM>) * nSlots);
 }
 
@@ -2251,6 +2265,7 @@ void engineAdmit(Engine& E, int slot, Scene& s) {
   if (E.mixed) prepareScene<float>(s, slotArgs<float>(E, slot));
   else prepareScene<double>(s, slotArgs<double>(E, slot));
   E.slotScene[slot] = &s;
+  E.slotRun[slot] = Engine::SlotRun{};
   E.admit.hSlots.push_back(slot);
 }
 
@@ -2262,7 +2277,7 @@ void engineStartAdmitted(Engine& E, hipStream_t st) {
 void engineRunChunk(Engine& E, hipStream_t st) {
   // resident, unless the last such launch made no progress (enginePoll)
   const bool resident = E.teamRows && !E.noGraph && E.teamSkip == 0;
-  E.ranResident = resident;
+  E.ranRows = resident ? E.teamRows : 0;
   if (E.teamSkip > 0) --E.teamSkip;
   if (resident) {
     if (E.mixed) launchTeams<float>(E, st, kTeamPassesServed);
@@ -2282,13 +2297,14 @@ std::vector<int> enginePoll(Engine& E, hipStream_t st) {
   bool some = false;
   for (int i = 0; i < E.nSlots; ++i)
     if (E.slotScene[i]) {
+      notePasses(E, i, outH[i].passes, E.ranRows);
       if (outH[i].done) done.push_back(i);
       passes += outH[i].passes;
       some = some || outH[i].passes > 0;
     }
-  if (E.ranResident && some && done.empty() && passes == E.polledPasses) E.teamSkip = kTeamSkip;
+  if (E.ranRows && some && done.empty() && passes == E.polledPasses) E.teamSkip = kTeamSkip;
   E.polledPasses = passes;
-  E.ranResident = false;
+  E.ranRows = 0;
   return done;
 }
 
@@ -2353,7 +2369,7 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
   // a chunk, then the copy of the states after it into buf[b]; while the
   // class is being measured, the chunk runs the next unmeasured candidate
   // schedule between two timing events
-  bool ranResident[2] = {false, false};
+  int ranRows[2] = {0, 0};
   auto launch = [&](int b, bool timed) {
     const int ci = tc ? nextCandidate(*tc, E.chunkCand[b ^ 1]) : -1;
     if (ci >= 0) {
@@ -2368,7 +2384,7 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
     } else {
       runChunk<TM>(E, st, timed ? ev : nullptr, prof);
     }
-    ranResident[b] = resident;
+    ranRows[b] = resident ? E.teamRows : 0;
     if (ci >= 0) DV_HIP(hipEventRecord(E.tev[b][1], st));
     DV_HIP(hipMemcpyAsync(buf[b], E.out.p, sizeof(ApgdState) * E.nSlots, hipMemcpyDeviceToHost, st));
     DV_HIP(hipEventRecord(E.polled[b], st));
@@ -2401,6 +2417,7 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
     long passesNow = 0;
     int passesMost = 0;
     for (int i = 0; i < n; ++i) {
+      notePasses(E, i, last[i].passes, ranRows[cur]);
       passesNow += last[i].passes;
       passesMost = std::max(passesMost, last[i].passes);
     }
@@ -2410,7 +2427,7 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
       if (last[i].done) ++doneNow;
       else rowsLeft += (double)slotRows[i];
     }
-    if (ranResident[cur]) {
+    if (ranRows[cur]) {
       E.launched = passesMost;
       if (passesNow == passesBefore && doneNow < n) {
         resident = false;
@@ -2428,7 +2445,7 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
     activeRows = rowsLeft;
     if (doneNow == n) {
       if (tc) endMeasuredSolve(E, *tc);
-      if (n == 1 && ranResident[cur]) {
+      if (n == 1 && ranRows[cur]) {
         recordSlots<TM>(E, {0}, last);
         return;
       }

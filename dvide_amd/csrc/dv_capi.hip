@@ -224,6 +224,7 @@ int solveBuild(const Scene& s) {
 }
 
 void runSolver(Scene& s) {
+  s.residentPasses = s.teamRows = 0;
   switch (solveBuild(s)) {
     case DV_APGD_PLAIN: solvePlain(s); break;
     case DV_APGD_MIXED: solveFused(s, true); break;
@@ -240,6 +241,7 @@ void runSolver(Scene& s) {
 void stepAssembleBegin(Scene& s) {
   if (!s.initialized) throw DvError{DV_ERR_STATE, "DoTimeStep before initializeSystem"};
   s.stats = dv_stats{};
+  s.residentPasses = s.teamRows = 0;
   DV_HIP(hipEventRecord(s.ev[0], s.stream));
   collideCount(s);
 }
@@ -566,6 +568,8 @@ int dv_set_param(dv_scene* h, int param, double v) {
         if (v != 0 && v != 1 && v != 2) return dv::fail(s, DV_ERR_ARG, "rows per thread is 0 (tuned), 1 or 2");
         s.rowsPerThread = (int)v;
         break;
+      case DV_PARAM_RESIDENT_PASSES:
+      case DV_PARAM_TEAM_ROWS: return dv::fail(s, DV_ERR_ARG, "the parameter is read only");
       default: return dv::fail(s, DV_ERR_ARG, "unknown parameter");
     }
     return DV_OK;
@@ -592,6 +596,8 @@ int dv_get_param(const dv_scene* hc, int param, double* v) {
       case DV_PARAM_GRID: *v = s.grid; break;
       case DV_PARAM_PROFILE: *v = s.profKernel; break;
       case DV_PARAM_ROWS_PER_THREAD: *v = s.rowsPerThread; break;
+      case DV_PARAM_RESIDENT_PASSES: *v = s.residentPasses; break;
+      case DV_PARAM_TEAM_ROWS: *v = s.teamRows; break;
       default: return dv::fail(s, DV_ERR_ARG, "unknown parameter");
     }
     return DV_OK;

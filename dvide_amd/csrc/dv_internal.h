@@ -144,6 +144,12 @@ struct Engine {
   int nSlots = 0;
   std::vector<char> hostTable;  // Args<TM>[nSlots]
   std::vector<Scene*> slotScene;
+  // per slot: its passes when last read, and of them those that ran resident,
+  // with the row tiles per workgroup they ran with last
+  struct SlotRun {
+    int passes = 0, resident = 0, teamRows = 0;
+  };
+  std::vector<SlotRun> slotRun;
   DevBuf<char> table;
   TileSet active, admit, retire;
   DevBuf<char> out;     // ApgdState[nSlots]
@@ -156,7 +162,7 @@ struct Engine {
   int teamRows = 0;     // their row tiles per workgroup (0: some slot has no team)
   bool teamBil = false; // some have bilateral rows
   int teamSkip = 0;     // solves (or chunks) to run as launches: no team could be placed
-  bool ranResident = false;  // a server's last chunk
+  int ranRows = 0;           // teamRows of a server's last chunk (0: it ran as launches)
   long polledPasses = 0;     // of its slots, when last polled
   void* outHost = nullptr;  // pinned copies of out: two halves, by chunk parity
   hipEvent_t polled[2] = {nullptr, nullptr};  // after each half's copy
@@ -269,6 +275,7 @@ struct Scene {
 
   // --- statistics of the last step
   dv_stats stats{};
+  int residentPasses = 0, teamRows = 0;  // of the last solve (DV_PARAM_RESIDENT_PASSES, DV_PARAM_TEAM_ROWS)
   hipEvent_t ev[7] = {};  // [0..4] phases of a step, [5], [6] the plain solver's chunks
 };
 

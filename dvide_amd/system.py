@@ -25,7 +25,7 @@ SOLVER_APGD = 1  # System(int solverType): 2..7 (PDIP .. PJKIP) are rejected
 BUILD_FP64, BUILD_MIXED, BUILD_PLAIN = 0, 1, 2  # DV_APGD_*
 (PARAM_H, PARAM_MU, PARAM_TOL, PARAM_MAX_ITER, PARAM_GX, PARAM_GY, PARAM_GZ, PARAM_ENVELOPE,
  PARAM_WARM_START, PARAM_APGD_BUILD, PARAM_GEOM_MODE, PARAM_TIME, PARAM_VERBOSE, PARAM_GRID,
- PARAM_PROFILE, PARAM_ROWS_PER_THREAD, PARAM_ANTI_RELAX) = range(17)
+ PARAM_PROFILE, PARAM_ROWS_PER_THREAD, PARAM_ANTI_RELAX, PARAM_RESIDENT_PASSES, PARAM_TEAM_ROWS) = range(19)
 PROFILE_OFF, PROFILE_P1, PROFILE_P2, PROFILE_DECIDE = 0, 1, 2, 4  # DV_PARAM_PROFILE values
 VEC_P, VEC_V, VEC_GAMMA, VEC_F_CONTACT, VEC_R, VEC_K, VEC_B = range(7)
 
@@ -304,6 +304,16 @@ class System:
     def setRowsPerThread(self, r):
         """Contacts per thread of the solver's contact kernels (0 tuned, 1 or 2)."""
         self._set(PARAM_ROWS_PER_THREAD, r)
+
+    @property
+    def residentPasses(self):
+        """Passes of the last solve that ran resident (DV_PARAM_RESIDENT_PASSES)."""
+        return int(self._get(PARAM_RESIDENT_PASSES))
+
+    @property
+    def teamRows(self):
+        """Contact rows per thread of those passes (DV_PARAM_TEAM_ROWS)."""
+        return int(self._get(PARAM_TEAM_ROWS))
 
     def setProfileKernel(self, k):
         """Time one solver kernel per pass with HIP events (PROFILE_*)."""

@@ -91,6 +91,11 @@ typedef struct dv_scene dv_scene;
 #define DV_PARAM_ANTI_RELAX 16 /* 0/1                  APGD::setAntiRelaxation, APGD.cuh:63
                                   (APGD.cu:104-114, 335-345); runs on DV_APGD_PLAIN, and a
                                   DV_APGD_FP64 scene with it on is solved by that build */
+#define DV_PARAM_RESIDENT_PASSES 17 /* read only: of the last solve's passes, those that ran in
+                                       one kernel of a team of workgroups, the contacts' state
+                                       in registers; the others ran as two launches each (the
+                                       results are the same bits) */
+#define DV_PARAM_TEAM_ROWS 18 /* read only: contact rows per thread of those passes */
 
 /* state vectors (dv_get_vector / dv_set_vector) */
 #define DV_VEC_P 0         /* System::p_d        3*nb */

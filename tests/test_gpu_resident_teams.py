@@ -1,0 +1,123 @@
+"""Which solves run resident, and teams of the sizes between a few workgroups
+and half the chip.
+
+A comparison of resident passes with passes as launches says nothing where
+both sides are launches, so every case here states how many rows per thread
+its team has (0: none, the scene runs as launches) and the passes that ran
+resident are counted.  The sizes are those at which the kernel takes another
+branch: a team of more than 64 members (FP64 forms a unit's sums ahead of the
+decision up to there), members with several body tiles (a shell's contact
+points), one, two and three rows per thread, and FP64 past its last."""
+import copy
+
+import numpy as np
+import pytest
+
+from dvide_amd import scenes, system
+
+pytestmark = pytest.mark.gpu
+
+FP64, MIXED = system.BUILD_FP64, system.BUILD_MIXED
+
+
+def bits_equal(x, y):
+    x = np.asarray(x, np.float64)
+    y = np.asarray(y, np.float64)
+    return x.shape == y.shape and np.array_equal(x.view(np.uint64), y.view(np.uint64))
+
+
+def box(n):
+    return scenes.compaction(2002, n=n, width=5.0 * (n / 112000.0) ** (1.0 / 3.0), lid=scenes.LID_NONE)
+
+
+def wide_shell():
+    """640 spheres landed on a shell of 480 elements: few contacts, 70 body tiles."""
+    sc = scenes.shell_bed(3, nx=16, ny=30, per_side=(16, 40), layers=1)
+    sc.pos[:, 1] -= 1e-4
+    return sc
+
+
+SCENES = {
+    "ball": scenes.ball_on_box,
+    "pile_6000": lambda: scenes.pile(31, 6000),
+    "wide_shell": wide_shell,
+    "box_8000": lambda: box(8000),     # 36 members
+    "box_17000": lambda: box(17000),   # 77
+    "box_58000": lambda: box(58000),   # two rows a thread on 256 CUs
+    "box_118000": lambda: box(118000),  # mixed three, FP64 none
+    "bilateral_lid": lambda: scenes.compaction(5, n=1200, width=1.2, lid=scenes.LID_BILATERAL),
+}
+
+
+def _stepped(sc, build, rows, steps=2):
+    g = system.from_scene(copy.deepcopy(sc), build, tol=1e-7, max_iterations=150)
+    g.setRowsPerThread(rows)
+    out = []
+    for _ in range(steps):
+        g.step()
+        st = g.stats()
+        out.append((st.num_contacts, st.iterations, st.passes, st.backtracks, st.residual, st.objective))
+    ran = (g.residentPasses, g.teamRows, g.stats().passes)
+    vectors = (g.gamma, g.v, g.p)
+    g.close()
+    return out, vectors, ran
+
+
+@pytest.mark.parametrize("name,build,rows", [
+    ("ball", FP64, 1), ("wide_shell", FP64, 1), ("wide_shell", MIXED, 1),
+    ("box_8000", FP64, 1), ("box_8000", MIXED, 1), ("box_17000", FP64, 1), ("box_17000", MIXED, 1),
+    ("box_58000", FP64, 2), ("box_58000", MIXED, 2), ("box_118000", FP64, 0), ("box_118000", MIXED, 3)])
+def test_team_sizes_equal_the_launches(gpu, monkeypatch, name, build, rows):
+    monkeypatch.setenv("DVIDE_TUNE", "0")
+    sc = SCENES[name]()
+    launched, ref, ran = _stepped(sc, build, 1)
+    assert ran[0] == 0 and ran[1] == 0 and ran[2] > 0  # fixed rows per thread: as launches
+    assert launched[0][0] > 0
+    stats, vectors, ran = _stepped(sc, build, 0)
+    assert ran == ((ran[2], rows, ran[2]) if rows else (0, 0, ran[2]))
+    assert stats == launched
+    for a, b in zip(ref, vectors):
+        assert bits_equal(a, b)
+
+
+@pytest.mark.parametrize("how", ["batch", "server"])
+@pytest.mark.parametrize("build", [FP64, MIXED])
+def test_scenes_side_by_side_run_resident(gpu, monkeypatch, build, how):
+    """One row per thread beside each other, and with a scene past the chip's
+    CUs two for all."""
+    monkeypatch.setenv("DVIDE_TUNE", "0")
+    for names, rows in ((("ball", "pile_6000", "bilateral_lid", "wide_shell"), 1), (("pile_6000", "box_58000", "ball"), 2)):
+        scs = [SCENES[n]() for n in names]
+        members = [system.from_scene(copy.deepcopy(sc), build, tol=1e-7, max_iterations=150) for sc in scs]
+        if how == "batch":
+            b = system.Batch(build)
+            for g in members:
+                b.add(g)
+            b.step()
+            b.close()
+        else:
+            srv = system.Server(build, max_slots=4)
+            for g in members:
+                srv.submit(g)
+            assert len(srv.drain()) == len(members)
+            srv.close()
+        for n, sc, g in zip(names, scs, members):
+            launched, ref, _ = _stepped(sc, build, 1, steps=1)
+            st = g.stats()
+            assert g.residentPasses == st.passes > 0, n
+            # (a server's slots end at different times, and a team is formed for those left)
+            assert g.teamRows == rows if how == "batch" else g.teamRows in (1, rows), n
+            assert (st.num_contacts, st.iterations, st.passes) == launched[0][:3], n
+            for x, y in zip((g.gamma, g.v, g.p), ref):
+                assert bits_equal(x, y), n
+            g.close()
+
+
+def test_passes_counts_are_read_only(gpu):
+    g = system.from_scene(SCENES["ball"](), FP64)
+    assert g.residentPasses == 0 and g.teamRows == 0
+    for p in (system.PARAM_RESIDENT_PASSES, system.PARAM_TEAM_ROWS):
+        with pytest.raises(system.DvideError) as e:
+            g._set(p, 1)
+        assert e.value.code == system.DV_ERR_ARG
+    g.close()
