@@ -2095,7 +2095,7 @@ void launchTeams(Engine& E, hipStream_t st, int passes) {
   hipLaunchKernelGGL(kernel, dim3((unsigned)(places * stride)), dim3(kTC), 0, st,
                      reinterpret_cast<const Args<TM>*>(E.table.p), T,
                      E.nSlots == 1 ? nullptr : reinterpret_cast<const TeamItem*>(E.teamItems.p), stride, E.teamSync.p,
-                     ++E.teamLaunch, passes, E.nSlots == 1 ? kFormTicks : kFormTicksMany);
+                     ++E.teamLaunch, passes, (u64)(kTicksPerMs * (E.teamWaitMs >= 0 ? E.teamWaitMs : E.nSlots == 1 ? kFormMs : kFormMsMany)));
   DV_HIP(hipGetLastError());
 }
 
@@ -2244,6 +2244,12 @@ void engineOpen(Engine& E, int nSlots, bool mixed, int numCU, bool noGraph, int 
   E.nSlots = nSlots;
   E.numCU = numCU;
   E.noGraph = noGraph;
+  E.teamWaitMs = -1;
+  if (const char* wait = getenv("DVIDE_TEAM_WAIT_MS")) {
+    char* end = nullptr;
+    const double ms = strtod(wait, &end);
+    if (end != wait && ms >= 0) E.teamWaitMs = std::min(ms, kFormMsMost);
+  }
   E.launched = 0;
   E.admit.hSlots.clear();
   if (mixed) openT<float>(E, nSlots);

@@ -41,10 +41,12 @@ struct TeamItem {
 // cleared between launches.
 constexpr int kTeamMax = 256;
 constexpr int kTeamSync = 16 + kTeamMax;
-// A team whose members are not all running after this long gives up (the
-// 100 MHz wall clock): the slot's passes then run as launches.
-constexpr unsigned long long kFormTicks = 200000ull;         // 2 ms
-constexpr unsigned long long kFormTicksMany = 10000000ull;   // 100 ms: several scenes' teams wait for room
+// A team whose members are not all running after this long gives up (0: at
+// once): the slot's passes then run as launches.
+constexpr double kFormMs = 2;
+constexpr double kFormMsMany = 100;  // several scenes' teams wait for room
+constexpr double kFormMsMost = 1000;
+constexpr double kTicksPerMs = 1e5;  // of the wall clock
 
 using u64 = unsigned long long;
 
@@ -282,13 +284,13 @@ __device__ __forceinline__ void drainStores() {
 __device__ __forceinline__ bool teamForm(u64* sync, int rank, int W, u64 launch, u64 ticks) {
   __shared__ u64 outcome;
   __shared__ int late;
-  if (threadIdx.x == 0) late = 0;
+  if (threadIdx.x == 0) late = ticks == 0;
   drainStores();
   __syncthreads();
   if (W == 1) return true;
   u64* flags = sync + 16;
   if (threadIdx.x == 0) coStore(flags + rank, launch);
-  for (int i = threadIdx.x; i < W; i += kTC) {
+  for (int i = threadIdx.x; ticks && i < W; i += kTC) {
     const u64 t0 = wall_clock64();
     for (int k = 1; coLoad(flags + i) < launch; ++k)
       if ((k & 63) == 0 && wall_clock64() - t0 > ticks) {

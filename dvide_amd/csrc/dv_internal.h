@@ -161,6 +161,7 @@ struct Engine {
   std::vector<char> hTeams;
   int teamRows = 0;     // their row tiles per workgroup (0: some slot has no team)
   bool teamBil = false; // some have bilateral rows
+  double teamWaitMs = -1;  // how long a team's members wait for each other (DVIDE_TEAM_WAIT_MS; < 0: the default)
   int teamSkip = 0;     // solves (or chunks) to run as launches: no team could be placed
   int ranRows = 0;           // teamRows of a server's last chunk (0: it ran as launches)
   long polledPasses = 0;     // of its slots, when last polled

@@ -299,7 +299,16 @@ int dv_solve(dv_scene* s);
  * warm-start gamma) and remain usable alone.  A scene's result is
  * bit-identical whether it is stepped alone (dv_step with the same build) or
  * in a batch or a server mix: its partial sums are formed per tile of its
- * own rows and reduced in a fixed order. */
+ * own rows and reduced in a fixed order.
+ *
+ * A scene's passes run in one kernel whose workgroups (one per 512 contact
+ * rows, or 1,024 or 1,536) must all be on the chip at once, each filling a
+ * CU.  Where other work holds part of the chip (another batch, server or
+ * scene on a stream of its own, another process), those that have found a
+ * place wait for the rest: up to 100 ms in batches and servers, 2 ms for a
+ * scene alone, or what the environment's DVIDE_TEAM_WAIT_MS says (0: not at
+ * all; at most 1000).  The solve's passes, and those of the next 16 solves
+ * (a server: turns), then run as launches, with the same results. */
 
 typedef struct dv_batch dv_batch;
 typedef struct dv_server dv_server;

@@ -121,3 +121,61 @@ def test_passes_counts_are_read_only(gpu):
             g._set(p, 1)
         assert e.value.code == system.DV_ERR_ARG
     g.close()
+
+
+def layer(n):
+    """n spheres on a floor, one contact each."""
+    sc = scenes.layer(7, per_side=int(np.ceil(np.sqrt(n))))
+    for k in ("pos", "vel", "mass", "geom", "fixed", "family"):
+        setattr(sc, k, getattr(sc, k)[:n + 1].copy())
+    return sc
+
+
+@pytest.mark.parametrize("build", [FP64, MIXED])
+def test_a_team_that_cannot_be_placed_runs_as_launches(gpu, monkeypatch, build):
+    """With no time to wait for its members a team of several workgroups gives
+    up (every kernel exits at once): the step's passes run as launches, the
+    next 16 solves do not try, and then the team forms."""
+    monkeypatch.setenv("DVIDE_TUNE", "0")
+    sc = layer(1025)
+    ref = system.from_scene(copy.deepcopy(sc), build, tol=1e-7, max_iterations=40)
+    ref.setRowsPerThread(1)
+    g = system.from_scene(copy.deepcopy(sc), build, tol=1e-7, max_iterations=40)
+    ran = []
+    for k in range(18):
+        if k == 0:
+            monkeypatch.setenv("DVIDE_TEAM_WAIT_MS", "0")
+        else:
+            monkeypatch.delenv("DVIDE_TEAM_WAIT_MS", raising=False)
+        ref.step()
+        g.step()
+        assert (g.stats().iterations, g.stats().residual) == (ref.stats().iterations, ref.stats().residual)
+        for a, b in zip((g.gamma, g.v, g.p), (ref.gamma, ref.v, ref.p)):
+            assert bits_equal(a, b)
+        ran.append(g.residentPasses)
+    assert ran[:17] == [0] * 17 and ran[17] == g.stats().passes > 0
+    ref.close()
+    g.close()
+
+
+@pytest.mark.parametrize("build", [FP64, MIXED])
+def test_a_batch_whose_teams_cannot_be_placed_runs_as_launches(gpu, monkeypatch, build):
+    """A team of one workgroup needs no wait and runs on, those of several
+    give up; every scene's result is that of its launches."""
+    monkeypatch.setenv("DVIDE_TUNE", "0")
+    monkeypatch.setenv("DVIDE_TEAM_WAIT_MS", "0")
+    names = ("pile_6000", "ball", "bilateral_lid")
+    members = [system.from_scene(SCENES[n](), build, tol=1e-7, max_iterations=150) for n in names]
+    b = system.Batch(build)
+    for g in members:
+        b.add(g)
+    b.step()
+    b.close()
+    for n, g in zip(names, members):
+        launched, ref, _ = _stepped(SCENES[n](), build, 1, steps=1)
+        st = g.stats()
+        assert (st.num_contacts, st.iterations, st.passes) == launched[0][:3], n
+        assert g.residentPasses == (st.passes if n == "ball" else 0), n
+        for x, y in zip((g.gamma, g.v, g.p), ref):
+            assert bits_equal(x, y), n
+        g.close()
