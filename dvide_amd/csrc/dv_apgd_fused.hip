@@ -2099,15 +2099,20 @@ void launchTeams(Engine& E, hipStream_t st, int passes) {
   DV_HIP(hipGetLastError());
 }
 
-// A slot's passes as read after a chunk that ran with ranRows row tiles per
-// workgroup (0: as launches).
-void notePasses(Engine& E, int slot, int passes, int ranRows) {
+// A slot's state as read after a chunk that ran with ranRows row tiles per
+// workgroup (0: as launches).  True if its team could not be placed: a team
+// that forms runs a pass at least.  (Slot by slot: the others' passes say
+// nothing about it, and a slot just admitted has had none before either.)
+bool teamStalled(Engine& E, int slot, const ApgdState& S, int ranRows) {
   Engine::SlotRun& r = E.slotRun[slot];
-  if (ranRows && passes > r.passes) {
-    r.resident += passes - r.passes;
+  const int more = S.passes - r.passes;
+  r.passes = S.passes;
+  if (!ranRows) return false;
+  if (more > 0) {
+    r.resident += more;
     r.teamRows = ranRows;
   }
-  r.passes = passes;
+  return more == 0 && !S.done;
 }
 
 template <typename TM>
@@ -2281,9 +2286,10 @@ void engineStartAdmitted(Engine& E, hipStream_t st) {
 }
 
 void engineRunChunk(Engine& E, hipStream_t st) {
-  // resident, unless the last such launch made no progress (enginePoll)
+  // resident, unless a team of the last such launch could not be placed (enginePoll)
   const bool resident = E.teamRows && !E.noGraph && E.teamSkip == 0;
   E.ranRows = resident ? E.teamRows : 0;
+  for (int i = 0; i < E.nSlots; ++i) E.slotRun[i].inChunk = E.slotScene[i] != nullptr;
   if (E.teamSkip > 0) --E.teamSkip;
   if (resident) {
     if (E.mixed) launchTeams<float>(E, st, kTeamPassesServed);
@@ -2299,17 +2305,11 @@ std::vector<int> enginePoll(Engine& E, hipStream_t st) {
   DV_HIP(hipMemcpyAsync(outH, E.out.p, sizeof(ApgdState) * E.nSlots, hipMemcpyDeviceToHost, st));
   DV_HIP(hipStreamSynchronize(st));
   std::vector<int> done;
-  long passes = 0;
-  bool some = false;
   for (int i = 0; i < E.nSlots; ++i)
     if (E.slotScene[i]) {
-      notePasses(E, i, outH[i].passes, E.ranRows);
+      if (teamStalled(E, i, outH[i], E.slotRun[i].inChunk ? E.ranRows : 0)) E.teamSkip = kTeamSkip;
       if (outH[i].done) done.push_back(i);
-      passes += outH[i].passes;
-      some = some || outH[i].passes > 0;
     }
-  if (E.ranRows && some && done.empty() && passes == E.polledPasses) E.teamSkip = kTeamSkip;
-  E.polledPasses = passes;
   E.ranRows = 0;
   return done;
 }
@@ -2362,9 +2362,9 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
   int maxIt = 1;
   for (Scene* s : scenes) maxIt = std::max(maxIt, s->maxIt);
   const long passCap = (long)maxIt * 64 + 4096;
-  long passesBefore = 0;
-  // a class whose schedule is decided runs resident, until a launch makes no
-  // progress (no team could be placed)
+  int passesBefore = 0;  // of the first slot
+  // a class whose schedule is decided runs resident, until a team could not
+  // be placed
   const bool mayReside = !tc && !E.noGraph && !E.forcedRpt && E.teamRows && E.teamSkip == 0;
   if (E.teamSkip > 0) --E.teamSkip;
   bool resident = mayReside && !ev;  // (profiling: once the sample is taken)
@@ -2420,11 +2420,11 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
       profStats->prof_kernel_ms += ms;
       profStats->prof_kernel_count += prof == 4 ? 1 : kProfBurst;
     }
-    long passesNow = 0;
+    passesBefore = last[0].passes;
     int passesMost = 0;
+    bool stalled = false;
     for (int i = 0; i < n; ++i) {
-      notePasses(E, i, last[i].passes, ranRows[cur]);
-      passesNow += last[i].passes;
+      if (teamStalled(E, i, last[i], ranRows[cur])) stalled = true;
       passesMost = std::max(passesMost, last[i].passes);
     }
     int doneNow = 0;
@@ -2435,12 +2435,11 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
     }
     if (ranRows[cur]) {
       E.launched = passesMost;
-      if (passesNow == passesBefore && doneNow < n) {
+      if (stalled) {
         resident = false;
         E.teamSkip = kTeamSkip;
       }
     }
-    passesBefore = passesNow;
     if (tc && E.chunkCand[cur] >= 0 && doneNow == doneBefore && doneNow < n) {
       float ms = 0;
       DV_HIP(hipEventElapsedTime(&ms, E.tev[cur][0], E.tev[cur][1]));

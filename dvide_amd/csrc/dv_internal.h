@@ -148,6 +148,7 @@ struct Engine {
   // with the row tiles per workgroup they ran with last
   struct SlotRun {
     int passes = 0, resident = 0, teamRows = 0;
+    bool inChunk = false;  // a server's: it was there when the last chunk was launched
   };
   std::vector<SlotRun> slotRun;
   DevBuf<char> table;
@@ -162,9 +163,8 @@ struct Engine {
   int teamRows = 0;     // their row tiles per workgroup (0: some slot has no team)
   bool teamBil = false; // some have bilateral rows
   double teamWaitMs = -1;  // how long a team's members wait for each other (DVIDE_TEAM_WAIT_MS; < 0: the default)
-  int teamSkip = 0;     // solves (or chunks) to run as launches: no team could be placed
+  int teamSkip = 0;     // solves (or chunks) to run as launches: a team could not be placed
   int ranRows = 0;           // teamRows of a server's last chunk (0: it ran as launches)
-  long polledPasses = 0;     // of its slots, when last polled
   void* outHost = nullptr;  // pinned copies of out: two halves, by chunk parity
   hipEvent_t polled[2] = {nullptr, nullptr};  // after each half's copy
   int outHostCap = 0;

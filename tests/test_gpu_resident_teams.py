@@ -179,3 +179,39 @@ def test_a_batch_whose_teams_cannot_be_placed_runs_as_launches(gpu, monkeypatch,
         for x, y in zip((g.gamma, g.v, g.p), ref):
             assert bits_equal(x, y), n
         g.close()
+
+
+@pytest.mark.parametrize("build", [FP64, MIXED])
+def test_a_server_whose_teams_cannot_be_placed_runs_as_launches(gpu, monkeypatch, build):
+    """Freshly admitted slots whose teams give up, alone and beside a slot
+    whose team (one workgroup) forms in every turn: the next turns run as
+    launches.  The turns are bounded, so that a server that tries the teams
+    for ever fails here."""
+    monkeypatch.setenv("DVIDE_TUNE", "0")
+    monkeypatch.setenv("DVIDE_TEAM_WAIT_MS", "0")
+    for names in (("pile_6000", "bilateral_lid"), ("ball", "pile_6000")):
+        members = [system.from_scene(SCENES[n](), build, tol=1e-7, max_iterations=150) for n in names]
+        if names[0] == "ball":  # this one iterates for long
+            members[0].solver.tolerance, members[0].solver.maxIterations = 1e-300, 20000
+        srv = system.Server(build, max_slots=2)
+        for g in members:
+            srv.submit(g)
+        done, turns = [], 0
+        while srv.pending() and turns < 2000:
+            done += srv.poll()
+            turns += 1
+            if len(done) == 1 and names[0] == "ball":  # the pile, beside the ball
+                assert members[1].stats().iterations > 0 and members[0].stats().iterations == 0
+        assert sorted(done) == [1, 2]
+        srv.close()
+        for n, g in zip(names, members):
+            if n == "ball":
+                continue
+            launched, ref, _ = _stepped(SCENES[n](), build, 1, steps=1)
+            st = g.stats()
+            assert (st.num_contacts, st.iterations, st.passes) == launched[0][:3], n
+            assert g.residentPasses == 0, n
+            for x, y in zip((g.gamma, g.v, g.p), ref):
+                assert bits_equal(x, y), n
+        for g in members:
+            g.close()
