@@ -214,11 +214,11 @@ constexpr int kList = 24;
 constexpr int kLanes = 16;
 constexpr int kGroups = kT / kLanes;
 template <bool kCsr>
-__device__ void walkSmall(const CdArgs& a, int* cntUp, int* cntDown, int* lists, int* over, const int* iStart,
+__device__ void walkSmall(const CdArgs& a, int block, int* cntUp, int* cntDown, int* lists, int* over, const int* iStart,
                           int* csr) {
   __shared__ int found[kGroups], above[kGroups], ids[kGroups][kList];
   const int lane = threadIdx.x % kLanes, grp = threadIdx.x / kLanes;
-  const int t = blockIdx.x * kGroups + grp;
+  const int t = block * kGroups + grp;
   const bool on = t < a.nsmall;
   if (lane == 0) found[grp] = above[grp] = 0;
   __syncthreads();
@@ -304,13 +304,38 @@ __device__ int blockSum(int v) {
 // geometry b in its chunk; a per-big scan over the chunks then gives each
 // block its output offsets, so the emit pass writes the row in order.  Two
 // rounds of a workgroup to a chunk: with eight, few workgroups each waited
-// for eight rounds in turn (26 + 11 us at 112,000 spheres).
-constexpr int kChunk = 512;
+// for eight rounds in turn (26 + 11 us at 112,000 spheres).  Past kChunksMany
+// chunks there are workgroups enough, and eight rounds to a chunk keep the
+// counts' memory, which grows with the square of the big geometries, small;
+// past kChunksMost larger chunks keep their number an int.
+constexpr int kChunk = 512, kChunkMany = 2048;
+constexpr long kChunksMany = 1L << 20, kChunksMost = 1L << 30;
+struct Chunks {
+  int size, n;  // partners of a chunk, chunks of a big geometry
+  int all;      // chunks of all of them
+};
+Chunks chunksOf(const CdArgs& a) {
+  auto all = [&](int size) { return (long)a.nbig * blocksFor(a.nb, size); };
+  Chunks c;
+  c.size = all(kChunk) > kChunksMany ? kChunkMany : kChunk;
+  while (all(c.size) > kChunksMost) c.size *= 2;
+  c.n = blocksFor(a.nb, c.size);
+  c.all = (int)all(c.size);
+  return c;
+}
 
-__device__ void countBigChunk(const CdArgs& a, int q, int chunk, int nchunks, int* chUp, int* chDown, int* cntUp,
+// A workgroup to each of `items`, in launches of at most 2^31 threads (a
+// dimension of a grid holds less than 2^32).
+template <class Launch>
+void launchItems(int items, const Launch& launch) {
+  constexpr int kMost = 1 << 23;
+  for (int first = 0; first < items; first += kMost) launch(first, dim3(std::min(kMost, items - first)));
+}
+
+__device__ void countBigChunk(const CdArgs& a, int q, int chunk, const Chunks& ch, int* chUp, int* chDown, int* cntUp,
                               int* cntDown) {
   const int b = a.bigIds[q];
-  const int j0 = chunk * kChunk, j1 = min(a.nb, j0 + kChunk);
+  const int j0 = chunk * ch.size, j1 = min(a.nb, j0 + ch.size);
   int up = 0, down = 0;
   for (int j = j0 + threadIdx.x; j < j1; j += kT) {
     if (j == b) continue;
@@ -321,9 +346,9 @@ __device__ void countBigChunk(const CdArgs& a, int q, int chunk, int nchunks, in
   up = blockSum(up);
   down = blockSum(down);
   if (threadIdx.x == 0) {
-    const bool only = nchunks == 1;  // then there is nothing to scan
-    chUp[q * nchunks + chunk] = only ? 0 : up;
-    chDown[q * nchunks + chunk] = only ? 0 : down;
+    const bool only = ch.n == 1;  // then there is nothing to scan
+    chUp[q * ch.n + chunk] = only ? 0 : up;
+    chDown[q * ch.n + chunk] = only ? 0 : down;
     if (only) {
       cntUp[b] = up;
       cntDown[b] = down;
@@ -333,17 +358,18 @@ __device__ void countBigChunk(const CdArgs& a, int q, int chunk, int nchunks, in
 
 // The walk of the small geometries in the first walkBlocks workgroups and the
 // big ones' chunks in the others, which need nothing of each other.
-__global__ __launch_bounds__(kT) void countPartners(CdArgs a, int walkBlocks, int nchunks, int* cntUp, int* cntDown,
-                                                    int* lists, int* over, int* chUp, int* chDown) {
-  if ((int)blockIdx.x < walkBlocks) {
-    walkSmall<false>(a, cntUp, cntDown, lists, over, nullptr, nullptr);
+__global__ __launch_bounds__(kT) void countPartners(CdArgs a, int first, int walkBlocks, Chunks ch, int* cntUp,
+                                                    int* cntDown, int* lists, int* over, int* chUp, int* chDown) {
+  const int w = first + (int)blockIdx.x;
+  if (w < walkBlocks) {
+    walkSmall<false>(a, w, cntUp, cntDown, lists, over, nullptr, nullptr);
   } else {
-    const int k = (int)blockIdx.x - walkBlocks;
-    countBigChunk(a, k / nchunks, k % nchunks, nchunks, chUp, chDown, cntUp, cntDown);
+    const int k = w - walkBlocks;
+    countBigChunk(a, k / ch.n, k % ch.n, ch, chUp, chDown, cntUp, cntDown);
   }
 }
-__global__ __launch_bounds__(kT) void listPartners(CdArgs a, int* over, const int* iStart, int* csr) {
-  walkSmall<true>(a, nullptr, nullptr, nullptr, over, iStart, csr);
+__global__ __launch_bounds__(kT) void listPartners(CdArgs a, int first, int* over, const int* iStart, int* csr) {
+  walkSmall<true>(a, first + (int)blockIdx.x, nullptr, nullptr, nullptr, over, iStart, csr);
 }
 
 // per big geometry: exclusive scan of its chunk counts (in place) and totals,
@@ -354,7 +380,8 @@ __global__ __launch_bounds__(64) void scanBigChunks(CdArgs a, int nchunks, int* 
   int baseUp = 0, baseDown = 0;
   for (int k0 = 0; k0 < nchunks; k0 += 64) {
     const int k = k0 + lane;
-    const int u = k < nchunks ? chUp[q * nchunks + k] : 0, d = k < nchunks ? chDown[q * nchunks + k] : 0;
+    const int at = q * nchunks + k;
+    const int u = k < nchunks ? chUp[at] : 0, d = k < nchunks ? chDown[at] : 0;
     int su = u, sd = d;  // inclusive over the wavefront
 #pragma unroll
     for (int w = 1; w < 64; w <<= 1) {
@@ -362,8 +389,8 @@ __global__ __launch_bounds__(64) void scanBigChunks(CdArgs a, int nchunks, int* 
       if (lane >= w) { su += yu; sd += yd; }
     }
     if (k < nchunks) {
-      chUp[q * nchunks + k] = baseUp + su - u;
-      chDown[q * nchunks + k] = baseDown + sd - d;
+      chUp[at] = baseUp + su - u;
+      chDown[at] = baseDown + sd - d;
     }
     baseUp += __shfl(su, 63, 64);
     baseDown += __shfl(sd, 63, 64);
@@ -538,8 +565,8 @@ __device__ __forceinline__ void writeRecord(const CdArgs& a, const EmitOut& o, i
 
 // Rows of the small geometries, in id order and four lanes to each, so that a
 // wavefront writes one run of contacts.
-__device__ void emitSmall(const CdArgs& a, const EmitOut& o) {
-  const int t = (blockIdx.x * blockDim.x + threadIdx.x) >> 2, lane = threadIdx.x & 3;
+__device__ void emitSmall(const CdArgs& a, const EmitOut& o, int block) {
+  const int t = (block * kT + (int)threadIdx.x) >> 2, lane = threadIdx.x & 3;
   if (t >= a.nsmall) return;
   const int g = a.smallIds[t];
   const int nu = o.cntUp[g], nd = o.cntDown[g], c0 = o.cStart[g], i0 = o.iStart[g];
@@ -567,14 +594,14 @@ __device__ __forceinline__ int contactWith(const EmitOut& o, int A, int B) {
 
 // big geometry rows: ordered stream compaction of each chunk's partners, and
 // its incidences as body B (of big partners below it, ~id for now: placeBig)
-__device__ void emitBigChunk(const CdArgs& a, const EmitOut& o, int q, int chunk, int nchunks, const int* chUp,
+__device__ void emitBigChunk(const CdArgs& a, const EmitOut& o, int q, int chunk, const Chunks& ch, const int* chUp,
                              const int* chDown) {
   const int b = a.bigIds[q];
-  const int j0 = chunk * kChunk, j1 = min(a.nb, j0 + kChunk);
+  const int j0 = chunk * ch.size, j1 = min(a.nb, j0 + ch.size);
   __shared__ int baseUp, baseDown;
   if (threadIdx.x == 0) {
-    baseUp = o.cStart[b] + chUp[q * nchunks + chunk];
-    baseDown = o.iStart[b] + chDown[q * nchunks + chunk];
+    baseUp = o.cStart[b] + chUp[q * ch.n + chunk];
+    baseDown = o.iStart[b] + chDown[q * ch.n + chunk];
   }
   __syncthreads();
   __shared__ int wUp[kT / 64], wDown[kT / 64];
@@ -618,13 +645,14 @@ __device__ void emitBigChunk(const CdArgs& a, const EmitOut& o, int q, int chunk
 }
 
 // All rows: the small geometries' in the first smallBlocks workgroups.
-__global__ __launch_bounds__(kT) void emitContacts(CdArgs a, EmitOut o, int smallBlocks, int nchunks, const int* chUp,
-                                                   const int* chDown) {
-  if ((int)blockIdx.x < smallBlocks) {
-    emitSmall(a, o);
+__global__ __launch_bounds__(kT) void emitContacts(CdArgs a, EmitOut o, int first, int smallBlocks, Chunks ch,
+                                                   const int* chUp, const int* chDown) {
+  const int w = first + (int)blockIdx.x;
+  if (w < smallBlocks) {
+    emitSmall(a, o, w);
   } else {
-    const int k = (int)blockIdx.x - smallBlocks;
-    emitBigChunk(a, o, k / nchunks, k % nchunks, nchunks, chUp, chDown);
+    const int k = w - smallBlocks;
+    emitBigChunk(a, o, k / ch.n, k % ch.n, ch, chUp, chDown);
   }
 }
 
@@ -748,16 +776,17 @@ void collideCount(Scene& s) {
     exclusiveScanU(s, s.slotCount.p, s.slotStart.p, (int)T);
     hipLaunchKernelGGL(scatterSmall, dim3(blocksFor(s.nsmall, kT)), dim3(kT), 0, st, a, (const unsigned*)s.slotOf.p);
   }
-  const int nchunks = blocksFor(s.nb, kChunk);
-  s.bigChunks.reserve((size_t)2 * std::max(1, s.nbig * nchunks));
+  const Chunks ch = chunksOf(a);
+  s.bigChunks.reserve(2 * (size_t)std::max(1, ch.all));
   int* chUp = s.bigChunks.p;
-  int* chDown = s.bigChunks.p + (size_t)std::max(1, s.nbig * nchunks);
+  int* chDown = s.bigChunks.p + std::max(1, ch.all);
   const int walkBlocks = s.nsmall ? blocksFor(s.nsmall, kGroups) : 0;
-  if (walkBlocks + s.nbig)
-    hipLaunchKernelGGL(countPartners, dim3(walkBlocks + s.nbig * nchunks), dim3(kT), 0, st, a, walkBlocks, nchunks,
-                       s.cntUp.p, s.cntDown.p, s.lists.p, s.counters.p + 3, chUp, chDown);
-  if (s.nbig && nchunks > 1)
-    hipLaunchKernelGGL(scanBigChunks, dim3(s.nbig), dim3(64), 0, st, a, nchunks, chUp, chDown, s.cntUp.p, s.cntDown.p);
+  launchItems(walkBlocks + ch.all, [&](int first, dim3 grid) {
+    hipLaunchKernelGGL(countPartners, grid, dim3(kT), 0, st, a, first, walkBlocks, ch, s.cntUp.p, s.cntDown.p,
+                       s.lists.p, s.counters.p + 3, chUp, chDown);
+  });
+  if (s.nbig && ch.n > 1)
+    hipLaunchKernelGGL(scanBigChunks, dim3(s.nbig), dim3(64), 0, st, a, ch.n, chUp, chDown, s.cntUp.p, s.cntDown.p);
   // contact rows and incidence offsets, heavy bodies, and the totals for the host
   const int tiles = blocksFor(s.nb, kBodyTile);
   s.scanTmp.reserve(3 * (size_t)tiles);
@@ -769,14 +798,15 @@ void collideCount(Scene& s) {
   hipLaunchKernelGGL(scanBodies, dim3(tiles), dim3(kT), 0, st, s.nb, (const int*)s.cntUp.p, (const int*)s.cntDown.p,
                      (const int*)s.scanTmp.p, tiles, s.cStart.p, s.iStart.p, s.heavy.p,
                      s.counters.p, s.pinned);
+  DV_HIP(hipGetLastError());
 }
 
 void collideEmit(Scene& s) {
   const hipStream_t st = s.stream;
   const CdArgs a = cdArgs(s);
-  const int nchunks = blocksFor(s.nb, kChunk);
+  const Chunks ch = chunksOf(a);
   int* chUp = s.bigChunks.p;
-  int* chDown = s.bigChunks.p + (size_t)std::max(1, s.nbig * nchunks);
+  int* chDown = s.bigChunks.p + std::max(1, ch.all);
   DV_HIP(hipStreamSynchronize(st));  // the counts of collideCount
   const int nc = s.pinned[0];
   const int ninc = s.pinned[1];
@@ -799,8 +829,10 @@ void collideEmit(Scene& s) {
   const bool csr = s.pinned[2] != 0;
   if (csr) {
     s.csr.reserve(std::max(1, ninc));
-    hipLaunchKernelGGL(listPartners, dim3(blocksFor(s.nsmall, kGroups)), dim3(kT), 0, st, a, s.counters.p + 3,
-                       (const int*)s.iStart.p, s.csr.p);
+    launchItems(blocksFor(s.nsmall, kGroups), [&](int first, dim3 grid) {
+      hipLaunchKernelGGL(listPartners, grid, dim3(kT), 0, st, a, first, s.counters.p + 3, (const int*)s.iStart.p,
+                         s.csr.p);
+    });
   }
   EmitOut o;
   o.cA = s.cA.p; o.cB = s.cB.p; o.frame = s.frame.p; o.gap = s.gap.p; o.loc = s.loc.p;
@@ -809,9 +841,10 @@ void collideEmit(Scene& s) {
   o.lists = s.lists.p; o.csr = csr ? s.csr.p : nullptr;
   o.cStart = s.cStart.p; o.iStart = s.iStart.p; o.cntUp = s.cntUp.p; o.cntDown = s.cntDown.p;
   const int smallBlocks = s.nsmall ? blocksFor(4L * s.nsmall, kT) : 0;
-  if (smallBlocks + s.nbig)
-    hipLaunchKernelGGL(emitContacts, dim3(smallBlocks + s.nbig * nchunks), dim3(kT), 0, st, a, o, smallBlocks, nchunks,
-                       (const int*)chUp, (const int*)chDown);
+  launchItems(smallBlocks + ch.all, [&](int first, dim3 grid) {
+    hipLaunchKernelGGL(emitContacts, grid, dim3(kT), 0, st, a, o, first, smallBlocks, ch, (const int*)chUp,
+                       (const int*)chDown);
+  });
   if (s.bigPairs) hipLaunchKernelGGL(placeBig, dim3(16, s.nbig), dim3(kT), 0, st, a, o);
   DV_HIP(hipGetLastError());
 }
