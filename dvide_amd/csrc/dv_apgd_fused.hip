@@ -1850,33 +1850,57 @@ void Engine::release() {
 
 namespace {
 
+// capacities of a scene's rows, of their tiles and of P2's Lipschitz sums
+struct SolverCaps {
+  long rows, tiles, lq;
+  explicit SolverCaps(const Scene& s)
+      : rows(std::max<long>(3L * s.ncCap + s.nbil, 1)),
+        tiles(std::max<long>(1, ((long)s.ncCap + s.nbil + kTC - 1) / kTC)) {
+    const long bodyTiles = std::max<long>(1, ((long)s.nb + kTB - 1) / kTB);
+    // a body reduced by a workgroup has more than kHeavyDegree of the 2 nc incidences
+    lq = (bodyTiles + 2L * std::max(s.ncCap, 1) / kHeavyDegree + 2) / 2 * 2;
+  }
+};
+
+}  // namespace
+
+SolverSizes solverSizes(const Scene& s, bool mixed) {
+  const SolverCaps cap(s);
+  const size_t nc = (size_t)std::max(s.ncCap, 1), nb = (size_t)std::max(s.nb, 1);
+  SolverSizes z;
+  z.partials = (size_t)(4 + 4) * kSlots * cap.tiles + 2 * kSlots + (2 + 4) * cap.lq;  // (exchanged: 16 bytes)
+  z.work = (size_t)5 * cap.rows + 16;  // ring[4], gHat: FP64 in both solvers
+  // rn[4], r, then J and JB (per contact; J as the resident passes exchange it
+  // takes the bilateral rows too), tmp, tmp exchanged and (mixed) the four
+  // ring slots of D^T gamma (per body) of 4 components 32-byte aligned, then
+  // (mixed) M^-1
+  z.products = (size_t)5 * cap.rows + 8 + 4 * (2 * nc + s.nbil + (mixed ? 6 : 2) * nb) + (mixed ? nb + 1 : 0) + 16;
+  z.frames = mixed ? 6 * nc : 0;  // n, u
+  z.bytes = sizeof(double) * (z.partials + z.work) + (mixed ? sizeof(float) : sizeof(double)) * z.products +
+            sizeof(float) * z.frames;
+  return z;
+}
+
+namespace {
+
 // Per-scene buffers and table entry.  Work buffers are sized by capacity, so
 // that a captured graph stays valid while counts drift.
 template <typename TM>
 void prepareScene(Scene& s, Args<TM>& a) {
   constexpr bool kMixed = sizeof(TM) < sizeof(double);
-  const long RsCap = std::max<long>(3L * s.ncCap + s.nbil, 1);
-  const long itemsCap = (long)s.ncCap + s.nbil;
-  const long tilesCap = std::max<long>(1, (itemsCap + kTC - 1) / kTC);
-  const long bodyTiles = std::max<long>(1, ((long)s.nb + kTB - 1) / kTB);
-  // a body reduced by a workgroup has more than kHeavyDegree of the 2 nc incidences
-  const long lqCap = (bodyTiles + 2L * std::max(s.ncCap, 1) / kHeavyDegree + 2) / 2 * 2;
-  s.partials.reserve((size_t)(4 + 4) * kSlots * tilesCap + 2 * kSlots + (2 + 4) * lqCap);  // (exchanged: 16 bytes)
-  s.work.reserve((size_t)5 * RsCap + 16);  // ring[4], gHat: FP64 in both solvers
-  // TM block: rn[4], r, then J and JB (per contact; J as the resident passes
-  // exchange it takes the bilateral rows too), tmp, tmp exchanged and (mixed)
-  // the four ring slots of D^T gamma (per body) of 4 components 32-byte
-  // aligned, then (mixed) M^-1
+  const SolverCaps cap(s);
+  const SolverSizes sizes = solverSizes(s, kMixed);
+  const long RsCap = cap.rows, tilesCap = cap.tiles, lqCap = cap.lq;
   const size_t nbc = (size_t)std::max(s.nb, 1);
-  const size_t tmElems = (size_t)5 * RsCap + 8 + 4 * (2 * (size_t)std::max(s.ncCap, 1) + s.nbil + 2 * nbc + (kMixed ? 4 : 0) * nbc) +
-                         (kMixed ? nbc + 1 : 0) + 16;
+  s.partials.reserve(sizes.partials);
+  s.work.reserve(sizes.work);
   TM* WM;
   if (kMixed) {
-    s.frame32.reserve((size_t)6 * std::max(s.ncCap, 1));  // n, u
-    s.work32.reserve(tmElems);
+    s.frame32.reserve(sizes.frames);
+    s.work32.reserve(sizes.products);
     WM = reinterpret_cast<TM*>(s.work32.p);
   } else {
-    s.workM64.reserve(tmElems);
+    s.workM64.reserve(sizes.products);
     WM = reinterpret_cast<TM*>(s.workM64.p);
   }
   std::memset(&a, 0, sizeof(a));

@@ -1062,19 +1062,6 @@ void needScene(dv_scene* h) {
     throw DvError{DV_ERR_UNSUPPORTED, "anti-relaxation runs on the plain build, not in batches or servers"};
 }
 
-// Device memory the solver of a slot needs beyond the scene's own state:
-// the FP64 iterate ring (4 slots + gammaHat), the product vectors (4 N gamma,
-// r), J and JB, tmp, (FP64) its exchanged form, (mixed) the ring of D^T gamma,
-// M^-1 and the FP32 frames, and the partial sums (per contact tile, per body
-// tile and its four units, and per heavy body).
-double solverBytes(const Scene& s, bool mixed) {
-  const double rows = 3.0 * std::max(s.ncCap, 1) + s.nbil;
-  const double nc = std::max(s.ncCap, 1), nb = std::max(s.nb, 1);
-  const double tm = mixed ? 4 : 8;
-  return rows * (5 * 8 + 5 * tm) + nc * (8 * tm + (mixed ? 24 : 0)) + nb * ((mixed ? 21 : 8) * tm) +
-         4.0 * 8 * 8 * (1 + (rows / 3 + 1023) / 1024) + 2 * 8 * (5 * (nb / 256 + 1) + 2 * nc / kHeavyDegree + 2) + 256;
-}
-
 // f(i) for i in [0, n) on up to eight host threads (each scene has its own
 // stream and buffers, and the HIP runtime takes launches from several
 // threads), so that the per-scene launch and read-back latencies of a
@@ -1212,7 +1199,7 @@ void serverPoll(dv_server& S) {
     }
     if (free < 0) break;
     dv_server::Request r = S.waiting.front();
-    r.bytes = solverBytes(r.scene->s, S.build == DV_APGD_MIXED);
+    r.bytes = (double)solverSizes(r.scene->s, S.build == DV_APGD_MIXED).bytes;
     if (used + r.bytes > S.budget && (busy || !take.empty())) break;
     S.waiting.pop_front();
     used += r.bytes;

@@ -311,6 +311,15 @@ void solveFused(Scene& s, bool mixed);
 // N x by the graph-driven solver's own pass kernels (J store, P2, contact rows) on the
 // assembled scene; x is a flat device array, y a flat host array
 void passProduct(Scene& s, bool mixed, const double* xDev, double* yHost);
+// What the graph-driven solver of a scene holds beyond the scene's own state,
+// in entries, by the scene's capacities (an allocation may round them up).
+struct SolverSizes {
+  size_t partials, work;  // doubles
+  size_t products;        // in the build's precision
+  size_t frames;          // floats (mixed)
+  size_t bytes;           // of all
+};
+SolverSizes solverSizes(const Scene& s, bool mixed);
 // one solve of several scenes in the same launches (on stream st); each
 // scene's results equal those of solveFused on it alone
 void solveFusedMany(Engine& E, const std::vector<Scene*>& scenes, bool mixed, hipStream_t st, int numCU,
