@@ -80,53 +80,169 @@ void upload(DevBuf<T>& d, const std::vector<T>& h, hipStream_t st) {
   if (!h.empty()) DV_HIP(hipMemcpyAsync(d.p, h.data(), sizeof(T) * h.size(), hipMemcpyHostToDevice, st));
 }
 
-// Vectors of up to 1 MB travel between the caller's memory and the device
-// through pinned memory of the scene's that a kernel reads or writes: with the
-// runtime's own copies from and to pageable memory a call took 17 us in and 23
-// out for 48 bytes, now 14 and 14; 31 and 34 for 24 to 190 KB, now 17 and 17.
-// Past 1 MB the host's copy costs more than the runtime's, which pins the
-// caller's pages.
-constexpr size_t kStagingMost = 1 << 17;  // doubles
+// Memory that a call needs while it runs is borrowed from a pool instead of
+// being kept by every scene: a fresh allocation takes 35 to 340 us here (pinned
+// or past 2 MB), which a scene's first call would pay.  A block belongs to one call
+// at a time; idle ones are kept up to `most` bytes, largest first, and freed
+// when the last scene is destroyed.
+struct Block {
+  void* p = nullptr;
+  size_t cap = 0;
+  int device = 0;
+};
+class Pool {
+ public:
+  Pool(bool pinned, size_t most) : pinned(pinned), most(most) { idle.reserve(kIdleMost + 1); }
+  // a block of at least `bytes`; none (p null) for no bytes, or if it cannot be
+  // allocated
+  Block take(int device, size_t bytes) {
+    if (!bytes) return Block{};
+    {
+      std::lock_guard<std::mutex> lock(m);
+      size_t best = idle.size();
+      for (size_t i = 0; i < idle.size(); ++i)
+        if (idle[i].device == device && idle[i].cap >= bytes && (best == idle.size() || idle[i].cap < idle[best].cap))
+          best = i;
+      if (best < idle.size()) return remove(best);
+    }
+    Block b;
+    b.device = device;
+    b.cap = size_t(1) << 16;
+    while (b.cap < bytes) b.cap *= 2;
+    if (b.cap > most) b.cap = bytes;  // (which is not kept)
+    const hipError_t e = pinned ? hipHostMalloc(&b.p, b.cap, hipHostMallocDefault) : hipMalloc(&b.p, b.cap);
+    if (e != hipSuccess) {
+      (void)hipGetLastError();
+      b.p = nullptr;
+    }
+    return b;
+  }
+  void give(const Block& b) {
+    if (b.cap > most) return free(b);
+    std::lock_guard<std::mutex> lock(m);
+    idle.push_back(b);
+    held += b.cap;
+    while (held > most || idle.size() > kIdleMost) {
+      size_t least = 0;
+      for (size_t i = 1; i < idle.size(); ++i)
+        if (idle[i].cap < idle[least].cap) least = i;
+      free(remove(least));
+    }
+  }
+  void drop() {
+    std::lock_guard<std::mutex> lock(m);
+    while (!idle.empty()) free(remove(idle.size() - 1));
+  }
+
+ private:
+  static constexpr size_t kIdleMost = 64;
+  Block remove(size_t i) {
+    const Block b = idle[i];
+    idle.erase(idle.begin() + i);
+    held -= b.cap;
+    return b;
+  }
+  void free(const Block& b) { (void)(pinned ? hipHostFree(b.p) : hipFree(b.p)); }
+  std::mutex m;
+  std::vector<Block> idle;
+  size_t held = 0;
+  const bool pinned;
+  const size_t most;
+};
+// (never destroyed: at exit the runtime may be gone before them)
+Pool& pinnedPool() {
+  static Pool& p = *new Pool(true, size_t(16) << 20);
+  return p;
+}
+Pool& productPool() {
+  static Pool& p = *new Pool(false, size_t(16) << 20);
+  return p;
+}
+std::mutex scenesMutex;
+long scenesAlive = 0;
+void sceneBorn() {
+  std::lock_guard<std::mutex> lock(scenesMutex);
+  ++scenesAlive;
+}
+void sceneGone() {
+  std::lock_guard<std::mutex> lock(scenesMutex);
+  if (--scenesAlive) return;
+  pinnedPool().drop();
+  productPool().drop();
+}
+// A block for one call on scene s.  What the call queued on the scene's stream
+// has ended when the block goes back: the call waits for it, or this does.
+class Lease {
+ public:
+  Lease(Pool& pool, Scene& s, size_t bytes) : pool(pool), s(s), b(pool.take(s.device, bytes)) {}
+  Lease(const Lease&) = delete;
+  Lease& operator=(const Lease&) = delete;
+  ~Lease() {
+    if (!b.p) return;
+    if (!waited) (void)hipStreamSynchronize(s.stream);
+    pool.give(b);
+  }
+  double* p() const { return static_cast<double*>(b.p); }
+  void wait() {
+    DV_HIP(hipStreamSynchronize(s.stream));
+    waited = true;
+  }
+  void ended() { waited = true; }  // the call has waited for the stream
+
+ private:
+  Pool& pool;
+  Scene& s;
+  Block b;
+  bool waited = false;
+};
+
+// Vectors of up to 2 MB travel between the caller's memory and the device
+// through pinned memory that a kernel reads or writes: with the runtime's own
+// copies from and to pageable memory a call took 17 us in and 23 out for 48
+// bytes, now 14 and 14; 31 and 34 for 24 to 190 KB, now 17 and 17.  Past 1 MB
+// the runtime pins the caller's pages, which it does quickly or not as they
+// lie: 1.1 MB took 54 to 400 us in and 74 to 630 out, and so 52 and 72.
+constexpr size_t kStagingMost = 1 << 18;  // doubles
 __global__ void kMove(double* dst, const double* src, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = src[i];
 }
-bool stage(Scene& s, size_t n) {  // whether n doubles go that way
-  if (n > kStagingMost) return false;
-  if (s.stagingCap < n) {
-    if (s.staging) DV_HIP(hipHostFree(s.staging));
-    s.staging = nullptr;
-    s.stagingCap = 0;
-    const size_t cap = std::min(kStagingMost, std::max<size_t>(2 * n, 512));
-    DV_HIP(hipHostMalloc(&s.staging, sizeof(double) * cap, hipHostMallocDefault));
-    s.stagingCap = cap;
+class Staging {
+ public:
+  Staging(Scene& s, size_t n)
+      : s(s), n(n), lease(pinnedPool(), s, n <= kStagingMost ? sizeof(double) * n : 0) {}
+  // in: queued, and the caller's memory read; out: queued, and in the caller's
+  // memory after takeOut.  Both directions share the memory, in stream order.
+  void moveIn(double* dst, const double* in) {
+    if (!n) return;
+    if (staged()) {
+      std::memcpy(lease.p(), in, sizeof(double) * n);
+      move(dst, lease.p());
+    } else {
+      DV_HIP(hipMemcpyAsync(dst, in, sizeof(double) * n, hipMemcpyHostToDevice, s.stream));
+    }
   }
-  return true;
-}
-void move(Scene& s, double* dst, const double* src, size_t n) {
-  hipLaunchKernelGGL(kMove, dim3(blocksFor((long)n, 256)), dim3(256), 0, s.stream, dst, src, (long)n);
-  DV_HIP(hipGetLastError());
-}
-// in: queued, and the caller's memory read; out: queued, and in the caller's
-// memory after takeOut.  Both directions share the memory, in stream order.
-void moveIn(Scene& s, double* dst, const double* in, size_t n) {
-  if (!n) return;
-  if (stage(s, n)) {
-    std::memcpy(s.staging, in, sizeof(double) * n);
-    move(s, dst, s.staging, n);
-  } else {
-    DV_HIP(hipMemcpyAsync(dst, in, sizeof(double) * n, hipMemcpyHostToDevice, s.stream));
+  void moveOut(double* out, const double* src) {
+    if (!n) return;
+    if (staged()) move(lease.p(), src);
+    else DV_HIP(hipMemcpyAsync(out, src, sizeof(double) * n, hipMemcpyDeviceToHost, s.stream));
   }
-}
-void moveOut(Scene& s, double* out, const double* src, size_t n) {
-  if (!n) return;
-  if (stage(s, n)) move(s, s.staging, src, n);
-  else DV_HIP(hipMemcpyAsync(out, src, sizeof(double) * n, hipMemcpyDeviceToHost, s.stream));
-}
-void takeOut(Scene& s, double* out, size_t n) {
-  DV_HIP(hipStreamSynchronize(s.stream));
-  if (n && n <= kStagingMost) std::memcpy(out, s.staging, sizeof(double) * n);
-}
+  void wait() { lease.wait(); }
+  void takeOut(double* out) {
+    wait();
+    if (n && staged()) std::memcpy(out, lease.p(), sizeof(double) * n);
+  }
+
+ private:
+  bool staged() const { return n <= kStagingMost && lease.p(); }  // (no pinned memory left: the runtime's copies)
+  void move(double* dst, const double* src) {
+    hipLaunchKernelGGL(kMove, dim3(blocksFor((long)n, 256)), dim3(256), 0, s.stream, dst, src, (long)n);
+    DV_HIP(hipGetLastError());
+  }
+  Scene& s;
+  const size_t n;
+  Lease lease;
+};
 
 __global__ void kProjectN(double* g, long n, double mu) {
   long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -335,6 +451,7 @@ int dv_scene_create(dv_scene** out, int solverType) {
     dv_scene* h = new dv_scene();
     const char* ng = getenv("DVIDE_NO_GRAPH");
     h->s.noGraph = ng && ng[0] == '1';
+    dv::sceneBorn();
     *out = h;
     return DV_OK;
   } catch (...) {
@@ -348,7 +465,7 @@ int dv_scene_destroy(dv_scene* h) {
   if (s.stream) (void)hipStreamSynchronize(s.stream);
   dv::DevBuf<double>* dbufs[] = {&s.p, &s.v, &s.f, &s.k, &s.fContact, &s.tmp, &s.minv, &s.geom, &s.bilVel,
                                  &s.bilT0, &s.bilP0, &s.cellPosR, &s.frame, &s.gap, &s.loc, &s.r,
-                                 &s.b, &s.gamma, &s.work, &s.partials, &s.product, &s.shellNodes, &s.ptS, &s.shellF};
+                                 &s.b, &s.gamma, &s.work, &s.partials, &s.shellNodes, &s.ptS, &s.shellF};
   for (auto* b : dbufs) b->release();
   dv::DevBuf<int>* ibufs[] = {&s.family, &s.smallIds, &s.bigIds, &s.bilA, &s.bilB, &s.bilIncStart,
                               &s.bilInc, &s.cellMeta, &s.lists, &s.csr, &s.cntUp, &s.cntDown, &s.cStart, &s.iStart,
@@ -364,12 +481,12 @@ int dv_scene_destroy(dv_scene* h) {
   if (s.plainHost) (void)hipHostFree(s.plainHost);
   s.workM64.release();
   if (s.pinned) (void)hipHostFree(s.pinned);
-  if (s.staging) (void)hipHostFree(s.staging);
   for (auto& e : s.ev)
     if (e) (void)hipEventDestroy(e);
   for (auto& e : s.profEv) (void)hipEventDestroy(e);
   if (s.stream) (void)hipStreamDestroy(s.stream);
   delete h;
+  dv::sceneGone();
   return DV_OK;
 }
 
@@ -685,7 +802,8 @@ int dv_get_vector(dv_scene* h, int which, double* out, size_t n, size_t* len) {
     if (len) *len = L;
     if (!out || !n) return DV_OK;
     const size_t m = std::min(n, dof ? nBody : L);
-    dv::moveOut(s, out, src, m);
+    dv::Staging staging(s, m);
+    staging.moveOut(out, src);
     std::vector<double> sh;
     if (dof && n > nBody && nShell) {  // the shell DOFs: fixed nodes, no velocity
       if (which == DV_VEC_P) sh = s.hShellNodes;
@@ -696,7 +814,7 @@ int dv_get_vector(dv_scene* h, int which, double* out, size_t n, size_t* len) {
         DV_HIP(hipMemcpyAsync(sh.data(), s.shellF.p, sizeof(double) * nShell, hipMemcpyDeviceToHost, s.stream));
       }
     }
-    dv::takeOut(s, out, m);
+    staging.takeOut(out);
     if (!sh.empty()) std::copy(sh.begin(), sh.begin() + std::min(nShell, n - nBody), out + nBody);
     return DV_OK;
   });
@@ -722,8 +840,9 @@ int dv_set_vector(dv_scene* h, int which, const double* in, size_t n) {
       n = nBody;
     }
     if (n) {
-      dv::moveIn(s, dst, in, n);
-      DV_HIP(hipStreamSynchronize(s.stream));
+      dv::Staging staging(s, n);
+      staging.moveIn(dst, in);
+      staging.wait();
     }
     return DV_OK;
   });
@@ -915,15 +1034,14 @@ int dv_schur_product(dv_scene* h, const double* x, double* y, size_t n) {
   return dv::guarded(h, [&](Scene& s) {
     if (n != (size_t)s.R || !x || !y) return dv::fail(s, DV_ERR_ARG, "x and y need nbil + 3*nc entries");
     if (n == 0) return DV_OK;
-    // the scene keeps the vectors up to 16 MB (a product of 60,000 rows took 228
-    // us with an allocation and copies of pageable memory, 172 so)
-    dv::DevBuf<double>& buf = s.product;
-    buf.reserve(2 * n);
-    dv::moveIn(s, buf.p, x, n);
-    dv::schurExact(s, buf.p, buf.p + n);
-    dv::moveOut(s, y, buf.p + n, n);
-    dv::takeOut(s, y, n);
-    if (buf.cap > (size_t)1 << 21) buf.release();
+    dv::Lease buf(dv::productPool(), s, 2 * sizeof(double) * n);
+    if (!buf.p()) throw dv::DvError{DV_ERR_NOMEM, "device allocation of the product's vectors failed"};
+    dv::Staging staging(s, n);
+    staging.moveIn(buf.p(), x);
+    dv::schurExact(s, buf.p(), buf.p() + n);
+    staging.moveOut(y, buf.p() + n);
+    staging.takeOut(y);
+    buf.ended();
     return DV_OK;
   });
 }

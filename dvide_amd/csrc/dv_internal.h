@@ -244,9 +244,6 @@ struct Scene {
   DevBuf<int> cntUp, cntDown, cStart, iStart, scanTmp;
   DevBuf<int> counters;     // [2] nHeavy, [3] a partner list overflowed
   int* pinned = nullptr;    // pinned: contacts, incidences, overflow of the last count
-  double* staging = nullptr;  // pinned: a vector on its way between the caller and the device
-  size_t stagingCap = 0;
-  DevBuf<double> product;     // dv_schur_product: x and y
 
   // --- contacts (canonical (idA, idB) order)
   int nc = 0, ncCap = 0;
