@@ -1632,7 +1632,7 @@ constexpr int kManySlotsN = (int)(sizeof(kManySlots) / sizeof(kManySlots[0]));
 struct TuneClass {
   std::vector<double> score;  // per candidate: us per pass per million active rows (< 0: not measured)
   int best = -1;              // the chosen candidate (-1: still measuring)
-  int solves = 0;             // finished while measuring
+  int solves = 0;             // measured to their end without a decision
   Schedule sched;             // its schedule (also when read from the file)
 };
 
@@ -1766,15 +1766,17 @@ bool recordCandidate(Engine& E, TuneClass& c, int i, double score) {
   return true;
 }
 
-// Solves of a few passes end before a candidate's chunk counts; after
-// kMeasuredSolves of them the class takes the first candidate for this
-// process (nothing is written to the file).
+// Solves of a few passes end before a candidate's chunk counts.  After
+// kMeasuredSolves of them the class's solves that can run resident do, and
+// only those that run as launches measure on.
 constexpr int kMeasuredSolves = 8;
-void endMeasuredSolve(Engine& E, TuneClass& c) {
+void endMeasuredSolve(TuneClass& c) {
   std::lock_guard<std::mutex> lock(tuner().m);
-  if (c.best >= 0 || ++c.solves < kMeasuredSolves) return;
-  c.best = 0;
-  c.sched = (E.nSlots == 1 ? kOneSlot : kManySlots)[0];
+  if (c.best < 0 && c.solves < kMeasuredSolves) ++c.solves;
+}
+bool measuredEnough(TuneClass& c) {
+  std::lock_guard<std::mutex> lock(tuner().m);
+  return c.solves >= kMeasuredSolves;
 }
 
 const Schedule& candidate(const Engine& E, int i) { return (E.nSlots == 1 ? kOneSlot : kManySlots)[i]; }
@@ -2367,13 +2369,15 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
   std::vector<long> slotRows(n);
   for (int i = 0; i < n; ++i) rows += slotRows[i] = (long)scenes[i]->nc + scenes[i]->nbil;
   TuneClass* tc = chooseSchedule(E, rows, prof == 0);
+  startAdmitted<TM>(E, st);
+  const bool hasTeams = !E.noGraph && !E.forcedRpt && E.teamRows && E.teamSkip == 0;
+  if (tc && hasTeams && measuredEnough(*tc)) tc = nullptr;
   E.tuning = tc ? 1 : 0;
   if (tc)
     for (auto& pair : E.tev)
       for (hipEvent_t& e : pair)
         if (!e) DV_HIP(hipEventCreate(&e));
   E.chunkCand[0] = E.chunkCand[1] = -1;
-  startAdmitted<TM>(E, st);
   hipEvent_t* ev = nullptr;
   if (prof && profEv) {
     while (profEv->size() < 2) {
@@ -2387,9 +2391,9 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
   for (Scene* s : scenes) maxIt = std::max(maxIt, s->maxIt);
   const long passCap = (long)maxIt * 64 + 4096;
   int passesBefore = 0;  // of the first slot
-  // a class whose schedule is decided runs resident, until a team could not
-  // be placed
-  const bool mayReside = !tc && !E.noGraph && !E.forcedRpt && E.teamRows && E.teamSkip == 0;
+  // a solve that does not measure runs resident, until a team could not be
+  // placed
+  const bool mayReside = !tc && hasTeams;
   if (E.teamSkip > 0) --E.teamSkip;
   bool resident = mayReside && !ev;  // (profiling: once the sample is taken)
   ApgdState* outH = reinterpret_cast<ApgdState*>(E.outHost);
@@ -2473,7 +2477,7 @@ void solveAll(Engine& E, const std::vector<Scene*>& scenes, hipStream_t st, int 
     doneBefore = doneNow;
     activeRows = rowsLeft;
     if (doneNow == n) {
-      if (tc) endMeasuredSolve(E, *tc);
+      if (tc) endMeasuredSolve(*tc);
       if (n == 1 && ranRows[cur]) {
         recordSlots<TM>(E, {0}, last);
         return;
