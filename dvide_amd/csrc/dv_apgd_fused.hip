@@ -109,7 +109,6 @@ struct SolveDims {
 namespace {
 
 constexpr int kTC = 512;   // contact kernels: 8 wavefronts, one tile of rows
-constexpr int kTB = 256;   // body kernel: one tile of bodies
 constexpr int kTD = 64;    // setup and final decisions: one wavefront per scene
 constexpr int kBacktrackCap = 1100;  // L doubles past 1e308 long before this
 constexpr int kPassesPerChunk = 16;  // even: a chunk ends on parity 0
@@ -2072,6 +2071,18 @@ Plan<TM> activePlan(Engine& E) {
 // and mixed, 3 tiles 7.4 and 7.0, 5.5 and 5.2; 5 tiles 7.5 and 7.0, 5.8 and
 // 5.3; 10 tiles 7.5 and 7.3, 5.8 and 5.5; 19 tiles 7.7 and 8.7, 5.8 and 6.0.
 constexpr int kXcdMost = 10;
+// Where bodies outnumber contacts, a member's share of them is what a pass
+// waits for (units of movable bodies, in contact or not).  Past kBodiesMany
+// tiles to a member a team gets members without rows: one to every kBodiesEach
+// tiles if the chip holds all teams so, or else to the fewest more (twice,
+// four times as many, ...) with which it does.  us per pass of 100 contacts among 1,024, 4,096 and 7,936 movable bodies
+// as launches, on one member and so: FP64 9.2, 8.1 and 7.3; 9.0, 12.8 and 7.3;
+// 9.0, 18.4 and 7.6; mixed 8.1, 7.0 and 5.8; 8.3, 12.8 and 5.8; 8.0, 21.3 and
+// 6.0.  (Past the chip a batch's teams would wait for each other: 128 scenes of
+// 4,096 bodies 25.4 as launches, 13.3 on a member each, 38 on eight.)  A scene
+// alone with more than kBodiesMost tiles to a member runs as launches: with 14
+// they take 19.6 against 16.1, with 53 36.2 against 45.9.
+constexpr int kBodiesMany = 4, kBodiesEach = 2, kBodiesMost = 16;
 constexpr int kTeamPasses = 2048;     // of one launch of a single scene (tags: 2 p + 3 < 65,536)
 constexpr int kTeamPassesMany = 512;  // of several scenes: a team waits for the room of those before it
 constexpr int kTeamPassesServed = 64; // of a server, which admits and completes between launches
@@ -2088,13 +2099,25 @@ void buildTeams(Engine& E, hipStream_t st) {
   if (E.mixed)  // (three rows in FP64 have no room in LDS)
     for (int slot : E.active.hSlots)
       if (slotArgs<TM>(E, slot).nTiles > 2L * most) R = 3;
+  int each = kBodiesEach;  // body tiles to a member where they decide; 0: the rows do
+  auto membersOf = [&](int slot) {
+    const int rows = (slotArgs<TM>(E, slot).nTiles + R - 1) / R, bodies = E.slotScene[slot]->freeTiles;
+    return each && bodies > kBodiesMany * rows ? std::max(rows, std::min(most, (bodies + each - 1) / each)) : rows;
+  };
+  for (;; each *= 2) {
+    long places = 0;
+    for (int slot : E.active.hSlots) places += membersOf(slot);
+    if (places <= E.numCU || !each) break;
+    if (each >= 64) each = 0;
+  }
   std::vector<TeamItem> items;
   E.teamRows = E.active.hSlots.empty() ? 0 : R;
   E.teamBil = false;
   for (int slot : E.active.hSlots) {
     const Args<TM>& a = slotArgs<TM>(E, slot);
-    const int members = (a.nTiles + R - 1) / R;
+    const int members = membersOf(slot);
     if (members > most || a.nBodyTiles > 64L * members) E.teamRows = 0;  // (32 rounds of body units)
+    if (E.nSlots == 1 && E.slotScene[slot]->freeTiles > kBodiesMost * members) E.teamRows = 0;
     if (a.cap + a.dims.nbil > 1L << 26) E.teamRows = 0;  // (32-bit offsets into the exchanged J)
     for (int k = 0; k < members; ++k) items.push_back(TeamItem{slot, k, members, 0});
     E.teamBil = E.teamBil || a.dims.nbil > 0;

@@ -274,6 +274,12 @@ void initialize(Scene& s) {
     for (int c = 0; c < 3; ++c) f[3 * j + c] = s.hFixed[j] ? 0.0 : s.hMass[j] * s.g[c];
     minv[j] = s.hFixed[j] ? 0.0 : 1.0 / s.hMass[j];
   }
+  s.freeTiles = 0;
+  for (int j = 0, last = -1; j < nb; ++j)
+    if (minv[j] != 0 && j / kTB != last) {
+      last = j / kTB;
+      ++s.freeTiles;
+    }
   const hipStream_t st = s.stream;
   upload(s.p, s.hPos, st);
   upload(s.v, s.hVel, st);

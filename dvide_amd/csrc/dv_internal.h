@@ -69,6 +69,7 @@ struct DevBuf {
 constexpr int kHeavyDegree = 128;
 
 constexpr int kSlots = 8;  // reduction slots of the solver kernels
+constexpr int kTB = 256;   // the solvers' body tile
 
 // Most contact points a shell mesh may add (elements x (points per side - 2)^2).
 constexpr long kMaxShellPoints = 1L << 26;
@@ -225,6 +226,7 @@ struct Scene {
   hipStream_t stream = nullptr;
   int device = 0, numCU = 0;
   int nb = 0, nbil = 0;
+  int freeTiles = 0;     // body tiles with a movable body
   int nsmall = 0, nbig = 0;
   double cellSize = 0;
   unsigned hashSize = 0;

@@ -37,8 +37,31 @@ def wide_shell():
     return sc
 
 
+def layer(n):
+    """n spheres on a floor, one contact each."""
+    sc = scenes.layer(7, per_side=int(np.ceil(np.sqrt(n))))
+    for k in ("pos", "vel", "mass", "geom", "fixed", "family"):
+        setattr(sc, k, getattr(sc, k)[:n + 1].copy())
+    return sc
+
+
+def among(sc, n):
+    """The scene and n free spheres far above it that touch nothing."""
+    k, r = np.arange(n), 0.05
+    side = int(np.ceil(np.sqrt(n)))
+    pos = np.stack([3 * r * (k % side), np.full(n, 50.0), 3 * r * (k // side)], 1)
+    for name, more in (("pos", pos), ("vel", np.zeros((n, 3))), ("mass", np.ones(n)), ("geom", np.tile([[r, 0.0, 0.0]], (n, 1))),
+                       ("fixed", np.zeros(n, np.int32)), ("family", np.full(n, -1, np.int32))):
+        setattr(sc, name, np.concatenate([getattr(sc, name), more]).astype(more.dtype))
+    return sc
+
+
 SCENES = {
     "ball": scenes.ball_on_box,
+    # bodies decide the team's size: 16 members of which one has rows, and 256
+    # of which 134 have two tiles each
+    "few_contacts": lambda: among(layer(100), 7900),
+    "many_bodies": lambda: among(box(58000), 150000),
     "pile_6000": lambda: scenes.pile(31, 6000),
     "wide_shell": wide_shell,
     "box_8000": lambda: box(8000),     # 36 members
@@ -66,6 +89,7 @@ def _stepped(sc, build, rows, steps=2):
 @pytest.mark.parametrize("name,build,rows", [
     ("ball", FP64, 1), ("wide_shell", FP64, 1), ("wide_shell", MIXED, 1),
     ("box_8000", FP64, 1), ("box_8000", MIXED, 1), ("box_17000", FP64, 1), ("box_17000", MIXED, 1),
+    ("few_contacts", FP64, 1), ("few_contacts", MIXED, 1), ("many_bodies", FP64, 2), ("many_bodies", MIXED, 2),
     ("box_58000", FP64, 2), ("box_58000", MIXED, 2), ("box_118000", FP64, 0), ("box_118000", MIXED, 3)])
 def test_team_sizes_equal_the_launches(gpu, monkeypatch, name, build, rows):
     monkeypatch.setenv("DVIDE_TUNE", "0")
@@ -86,7 +110,7 @@ def test_scenes_side_by_side_run_resident(gpu, monkeypatch, build, how):
     """One row per thread beside each other, and with a scene past the chip's
     CUs two for all."""
     monkeypatch.setenv("DVIDE_TUNE", "0")
-    for names, rows in ((("ball", "pile_6000", "bilateral_lid", "wide_shell"), 1), (("pile_6000", "box_58000", "ball"), 2)):
+    for names, rows in ((("ball", "pile_6000", "bilateral_lid", "wide_shell", "few_contacts"), 1), (("pile_6000", "box_58000", "ball"), 2)):
         scs = [SCENES[n]() for n in names]
         members = [system.from_scene(copy.deepcopy(sc), build, tol=1e-7, max_iterations=150) for sc in scs]
         if how == "batch":
@@ -123,12 +147,23 @@ def test_passes_counts_are_read_only(gpu):
     g.close()
 
 
-def layer(n):
-    """n spheres on a floor, one contact each."""
-    sc = scenes.layer(7, per_side=int(np.ceil(np.sqrt(n))))
-    for k in ("pos", "vel", "mass", "geom", "fixed", "family"):
-        setattr(sc, k, getattr(sc, k)[:n + 1].copy())
-    return sc
+@pytest.mark.parametrize("build", [FP64, MIXED])
+def test_few_contacts_among_many_bodies_take_no_longer(gpu, monkeypatch, build):
+    """100 contacts among 8,000 movable bodies: a pass on the one member that
+    the rows need took 2.0 (FP64) and 2.6 times as long as one as launches,
+    and on the sixteen that the bodies get takes 0.8 and 0.7 times as long."""
+    monkeypatch.setenv("DVIDE_TUNE", "0")
+    us = []
+    for rows in (1, 0):
+        g = system.from_scene(SCENES["few_contacts"](), build, tol=1e-300, max_iterations=200)
+        g.setRowsPerThread(rows)
+        best = np.inf
+        for _ in range(6):
+            g.step()
+            best = min(best, 1e3 * g.stats().ms_solve / g.stats().passes)
+        us.append(best)
+        g.close()
+    assert us[1] < 1.3 * us[0], us
 
 
 @pytest.mark.parametrize("build", [FP64, MIXED])
