@@ -2083,6 +2083,13 @@ constexpr int kXcdMost = 10;
 // alone with more than kBodiesMost tiles to a member runs as launches: with 14
 // they take 19.6 against 16.1, with 53 36.2 against 45.9.
 constexpr int kBodiesMany = 4, kBodiesEach = 2, kBodiesMost = 16;
+// A body's bilateral rows are awaited one after another.  us per pass of a body
+// with 7, 15, 26 and 49 of them as launches and resident: FP64 9.0 and 7.8,
+// 10.2 and 11.6, 12.2 and 16.5, 16.0 and 30; mixed 8.5 and 5.9, 9.9 and 9.0,
+// 11.8 and 14, 15.8 and 26; several scenes' launches take 18 to 20.  (Four rows
+// awaited together: 23 and 20 with 49, but in FP64 6.8 became 7.6 where bodies
+// have two, for want of registers.)
+constexpr int kBilMost = 12, kBilMostMany = 32;
 constexpr int kTeamPasses = 2048;     // of one launch of a single scene (tags: 2 p + 3 < 65,536)
 constexpr int kTeamPassesMany = 512;  // of several scenes: a team waits for the room of those before it
 constexpr int kTeamPassesServed = 64; // of a server, which admits and completes between launches
@@ -2117,6 +2124,7 @@ void buildTeams(Engine& E, hipStream_t st) {
     const Args<TM>& a = slotArgs<TM>(E, slot);
     const int members = membersOf(slot);
     if (members > most || a.nBodyTiles > 64L * members) E.teamRows = 0;  // (32 rounds of body units)
+    if (E.slotScene[slot]->bilMost > (E.nSlots == 1 ? kBilMost : kBilMostMany)) E.teamRows = 0;
     if (E.nSlots == 1 && E.slotScene[slot]->freeTiles > kBodiesMost * members) E.teamRows = 0;
     if (a.cap + a.dims.nbil > 1L << 26) E.teamRows = 0;  // (32-bit offsets into the exchanged J)
     for (int k = 0; k < members; ++k) items.push_back(TeamItem{slot, k, members, 0});

@@ -315,7 +315,9 @@ void initialize(Scene& s) {
     if (s.hBilB[i] >= 0) per[s.hBilB[i] / 3].push_back((i << 3) | ((s.hBilB[i] % 3) << 1) | 1);
   }
   std::vector<int> bs(nb + 1, 0), bl;
+  s.bilMost = 0;
   for (int j = 0; j < nb; ++j) {
+    s.bilMost = std::max(s.bilMost, (int)per[j].size());
     bs[j + 1] = bs[j] + (int)per[j].size();
     for (int e : per[j]) bl.push_back(e);
   }

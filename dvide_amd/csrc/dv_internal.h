@@ -227,6 +227,7 @@ struct Scene {
   int device = 0, numCU = 0;
   int nb = 0, nbil = 0;
   int freeTiles = 0;     // body tiles with a movable body
+  int bilMost = 0;       // most bilateral rows of a body
   int nsmall = 0, nbig = 0;
   double cellSize = 0;
   unsigned hashSize = 0;

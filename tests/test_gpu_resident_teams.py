@@ -14,6 +14,7 @@ import numpy as np
 import pytest
 
 from dvide_amd import scenes, system
+from tests.helpers import tiny_scene
 
 pytestmark = pytest.mark.gpu
 
@@ -164,6 +165,38 @@ def test_few_contacts_among_many_bodies_take_no_longer(gpu, monkeypatch, build):
         us.append(best)
         g.close()
     assert us[1] < 1.3 * us[0], us
+
+
+def star(n):
+    """A sphere whose x is tied to those of n others: n bilateral rows of one body."""
+    pos = np.stack([0.3 * np.arange(n + 1), np.full(n + 1, 5.0), np.zeros(n + 1)], 1)
+    return tiny_scene(pos, [[0.05, 0, 0]] * (n + 1), bilaterals=[(0, 3 * i, 0.0, 0.0) for i in range(1, n + 1)])
+
+
+@pytest.mark.parametrize("build", [FP64, MIXED])
+@pytest.mark.parametrize("n,alone,beside", [(12, 1, 1), (13, 0, 1), (32, 0, 1), (33, 0, 0)])
+def test_bodies_with_many_bilateral_rows_run_as_launches(gpu, monkeypatch, build, n, alone, beside):
+    """A body's bilateral rows are awaited in turn: past 12 a scene alone, past
+    32 scenes beside each other take longer resident (with 49 rows 30 us a pass
+    against 16 as launches)."""
+    monkeypatch.setenv("DVIDE_TUNE", "0")
+    launched, ref, _ = _stepped(star(n), build, 1)
+    stats, vectors, ran = _stepped(star(n), build, 0)
+    assert (ran[0] > 0) == bool(alone) and stats == launched
+    for a, b in zip(ref, vectors):
+        assert bits_equal(a, b)
+    members = [system.from_scene(sc, build, tol=1e-7, max_iterations=150) for sc in (star(n), SCENES["ball"]())]
+    b = system.Batch(build)
+    for g in members:
+        b.add(g)
+    for _ in range(2):
+        b.step()
+    b.close()
+    assert (members[0].residentPasses > 0) == bool(beside)
+    for x, y in zip((members[0].gamma, members[0].v, members[0].p), ref):
+        assert bits_equal(x, y)
+    for g in members:
+        g.close()
 
 
 @pytest.mark.parametrize("build", [FP64, MIXED])
