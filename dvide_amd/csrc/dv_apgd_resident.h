@@ -44,7 +44,11 @@ constexpr int kTeamSync = 16 + kTeamMax;
 // A team whose members are not all running after this long gives up (0: at
 // once): the slot's passes then run as launches.
 constexpr double kFormMs = 2;
-constexpr double kFormMsMany = 100;  // several scenes' teams wait for room
+// Several scenes' teams wait for room: until a team before them has run its
+// 512 passes, 13 ms at most.  (With 100 ms, two batches of two 112,000-sphere
+// scenes on threads of their own, whose teams of 250 can each hold half of the
+// chip, made 187 scene-steps/s in such a run, with 30 229, as launches 201.)
+constexpr double kFormMsMany = 30;
 constexpr double kFormMsMost = 1000;
 constexpr double kTicksPerMs = 1e5;  // of the wall clock
 

@@ -305,7 +305,7 @@ int dv_solve(dv_scene* s);
  * rows, or 1,024 or 1,536) must all be on the chip at once, each filling a
  * CU.  Where other work holds part of the chip (another batch, server or
  * scene on a stream of its own, another process), those that have found a
- * place wait for the rest: up to 100 ms in batches and servers, 2 ms for a
+ * place wait for the rest: up to 30 ms in batches and servers, 2 ms for a
  * scene alone, or what the environment's DVIDE_TEAM_WAIT_MS says (0: not at
  * all; at most 1000).  The solve's passes, and those of the next 16 solves
  * (a server: turns), then run as launches, with the same results. */
