@@ -283,3 +283,38 @@ def test_a_server_whose_teams_cannot_be_placed_runs_as_launches(gpu, monkeypatch
                 assert bits_equal(x, y), n
         for g in members:
             g.close()
+
+
+@pytest.mark.parametrize("build", [FP64, MIXED])
+@pytest.mark.parametrize("name", ["pile_400", "bilateral_box"])
+def test_a_solve_that_changes_between_resident_and_launches(gpu, monkeypatch, name, build):
+    """A scene of one workgroup in a server starts resident, goes on as
+    launches while another scene's team gives up beside it, and ends resident:
+    the bits of its launches alone."""
+    monkeypatch.setenv("DVIDE_TUNE", "0")
+    sc = scenes.pile(33, 400) if name == "pile_400" else scenes.compaction(5, n=150, width=0.6, lid=scenes.LID_BILATERAL)
+
+    def made():
+        return system.from_scene(copy.deepcopy(sc), build, tol=1e-300, max_iterations=3000)
+
+    ref = made()
+    ref.setRowsPerThread(1)
+    ref.step()
+    assert 0 < ref.stats().num_contacts <= 512 - 3
+    g, other = made(), system.from_scene(SCENES["pile_6000"](), build, tol=1e-300, max_iterations=100)
+    monkeypatch.setenv("DVIDE_TEAM_WAIT_MS", "0")
+    srv = system.Server(build, max_slots=2)
+    srv.submit(g)
+    for _ in range(4):
+        srv.poll()
+    srv.submit(other)
+    assert len(srv.drain()) == 2
+    srv.close()
+    st = g.stats()
+    assert (st.iterations, st.passes, st.backtracks, st.residual) == (
+        ref.stats().iterations, ref.stats().passes, ref.stats().backtracks, ref.stats().residual)
+    assert 0 < g.residentPasses < st.passes and other.residentPasses == 0
+    for a, b in zip((g.gamma, g.v, g.p), (ref.gamma, ref.v, ref.p)):
+        assert bits_equal(a, b)
+    for s in (ref, g, other):
+        s.close()
