@@ -65,12 +65,6 @@ __device__ __forceinline__ u64 coLoad(const u64* p) {
 __device__ __forceinline__ void coStore(u64* p, u64 v) {
   __hip_atomic_store(gl(p), v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-__device__ __forceinline__ double coLoad(const double* p) {
-  return __builtin_bit_cast(double, coLoad(reinterpret_cast<const u64*>(p)));
-}
-__device__ __forceinline__ void coStore(double* p, double v) {
-  coStore(reinterpret_cast<u64*>(p), __builtin_bit_cast(u64, v));
-}
 typedef int i32x2 __attribute__((ext_vector_type(2)));
 typedef int i32x4 __attribute__((ext_vector_type(4)));
 template <typename TM>
@@ -240,15 +234,16 @@ __device__ __forceinline__ void waitFor(int* bad, unsigned least, const Missing&
   if (left <= 0) __hip_atomic_store(bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 // N entries of an array, once each carries the tag (kNone: nothing to wait
-// for); awaitRest where they have been loaded once already.
+// for).
 template <typename TM, int N>
 __device__ __forceinline__ void loadEntries(const CoArray<TM>& A, const int (&id)[N], typename CoArray<TM>::Raw (&w)[N]) {
 #pragma unroll
   for (int k = 0; k < N; ++k) w[k] = A.ld(id[k]);
 }
 template <bool kLanes, typename TM, int N>
-__device__ __forceinline__ void awaitRest(const CoArray<TM>& A, const int (&id)[N], unsigned tag, int* bad,
-                                          typename CoArray<TM>::Raw (&w)[N], unsigned least = 0x10000u) {
+__device__ __forceinline__ void await(const CoArray<TM>& A, const int (&id)[N], unsigned tag, int* bad,
+                                      typename CoArray<TM>::Raw (&w)[N], unsigned least = 0x10000u) {
+  loadEntries(A, id, w);
   waitFor<kLanes>(
       bad, least,
       [&] {
@@ -262,12 +257,6 @@ __device__ __forceinline__ void awaitRest(const CoArray<TM>& A, const int (&id)[
   for (int k = 0; k < N; ++k)
 #pragma unroll
     for (int h = 0; h < CoArray<TM>::kHalves; ++h) pinned(w[k].h[h]);
-}
-template <bool kLanes, typename TM, int N>
-__device__ __forceinline__ void await(const CoArray<TM>& A, const int (&id)[N], unsigned tag, int* bad,
-                                      typename CoArray<TM>::Raw (&w)[N], unsigned least = 0x10000u) {
-  loadEntries(A, id, w);
-  awaitRest<kLanes>(A, id, tag, bad, w, least);
 }
 
 // Waits until this wavefront's stores have reached device scope (vmcnt 0;
