@@ -99,7 +99,7 @@ def run_gpu(scene, solver, steps, warmup, profile_kernel=0, max_iterations=None)
         g.setProfileKernel(profile_kernel)
         hip.hipDeviceSynchronize()
         lat, its, res, nc, passes, solve, kms, kcnt, kstep = [], [], [], [], [], [], 0.0, 0, []
-        any_tuning = False
+        any_tuning, resident, team_rows = False, 0, 0
         t0 = time.perf_counter()
         for _ in range(steps):
             ts = time.perf_counter()
@@ -115,6 +115,8 @@ def run_gpu(scene, solver, steps, warmup, profile_kernel=0, max_iterations=None)
             kcnt += st.prof_kernel_count
             kstep.append(round(1e3 * st.prof_kernel_ms / st.prof_kernel_count, 3) if st.prof_kernel_count else None)
             any_tuning = any_tuning or bool(st.schedule_tuning)
+            resident += g.residentPasses
+            team_rows = max(team_rows, g.teamRows)
         hip.hipDeviceSynchronize()
         elapsed = time.perf_counter() - t0
         last = g.stats()
@@ -126,7 +128,9 @@ def run_gpu(scene, solver, steps, warmup, profile_kernel=0, max_iterations=None)
                         update=last.ms_update),
             nb=g.numBodies, v=g.v, p=g.p,
             schedule=dict(rows_per_thread=last.rows_per_thread, xcd_order=last.xcd_order,
-                          measured_in_timed_steps=int(any_tuning)),
+                          measured_in_timed_steps=int(any_tuning),
+                          # passes in one kernel of a team of workgroups, and their rows per thread
+                          resident_pass_share=round(resident / max(sum(passes), 1), 4), team_rows=team_rows),
         )
     finally:
         g.close()
@@ -738,7 +742,9 @@ def main():
         "schedule": mixed["schedule"],
         "roofline": {
             "bound": "hbm",
-            "kernel": "kP1<float> (contact pass: previous decision, momentum, projection, F^T gamma)",
+            # timed on a chunk of each solve that runs as launches; the other passes run resident
+            # (schedule.resident_pass_share, us_per_pass)
+            "kernel": "kP1<float> (contact pass as a launch: previous decision, momentum, projection, F^T gamma)",
             "achieved": round(achieved, 1),
             "peak": HBM_PEAK_GBS,
             "unit": "GB/s",
@@ -767,6 +773,12 @@ def main():
             "achieved_gbs": round(b_pass / (t_pass * 1e-6) / 1e9, 1),
             "frac": round(b_pass / (t_pass * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),
         }
+    def us_per_pass(r):  # (the plain build counts no passes)
+        n = int(np.sum(r["passes"]))
+        return round(1e3 * float(np.sum(r["solve_ms"])) / n, 2) if n else None
+
+    line["us_per_pass"] = us_per_pass(mixed)
+
     def us_per_iteration(r):
         return round(1e3 * float(np.sum(r["solve_ms"])) / max(int(np.sum(r["iterations"])), 1), 2)
 
@@ -781,6 +793,7 @@ def main():
             "residual_max": float(np.max(r["residual"])),
             "steps_converged": int(np.sum(r["residual"] < TOL)),
             "us_per_iteration": us_per_iteration(r),
+            "us_per_pass": us_per_pass(r),
             "schedule": r["schedule"],
         }
     # ratios over the same steps from the same state: the plain path runs the

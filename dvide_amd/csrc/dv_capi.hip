@@ -196,13 +196,15 @@ class Lease {
   bool waited = false;
 };
 
-// Vectors of up to 2 MB travel between the caller's memory and the device
+// Vectors of up to 1.5 MB travel between the caller's memory and the device
 // through pinned memory that a kernel reads or writes: with the runtime's own
 // copies from and to pageable memory a call took 17 us in and 23 out for 48
 // bytes, now 14 and 14; 31 and 34 for 24 to 190 KB, now 17 and 17.  Past 1 MB
 // the runtime pins the caller's pages, which it does quickly or not as they
-// lie: 1.1 MB took 54 to 400 us in and 74 to 630 out, and so 52 and 72.
-constexpr size_t kStagingMost = 1 << 18;  // doubles
+// lie: 1.1 MB took 54 to 400 us in and 74 to 630 out, and so 52 and 72.  Reading
+// a vector again and again takes the same either way at 1.4 MB, and at 2 MB 127
+// us with the runtime's copies and 144 so.
+constexpr size_t kStagingMost = 3 << 16;  // doubles
 __global__ void kMove(double* dst, const double* src, long n) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = src[i];
