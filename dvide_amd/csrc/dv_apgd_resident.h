@@ -435,7 +435,9 @@ __device__ __forceinline__ PassView uniformView(const PassView& s) {
 // leaves the registers.
 // Two wavefronts per SIMD (up to 256 VGPRs, one workgroup to a CU): held to
 // 128, so that a CU takes two, the mixed kernel spilled 20 and took 26.3 us
-// per pass on 256,000 contacts, where two rows per thread take 10.7.
+// per pass on 256,000 contacts, where two rows per thread take 10.7.  So, two
+// rows mixed spill 4 VGPRs (15 with bilateral rows), three 26 (39), one in FP64
+// 5 (8), the others none.
 // Two rows in FP64 have room for the second step with gamma_{k-1} and its
 // N gamma in LDS and five contacts of a body in flight: 17.4 us without the
 // step, 14.6 with it.  (Mixed they stay in registers: 9.4 us, in LDS 9.6.)

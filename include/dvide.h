@@ -85,9 +85,10 @@ typedef struct dv_scene dv_scene;
                                  last pass for one scene); the rest run as without
                                  profiling */
 #define DV_PARAM_ROWS_PER_THREAD 15 /* contact kernels of the graph-driven solvers: 0 the
-                                       tuned choice (default), 1 or 2 contacts per thread
-                                       (results agree to rounding, each choice is
-                                       deterministic) */
+                                       tuned choice (default), 1 or 2 contacts per thread,
+                                       which also keeps the passes of the scene, or of a
+                                       batch whose first scene it is, as launches (the
+                                       results are the same bits) */
 #define DV_PARAM_ANTI_RELAX 16 /* 0/1                  APGD::setAntiRelaxation, APGD.cuh:63
                                   (APGD.cu:104-114, 335-345); runs on DV_APGD_PLAIN, and a
                                   DV_APGD_FP64 scene with it on is solved by that build */
@@ -124,7 +125,8 @@ typedef struct dv_stats {
   int prof_kernel_count;  /* ... and their number */
   int passes;             /* solver passes (Schur products) of the step */
   /* launch schedule of the graph-driven builds' last chunk of passes (none
-     changes a result): contact rows per thread, XCD-contiguous tile order,
+     changes a result; resident passes, DV_PARAM_RESIDENT_PASSES, use none of
+     it): contact rows per thread, XCD-contiguous tile order,
      and, for several slots, workgroups per CU of the contact and body
      kernels; schedule_tuning is 1 when the solve measured candidate
      schedules (see DVIDE_SCHEDULE_FILE in dvide_amd/csrc/dv_apgd_fused.hip) */
