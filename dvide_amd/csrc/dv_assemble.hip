@@ -307,6 +307,8 @@ void schurExact(Scene& s, const double* x, double* y) {
   if (items)
     hipLaunchKernelGGL(kRowsD, dim3(blocksFor(items, kT)), dim3(kT), 0, s.stream, rowArgs(s), (const double*)s.tmp.p,
                        (const double*)nullptr, y);
+  else  // (the vectors keep the last step's length, whose rows are gone)
+    fillDevice(s, y, s.R, 0.0);
 }
 
 void rowsD(Scene& s, const double* x, const double* badd, double* y) {

@@ -63,3 +63,24 @@ def test_threads_borrow_blocks_of_their_own(gpu):
     assert not wrong
     for g in systems:
         g.close()
+
+
+def test_product_without_rows_is_zero(gpu):
+    """A scene whose contacts have gone keeps r's length; no row writes the
+    product, which must not be what the vectors' memory held before."""
+    other = system.from_scene(scenes.pile(31, 900), system.BUILD_FP64)
+    other.assemble()
+    g = system.from_scene(scenes.ball_on_box(), system.BUILD_FP64)
+    g.step()
+    n = g.vector(system.VEC_R).size
+    assert n == 3
+    p = g.p
+    p[1::3][np.asarray(g.fixed()) == 0] += 10.0
+    g.set_vector(system.VEC_P, p)
+    assert g.assemble() == 0
+    for product in (g.schur_product, g.schur_product_noalloc):
+        other_product = other.schur_product if product == g.schur_product else other.schur_product_noalloc
+        assert np.abs(other_product(np.ones(other.vector(system.VEC_R).size))).max() > 0
+        assert np.array_equal(product(np.ones(n)), np.zeros(n))
+    other.close()
+    g.close()
